@@ -5,8 +5,7 @@
 // states).  Same kernels, same arguments, same bits; what it saves is the host: one foreign call and one allocation per
 // forward instead of four calls and nine allocations, which is what bounds small shapes (B1 T2048 H8: the kernels take
 // 30 us, issuing them from Python 50).
-#include "zoo_common.h"
-#include "../../include/linquant_hip.h"
+#include "zoo_params.h"
 
 namespace {
 
@@ -96,11 +95,13 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // ---- the other cells: chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry each way round: the stage entry points in
 // the order the Python wrappers issue them, over one workspace.  64-token chunks take the fused pre-passes (the cumsum / WY
-// launch also makes the write codes), 128-token chunks the separate write-codes launch.
+// launch also makes the write codes), 128-token chunks the separate write-codes launch.  Under per-channel decay 64-token
+// chunks run the recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).
 namespace {
 
 struct FLayout {
-  int64_t gc, logenv, kqT, vqT, wq, ev, gam, pack, A, Ax, qg, Hw, W, U, fw, e_out, h_i8, cross, total;
+  int64_t gc, logenv, kqT, vqT, vcT, wq, ev, gam, pack, A, Ax, qg, Hw, W, U, fw, e_out, h_i8, cross, total;
+  bool scan;  // recurrence and output in one launch
 };
 
 int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
@@ -125,12 +126,14 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->A, diag ? B * T * H * 64 * 2 : 0);
   take(l->Ax, diag && big ? B * T * H * 64 * 2 : 0);
   take(l->qg, diag ? B * T * H * K : 0);
+  l->scan = diag && !big;
+  take(l->vcT, l->scan && !delta ? B * NT * H * V * 64 : 0);
   take(l->Hw, delta ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
   take(l->U, delta ? B * T * H * V * 2 : 0);
   take(l->fw, delta ? B * T * H * 4 : 0);
-  take(l->e_out, delta ? B * T * H * V * 2 : 0);
-  take(l->h_i8, B * (T / cs) * H * V * K);
+  take(l->e_out, delta && !l->scan ? B * T * H * V * 2 : 0);
+  take(l->h_i8, l->scan ? 0 : B * (T / cs) * H * V * K);
   take(l->cross, big ? B * T * H * V * 4 : 0);
   l->total = off;
   return LQ_OK;
@@ -179,6 +182,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   void* A = diag ? ws + l.A : nullptr;
   void* Ax = diag && big ? ws + l.Ax : nullptr;
   int8_t* qg = diag ? (int8_t*)(ws + l.qg) : nullptr;
+  int8_t* vcT = l.scan && !delta ? (int8_t*)(ws + l.vcT) : nullptr;
   float* cross = big ? (float*)(ws + l.cross) : nullptr;
 
   // (every stage validates its own arguments before it launches: see lq_zoo_simple_gla)
@@ -190,7 +194,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
       c.k = a->k, c.v = a->v, c.kqT = kqT, c.vqT = vqT, c.ev = ev, c.gam = gam, c.skw = a->skw, c.svw = a->svw;
       c.eta = a->eta, c.qmax = a->qmax, c.vdim = a->vdim, c.act_dtype = a->act_dtype;
     }
-    if ((rc = lq_zoo_cumsum(&c, stream)) != LQ_OK) return rc;
+    if ((rc = zoo_cumsum_launch(&c, vcT, a->svl, stream)) != LQ_OK) return rc;
   }
   if (delta) {
     lq_zoo_wy_prep_args w = {};
@@ -201,7 +205,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
       w.kqT = kqT, w.wq = wq, w.ev = ev, w.gam = gam, w.logenv = logenv, w.skw = a->skw, w.sw = a->sw, w.eta = a->eta, w.qmax = a->qmax;
       w.dk_div = a->dq, w.dk_rcp = a->dq_rcp, w.pack = pack;
     }
-    if ((rc = lq_zoo_wy_prep(&w, stream)) != LQ_OK) return rc;
+    if ((rc = zoo_wy_prep_launch(&w, l.scan, stream)) != LQ_OK) return rc;
   }
   if (big) {
     lq_zoo_write_codes_args w = {};
@@ -216,7 +220,15 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     g.q = a->q, g.k = delta ? Hw : a->k, g.g = gc, g.A = A, g.qg = qg, g.rot = a->rot, g.sq = a->sq, g.sk = a->sk, g.scale = a->scale;
     g.qmax = a->qmax, g.batch = a->batch, g.seqlen = a->seqlen, g.nheads = a->nheads, g.kdim = a->kdim, g.chunk_size = a->chunk_size;
     g.act_dtype = a->act_dtype, g.dq = a->dq, g.A_cross = Ax;
-    if ((rc = lq_zoo_gla_A(&g, stream)) != LQ_OK) return rc;
+    if ((rc = zoo_gla_A_launch(&g, l.scan, stream)) != LQ_OK) return rc;
+  }
+  if (l.scan) {
+    ZooScanParams s = {};
+    s.kqT = kqT, s.vqT = vqT, s.vcT = vcT, s.wq = wq, s.u = (const _Float16*)U, s.pack = pack, s.gam = gam;
+    s.qc = qg, s.A = (const _Float16*)A, s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
+    s.skw = a->skw, s.svw = a->svw, s.sw = a->sw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
+    s.qmax = a->qmax, s.bf = a->act_dtype == LQ_DT_BF16, s.T = a->seqlen, s.H = a->nheads, s.V = a->vdim, s.NT = a->seqlen / 64;
+    return zoo_scan_launch(s, delta, false, a->kdim, a->batch, stream);
   }
   {
     lq_zoo_state_args s = {};

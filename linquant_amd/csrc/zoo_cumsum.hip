@@ -5,7 +5,7 @@
 //   logenv[b, t, h] = max_k (gc_last[k] - gc[t, k])                     (diagonal decay only)
 // One thread walks one (batch, chunk, head[, channel]) column; threads of a workgroup cover adjacent
 // channels, so every step is a coalesced row access.
-#include "zoo_common.h"
+#include "zoo_params.h"
 #include "../../include/linquant_hip.h"
 
 namespace {
@@ -49,16 +49,19 @@ __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* _
 // Write operands of the linear family's state kernel under per-channel decay, made by the cumsum launch from the decay
 // tile it holds (what lq_zoo_write_codes would make from the stored gc and logenv; same arithmetic, same bits):
 //   kqT[k][t] = q8(key[t][k] * exp(gk_last - gk_t - eta*le_t), 1/skw[k]),  vqT[v][t] = q8(val[t][v] * exp(eta*le_t), 1/svw[v]),
-//   ev[t] = exp(eta*le_t),  gam[k] = exp(gk_last).
+//   ev[t] = exp(eta*le_t),  gam[k] = exp(gk_last),
+// and, when vcT is set, the local value codes q8(val[t][v], 1/svl[v]) that the output wants (zoo_op_values).
 struct CumsumCodes {
   const uint16_t* k;
   const uint16_t* v;
   int8_t* kqT;
   int8_t* vqT;
+  int8_t* vcT;
   float* ev;
   float* gam;
   const float* skw;
   const float* svw;
+  const float* svl;
   float eta;
   int qmax;
   int V;
@@ -190,13 +193,23 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
 #pragma unroll
       for (int d = 0; d < 4; ++d) o[d] = (int)zoo_pack_codes(code[4 * d], code[4 * d + 1], code[4 * d + 2], code[4 * d + 3]);
       *(lq_v4i*)(cc.vqT + (cb * V + c) * 64 + 16 * q) = o;
+      if (cc.vcT) {
+        const float inv_svl = 1.0f / cc.svl[h * V + c];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf), inv_svl, cc.qmax);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) o[d] = (int)zoo_pack_codes(code[4 * d], code[4 * d + 1], code[4 * d + 2], code[4 * d + 3]);
+        int8_t* dst = cc.vcT + cb * V * 64 + zoo_op_values(c, 16 * q);
+        *(lq_v2i*)dst = lq_v2i{o[0], o[1]};
+        *(lq_v2i*)(dst + 256) = lq_v2i{o[2], o[3]};  // the next group of eight tokens
+      }
     }
   }
 }
 
 }  // namespace
 
-extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) {
+int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl, hipStream_t stream) {
   if (!a || !a->g || !a->gc) return LQ_ERR_NULL;
   if (a->batch <= 0 || a->seqlen <= 0 || a->nheads <= 0 || a->chunk_size <= 0 || a->kdim < 0) return LQ_ERR_SHAPE;
   if (a->seqlen % a->chunk_size != 0) return LQ_ERR_SHAPE;
@@ -236,6 +249,7 @@ extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) {
       if (!zoo_al(a->kqT, 16) || !zoo_al(a->vqT, 16)) return LQ_ERR_SHAPE;
       cc.k = (const uint16_t*)a->k, cc.v = (const uint16_t*)a->v, cc.kqT = a->kqT, cc.vqT = a->vqT, cc.ev = a->ev, cc.gam = a->gam;
       cc.skw = a->skw, cc.svw = a->svw, cc.eta = a->eta, cc.qmax = a->qmax, cc.V = a->vdim, cc.bf = a->act_dtype == LQ_DT_BF16;
+      cc.vcT = vcT, cc.svl = svl;
       hipLaunchKernelGGL(cumsum_diag_kernel<true>, grid, block, lds, stream, a->g, a->gc, a->logenv, a->seqlen, a->nheads,
                          a->kdim, a->chunk_size, cc);
     } else if (big) {
@@ -248,3 +262,5 @@ extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) {
   }
   return lq_check_launch();
 }
+
+extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) { return zoo_cumsum_launch(a, nullptr, nullptr, stream); }

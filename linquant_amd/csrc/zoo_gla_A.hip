@@ -51,9 +51,9 @@ LQ_DEV float wave_max(float m) {
 
 // Diagonal block, every (i, j, n) weight evaluated on its own and masked before use (any decay spread):
 // lane (i = rl, j = 4kg + jj), 8 channels per step.
-template <int K, bool BF>
+template <int K, bool BF, bool SCAN>
 LQ_DEV void diag_exact(const AParams& p, float sq, float sk, float inv_sq, float inv_sk, int rl, int kg, int64_t row0, int h,
-                       int i0) {
+                       int i0, int64_t cb) {
   const int H = p.H, qmax = p.qmax;
   constexpr bool bf = BF;
   float s[4] = {0.f, 0.f, 0.f, 0.f};
@@ -90,14 +90,15 @@ LQ_DEV void diag_exact(const AParams& p, float sq, float sk, float inv_sq, float
     lq_v2i oh;
     oh[0] = (int)zoo_pack_h2(o[0], o[1]);
     oh[1] = (int)zoo_pack_h2(o[2], o[3]);
-    *(lq_v2i*)(p.A + ((row0 + rl) * H + h) * 64 + i0 + 4 * kg) = oh;
+    *(lq_v2i*)(SCAN ? p.A + cb * 4096 + zoo_op_A(i0 + rl, i0 + 4 * kg) : p.A + ((row0 + rl) * H + h) * 64 + i0 + 4 * kg) = oh;
   }
 }
 
 // QG: the state-read codes are wanted (p.qg is set); a compile-time flag keeps the own-rows loop
 // one basic block.
+// SCAN: A and the state-read codes leave in operand order (zoo_params.h), for zoo_scan.hip.
 // DQ: q is rescaled per (head, channel) as it is loaded (a compile-time flag: the kernel sits at its register limit).
-template <int K, bool ROT, bool BF, bool QG, bool DQ>
+template <int K, bool ROT, bool BF, bool QG, bool DQ, bool SCAN>
 __global__ __launch_bounds__(256, 3) void zoo_gla_A_kernel(AParams p) {
   constexpr int RS = K + 8;  // halves per row of the transposed rotation
   __shared__ __align__(16) _Float16 RT[ROT ? K * RS : 8];  // RT[m][n] = R[n][m]
@@ -159,6 +160,11 @@ __global__ __launch_bounds__(256, 3) void zoo_gla_A_kernel(AParams p) {
   const int rl = lane_o & 15, kg = lane_o >> 4;
   const int i0 = 16 * blk;
   const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
+  const int64_t cb = ((int64_t)b * nchunks + ct) * H + h;
+  // element (row, col) of this chunk's A
+  auto a_at = [&](int row, int col) {
+    return SCAN ? p.A + cb * 4096 + zoo_op_A(row, col) : p.A + ((t0 + row) * H + h) * 64 + col;
+  };
 
   {
     // ---- The wave loads its own sub-block (q, k, g rows) once, in the layout of the rotation
@@ -250,7 +256,7 @@ __global__ __launch_bounds__(256, 3) void zoo_gla_A_kernel(AParams p) {
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        p.A[((t0 + 16 * I + 4 * kg + r) * H + h) * 64 + i0 + rl] = (_Float16)((float)acc[r] * sqk);
+        *a_at(16 * I + 4 * kg + r, i0 + rl) = (_Float16)((float)acc[r] * sqk);
     };
 
     // own rows, fetched once: state-read codes, diagonal block (factorized around the first row while the spread is
@@ -298,7 +304,8 @@ __global__ __launch_bounds__(256, 3) void zoo_gla_A_kernel(AParams p) {
         lq_v2i o;
         o[0] = (int)zoo_pack_codes(cs[0], cs[1], cs[2], cs[3]);
         o[1] = (int)zoo_pack_codes(cs[4], cs[5], cs[6], cs[7]);
-        *(lq_v2i*)(p.qg + roff + 32 * ks) = o;
+        // (operand order: 32 channels further is 512 bytes further)
+        *(lq_v2i*)(SCAN ? p.qg + cb * 64 * K + zoo_op_codes(i0 + rl, 8 * kg, K) + 512 * ks : p.qg + roff + 32 * ks) = o;
       }
       if constexpr (!ROT) {
         cq[2 * ks] = zoo_pack_codes(iq[0], iq[1], iq[2], iq[3]), cq[2 * ks + 1] = zoo_pack_codes(iq[4], iq[5], iq[6], iq[7]);
@@ -356,26 +363,27 @@ __global__ __launch_bounds__(256, 3) void zoo_gla_A_kernel(AParams p) {
       // lane holds column j = rl, rows i = 4kg + r
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        p.A[((t0 + i0 + 4 * kg + r) * H + h) * 64 + i0 + rl] = (_Float16)((rl <= 4 * kg + r) ? dacc[r] : 0.0f);
+        *a_at(i0 + 4 * kg + r, i0 + rl) = (_Float16)((rl <= 4 * kg + r) ? dacc[r] : 0.0f);
     } else {
-      diag_exact<K, BF>(p, sq, sk, inv_sq, inv_sk, rl, kg, t0 + i0, h, i0);  // (applies p.dq itself)
+      diag_exact<K, BF, SCAN>(p, sq, sk, inv_sq, inv_sk, rl, kg, t0 + i0, h, i0, cb);  // (applies p.dq itself)
     }
   }
   // zero blocks above the diagonal
   for (int J = blk + 1; J < 4; ++J)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) p.A[((t0 + i0 + 4 * kg + r) * H + h) * 64 + 16 * J + rl] = (_Float16)0.0f;
+    for (int r = 0; r < 4; ++r) *a_at(i0 + 4 * kg + r, 16 * J + rl) = (_Float16)0.0f;
   }  // pass
 }
 
 }  // namespace
 
-extern "C" int lq_zoo_gla_A(const lq_zoo_gla_A_args* a, hipStream_t stream) {
+int zoo_gla_A_launch(const lq_zoo_gla_A_args* a, bool scan, hipStream_t stream) {
   if (!a || !a->q || !a->k || !a->g || !a->A || !a->sq || !a->sk) return LQ_ERR_NULL;
   if (a->batch <= 0 || a->seqlen <= 0 || a->nheads <= 0) return LQ_ERR_SHAPE;
   // 128-token chunks: the blocks inside either half are those of 64-token chunks (g cumulated over the 128 tokens), the
   // blocks between the halves come from a second launch into A_cross
   const bool pair = a->chunk_size == 128;
+  if (scan && (pair || !a->qg)) return LQ_ERR_SHAPE;
   if (pair && !a->A_cross) return LQ_ERR_NULL;
   if (pair && !zoo_al(a->A_cross, 16)) return LQ_ERR_SHAPE;
   if ((a->chunk_size != 64 && !pair) || a->seqlen % a->chunk_size != 0) return LQ_ERR_SHAPE;
@@ -394,30 +402,34 @@ extern "C" int lq_zoo_gla_A(const lq_zoo_gla_A_args* a, hipStream_t stream) {
   p.B = a->batch, p.T = a->seqlen, p.H = a->nheads;
   if ((int64_t)((a->seqlen / 64 + 1) / 2) * a->batch * a->nheads > 0x7fffffff) return LQ_ERR_SHAPE;
   dim3 grid((uint32_t)(((a->seqlen / 64 + 1) / 2) * a->batch * a->nheads));
-#define LQ_A_LAUNCH3(KV, ROTV, BFV, QGV)                                                                   \
-  do {                                                                                                     \
-    if (p.dq)                                                                                              \
-      hipLaunchKernelGGL((zoo_gla_A_kernel<KV, ROTV, BFV, QGV, true>), grid, dim3(256), 0, stream, p);     \
-    else                                                                                                   \
-      hipLaunchKernelGGL((zoo_gla_A_kernel<KV, ROTV, BFV, QGV, false>), grid, dim3(256), 0, stream, p);    \
+#define LQ_A_LAUNCH3(KV, ROTV, BFV, QGV, SCANV)                                                                \
+  do {                                                                                                         \
+    if (p.dq)                                                                                                  \
+      hipLaunchKernelGGL((zoo_gla_A_kernel<KV, ROTV, BFV, QGV, true, SCANV>), grid, dim3(256), 0, stream, p);  \
+    else                                                                                                       \
+      hipLaunchKernelGGL((zoo_gla_A_kernel<KV, ROTV, BFV, QGV, false, SCANV>), grid, dim3(256), 0, stream, p); \
   } while (0)
-#define LQ_A_LAUNCH2(KV, ROTV, QGV)                                                                        \
-  do {                                                                                                     \
-    if (p.bf)                                                                                              \
-      LQ_A_LAUNCH3(KV, ROTV, true, QGV);                                                                   \
-    else                                                                                                   \
-      LQ_A_LAUNCH3(KV, ROTV, false, QGV);                                                                  \
+#define LQ_A_LAUNCH2(KV, ROTV, QGV, SCANV)       \
+  do {                                           \
+    if (p.bf)                                    \
+      LQ_A_LAUNCH3(KV, ROTV, true, QGV, SCANV);  \
+    else                                         \
+      LQ_A_LAUNCH3(KV, ROTV, false, QGV, SCANV); \
   } while (0)
-#define LQ_A_LAUNCH(KV)                 \
-  do {                                  \
-    if (a->rot && p.qg)                 \
-      LQ_A_LAUNCH2(KV, true, true);     \
-    else if (a->rot)                    \
-      LQ_A_LAUNCH2(KV, true, false);    \
-    else if (p.qg)                      \
-      LQ_A_LAUNCH2(KV, false, true);    \
-    else                                \
-      LQ_A_LAUNCH2(KV, false, false);   \
+#define LQ_A_LAUNCH(KV)                       \
+  do {                                        \
+    if (a->rot && scan)                       \
+      LQ_A_LAUNCH2(KV, true, true, true);     \
+    else if (scan)                            \
+      LQ_A_LAUNCH2(KV, false, true, true);    \
+    else if (a->rot && p.qg)                  \
+      LQ_A_LAUNCH2(KV, true, true, false);    \
+    else if (a->rot)                          \
+      LQ_A_LAUNCH2(KV, true, false, false);   \
+    else if (p.qg)                            \
+      LQ_A_LAUNCH2(KV, false, true, false);   \
+    else                                      \
+      LQ_A_LAUNCH2(KV, false, false, false);  \
   } while (0)
   if (a->kdim == 128)
     LQ_A_LAUNCH(128);
@@ -436,3 +448,5 @@ extern "C" int lq_zoo_gla_A(const lq_zoo_gla_A_args* a, hipStream_t stream) {
   }
   return lq_check_launch();
 }
+
+extern "C" int lq_zoo_gla_A(const lq_zoo_gla_A_args* a, hipStream_t stream) { return zoo_gla_A_launch(a, false, stream); }

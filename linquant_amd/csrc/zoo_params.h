@@ -3,6 +3,7 @@
 #pragma once
 
 #include "zoo_common.h"
+#include "../../include/linquant_hip.h"
 
 struct ZooStateParams {
   const int8_t* kqT;
@@ -75,3 +76,58 @@ int zoo_gla_A_cross_launch(const ZooACrossParams& p, int K, hipStream_t stream);
 // canonical storage: one workgroup spans all V value channels (V = 64 or 128); defined in zoo_unrot.hip
 int zoo_state_unrot_launch(const ZooStateParams& p, bool delta, int K, int batch, bool pair, hipStream_t stream);
 int zoo_output_unrot_launch(const ZooOutParams& p, int decay, int K, hipStream_t stream);
+
+// ---- Operand order: the layouts in which the pre-pass kernels leave the operands of zoo_scan.hip.  Tiles of one (batch, chunk,
+// head) are contiguous, and inside a tile the 16 bytes that lane l of a wave wants as its MFMA operand (row l & 15, contraction
+// group l >> 4) lie at 16 l: a wave's request is 1 KB of whole cache lines.  From token-major rows (16 rows of 64 bytes, H * K
+// bytes apart) the same requests kept the vector memory pipeline of a compute unit busy for 1055 of a step's 2790 cycles, in this
+// order for 640 of 2100 (linear family, K = V = 128).
+// INT8 codes of 64 tokens x K channels: element (token, ch)
+LQ_DEV int zoo_op_codes(int token, int ch, int K) {
+  return ((token >> 4) * (K >> 6) + (ch >> 6)) * 1024 + ((ch >> 4) & 3) * 256 + (token & 15) * 16 + (ch & 15);
+}
+// fp16 A of 64 x 64: element (row, col), in halves
+LQ_DEV int zoo_op_A(int row, int col) {
+  return ((row >> 4) * 2 + (col >> 5)) * 512 + ((col >> 3) & 3) * 128 + (row & 15) * 8 + (col & 7);
+}
+// INT8 local value codes of V channels x 64 tokens: element (channel, token)
+LQ_DEV int zoo_op_values(int ch, int token) {
+  return (ch >> 5) * 2048 + (ch & 1) * 1024 + ((token >> 3) & 3) * 256 + ((ch >> 1) & 15) * 16 + (token >> 5) * 8 + (token & 7);
+}
+// 16-bit U of 64 tokens x V channels, in elements: element (token, channel)
+LQ_DEV int zoo_op_U(int token, int ch) { return (ch >> 5) * 2048 + token * 32 + (ch & 31); }
+
+// recurrence and output in one launch (rotated storage, 64-token chunks); defined in zoo_scan.hip
+struct ZooScanParams {
+  const int8_t* kqT;    // key write codes (B,NT,H,K,64)
+  const int8_t* vqT;    // linear: value write codes (B,NT,H,V,64)
+  const int8_t* vcT;    // linear: local value codes (B,NT,H, zoo_op_values)
+  const int8_t* wq;     // delta: state-read codes of W (B,NT,H, zoo_op_codes)
+  const _Float16* u;    // delta: (B,NT,H, zoo_op_U)
+  const float* pack;    // delta: fw[64] | ev[64] | gam[K] per (batch, chunk, head)
+  const float* gam;     // linear: (B,NT,H,K)
+  const int8_t* qc;     // codes of q that read the state (B,NT,H, zoo_op_codes)
+  const _Float16* A;    // intra-chunk product (B,NT,H, zoo_op_A), zeros above the diagonal
+  const float* gpk;     // scalar decay: cumulative log decay (B,NT,H,64)
+  void* o;
+  int o_is_f32;
+  float* ht;
+  const float* skw;
+  const float* svw;
+  const float* sw;
+  const float* ss;
+  const float* sq;
+  const float* svl;
+  int qmax;
+  int bf;
+  int T, H, V, NT;
+};
+int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, int batch, hipStream_t stream);
+
+// The pre-pass entry points with what zoo_scan.hip wants on top of their public arguments.
+// cumsum (GLA): also the local value codes (zoo_op_values)
+int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl, hipStream_t stream);
+// A kernel: A and qg in operand order (scan = true)
+int zoo_gla_A_launch(const lq_zoo_gla_A_args* a, bool scan, hipStream_t stream);
+// WY prep with the write codes: wq and U in operand order (scan = true)
+int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stream);

@@ -1,0 +1,443 @@
+// The chunk recurrence and the output of a zoo cell in one launch (rotated storage, 64-token chunks): what zoo_state.hip and
+// zoo_output.hip do one after the other, without the stored states and the pseudo-values E ever reaching memory.
+// Covers the state bodies linquant/kernels/zoo/simple_gla.py:23-75, gla.py:102-148, gated_delta_rule.py:50-115, kda.py:68-130
+// and the output bodies simple_gla.py:98-153, gla.py:170-213, with the arithmetic of the two kernels named above in their
+// order, so the outputs are theirs bit for bit.
+//
+// What bounds it: the chain of chunk steps (64 at T = 4096).  One 8-wave workgroup per (BV-column V tile, batch*head); per
+// step
+//   waves 0..3 (chain) quantize the fp32 carry they hold in registers (wave w owns K/4 rows) into LDS, read the state for
+//     the delta family, form E and its write codes, and apply the INT8 write product to the carry;
+//   waves 4..7 (output; wave 4 + w owns token rows 16w .. 16w + 15) read the same stored copy from LDS with the codes of q,
+//     and add the intra-chunk product of A with the local codes of v (linear family) or E (delta family).
+// Every SIMD holds one wave of each kind, so the output's instructions fill the issue slots that the chain leaves while it
+// waits for its rendezvous.  The output's operands do not depend on the carry; it has no rendezvous of its own: the chain's
+// (one per step for the linear family, two for the delta family) hand it the stored copy and E.  The delta family's output
+// runs half a step behind: E of a chunk becomes local codes between the chain's second and the next first rendezvous, and the
+// chunk's local product and store follow after that one.
+//
+// Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 64 us, KDA B2 T8192 H32 157 +
+// 128 -> 135 us, KDA B1 T2048 H8 41 + 7 -> 36 us.  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
+// carry, 300 to issue its requests, 1000 for state read and E, 300 for the update; one workgroup of 32 columns per compute unit
+// at the first two shapes.
+//
+// Nothing inside an output step branches (A holds zeros above the diagonal and both 32-token slabs are always multiplied, the
+// output type is a template parameter, the first step is peeled off): memory operations retire in issue order and the compiler
+// derives each wait from a count of those issued since, merged over all paths, so a branch around a store or a product made
+// every step wait for the operands it had just requested (seen in its assembly: vmcnt(2) .. vmcnt(4)
+// where vmcnt(27) is meant).
+#include <type_traits>
+
+#include "zoo_params.h"
+
+namespace {
+
+using ScanParams = ZooScanParams;
+
+constexpr int BV = 32;  // value columns per workgroup
+
+template <bool DELTA, int K>
+struct ChainOps {
+  lq_v4i kop[K / 64];                 // key write codes: rows of this wave, 16 token slots of the lane's group
+  lq_v4i vop[DELTA ? 1 : BV / 16];    // linear: value write codes
+  lq_v4i wop[DELTA ? K / 64 : 1];     // delta: state-read codes of token 16*wave + (lane & 15)
+  lq_v4i uraw;                        // delta: U of token 16*wave + (lane >> 2), columns 8 * (lane & 3) .. + 7
+  float misc;                         // lanes 0..15 fw, 16..31 ev of the wave's tokens (delta), 32.. decay of the carry rows
+};
+
+template <bool DELTA, bool SCALAR, int K>
+struct OutOps {
+  lq_v4i qop[K / 64];                     // codes of q: token 16*w + (lane & 15)
+  lq_v4i aop[2];                          // A (fp16): the same token, columns 32 js + 8 kg ..
+  lq_v4i vop[DELTA ? 1 : BV / 16];        // linear: local value codes of column NJ rl + jj, tokens 8 kg .. and 32 + 8 kg ..
+  lq_v4f g;                               // scalar decay: cumulative log decay of tokens 16*w + 4 kg ..
+};
+
+template <int I, int N, typename F>
+LQ_DEV void scan_for_from(const F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    scan_for_from<I + 1, N>(f);
+  }
+}
+template <int N, typename F>
+LQ_DEV void scan_for(const F& f) {
+  scan_for_from<0, N>(f);
+}
+
+// eight int8 codes -> eight exact fp16 values
+LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
+  uint32_t w[4];
+  zoo_i8x4_to_f16x4((uint32_t)c[0], w[0], w[1]);
+  zoo_i8x4_to_f16x4((uint32_t)c[1], w[2], w[3]);
+  return __builtin_bit_cast(lq_v8h, lq_v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]});
+}
+
+// Operand sets in rotation: a set is requested D - 1 steps ahead of its use, and the loop is unrolled by D so that the sets
+// keep their registers.  Its body has no exit in it (what does not fill D steps follows behind): an exit inside merged, in the
+// compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
+constexpr int scan_sets(bool delta) { return delta ? 3 : 5; }
+
+template <bool DELTA, bool SCALAR, int K, bool BF, bool OF32>
+__global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
+  constexpr int D = scan_sets(DELTA);
+  constexpr int KR = K / 4;        // carry rows per chain wave
+  constexpr int KT = K / 64;       // 16-row tiles per chain wave
+  constexpr int VT = BV / 16;      // 16-column tiles
+  constexpr int NJ = BV / 16;      // adjacent value columns per lane in the state reads
+  constexpr int HS = K + 16;       // byte stride of a stored-state row in LDS
+  constexpr int ES = 64 + 16;      // byte stride of a pseudo-value write-code row
+  constexpr int US = 2 * BV + 16;  // byte stride of a token row of the chain's wave-private U tile
+  constexpr int LS = 128 + 16;     // byte stride of a channel row of E / of its local codes (64 tokens, 2 bytes each)
+
+  __shared__ __align__(16) unsigned char hT[(DELTA ? 1 : 2) * BV * HS];
+  __shared__ __align__(16) unsigned char eT[DELTA ? BV * ES : 16];
+  __shared__ __align__(16) unsigned char eB[DELTA ? BV * LS : 16];  // E in the activation dtype, channel-major
+  __shared__ __align__(16) unsigned char eL[DELTA ? BV * LS : 16];  // its local codes as fp16, channel-major
+  __shared__ __align__(16) unsigned char ue_lds[DELTA ? 4 * 16 * US : 16];
+  __shared__ __align__(16) float misc_lds[256];                     // 64 floats per chain wave
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rl = lane & 15, kg = lane >> 4;
+  // the V tiles of one (batch, head) read the same key, query, state-read and decay operands at the same time: renumbered
+  // onto one XCD (workgroups are dealt to the 8 XCDs round-robin) whenever the grid divides evenly
+  int vtile = blockIdx.x, bh = blockIdx.y;
+  {
+    const int nv = gridDim.x, total = gridDim.x * gridDim.y;
+    if (total % 8 == 0 && (total / 8) % nv == 0) {
+      const int lid = blockIdx.x + nv * blockIdx.y;
+      const int vid = (lid % 8) * (total / 8) + lid / 8;
+      vtile = vid % nv, bh = vid / nv;
+    }
+  }
+  const int v0 = vtile * BV;
+  const int b = bh / p.H, h = bh % p.H;
+  const int H = p.H, V = p.V, T = p.T, NT = p.NT;
+  const int qmax = p.qmax;
+  constexpr bool bf = BF;
+
+  if (wv < 4) {
+    // ------------------------------------------------------------------------------------------------------- chain
+    const int wave = wv;
+    __builtin_amdgcn_s_setprio(2);  // the chain is what the launch lasts: it issues first where both waves of a SIMD can
+    float skw_r[KT][4], svw_c[VT], inv_ss_c[VT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) skw_r[kt][r] = p.skw[h * K + KR * wave + 16 * kt + 4 * kg + r];
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) {
+      svw_c[vt] = p.svw[h * V + v0 + 16 * vt + rl];
+      inv_ss_c[vt] = 1.0f / p.ss[h * V + v0 + 16 * vt + rl];
+    }
+    float ss_d[NJ], inv_ew_d[NJ], sw = 0.f;
+    if (DELTA) {
+      sw = p.sw[h];
+#pragma unroll
+      for (int jj = 0; jj < NJ; ++jj) {
+        ss_d[jj] = p.ss[h * V + v0 + NJ * rl + jj];
+        inv_ew_d[jj] = 1.0f / p.svw[h * V + v0 + NJ * rl + jj];
+      }
+    }
+    using Ops = ChainOps<DELTA, K>;
+    // part: 0 = everything, 1 = key codes, decays and per-token factors, 2 = state-read codes and U
+    auto load_part = [&](auto part_c, int ct, Ops& o) __attribute__((always_inline)) {
+      constexpr int part = decltype(part_c)::value;
+      const int64_t cb = ((int64_t)b * NT + ct) * H + h;
+      const int64_t t0 = (int64_t)b * T + (int64_t)ct * 64;
+      if constexpr (part == 0 || part == 1) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) o.kop[kt] = *(const lq_v4i*)(p.kqT + (cb * K + KR * wave + 16 * kt + rl) * 64 + 16 * kg);
+        if constexpr (DELTA) {  // fw[64] | ev[64] | gam[K]
+          const float* pk = p.pack + cb * (128 + K);
+          o.misc = *(lane < 32 ? pk + 64 * (lane >> 4) + 16 * wave + (lane & 15) : pk + 128 + KR * wave + min(lane - 32, KR - 1));
+        } else {
+          o.misc = p.gam[cb * K + KR * wave + min(max(lane - 32, 0), KR - 1)];
+#pragma unroll
+          for (int vt = 0; vt < VT; ++vt) o.vop[vt] = *(const lq_v4i*)(p.vqT + (cb * V + v0 + 16 * vt + rl) * 64 + 16 * kg);
+        }
+      }
+      if constexpr (DELTA && (part == 0 || part == 2)) {
+#pragma unroll
+        for (int ks = 0; ks < K / 64; ++ks)
+          o.wop[ks] = *(const lq_v4i*)(p.wq + cb * 64 * K + ((wave * (K / 64) + ks) * 64 + lane) * 16);
+        o.uraw = *(const lq_v4i*)(p.u + cb * 64 * V + 64 * v0 + (wave * 64 + lane) * 8);  // token lane >> 2, a quarter of the columns
+      }
+    };
+    float hc[KT][VT][4];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) hc[kt][vt][r] = 0.0f;
+    float* misc_s = misc_lds + 64 * wave;
+    unsigned char* ue_s = ue_lds + wave * 16 * US;
+
+    // one chunk step; the operands of chunk ct + D - 1 are requested into `pre` (unconditionally: the last chunks re-request the
+    // final one, so that the compiler's count of outstanding requests does not depend on the path)
+    auto do_step = [&](int ct, Ops& cur, Ops& pre) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);  // a request hoisted over the last use of its set would need registers of its own
+      unsigned char* hTb = hT + (DELTA ? 0 : (ct & 1) * BV * HS);
+      misc_s[lane] = cur.misc;
+      if constexpr (DELTA) {
+        *(lq_v4i*)(ue_s + (lane >> 2) * US + 16 * (lane & 3)) = cur.uraw;
+      }
+      // stored copy of the incoming state -> LDS (V-major)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) {
+          int cd[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) cd[r] = zoo_q8(hc[kt][vt][r], inv_ss_c[vt], 127);
+          *(uint32_t*)(hTb + (16 * vt + rl) * HS + KR * wave + 16 * kt + 4 * kg) = zoo_pack_codes(cd[0], cd[1], cd[2], cd[3]);
+        }
+      const int ctn = min(ct + D - 1, NT - 1);
+      load_part(std::integral_constant<int, 1>{}, ctn, pre);
+      __syncthreads();
+
+      if constexpr (DELTA) {
+        // state read against the stored copy, pseudo-values E, their write codes
+        lq_v4i aw[NJ];
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) aw[jj] = lq_v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int ks = 0; ks < K / 64; ++ks)
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj) {
+            const lq_v4i hop = *(const lq_v4i*)(hTb + (NJ * rl + jj) * HS + 64 * ks + 16 * kg);
+            aw[jj] = lq_mfma_i8(cur.wop[ks], hop, aw[jj]);
+          }
+        load_part(std::integral_constant<int, 2>{}, ctn, pre);
+        uint32_t ecode[NJ][4];
+        float ef[NJ][4];
+        const lq_v4f fw4 = *(const lq_v4f*)(misc_s + 4 * kg), ev4 = *(const lq_v4f*)(misc_s + 16 + 4 * kg);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const unsigned char* cell = ue_s + (4 * kg + r) * US + 2 * NJ * rl;
+          const uint32_t uw = *(const uint32_t*)cell;
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj) {
+            float ws = (float)aw[jj][r] * sw;
+            ws = ws * ss_d[jj];
+            const float u = zoo_dec1(jj ? uw >> 16 : uw & 0xffffu, bf);
+            ef[jj][r] = (u - ws) * fw4[r];
+            ecode[jj][r] = (uint32_t)zoo_q8(ef[jj][r] * ev4[r], inv_ew_d[jj], qmax);
+          }
+        }
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          *(uint32_t*)(eT + (NJ * rl + jj) * ES + 16 * wave + 4 * kg) =
+              zoo_pack_codes((int)ecode[jj][0], (int)ecode[jj][1], (int)ecode[jj][2], (int)ecode[jj][3]);
+          lq_v2i eo;
+          eo[0] = (int)zoo_enc2(ef[jj][0], ef[jj][1], bf);
+          eo[1] = (int)zoo_enc2(ef[jj][2], ef[jj][3], bf);
+          *(lq_v2i*)(eB + (NJ * rl + jj) * LS + 2 * (16 * wave + 4 * kg)) = eo;
+        }
+        __syncthreads();
+      }
+
+      // write product and carry update
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        lq_v4i bop;
+        if constexpr (DELTA)
+          bop = *(const lq_v4i*)(eT + (16 * vt + rl) * ES + 16 * kg);
+        else
+          bop = cur.vop[vt];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const lq_v4i a = lq_mfma_i8(cur.kop[kt], bop, lq_v4i{0, 0, 0, 0});
+          const lq_v4f gam4 = *(const lq_v4f*)(misc_s + 32 + 16 * kt + 4 * kg);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float prod = (float)a[r] * skw_r[kt][r];
+            prod = prod * svw_c[vt];
+            hc[kt][vt][r] = hc[kt][vt][r] * gam4[r] + prod;
+          }
+        }
+      }
+    };
+
+    Ops st[D];
+    load_part(std::integral_constant<int, 0>{}, 0, st[0]);
+    scan_for<D - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
+    scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load_part(std::integral_constant<int, 0>{}, min(i + 1, NT - 1), st[i + 1]); });
+    // everything requested so far is waited for once, in front of the loop (a load still outstanding at loop entry would make
+    // every iteration wait until almost nothing is in flight)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    asm volatile("" ::: "memory");
+    int ct = 0;
+    for (; ct + D <= NT; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(ct + i, st[i], st[(i + D - 1) % D]); });
+    scan_for<D - 1>([&](auto i) __attribute__((always_inline)) {
+      if (ct + i < NT) do_step(ct + i, st[i], st[(i + D - 1) % D]);
+    });
+    if constexpr (DELTA) __syncthreads();  // the output's last local codes (its rendezvous below)
+
+    if (p.ht) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            p.ht[(((int64_t)b * H + h) * K + KR * wave + 16 * kt + 4 * kg + r) * V + v0 + 16 * vt + rl] = hc[kt][vt][r];
+    }
+  } else {
+    // ------------------------------------------------------------------------------------------------------ output
+    const int w = wv - 4;      // token rows 16w .. 16w + 15 of every chunk
+    const int ot = tid - 256;  // thread of the output waves
+    const float sq = p.sq[h];
+    float ss_o[NJ], svl_o[NJ], inv_el = 0.0f;
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) ss_o[jj] = p.ss[h * V + v0 + NJ * rl + jj], svl_o[jj] = p.svl[h * V + v0 + NJ * rl + jj];
+    if constexpr (DELTA) inv_el = 1.0f / p.svl[h * V + v0 + (ot >> 3)];  // E -> local codes: this thread's column
+    using Ops = OutOps<DELTA, SCALAR, K>;
+    auto load = [&](int ct, Ops& o) __attribute__((always_inline)) {
+      const int64_t cb = ((int64_t)b * NT + ct) * H + h;
+#pragma unroll
+      for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = *(const lq_v4i*)(p.qc + cb * 64 * K + ((w * (K / 64) + ks) * 64 + lane) * 16);
+#pragma unroll
+      for (int js = 0; js < 2; ++js) o.aop[js] = *(const lq_v4i*)(p.A + cb * 4096 + ((w * 2 + js) * 64 + lane) * 8);
+      if constexpr (!DELTA) {
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) o.vop[jj] = *(const lq_v4i*)(p.vcT + cb * 64 * V + 64 * v0 + (jj * 64 + lane) * 16);
+      }
+      if constexpr (SCALAR) o.g = *(const lq_v4f*)(p.gpk + cb * 64 + 16 * w + 4 * kg);
+    };
+    float of[NJ][4];
+    // state read of chunk ct
+    auto read_state = [&](int ct, const Ops& o) __attribute__((always_inline)) {
+      const unsigned char* hTb = hT + (DELTA ? 0 : (ct & 1) * BV * HS);
+      lq_v4i a[NJ];
+#pragma unroll
+      for (int jj = 0; jj < NJ; ++jj) a[jj] = lq_v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < K / 64; ++ks)
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          const lq_v4i hop = *(const lq_v4i*)(hTb + (NJ * rl + jj) * HS + 64 * ks + 16 * kg);
+          a[jj] = lq_mfma_i8(o.qop[ks], hop, a[jj]);
+        }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float eg = SCALAR ? zoo_exp(o.g[r]) : 1.0f;
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          float x = (float)a[jj][r] * sq;
+          x = x * ss_o[jj];
+          of[jj][r] = SCALAR ? x * eg : x;
+        }
+      }
+    };
+    // local product of chunk ct on the fp16 MFMA, output
+    auto finish = [&](int ct, const Ops& o) __attribute__((always_inline)) {
+      lq_v4f loc[NJ];
+#pragma unroll
+      for (int jj = 0; jj < NJ; ++jj) loc[jj] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int js = 0; js < 2; ++js) {
+        const lq_v8h aop = __builtin_bit_cast(lq_v8h, o.aop[js]);
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          lq_v8h x;
+          if constexpr (DELTA)
+            x = *(const lq_v8h*)(eL + (NJ * rl + jj) * LS + 2 * (32 * js + 8 * kg));
+          else
+            x = scan_i8x8_to_f16x8(lq_v2i{o.vop[jj][2 * js], o.vop[jj][2 * js + 1]});
+          loc[jj] = lq_mfma_f16(aop, x, loc[jj]);
+        }
+      }
+      const int64_t t0 = (int64_t)b * T + (int64_t)ct * 64;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t off = ((t0 + 16 * w + 4 * kg + r) * H + h) * V + v0 + NJ * rl;
+        float res[NJ];
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) res[jj] = of[jj][r] + loc[jj][r] * svl_o[jj];
+        if constexpr (OF32) {
+          float* op = (float*)p.o + off;
+          *(lq_v2i*)op = lq_v2i{__float_as_int(res[0]), __float_as_int(res[1])};
+        } else {
+          _Float16* op = (_Float16*)p.o + off;
+          *(uint32_t*)op = zoo_enc2(res[0], res[1], bf);
+        }
+      }
+    };
+    // E of the chunk the chain has just formed -> its local codes (fp16), eight tokens of a column per thread
+    auto convert = [&]() __attribute__((always_inline)) {
+      const int col = ot >> 3;
+      const lq_v4i raw = *(const lq_v4i*)(eB + col * LS + 16 * (ot & 7));
+      lq_v4i o;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        float e0, e1;
+        zoo_dec2((uint32_t)raw[d], bf, e0, e1);
+        o[d] = (int)zoo_pack_h2((float)zoo_q8(e0, inv_el, qmax), (float)zoo_q8(e1, inv_el, qmax));
+      }
+      *(lq_v4i*)(eL + col * LS + 16 * (ot & 7)) = o;
+    };
+    // One step: `cur` holds chunk ct, `prev` chunk ct - 1, into which chunk ct + D - 1 is requested once its last use is past.
+    auto do_step = [&](auto first_c, int ct, Ops& cur, Ops& prev) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();  // the stored copy of chunk ct is in LDS
+      if constexpr (DELTA && !decltype(first_c)::value) finish(ct - 1, prev);
+      load(min(ct + D - 1, NT - 1), prev);
+      read_state(ct, cur);
+      if constexpr (DELTA) {
+        __syncthreads();  // E of chunk ct is in LDS
+        convert();
+      } else {
+        finish(ct, cur);
+      }
+    };
+    Ops st[D];
+    load(0, st[0]);
+    scan_for<D - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
+    scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load(min(i + 1, NT - 1), st[i + 1]); });
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
+    asm volatile("" ::: "memory");
+    do_step(std::true_type{}, 0, st[0], st[D - 1]);
+    int ct = 1;
+    for (; ct + D <= NT; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]); });
+    scan_for<D - 1>([&](auto i) __attribute__((always_inline)) {
+      if (ct + i < NT) do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]);
+    });
+    if constexpr (DELTA) {
+      __syncthreads();  // the local codes of the last chunk, written by all four output waves
+      scan_for<D>([&](auto i) __attribute__((always_inline)) {
+        if ((NT - 1) % D == i) finish(NT - 1, st[i]);
+      });
+    }
+  }
+}
+
+template <bool DELTA, bool SCALAR, int K>
+int launch(const ScanParams& p, int B, hipStream_t stream) {
+  const dim3 grid(p.V / BV, B * p.H), block(512);
+  if (DELTA && p.o_is_f32 && p.bf)  // (the linear family reads codes only: the activation dtype is that of the output)
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, DELTA, true>), grid, block, 0, stream, p);
+  else if (p.o_is_f32)
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, false, true>), grid, block, 0, stream, p);
+  else if (p.bf)
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, true, false>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, false, false>), grid, block, 0, stream, p);
+  return lq_check_launch();
+}
+
+template <bool DELTA, bool SCALAR>
+int launch_k(const ScanParams& p, int K, int B, hipStream_t stream) {
+  return K == 128 ? launch<DELTA, SCALAR, 128>(p, B, stream) : launch<DELTA, SCALAR, 64>(p, B, stream);
+}
+
+}  // namespace
+
+int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, int batch, hipStream_t stream) {
+  if (delta) return scalar ? launch_k<true, true>(p, K, batch, stream) : launch_k<true, false>(p, K, batch, stream);
+  return scalar ? launch_k<false, true>(p, K, batch, stream) : launch_k<false, false>(p, K, batch, stream);
+}

@@ -17,8 +17,7 @@
 //   W, U: T . X on the bf16 MFMA with T and X each split in three bf16 pieces (six products per step); X is staged
 //     transposed in LDS, each wave takes row block w for the first half of the column tiles and row block 3 - w for
 //     the second half (equal work), and stores four adjacent channels per lane.
-#include "zoo_common.h"
-#include "../../include/linquant_hip.h"
+#include "zoo_params.h"
 
 namespace {
 
@@ -279,7 +278,8 @@ LQ_DEV void gram_rowblock(const WyParams& p, float* G_s, const float* bs_s, cons
 // CODES: the kernel also emits what lq_zoo_write_codes would make from the stored Hw and W (same arithmetic on the same
 // rounded values, so the same bits): channel-major key write codes, token-major state-read codes of W, the per-token
 // value factor and the per-channel chunk decay.  W itself is then stored only when p.W is set.
-template <int DECAY, int K, bool BF, bool CODES, bool DK>
+// SCAN (with CODES): wq and U leave in operand order (zoo_params.h), for zoo_scan.hip.
+template <int DECAY, int K, bool BF, bool CODES, bool DK, bool SCAN>
 __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
   constexpr int LS = 64 + 16;  // floats per row of the buffer that holds the Gram tile and then the X tiles
   static_assert(LS >= kGS, "the Gram tile lives in the X buffer until the inverse is done");
@@ -323,6 +323,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
   const int ct = (int)(group % (uint32_t)p.NT), b = (int)(group / (uint32_t)p.NT);
   const int H = p.H, V = p.V;
   const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
+  const int64_t cb = ((int64_t)b * p.NT + ct) * H + h;
   const float sigma = p.sigma, tau = p.tau;
   constexpr bool bf = BF;
 
@@ -694,8 +695,9 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
       lq_v2i o;
       o[0] = (int)zoo_enc2(a[0], a[1], bf);
       o[1] = (int)zoo_enc2(a[2], a[3], bf);
-      const int64_t woff = ((t0 + 16 * I + rl) * H + h) * K + kc + 16 * nt + 4 * kg;
-      if (!CODES || p.W) *(lq_v2i*)(p.W + woff) = o;
+      const int64_t woff = SCAN ? cb * 64 * K + zoo_op_codes(16 * I + rl, kc + 16 * nt + 4 * kg, K)
+                                : ((t0 + 16 * I + rl) * H + h) * K + kc + 16 * nt + 4 * kg;
+      if (!SCAN && (!CODES || p.W)) *(lq_v2i*)(p.W + woff) = o;
       if constexpr (CODES) {  // state-read codes of the rounded W
         float w0, w1, w2, w3;
         zoo_dec2((uint32_t)o[0], bf, w0, w1);
@@ -734,7 +736,8 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
       lq_v2i o;
       o[0] = (int)zoo_enc2(a[0], a[1], bf);
       o[1] = (int)zoo_enc2(a[2], a[3], bf);
-      *(lq_v2i*)(p.U + ((t0 + 16 * I + rl) * H + h) * V + vc + 16 * nt + 4 * kg) = o;
+      *(lq_v2i*)(SCAN ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vc + 16 * nt + 4 * kg)
+                      : p.U + ((t0 + 16 * I + rl) * H + h) * V + vc + 16 * nt + 4 * kg) = o;
     }
   }
 }
@@ -917,37 +920,41 @@ int launch128_decay(const WyParams& p, int decay, hipStream_t stream) {
   return LQ_ERR_SHAPE;
 }
 
-template <int DECAY, int K, bool CODES, bool DK>
+template <int DECAY, int K, bool CODES, bool DK, bool SCAN = false>
 int launch_c(const WyParams& p, dim3 grid, hipStream_t stream) {
   if (p.bf)
-    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, true, CODES, DK>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, true, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, false, CODES, DK>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, false, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
   return lq_check_launch();
 }
 
 template <int DECAY, int K>
-int launch(const WyParams& p, dim3 grid, hipStream_t stream) {
+int launch(const WyParams& p, bool scan, dim3 grid, hipStream_t stream) {
+  if constexpr (DECAY == LQ_DECAY_DIAGONAL) {
+    if (scan) return p.dk_div ? launch_c<DECAY, K, true, true, true>(p, grid, stream) : launch_c<DECAY, K, true, false, true>(p, grid, stream);
+  }
   if (p.dk_div) return launch_c<DECAY, K, true, true>(p, grid, stream);  // the rescaling comes with the codes (checked)
   return p.kqT ? launch_c<DECAY, K, true, false>(p, grid, stream) : launch_c<DECAY, K, false, false>(p, grid, stream);
 }
 
 template <int K>
-int launch_decay(const WyParams& p, int decay, dim3 grid, hipStream_t stream) {
+int launch_decay(const WyParams& p, int decay, bool scan, dim3 grid, hipStream_t stream) {
   switch (decay) {
-    case LQ_DECAY_NONE: return launch<LQ_DECAY_NONE, K>(p, grid, stream);
-    case LQ_DECAY_SCALAR: return launch<LQ_DECAY_SCALAR, K>(p, grid, stream);
-    case LQ_DECAY_DIAGONAL: return launch<LQ_DECAY_DIAGONAL, K>(p, grid, stream);
+    case LQ_DECAY_NONE: return launch<LQ_DECAY_NONE, K>(p, scan, grid, stream);
+    case LQ_DECAY_SCALAR: return launch<LQ_DECAY_SCALAR, K>(p, scan, grid, stream);
+    case LQ_DECAY_DIAGONAL: return launch<LQ_DECAY_DIAGONAL, K>(p, scan, grid, stream);
   }
   return LQ_ERR_SHAPE;
 }
 
 }  // namespace
 
-extern "C" int lq_zoo_wy_prep(const lq_zoo_wy_prep_args* a, hipStream_t stream) {
+int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stream) {
   if (!a || !a->k || !a->v || !a->beta || !a->Hw || !a->U || !a->fw) return LQ_ERR_NULL;
   if (a->decay != LQ_DECAY_NONE && !a->g) return LQ_ERR_NULL;
   const bool codes = a->kqT != nullptr;
+  if (scan && (!codes || a->decay != LQ_DECAY_DIAGONAL)) return LQ_ERR_SHAPE;
   if (!codes && !a->W) return LQ_ERR_NULL;
   if (codes && (!a->wq || !a->ev || !a->gam || !a->skw || !a->sw)) return LQ_ERR_NULL;
   if (codes && a->decay == LQ_DECAY_DIAGONAL && !a->logenv) return LQ_ERR_NULL;
@@ -979,5 +986,7 @@ extern "C" int lq_zoo_wy_prep(const lq_zoo_wy_prep_args* a, hipStream_t stream) 
   if ((int64_t)(a->seqlen / 64) * a->batch * a->nheads > 0x7fffffff) return LQ_ERR_SHAPE;
   if (big) return a->kdim == 128 ? launch128_decay<128>(p, a->decay, stream) : launch128_decay<64>(p, a->decay, stream);
   dim3 grid((uint32_t)((a->seqlen / 64) * a->batch * a->nheads));
-  return a->kdim == 128 ? launch_decay<128>(p, a->decay, grid, stream) : launch_decay<64>(p, a->decay, grid, stream);
+  return a->kdim == 128 ? launch_decay<128>(p, a->decay, scan, grid, stream) : launch_decay<64>(p, a->decay, scan, grid, stream);
 }
+
+extern "C" int lq_zoo_wy_prep(const lq_zoo_wy_prep_args* a, hipStream_t stream) { return zoo_wy_prep_launch(a, false, stream); }

@@ -1,0 +1,45 @@
+"""GPU test of the launch that runs the chunk recurrence and the output together (zoo_scan.hip) at the edges of its loops and
+grids, against the stage-by-stage kernels, which the float64 oracle pins in test_zoo_gpu.py: every value is the same arithmetic
+in the same order, so outputs and final states are equal bit for bit."""
+
+import pytest
+import torch
+
+from tests import zoo_cases as zc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cell", list(zc.CELLS))
+# chunks: fewer than the operand sets in rotation (3 and 5), exactly as many, remainders of one and of all but one; grids that
+# do and do not divide over the 8 XCDs; one and several V tiles per head, a V the operand prologue is not built for (192)
+@pytest.mark.parametrize("NT,B,H,K,V,dtype,out_dtype", [
+    (1, 1, 1, 128, 64, torch.float16, None), (2, 1, 8, 64, 128, torch.bfloat16, None), (3, 2, 3, 128, 192, torch.float16, None),
+    (5, 1, 5, 64, 64, torch.float16, torch.float32), (6, 3, 2, 128, 128, torch.bfloat16, torch.float32),
+    (11, 2, 4, 128, 128, torch.float16, None)])
+def test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype):
+    from linquant_amd.kernels import zoo
+    from oracle.zoo_reference import signed_hadamard
+
+    q, k, v, g, beta = [t.to(cuda) if t is not None else None for t in zc.inputs(cell, B=B, T=64 * NT, H=H, K=K, V=V, seed=NT, dtype=dtype)]
+    gen = torch.Generator().manual_seed(NT)
+    r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
+    sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.01), "w": r(H, lo=0.02, hi=0.04), "kw": r(H, K, lo=0.005, hi=0.015),
+          "vw": r(H, V, lo=0.02, hi=0.04), "vl": r(H, V, lo=0.02, hi=0.04), "el": r(H, V, lo=0.04, hi=0.06),
+          "ew": r(H, V, lo=0.04, hi=0.06), "state": r(H, V, lo=0.02, hi=0.07)}
+    fam, dec = zc.CELLS[cell]
+    kw = dict(eta=0.25, output_final_state=True, out_dtype=out_dtype)
+    if dec == "diagonal":
+        kw["rot"] = signed_hadamard(K, 2).float().to(cuda)
+    if fam == "delta":
+        kw.update(sigma=0.5, tau=0.5)
+        fn = zoo.chunk_kda_int8 if dec == "diagonal" else zoo.chunk_delta_int8
+        args = (q, k, v, g, beta, sc)
+    else:
+        fn = zoo.chunk_gla_int8 if dec == "diagonal" else zoo.chunk_simple_gla_int8
+        args = (q, k, v, g, sc)
+    o1, h1 = fn(*args, **kw)
+    o0, h0 = fn(*args, _debug={}, **kw)
+    torch.cuda.synchronize()
+    assert o1.dtype == (out_dtype or dtype) and float(o1.float().abs().max()) > 0
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
