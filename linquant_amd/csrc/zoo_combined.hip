@@ -95,12 +95,12 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // ---- the other cells: chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry each way round: the stage entry points in
 // the order the Python wrappers issue them, over one workspace.  64-token chunks take the fused pre-passes (the cumsum / WY
-// launch also makes the write codes), 128-token chunks the separate write-codes launch.  Under per-channel decay 64-token
-// chunks run the recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).
+// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks run the
+// recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).
 namespace {
 
 struct FLayout {
-  int64_t gc, logenv, kqT, vqT, vcT, wq, ev, gam, pack, A, Ax, qg, Hw, W, U, fw, e_out, h_i8, cross, total;
+  int64_t gc, logenv, kqT, vqT, vcT, wq, ev, gam, pack, gpk, A, Ax, qg, Hw, W, U, fw, e_out, h_i8, cross, total;
   bool scan;  // recurrence and output in one launch
 };
 
@@ -123,12 +123,13 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->ev, B * T * H * 4);
   take(l->gam, B * NT * H * K * 4);
   take(l->pack, delta && !big ? B * NT * H * (128 + K) * 4 : 0);
-  take(l->A, diag ? B * T * H * 64 * 2 : 0);
+  take(l->A, diag || !big ? B * T * H * 64 * 2 : 0);
   take(l->Ax, diag && big ? B * T * H * 64 * 2 : 0);
-  take(l->qg, diag ? B * T * H * K : 0);
-  l->scan = diag && !big;
+  take(l->qg, diag || !big ? B * T * H * K : 0);
+  take(l->gpk, a->decay == LQ_DECAY_SCALAR && !big ? B * NT * H * 64 * 4 : 0);
+  l->scan = !big;
   take(l->vcT, l->scan && !delta ? B * NT * H * V * 64 : 0);
-  take(l->Hw, delta ? B * T * H * K * 2 : 0);
+  take(l->Hw, delta && (diag || big) ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
   take(l->U, delta ? B * T * H * V * 2 : 0);
   take(l->fw, delta ? B * T * H * 4 : 0);
@@ -173,15 +174,16 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   float* ev = (float*)(ws + l.ev);
   float* gam = (float*)(ws + l.gam);
   float* pack = delta && !big ? (float*)(ws + l.pack) : nullptr;
-  void* Hw = delta ? ws + l.Hw : nullptr;
+  void* Hw = delta && (diag || big) ? ws + l.Hw : nullptr;
   void* W = delta && big ? ws + l.W : nullptr;
   void* U = delta ? ws + l.U : nullptr;
   float* fw = delta ? (float*)(ws + l.fw) : nullptr;
   void* e_out = delta ? ws + l.e_out : nullptr;
   int8_t* h_i8 = (int8_t*)(ws + l.h_i8);
-  void* A = diag ? ws + l.A : nullptr;
+  void* A = diag || !big ? ws + l.A : nullptr;
   void* Ax = diag && big ? ws + l.Ax : nullptr;
-  int8_t* qg = diag ? (int8_t*)(ws + l.qg) : nullptr;
+  int8_t* qg = diag || !big ? (int8_t*)(ws + l.qg) : nullptr;
+  float* gpk = a->decay == LQ_DECAY_SCALAR && !big ? (float*)(ws + l.gpk) : nullptr;
   int8_t* vcT = l.scan && !delta ? (int8_t*)(ws + l.vcT) : nullptr;
   float* cross = big ? (float*)(ws + l.cross) : nullptr;
 
@@ -205,7 +207,8 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
       w.kqT = kqT, w.wq = wq, w.ev = ev, w.gam = gam, w.logenv = logenv, w.skw = a->skw, w.sw = a->sw, w.eta = a->eta, w.qmax = a->qmax;
       w.dk_div = a->dq, w.dk_rcp = a->dq_rcp, w.pack = pack;
     }
-    if ((rc = zoo_wy_prep_launch(&w, l.scan, stream)) != LQ_OK) return rc;
+    const ZooWyLocal local = {a->q, qg, A, gpk, a->sq, a->sk, a->scale};
+    if ((rc = zoo_wy_prep_launch(&w, l.scan, l.scan && !diag ? &local : nullptr, stream)) != LQ_OK) return rc;
   }
   if (big) {
     lq_zoo_write_codes_args w = {};
@@ -225,10 +228,10 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   if (l.scan) {
     ZooScanParams s = {};
     s.kqT = kqT, s.vqT = vqT, s.vcT = vcT, s.wq = wq, s.u = (const _Float16*)U, s.pack = pack, s.gam = gam;
-    s.qc = qg, s.A = (const _Float16*)A, s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
+    s.qc = qg, s.A = (const _Float16*)A, s.gpk = gpk, s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
     s.skw = a->skw, s.svw = a->svw, s.sw = a->sw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
     s.qmax = a->qmax, s.bf = a->act_dtype == LQ_DT_BF16, s.T = a->seqlen, s.H = a->nheads, s.V = a->vdim, s.NT = a->seqlen / 64;
-    return zoo_scan_launch(s, delta, false, a->kdim, a->batch, stream);
+    return zoo_scan_launch(s, delta, a->decay == LQ_DECAY_SCALAR, a->kdim, a->batch, stream);
   }
   {
     lq_zoo_state_args s = {};

@@ -129,5 +129,54 @@ int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, int 
 int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl, hipStream_t stream);
 // A kernel: A and qg in operand order (scan = true)
 int zoo_gla_A_launch(const lq_zoo_gla_A_args* a, bool scan, hipStream_t stream);
-// WY prep with the write codes: wq and U in operand order (scan = true)
-int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stream);
+// WY prep.  scan (with the write codes): wq and U in operand order; no / scalar decay also the codes of q and A (`local`), and Hw is
+// not stored then
+struct ZooWyLocal {
+  const void* q;
+  int8_t* qc;   // zoo_op_codes
+  void* A;      // zoo_op_A
+  float* gpk;   // scalar decay: (B,NT,H,64)
+  const float* sq;
+  const float* sk;
+  float scale;
+};
+int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, const ZooWyLocal* local, hipStream_t stream);
+
+struct ZooWyParams {
+  const _Float16* k;
+  const _Float16* v;
+  const float* beta;
+  const float* g;
+  _Float16* Hw;
+  _Float16* W;
+  _Float16* U;
+  float* fw;
+  float sigma, tau;
+  int bf;
+  int B, T, H, V;
+  // write-operand codes of the state kernel, made here when kqT is set (otherwise lq_zoo_write_codes makes them from the
+  // stored Hw and W)
+  int8_t* kqT;
+  int8_t* wq;
+  float* ev;
+  float* gam;
+  const float* logenv;
+  const float* skw;
+  const float* sw;
+  float eta;
+  int qmax;
+  int NT;
+  const float* dk_div;  // (H,K) D_QK applied to k at load (k' = act(k / D)), with its reciprocal; or nullptr
+  const float* dk_rcp;
+  float* pack;  // fw | ev | gam per (batch, chunk, head), 64 + 64 + K floats, or nullptr
+  // ZooWyLocal
+  const _Float16* q;
+  int8_t* qc;
+  _Float16* A;
+  float* gpk;
+  const float* sq;
+  const float* sk;
+  float scale;
+};
+// no / scalar decay; defined in zoo_wy_ns.hip
+int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, dim3 grid, hipStream_t stream);

@@ -1,0 +1,482 @@
+// WY / UT transform of the delta family with no or scalar decay (DeltaNet, Gated DeltaNet), 64-token chunks, with everything the
+// chunk recurrence wants of a chunk made in the same launch.
+// Replaces the torch prep linquant/kernels/zoo/gated_delta_rule.py:20-47 and the operand preparation of the state and output
+// bodies (gated_delta_rule.py:85-105, simple_gla.py:125-140):
+//   G[i][j] = bs_i bh_j (k_i . k_j) * exp(g_i - g_j) for i > j,  bs = beta^sigma, bh = beta^(1-sigma);  T = (I + G)^-1
+//   W = T (bs k exp(g)),  U = T (bs v),  Hw = beta^((1-sigma) tau) k,  fw = beta^((1-sigma)(1-tau))
+//
+// Nothing but per-token factors separates the operands of these products from k and v themselves, and a per-token factor is an
+// index of T's columns.  So the half-precision rows stay exact and all arithmetic goes to T:
+//   Gram: k . k^T on the half-precision MFMA (exact products, fp32 accumulation), the factors applied to the 64 x 64 result;
+//   W, U: (T . diag(bs exp(g))) . k and (T . diag(bs)) . v with k and v as they are and only T split: two fp16 pieces of each
+//     row scaled by a power of two to just below fp16's range (so that neither piece of an entry down to 2^-18 of the row's largest
+//     is subnormal), three bf16 pieces for bf16 activations.  Share of W, U entries on the other side of a rounding boundary than
+//     the float64 result (B2 T512, unit keys): 2.5e-4, 3.5e-4 in fp16, 4e-5 in bf16; the fp32 form below 4.5e-4, 5.6e-4 and 1e-4.
+// An fp32 form of the same (operands scaled and staged as fp32, 32 fp32 MFMA steps per Gram block, T and X split in three bf16
+// pieces, six products) took 121 us at B4 T4096 H16 K = V = 128, of which the splitting and the fp32 steps were two thirds.
+//
+// One 8-wave workgroup per (chunk, batch*head), two to a compute unit (77 KB of LDS): load and quantize (every row is read once)
+// | Gram blocks and, MODE_SCAN, the blocks of the intra-chunk product A (20 blocks over the 8 waves) | G | inverse of the four
+// diagonal blocks by forward substitution | block columns of T, one wave each, in registers | products.  Bound by memory: 97 KB a
+// chunk.
+#include "zoo_params.h"
+
+namespace {
+
+enum { MODE_PLAIN = 0, MODE_CODES = 1, MODE_SCAN = 2 };
+// MODE_PLAIN: Hw, W, U, fw.  MODE_CODES: also the write operands of the state kernel (W stored only when p.W is set).
+// MODE_SCAN: what zoo_scan.hip wants: the write operands, wq and U in operand order, the codes of q and the product A; no Hw.
+
+LQ_DEV lq_v4f wn_mfma_f32(float a, float b, lq_v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+typedef __bf16 wn_v8bf __attribute__((ext_vector_type(8)));
+
+template <bool BF>
+LQ_DEV lq_v4f wn_mfma(lq_v4i a, lq_v4i b, lq_v4f c) {
+  if constexpr (BF) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wn_v8bf, a), __builtin_bit_cast(wn_v8bf, b), c, 0, 0, 0);
+  return lq_mfma_f16(__builtin_bit_cast(lq_v8h, a), __builtin_bit_cast(lq_v8h, b), c);
+}
+
+constexpr int kGS = 70;   // floats per row of the G / T tiles: an A-operand read (16 rows, 4 adjacent slots) takes one LDS pass at 2 mod 4
+constexpr int kXP = 36;   // dwords per column of the transposed tiles (32 token pairs + pad)
+constexpr int kCS = 80;   // bytes per channel row of the transposed write codes (64 tokens + pad)
+
+// dword of the transposed tile [column][token pair]; the pairs are permuted in groups of four (one 16-byte operand piece) so that
+// the writes of a wave (16 groups of eight columns x 4 pairs) fall on 64 different banks
+LQ_DEV int wn_xt(int col, int pair) { return col * kXP + (pair ^ (((col >> 4) & 7) << 2)); }
+
+LQ_DEV float wn_powb(float b, float e) {
+  if (e == 0.0f) return 1.0f;
+  if (e == 1.0f) return b;
+  return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(b));
+}
+
+// T operand of one row block and contraction step: eight values of a row, scaled, as NP pieces
+template <bool BF>
+struct TPieces {
+  static constexpr int NP = BF ? 3 : 2;
+  lq_v4i p[NP];
+};
+
+template <bool BF>
+LQ_DEV void wn_split(const float (&x)[8], TPieces<BF>& t) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const float x0 = x[2 * d], x1 = x[2 * d + 1];
+    if constexpr (BF) {  // upper 16 bits of what the pieces before leave: 24 significant bits in all
+      const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+      t.p[0][d] = (int)__builtin_amdgcn_perm(b1, b0, 0x07060302u);
+      const float r0 = x0 - __uint_as_float(b0 & 0xffff0000u), r1 = x1 - __uint_as_float(b1 & 0xffff0000u);
+      const uint32_t c0 = __float_as_uint(r0), c1 = __float_as_uint(r1);
+      t.p[1][d] = (int)__builtin_amdgcn_perm(c1, c0, 0x07060302u);
+      const float q0 = r0 - __uint_as_float(c0 & 0xffff0000u), q1 = r1 - __uint_as_float(c1 & 0xffff0000u);
+      t.p[2][d] = (int)__builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
+    } else {
+      const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+      t.p[0][d] = __builtin_bit_cast(int, lq_v2h{h0, h1});
+      t.p[1][d] = (int)zoo_pack_h2(x0 - (float)h0, x1 - (float)h1);
+    }
+  }
+}
+
+template <bool SCALAR, int K, bool BF, int MODE>
+__global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
+  constexpr bool CODES = MODE != MODE_PLAIN, SCAN = MODE == MODE_SCAN;
+  constexpr int FS = K + 16;                      // halves per row of the raw key tile (72 or 40 dwords: two-pass operand reads)
+  constexpr int QS = K == 128 ? 160 : 80;         // bytes per row of the code tiles
+  constexpr int kR1 = 64 * FS * 2 > 64 * kGS * 4 ? 64 * FS * 2 : 64 * kGS * 4;            // raw keys, then T
+  constexpr int kR2 = 2 * 64 * QS > 128 * kXP * 4 ? 2 * 64 * QS : 128 * kXP * 4;          // codes of q and k, then transposed v
+  constexpr int kR3 = K * kCS > 64 * kGS * 4 ? K * kCS : 64 * kGS * 4;                    // transposed write codes, then G
+  constexpr int kR4 = K * kXP * 4;                                                       // transposed keys
+  __shared__ __align__(16) unsigned char lds[kR1 + kR2 + kR3 + kR4];
+  _Float16* kF = (_Float16*)lds;
+  float* T_s = (float*)lds;
+  unsigned char* qI = lds + kR1;
+  unsigned char* kI = lds + kR1 + 64 * QS;
+  uint32_t* Xv = (uint32_t*)(lds + kR1);
+  unsigned char* cT = lds + kR1 + kR2;
+  float* G_s = (float*)(lds + kR1 + kR2);
+  uint32_t* Xk = (uint32_t*)(lds + kR1 + kR2 + kR3);
+  __shared__ float bs_s[64], bh_s[64], bw_s[64], el_s[64], fW_s[64], gs_s[64], iskw_s[CODES ? K : 1];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rl = lane & 15, kg = lane >> 4;
+  // Flat grid: workgroup L = x + 8 m (x = its XCD) takes head m % H of (batch, chunk) number x + 8 (m / H): the workgroups
+  // resident on one XCD cover all heads of a few (batch, chunk)s, so the (B, T, H) tensors are fetched and written as whole lines
+  const uint32_t ngroups = (uint32_t)p.B * (uint32_t)p.NT;
+  uint32_t group, hh;
+  if ((ngroups & 7u) == 0) {
+    const uint32_t m = blockIdx.x >> 3;
+    hh = m % (uint32_t)p.H;
+    group = (blockIdx.x & 7u) + 8u * (m / (uint32_t)p.H);
+  } else {
+    hh = blockIdx.x % (uint32_t)p.H;
+    group = blockIdx.x / (uint32_t)p.H;
+  }
+  const int h = (int)hh;
+  const int ct = (int)(group % (uint32_t)p.NT), b = (int)(group / (uint32_t)p.NT);
+  const int H = p.H, V = p.V, qmax = p.qmax;
+  const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
+  const int64_t cb = ((int64_t)b * p.NT + ct) * H + h;
+  constexpr bool bf = BF;
+
+  // ---- requests: a thread takes two adjacent tokens x 8 channels of k, q and (first 128 columns) v
+  constexpr int KP = K / 8;  // 16-byte pieces of a key row
+  const int krp = tid / KP, kc = tid % KP;
+  const bool kact = K == 128 || tid < 256;
+  const int vp = min(V, 128) / 8;  // pieces of a value row per pass
+  const int vrp = tid / vp, vc8 = tid % vp;
+  const bool vact = vrp < 32;
+  lq_v4i kraw[2], qraw[2], vraw[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int64_t row = (t0 + 2 * (kact ? krp : 0) + u) * H + h;
+    kraw[u] = *(const lq_v4i*)(p.k + row * K + 8 * kc);
+    if constexpr (SCAN) qraw[u] = *(const lq_v4i*)(p.q + row * K + 8 * kc);
+    vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * (vact ? vrp : 0) + u) * H + h) * V + 8 * vc8);
+  }
+  // ---- per-token factors
+  if (tid < 64) {
+    const float bt = p.beta[(t0 + tid) * H + h];
+    const float bs = wn_powb(bt, p.sigma);
+    const float fwv = wn_powb(bt, (1.0f - p.sigma) * (1.0f - p.tau));
+    float gv = 0.0f, gl = 0.0f;
+    if (SCALAR) gv = p.g[(t0 + tid) * H + h], gl = p.g[(t0 + 63) * H + h];
+    bs_s[tid] = bs;
+    bh_s[tid] = wn_powb(bt, 1.0f - p.sigma);
+    bw_s[tid] = wn_powb(bt, (1.0f - p.sigma) * p.tau);
+    gs_s[tid] = gv;
+    fW_s[tid] = SCALAR ? bs * zoo_exp(gv) : bs;
+    el_s[tid] = SCALAR ? zoo_exp((1.0f - p.eta) * (gl - gv)) : 1.0f;
+    float* pk = p.pack ? p.pack + cb * (128 + K) : nullptr;
+    if (!SCAN) p.fw[(t0 + tid) * H + h] = fwv;
+    if constexpr (CODES) {
+      const float evv = SCALAR ? zoo_exp(p.eta * (gl - gv)) : 1.0f;
+      if (!SCAN) p.ev[(t0 + tid) * H + h] = evv;
+      if (pk) pk[tid] = fwv, pk[64 + tid] = evv;
+      if (SCAN && SCALAR) p.gpk[cb * 64 + tid] = gv;
+    }
+  } else if (CODES && tid >= 128 && tid < 128 + K) {
+    const int n = tid - 128;
+    const float gm = SCALAR ? zoo_exp(p.g[(t0 + 63) * H + h]) : 1.0f;
+    if (!SCAN) p.gam[cb * K + n] = gm;
+    if (p.pack) p.pack[cb * (128 + K) + 128 + n] = gm;
+    iskw_s[n] = 1.0f / p.skw[h * K + n];
+  }
+  __syncthreads();
+
+  // ---- rows into LDS: raw keys by token (Gram) and by channel (W), codes of q and Hw, transposed write codes
+  if (kact) {
+    if (p.dk_div) {  // D_QK at load: k' = act(k / D), the quotient rounded once (uniform over the launch)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const int n = h * K + 8 * kc + 2 * d;
+          float x0, x1;
+          zoo_dec2((uint32_t)kraw[u][d], bf, x0, x1);
+          kraw[u][d] = (int)zoo_enc2(zoo_div_rn(x0, p.dk_div[n], p.dk_rcp[n]), zoo_div_rn(x1, p.dk_div[n + 1], p.dk_rcp[n + 1]), bf);
+        }
+    }
+    float inv_sq = 0.0f, inv_sk = 0.0f;
+    if constexpr (SCAN) inv_sq = 1.0f / p.sq[h], inv_sk = 1.0f / p.sk[h];
+    uint32_t wc[2][8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int t = 2 * krp + u;
+      *(lq_v4i*)(kF + t * FS + 8 * kc) = kraw[u];
+      const float bw = bw_s[t], el = el_s[t];
+      lq_v2i ok, oq;
+      lq_v4i hw;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        float x0, x1;
+        zoo_dec2((uint32_t)kraw[u][d], bf, x0, x1);
+        hw[d] = (int)zoo_enc2(bw * x0, bw * x1, bf);  // Hw as it would be stored
+      }
+      if constexpr (!SCAN) *(lq_v4i*)(p.Hw + ((t0 + t) * H + h) * K + 8 * kc) = hw;
+      if constexpr (CODES) {
+        int ck[8], cq[8];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          float x0, x1;
+          zoo_dec2((uint32_t)hw[d], bf, x0, x1);
+          if constexpr (SCAN) ck[2 * d] = zoo_q8(x0, inv_sk, qmax), ck[2 * d + 1] = zoo_q8(x1, inv_sk, qmax);
+          if (SCALAR) x0 = x0 * el, x1 = x1 * el;
+          wc[u][2 * d] = (uint32_t)zoo_q8(x0, iskw_s[8 * kc + 2 * d], qmax);
+          wc[u][2 * d + 1] = (uint32_t)zoo_q8(x1, iskw_s[8 * kc + 2 * d + 1], qmax);
+          if constexpr (SCAN) {
+            zoo_dec2((uint32_t)qraw[u][d], bf, x0, x1);
+            cq[2 * d] = zoo_q8(x0 * p.scale, inv_sq, qmax), cq[2 * d + 1] = zoo_q8(x1 * p.scale, inv_sq, qmax);
+          }
+        }
+        if constexpr (SCAN) {
+          ok[0] = (int)zoo_pack_codes(ck[0], ck[1], ck[2], ck[3]), ok[1] = (int)zoo_pack_codes(ck[4], ck[5], ck[6], ck[7]);
+          oq[0] = (int)zoo_pack_codes(cq[0], cq[1], cq[2], cq[3]), oq[1] = (int)zoo_pack_codes(cq[4], cq[5], cq[6], cq[7]);
+          *(lq_v2i*)(kI + t * QS + 8 * kc) = ok;
+          *(lq_v2i*)(qI + t * QS + 8 * kc) = oq;
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      Xk[wn_xt(8 * kc + 2 * d, krp)] = __builtin_amdgcn_perm((uint32_t)kraw[1][d], (uint32_t)kraw[0][d], 0x05040100u);
+      Xk[wn_xt(8 * kc + 2 * d + 1, krp)] = __builtin_amdgcn_perm((uint32_t)kraw[1][d], (uint32_t)kraw[0][d], 0x07060302u);
+    }
+    if constexpr (CODES) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        *(uint16_t*)(cT + (8 * kc + e) * kCS + 2 * krp) = (uint16_t)__builtin_amdgcn_perm(wc[1][e], wc[0][e], 0x0c0c0400u);
+    }
+  }
+  __syncthreads();
+
+  // ---- the write codes leave as whole rows
+  if constexpr (CODES) {
+    if (tid < K * 4) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(cT + (tid >> 2) * kCS + 16 * (tid & 3));
+  }
+  // ---- Gram blocks (tasks 0..9) and, MODE_SCAN, A blocks (tasks 10..19): task t belongs to wave t % 8
+  // block n of the lower triangle: (0,0) (1,0) (1,1) (2,0) (2,1) (2,2) (3,0) ..
+  auto blk_i = [](int n) { return n < 1 ? 0 : (n < 3 ? 1 : (n < 6 ? 2 : 3)); };
+  auto blk_j = [](int n) { return n < 1 ? 0 : (n < 3 ? n - 1 : (n < 6 ? n - 3 : n - 6)); };
+  lq_v4f gacc[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    gacc[s] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+    const int n = wave + 8 * s;
+    if (n >= 10) continue;
+    const _Float16* ra = kF + (16 * blk_i(n) + rl) * FS + 8 * kg;
+    const _Float16* rb = kF + (16 * blk_j(n) + rl) * FS + 8 * kg;
+#pragma unroll
+    for (int ks = 0; ks < K / 32; ++ks) gacc[s] = wn_mfma<BF>(*(const lq_v4i*)(ra + 32 * ks), *(const lq_v4i*)(rb + 32 * ks), gacc[s]);
+  }
+  if constexpr (SCAN) {
+    const float sqk = p.sq[h] * p.sk[h];
+#pragma unroll
+    for (int s = 1; s < 3; ++s) {
+      const int n = wave + 8 * s - 10;  // (A blocks: tasks 10 .. 19)
+      if (n < 0 || n >= 10) continue;
+      const int I = blk_i(n), J = blk_j(n);
+      lq_v4i acc = {0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < K / 64; ++ks)  // transposed: lane (rl, kg) holds row 16I + rl, columns 16J + 4kg + r
+        acc = lq_mfma_i8(*(const lq_v4i*)(kI + (16 * J + rl) * QS + 64 * ks + 16 * kg), *(const lq_v4i*)(qI + (16 * I + rl) * QS + 64 * ks + 16 * kg), acc);
+      const int i = 16 * I + rl, j0 = 16 * J + 4 * kg;
+      float x[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[r] = (float)acc[r] * sqk;
+        if (SCALAR) x[r] = x[r] * zoo_exp(gs_s[i] - gs_s[j0 + r]);
+        x[r] = j0 + r <= i ? x[r] : 0.0f;
+      }
+      *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(i, j0)) = lq_v2i{(int)zoo_pack_h2(x[0], x[1]), (int)zoo_pack_h2(x[2], x[3])};
+    }
+    // zero blocks above the diagonal (waves 4 .. 7, which have a task less) and the codes of q, operand by operand (waves 0 .. 3)
+    if (wave >= 4) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = wave - 4 + 4 * s;  // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
+        if (n >= 6) continue;
+        const int I = n < 3 ? 0 : (n < 5 ? 1 : 2), J = n < 3 ? n + 1 : (n < 5 ? n - 1 : 3);
+        *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(16 * I + rl, 16 * J + 4 * kg)) = lq_v2i{0, 0};
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < K / 64; ++ks)
+        *(lq_v4i*)(p.qc + cb * 64 * K + ((wave * (K / 64) + ks) * 64 + lane) * 16) = *(const lq_v4i*)(qI + (16 * wave + rl) * QS + 64 * ks + 16 * kg);
+    }
+  }
+  __syncthreads();  // raw keys, codes and transposed codes are dead
+
+  // ---- G, with the factors of its rows and columns; v transposed
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int n = wave + 8 * s;
+    if (n >= 10) continue;
+    const int j = 16 * blk_j(n) + rl;  // lane holds column j, rows i = 4kg + r of the block
+    const float bh = bh_s[j], gj = gs_s[j];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * blk_i(n) + 4 * kg + r;
+      float x = (bs_s[i] * bh) * gacc[s][r];
+      if (SCALAR) x = x * zoo_exp(gs_s[i] - gj);
+      G_s[i * kGS + j] = i > j ? x : 0.0f;
+    }
+  }
+  auto stage_v = [&]() {
+    if (vact) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        Xv[wn_xt(8 * vc8 + 2 * d, vrp)] = __builtin_amdgcn_perm((uint32_t)vraw[1][d], (uint32_t)vraw[0][d], 0x05040100u);
+        Xv[wn_xt(8 * vc8 + 2 * d + 1, vrp)] = __builtin_amdgcn_perm((uint32_t)vraw[1][d], (uint32_t)vraw[0][d], 0x07060302u);
+      }
+    }
+  };
+  stage_v();
+  __syncthreads();
+
+  // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w < 4, lane c < 16 holds column c of block w)
+  if (wave < 4 && lane < 16) {
+    const int o = 16 * wave;
+    float tc[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float a = (i == lane) ? 1.0f : 0.0f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) a = fmaf(-G_s[(o + i) * kGS + o + j], tc[j], a);
+      tc[i] = a;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) T_s[(o + i) * kGS + o + lane] = tc[i];
+  }
+  __syncthreads();
+  // block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes out of
+  // the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product), so the column stays in registers.
+  if (wave < 3) {
+    const int J = wave;
+    lq_v4f tcol[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) tcol[0][s] = T_s[(16 * J + 4 * kg + s) * kGS + 16 * J + rl];
+#pragma unroll
+    for (int di = 1; di < 4; ++di) {
+      const int I = J + di;
+      if (I > 3) break;
+      lq_v4f sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int dm = 0; dm < di; ++dm)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) sacc = wn_mfma_f32(G_s[(16 * I + rl) * kGS + 16 * (J + dm) + 4 * kg + s], tcol[dm][s], sacc);
+      lq_v4f tacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) tacc = wn_mfma_f32(T_s[(16 * I + rl) * kGS + 16 * I + 4 * kg + s], sacc[s], tacc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        tcol[di][r] = -tacc[r];
+        T_s[(16 * I + 4 * kg + r) * kGS + 16 * J + rl] = -tacc[r];
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- W and U: wave w takes row block I (w, or 7 - w: the two waves of a SIMD have the same work as any other two) and half of
+  // the column tiles of both
+  const int I = wave < 4 ? wave : 7 - wave, half = wave >> 2;
+  const int NST = (I >> 1) + 1;  // 32-token contraction steps that are not zero
+  TPieces<BF> tw[2], tu[2];  // (no decay: W and U share T . diag(bs), tu is not used)
+  float unw = 1.0f, unu = 1.0f;
+  {
+    float xw[2][8], xu[2][8];
+    float mw = 0.0f, mu = 0.0f;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      const int m0 = 32 * st + 8 * kg;
+      const bool live = m0 < 16 * (I + 1);  // blocks right of the diagonal were never written
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float t = live ? T_s[(16 * I + rl) * kGS + m0 + e] : 0.0f;
+        xw[st][e] = t * fW_s[m0 + e];
+        xu[st][e] = t * bs_s[m0 + e];
+        mw = fmaxf(mw, __builtin_fabsf(xw[st][e])), mu = fmaxf(mu, __builtin_fabsf(xu[st][e]));
+      }
+    }
+    if constexpr (!BF) {
+      // each row scaled so that its largest entry lies in [2^14, 2^15)
+      auto scale_of = [&](float m, float& un) {
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        const int e = min(max((int)(__float_as_uint(m) >> 23), 16), 252);  // largest entry 2^(e - 127) .. 2^(e - 126)
+        un = __uint_as_float((uint32_t)(e - 14) << 23);
+        return __uint_as_float((uint32_t)(268 - e) << 23);  // 2^(141 - e)
+      };
+      const float sw_ = scale_of(mw, unw);
+      float su_ = sw_;
+      if (SCALAR) su_ = scale_of(mu, unu); else unu = unw;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xw[st][e] = xw[st][e] * sw_, xu[st][e] = xu[st][e] * su_;
+    }
+    wn_split<BF>(xw[0], tw[0]), wn_split<BF>(xw[1], tw[1]);
+    if constexpr (SCALAR) wn_split<BF>(xu[0], tu[0]), wn_split<BF>(xu[1], tu[1]);
+  }
+  // D^T tile: lane (rl = token of block I, kg) gets columns 16nt + 4kg + r
+  auto tile = [&](const uint32_t* X, const TPieces<BF> (&t)[2], int nt) {
+    lq_v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      if (st >= NST) continue;  // (wave-uniform)
+      const lq_v4i x = *(const lq_v4i*)(X + wn_xt(16 * nt + rl, 16 * st + 4 * kg));
+#pragma unroll
+      for (int i = TPieces<BF>::NP - 1; i >= 0; --i) acc = wn_mfma<BF>(x, t[st].p[i], acc);
+    }
+    return acc;
+  };
+  const float inv_sw = CODES ? 1.0f / p.sw[h] : 0.0f;
+#pragma unroll
+  for (int q = 0; q < K / 32; ++q) {
+    const int nt = half * (K / 32) + q;
+    const lq_v4f a = tile(Xk, tw, nt);
+    lq_v2i o;
+    o[0] = (int)zoo_enc2(a[0] * unw, a[1] * unw, bf);
+    o[1] = (int)zoo_enc2(a[2] * unw, a[3] * unw, bf);
+    const int64_t woff = ((t0 + 16 * I + rl) * H + h) * K + 16 * nt + 4 * kg;
+    if (!SCAN && (!CODES || p.W)) *(lq_v2i*)(p.W + woff) = o;
+    if constexpr (CODES) {  // state-read codes of the rounded W
+      float w0, w1, w2, w3;
+      zoo_dec2((uint32_t)o[0], bf, w0, w1);
+      zoo_dec2((uint32_t)o[1], bf, w2, w3);
+      *(uint32_t*)(SCAN ? p.wq + cb * 64 * K + zoo_op_codes(16 * I + rl, 16 * nt + 4 * kg, K) : p.wq + woff) =
+          zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax), zoo_q8(w3, inv_sw, qmax));
+    }
+  }
+  for (int vb = 0; vb < V; vb += 128) {
+    if (vb > 0) {  // further passes of up to 128 value columns
+      __syncthreads();
+      const int rest = min(V - vb, 128) / 8;
+      if (vact && vc8 < rest) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * vrp + u) * H + h) * V + vb + 8 * vc8);
+        stage_v();
+      }
+      __syncthreads();
+    }
+    const int ntiles = min(V - vb, 128) / 32;  // column tiles per half
+    for (int q = 0; q < ntiles; ++q) {
+      const int nt = half * ntiles + q;
+      lq_v4f a;
+      if constexpr (SCALAR) a = tile(Xv, tu, nt); else a = tile(Xv, tw, nt);
+      lq_v2i o;
+      o[0] = (int)zoo_enc2(a[0] * unu, a[1] * unu, bf);
+      o[1] = (int)zoo_enc2(a[2] * unu, a[3] * unu, bf);
+      *(lq_v2i*)(SCAN ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vb + 16 * nt + 4 * kg)
+                      : p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
+    }
+  }
+}
+
+template <bool SCALAR, int K, bool BF>
+void launch_mode(const ZooWyParams& p, bool scan, dim3 grid, hipStream_t stream) {
+  if (scan)
+    hipLaunchKernelGGL((zoo_wy_ns_kernel<SCALAR, K, BF, MODE_SCAN>), grid, dim3(512), 0, stream, p);
+  else if (p.kqT)
+    hipLaunchKernelGGL((zoo_wy_ns_kernel<SCALAR, K, BF, MODE_CODES>), grid, dim3(512), 0, stream, p);
+  else
+    hipLaunchKernelGGL((zoo_wy_ns_kernel<SCALAR, K, BF, MODE_PLAIN>), grid, dim3(512), 0, stream, p);
+}
+
+template <bool SCALAR, int K>
+void launch_bf(const ZooWyParams& p, bool scan, dim3 grid, hipStream_t stream) {
+  if (p.bf) launch_mode<SCALAR, K, true>(p, scan, grid, stream); else launch_mode<SCALAR, K, false>(p, scan, grid, stream);
+}
+
+}  // namespace
+
+int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, dim3 grid, hipStream_t stream) {
+  if (scalar) {
+    if (K == 128) launch_bf<true, 128>(p, scan, grid, stream); else launch_bf<true, 64>(p, scan, grid, stream);
+  } else {
+    if (K == 128) launch_bf<false, 128>(p, scan, grid, stream); else launch_bf<false, 64>(p, scan, grid, stream);
+  }
+  return lq_check_launch();
+}

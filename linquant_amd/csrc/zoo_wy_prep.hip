@@ -1,6 +1,6 @@
-// WY / UT transform of the delta family, per chunk, in fp32.
-// Replaces the torch prep linquant/kernels/zoo/gated_delta_rule.py:20-47 (no / scalar decay) and
-// linquant/kernels/zoo/kda.py:22-53 (per-channel decay); the reference's default route through fla-core's
+// WY / UT transform of the delta family, per chunk, in fp32: per-channel decay (64-token chunks) and every decay kind for
+// 128-token chunks; no / scalar decay on 64-token chunks is zoo_wy_ns.hip.
+// Replaces the torch prep linquant/kernels/zoo/kda.py:22-53 (and, 128-token chunks, gated_delta_rule.py:20-47); the reference's default route through fla-core's
 // prep kernels for sigma = tau = 1 is served by the same native prep.
 //   L = beta^sigma k,  Hg = beta^(1-sigma) k
 //   G[i][j] = sum_n L[i][n] Hg[j][n] * decay(i,j,n)  for i > j, decay = 1 | exp(g_i - g_j) | exp(g_in - g_jn)
@@ -21,34 +21,7 @@
 
 namespace {
 
-struct WyParams {
-  const _Float16* k;
-  const _Float16* v;
-  const float* beta;
-  const float* g;
-  _Float16* Hw;
-  _Float16* W;
-  _Float16* U;
-  float* fw;
-  float sigma, tau;
-  int bf;
-  int B, T, H, V;
-  // write-operand codes of the state kernel, made here when kqT is set (otherwise lq_zoo_write_codes makes them from the
-  // stored Hw and W)
-  int8_t* kqT;
-  int8_t* wq;
-  float* ev;
-  float* gam;
-  const float* logenv;
-  const float* skw;
-  const float* sw;
-  float eta;
-  int qmax;
-  int NT;
-  const float* dk_div;  // (H,K) D_QK applied to k at load (k' = act(k / D)), with its reciprocal; or nullptr
-  const float* dk_rcp;
-  float* pack;  // fw | ev | gam per (batch, chunk, head), 64 + 64 + K floats, or nullptr
-};
+using WyParams = ZooWyParams;
 
 LQ_DEV float powb(float b, float e) {
   if (e == 0.0f) return 1.0f;
@@ -279,7 +252,7 @@ LQ_DEV void gram_rowblock(const WyParams& p, float* G_s, const float* bs_s, cons
 // rounded values, so the same bits): channel-major key write codes, token-major state-read codes of W, the per-token
 // value factor and the per-channel chunk decay.  W itself is then stored only when p.W is set.
 // SCAN (with CODES): wq and U leave in operand order (zoo_params.h), for zoo_scan.hip.
-template <int DECAY, int K, bool BF, bool CODES, bool DK, bool SCAN>
+template <int K, bool BF, bool CODES, bool DK, bool SCAN>
 __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
   constexpr int LS = 64 + 16;  // floats per row of the buffer that holds the Gram tile and then the X tiles
   static_assert(LS >= kGS, "the Gram tile lives in the X buffer until the inverse is done");
@@ -293,7 +266,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
   static_assert(2 * 64 * kOP <= 64 * kGS + 64 * LS, "the Gram operands live in the T / X buffers until G is written");
   float* Lg_s = lds_f;
   float* Hg_s = lds_f + 64 * kOP;
-  __shared__ float gs_s[DECAY == LQ_DECAY_SCALAR ? 64 : 1], bs_s[64], bh_s[64];
+  __shared__ float bs_s[64], bh_s[64];
   __shared__ float iskw_s[CODES ? K : 1], bw_s[CODES ? 64 : 1], el_s[CODES ? 64 : 1];
   // the last 1.5 KB of the big buffer lie beyond the Gram operands, the G / T tiles and the X tiles alike: the per-head
   // tables live there for the whole kernel (D_QK and its reciprocal, 128 floats each; the chunk's last decay row)
@@ -341,38 +314,26 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
     if constexpr (CODES) {
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + tid] = fwv;
     }
-    if (DECAY == LQ_DECAY_SCALAR) gs_s[tid] = p.g[(t0 + tid) * H + h];
   }
   if constexpr (CODES) {
     // per-token value factor and per-channel chunk decay, as lq_zoo_write_codes writes them
     if (tid < 64) {
-      float evv = 1.0f;
-      if (DECAY == LQ_DECAY_SCALAR) evv = zoo_exp(p.eta * (p.g[(t0 + 63) * H + h] - p.g[(t0 + tid) * H + h]));
-      if (DECAY == LQ_DECAY_DIAGONAL) evv = zoo_exp(p.eta * p.logenv[(t0 + tid) * H + h]);
+      const float evv = zoo_exp(p.eta * p.logenv[(t0 + tid) * H + h]);
       p.ev[(t0 + tid) * H + h] = evv;
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + 64 + tid] = evv;
     }
     if (tid < K) {
-      float gm = 1.0f, gl = 0.0f;
-      if (DECAY == LQ_DECAY_SCALAR) gm = zoo_exp(p.g[(t0 + 63) * H + h]);
-      if (DECAY == LQ_DECAY_DIAGONAL) {
-        gl = p.g[((t0 + 63) * H + h) * K + tid];
-        gm = zoo_exp(gl);
-      }
+      const float gl = p.g[((t0 + 63) * H + h) * K + tid], gm = zoo_exp(gl);
       p.gam[(((int64_t)b * p.NT + ct) * H + h) * K + tid] = gm;
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + 128 + tid] = gm;
-      if (DECAY == LQ_DECAY_DIAGONAL) glast_s[tid] = gl;
+      glast_s[tid] = gl;
       iskw_s[tid] = 1.0f / p.skw[h * K + tid];
     }
     if (tid >= 128 && tid < 192) {
-      // per token: the factor of Hw and the key-side factor of the write codes (scalar decay: exp((1-eta)(g_last - g_t));
-      // per-channel decay: eta * log envelope, subtracted in the exponent per element)
+      // per token: the factor of Hw and eta * log envelope, subtracted in the exponent of the write codes per element
       const int t = tid - 128;
       bw_s[t] = powb(p.beta[(t0 + t) * H + h], (1.0f - sigma) * tau);
-      float e = 1.0f;
-      if (DECAY == LQ_DECAY_SCALAR) e = zoo_exp((1.0f - p.eta) * (p.g[(t0 + 63) * H + h] - p.g[(t0 + t) * H + h]));
-      if (DECAY == LQ_DECAY_DIAGONAL) e = p.eta * p.logenv[(t0 + t) * H + h];
-      el_s[t] = e;
+      el_s[t] = p.eta * p.logenv[(t0 + t) * H + h];
     }
   }
   __syncthreads();
@@ -407,27 +368,16 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
         wy_dk8<BF, DK>(dk_s, 64 * ps + 8 * c8, kv);
         const float bs = bs_s[r], bh = bh_s[r];
         lq_v4f l0, l1, h0, h1;
-        lq_v4f g0 = {0.f, 0.f, 0.f, 0.f}, g1 = g0;
-        if (DECAY == LQ_DECAY_DIAGONAL) {
-          g0 = *(const lq_v4f*)(p.g + off), g1 = *(const lq_v4f*)(p.g + off + 4);
-          const lq_v4f a0 = *(const lq_v4f*)(p.g + arow + 64 * ps + 8 * c8), a1 = *(const lq_v4f*)(p.g + arow + 64 * ps + 8 * c8 + 4);
+        const lq_v4f g0 = *(const lq_v4f*)(p.g + off), g1 = *(const lq_v4f*)(p.g + off + 4);
+        const lq_v4f a0 = *(const lq_v4f*)(p.g + arow + 64 * ps + 8 * c8), a1 = *(const lq_v4f*)(p.g + arow + 64 * ps + 8 * c8 + 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float d0 = g0[e] - a0[e], d1 = g1[e] - a1[e];
-            spread = fmaxf(spread, fmaxf(__builtin_fabsf(d0), __builtin_fabsf(d1)));
-            l0[e] = (bs * kv[e]) * zoo_exp(d0);
-            l1[e] = (bs * kv[4 + e]) * zoo_exp(d1);
-            h0[e] = (bh * kv[e]) * zoo_exp(-d0);
-            h1[e] = (bh * kv[4 + e]) * zoo_exp(-d1);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            l0[e] = bs * kv[e];
-            l1[e] = bs * kv[4 + e];
-            h0[e] = bh * kv[e];
-            h1[e] = bh * kv[4 + e];
-          }
+        for (int e = 0; e < 4; ++e) {
+          const float d0 = g0[e] - a0[e], d1 = g1[e] - a1[e];
+          spread = fmaxf(spread, fmaxf(__builtin_fabsf(d0), __builtin_fabsf(d1)));
+          l0[e] = (bs * kv[e]) * zoo_exp(d0);
+          l1[e] = (bs * kv[4 + e]) * zoo_exp(d1);
+          h0[e] = (bh * kv[e]) * zoo_exp(-d0);
+          h1[e] = (bh * kv[4 + e]) * zoo_exp(-d1);
         }
         *(lq_v4f*)(Lg_s + r * kOP + 8 * c8) = l0;
         *(lq_v4f*)(Lg_s + r * kOP + 8 * c8 + 4) = l1;
@@ -435,7 +385,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
         *(lq_v4f*)(Hg_s + r * kOP + 8 * c8 + 4) = h1;
         if constexpr (CODES) {
           // Hw = beta^((1-sigma) tau) k rounded to the activation dtype, stored; its write codes
-          // q8(Hw * fk, 1 / skw), fk = 1 | exp((1-eta)(g_last - g_t)) | exp(gk_last - gk_t - eta * le_t), go out
+          // q8(Hw * fk, 1 / skw), fk = exp(gk_last - gk_t - eta * le_t), go out
           // channel-major: the four lanes that hold tokens 4Q .. 4Q+3 of these eight channels (eight lanes apart)
           // exchange codes so that lane j of them owns channels 2j, 2j+1 of all four tokens, one dword each
           const float bw = bw_s[r], el = el_s[r];
@@ -445,20 +395,16 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
           *(lq_v4i*)(p.Hw + off) = o;
           const int n8 = 64 * ps + 8 * c8;
           const lq_v4f is0 = *(const lq_v4f*)(iskw_s + n8), is1 = *(const lq_v4f*)(iskw_s + n8 + 4);
-          lq_v4f gl0 = {0.f, 0.f, 0.f, 0.f}, gl1 = gl0;
-          if (DECAY == LQ_DECAY_DIAGONAL) gl0 = *(const lq_v4f*)(glast_s + n8), gl1 = *(const lq_v4f*)(glast_s + n8 + 4);
+          const lq_v4f gl0 = *(const lq_v4f*)(glast_s + n8), gl1 = *(const lq_v4f*)(glast_s + n8 + 4);
           int kc8[8];
 #pragma unroll
           for (int d = 0; d < 4; ++d) {
             float x0, x1;
             zoo_dec2((uint32_t)o[d], bf, x0, x1);
-            if (DECAY == LQ_DECAY_SCALAR) x0 = x0 * el, x1 = x1 * el;
-            if (DECAY == LQ_DECAY_DIAGONAL) {
-              const float ga = d < 2 ? g0[(2 * d) & 3] : g1[(2 * d) & 3], gb = d < 2 ? g0[(2 * d + 1) & 3] : g1[(2 * d + 1) & 3];
-              const float la = d < 2 ? gl0[(2 * d) & 3] : gl1[(2 * d) & 3], lb = d < 2 ? gl0[(2 * d + 1) & 3] : gl1[(2 * d + 1) & 3];
-              x0 = x0 * zoo_exp(la - ga - el);
-              x1 = x1 * zoo_exp(lb - gb - el);
-            }
+            const float ga = d < 2 ? g0[(2 * d) & 3] : g1[(2 * d) & 3], gb = d < 2 ? g0[(2 * d + 1) & 3] : g1[(2 * d + 1) & 3];
+            const float la = d < 2 ? gl0[(2 * d) & 3] : gl1[(2 * d) & 3], lb = d < 2 ? gl0[(2 * d + 1) & 3] : gl1[(2 * d + 1) & 3];
+            x0 = x0 * zoo_exp(la - ga - el);
+            x1 = x1 * zoo_exp(lb - gb - el);
             const float ia = d < 2 ? is0[(2 * d) & 3] : is1[(2 * d) & 3], ib = d < 2 ? is0[(2 * d + 1) & 3] : is1[(2 * d + 1) & 3];
             kc8[2 * d] = zoo_q8(x0, ia, p.qmax), kc8[2 * d + 1] = zoo_q8(x1, ib, p.qmax);
           }
@@ -497,9 +443,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
         }
       }
     }
-    bool one_anchor = true;
-    if (DECAY == LQ_DECAY_DIAGONAL) one_anchor = __syncthreads_or(spread > 40.0f) == 0;
-    else __syncthreads();
+    const bool one_anchor = __syncthreads_or(spread > 40.0f) == 0;
     // the operand buffers are dead: G overlays them
     if (one_anchor) {
       // lane holds column j = rl of block J, rows i = 4kg + r of block I
@@ -509,16 +453,11 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = 16 * blk_i(q) + 4 * kg + r, j = 16 * blk_j(q) + rl;
-          float v = 0.0f;
-          if (i > j) {
-            v = acc[q][r];
-            if (DECAY == LQ_DECAY_SCALAR) v = v * zoo_exp(gs_s[i] - gs_s[j]);
-          }
-          G_s[i * kGS + j] = v;
+          G_s[i * kGS + j] = i > j ? acc[q][r] : 0.0f;
         }
       }
     } else {
-      gram_rowblock<DECAY, K, BF, DK>(p, G_s, bs_s, bh_s, gs_s, wave, rl, kg, t0, h, dk_s);
+      gram_rowblock<LQ_DECAY_DIAGONAL, K, BF, DK>(p, G_s, bs_s, bh_s, nullptr, wave, rl, kg, t0, h, dk_s);
     }
   }
   __syncthreads();
@@ -594,17 +533,15 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
     for (int u = 0; u < 2; ++u) {
       const int64_t off = ((tok0 + u) * H + h) * K + kc + 8 * c8;
       kraw[u] = *(const lq_v4i*)(p.k + off);
-      if (DECAY == LQ_DECAY_DIAGONAL) graw[u][0] = *(const lq_v4f*)(p.g + off), graw[u][1] = *(const lq_v4f*)(p.g + off + 4);
+      graw[u][0] = *(const lq_v4f*)(p.g + off), graw[u][1] = *(const lq_v4f*)(p.g + off + 4);
     }
   };
   auto request_v = [&](int vc) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((tok0 + u) * H + h) * V + vc + 8 * c8);
   };
-  // (per-channel decay: its kernel sits at the register limit of four waves per SIMD, and holding a pass of k and g
-  // across the products spilled: 272 -> 316 us; it requests at the point of use)
-  constexpr bool kAhead = DECAY != LQ_DECAY_DIAGONAL;
-  if (kAhead) request_k(0);
+  // (k and g of a pass are requested at the point of use: the kernel sits at the register limit of four waves per SIMD, and
+  // holding a pass of them across the products spilled: 272 -> 316 us)
   float inv_sw = 0.0f;
   if constexpr (CODES) inv_sw = 1.0f / p.sw[h];
 
@@ -612,7 +549,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
 #pragma unroll
   for (int kc = 0; kc < K; kc += 64) {
     if (kc > 0) __syncthreads();
-    if (!kAhead) request_k(kc);
+    request_k(kc);
     if constexpr (CODES) {
       // Hw and its codes were written while the Gram operands were staged: only X is formed here, two channels at a time
       // for both tokens of the thread (a token pair is one dword of the transposed tile), so that few values are live
@@ -620,7 +557,6 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         bl[u] = bs_s[2 * rp + u];
-        if (DECAY == LQ_DECAY_SCALAR) bl[u] = bl[u] * zoo_exp(gs_s[2 * rp + u]);
       }
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
@@ -635,12 +571,8 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
             k0 = zoo_round_act(zoo_div_rn(k0, dd[0], rr[0]), BF);
             k1 = zoo_round_act(zoo_div_rn(k1, dd[1], rr[1]), BF);
           }
-          float x0 = bl[u] * k0, x1 = bl[u] * k1;
-          if (DECAY == LQ_DECAY_DIAGONAL) {
-            x0 = x0 * zoo_exp(graw[u][d >> 1][(2 * d) & 3]);
-            x1 = x1 * zoo_exp(graw[u][d >> 1][(2 * d + 1) & 3]);
-          }
-          x[u][0] = x0, x[u][1] = x1;
+          x[u][0] = (bl[u] * k0) * zoo_exp(graw[u][d >> 1][(2 * d) & 3]);
+          x[u][1] = (bl[u] * k1) * zoo_exp(graw[u][d >> 1][(2 * d + 1) & 3]);
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -657,20 +589,15 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
       for (int u = 0; u < 2; ++u) {
         const int64_t off = ((tok0 + u) * H + h) * K + kc + 8 * c8;
         const float bw = powb(btr[u], (1.0f - sigma) * tau);
-        float bl = bs_s[2 * rp + u];
-        if (DECAY == LQ_DECAY_SCALAR) bl = bl * zoo_exp(gs_s[2 * rp + u]);
+        const float bl = bs_s[2 * rp + u];
         float hw[8], kk[8];
 #pragma unroll
         for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)kraw[u][d], bf, kk[2 * d], kk[2 * d + 1]);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           const float k0 = kk[2 * d], k1 = kk[2 * d + 1];
-          float x0 = bl * k0, x1 = bl * k1;
-          if (DECAY == LQ_DECAY_DIAGONAL) {
-            x0 = x0 * zoo_exp(graw[u][d >> 1][(2 * d) & 3]);
-            x1 = x1 * zoo_exp(graw[u][d >> 1][(2 * d + 1) & 3]);
-          }
-          xr[u][2 * d] = x0, xr[u][2 * d + 1] = x1;
+          xr[u][2 * d] = (bl * k0) * zoo_exp(graw[u][d >> 1][(2 * d) & 3]);
+          xr[u][2 * d + 1] = (bl * k1) * zoo_exp(graw[u][d >> 1][(2 * d + 1) & 3]);
           hw[2 * d] = bw * k0, hw[2 * d + 1] = bw * k1;
         }
         lq_v4i o;
@@ -681,11 +608,6 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
       stage(xr[0], xr[1]);
     }
     __syncthreads();
-    if (kc + 64 < K) {
-      if (kAhead) request_k(kc + 64);
-    } else if (kAhead) {
-      request_v(0);
-    }
     // W = T . X for these 64 columns
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
@@ -711,7 +633,7 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
   // ---- U = T . (beta^sigma v)
   for (int vc = 0; vc < V; vc += 64) {
     __syncthreads();
-    if (!kAhead) request_v(vc);
+    request_v(vc);
     {
       float xr[2][8];
 #pragma unroll
@@ -727,7 +649,6 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
       stage(xr[0], xr[1]);
     }
     __syncthreads();
-    if (kAhead) request_v(min(vc + 64, V - 64));  // unconditional: the last pass requests its own columns once more
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       const int u = nt < 2 ? 0 : 1;
@@ -920,41 +841,33 @@ int launch128_decay(const WyParams& p, int decay, hipStream_t stream) {
   return LQ_ERR_SHAPE;
 }
 
-template <int DECAY, int K, bool CODES, bool DK, bool SCAN = false>
+template <int K, bool CODES, bool DK, bool SCAN = false>
 int launch_c(const WyParams& p, dim3 grid, hipStream_t stream) {
   if (p.bf)
-    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, true, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((zoo_wy_prep_kernel<K, true, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((zoo_wy_prep_kernel<DECAY, K, false, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((zoo_wy_prep_kernel<K, false, CODES, DK, SCAN>), grid, dim3(256), 0, stream, p);
   return lq_check_launch();
 }
 
-template <int DECAY, int K>
-int launch(const WyParams& p, bool scan, dim3 grid, hipStream_t stream) {
-  if constexpr (DECAY == LQ_DECAY_DIAGONAL) {
-    if (scan) return p.dk_div ? launch_c<DECAY, K, true, true, true>(p, grid, stream) : launch_c<DECAY, K, true, false, true>(p, grid, stream);
-  }
-  if (p.dk_div) return launch_c<DECAY, K, true, true>(p, grid, stream);  // the rescaling comes with the codes (checked)
-  return p.kqT ? launch_c<DECAY, K, true, false>(p, grid, stream) : launch_c<DECAY, K, false, false>(p, grid, stream);
-}
-
 template <int K>
-int launch_decay(const WyParams& p, int decay, bool scan, dim3 grid, hipStream_t stream) {
-  switch (decay) {
-    case LQ_DECAY_NONE: return launch<LQ_DECAY_NONE, K>(p, scan, grid, stream);
-    case LQ_DECAY_SCALAR: return launch<LQ_DECAY_SCALAR, K>(p, scan, grid, stream);
-    case LQ_DECAY_DIAGONAL: return launch<LQ_DECAY_DIAGONAL, K>(p, scan, grid, stream);
-  }
-  return LQ_ERR_SHAPE;
+int launch(const WyParams& p, bool scan, dim3 grid, hipStream_t stream) {
+  if (scan) return p.dk_div ? launch_c<K, true, true, true>(p, grid, stream) : launch_c<K, true, false, true>(p, grid, stream);
+  if (p.dk_div) return launch_c<K, true, true>(p, grid, stream);  // the rescaling comes with the codes (checked)
+  return p.kqT ? launch_c<K, true, false>(p, grid, stream) : launch_c<K, false, false>(p, grid, stream);
 }
 
 }  // namespace
 
-int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stream) {
-  if (!a || !a->k || !a->v || !a->beta || !a->Hw || !a->U || !a->fw) return LQ_ERR_NULL;
+int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, const ZooWyLocal* local, hipStream_t stream) {
+  const bool no_hw = scan && local;  // Hw itself is not wanted
+  if (!a || !a->k || !a->v || !a->beta || (!a->Hw && !no_hw) || !a->U || !a->fw) return LQ_ERR_NULL;
   if (a->decay != LQ_DECAY_NONE && !a->g) return LQ_ERR_NULL;
   const bool codes = a->kqT != nullptr;
-  if (scan && (!codes || a->decay != LQ_DECAY_DIAGONAL)) return LQ_ERR_SHAPE;
+  if (scan && (!codes || !a->pack || (local != nullptr) != (a->decay != LQ_DECAY_DIAGONAL))) return LQ_ERR_SHAPE;
+  if (local && (!local->q || !local->qc || !local->A || !local->sq || !local->sk || (a->decay == LQ_DECAY_SCALAR && !local->gpk)))
+    return LQ_ERR_NULL;
+  if (local && !zoo_al(local->q, 16)) return LQ_ERR_SHAPE;
   if (!codes && !a->W) return LQ_ERR_NULL;
   if (codes && (!a->wq || !a->ev || !a->gam || !a->skw || !a->sw)) return LQ_ERR_NULL;
   if (codes && a->decay == LQ_DECAY_DIAGONAL && !a->logenv) return LQ_ERR_NULL;
@@ -971,7 +884,8 @@ int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stre
   if ((a->chunk_size != 64 && !big) || a->seqlen % a->chunk_size != 0) return LQ_ERR_SHAPE;
   if ((a->kdim != 64 && a->kdim != 128) || a->vdim % 64 != 0 || a->vdim <= 0) return LQ_ERR_SHAPE;
   if (a->act_dtype != LQ_DT_F16 && a->act_dtype != LQ_DT_BF16) return LQ_ERR_SHAPE;
-  if (!zoo_al(a->k, 16) || !zoo_al(a->v, 16) || !zoo_al(a->Hw, 16)) return LQ_ERR_SHAPE;
+  if (a->decay < LQ_DECAY_NONE || a->decay > LQ_DECAY_DIAGONAL) return LQ_ERR_SHAPE;
+  if (!zoo_al(a->k, 16) || !zoo_al(a->v, 16) || (!no_hw && !zoo_al(a->Hw, 16))) return LQ_ERR_SHAPE;
   if (a->decay == LQ_DECAY_DIAGONAL && !zoo_al(a->g, 16)) return LQ_ERR_SHAPE;
   if ((int64_t)a->batch * a->nheads > 65535) return LQ_ERR_SHAPE;
   WyParams p = {};
@@ -983,10 +897,15 @@ int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, hipStream_t stre
   p.eta = a->eta, p.qmax = a->qmax, p.NT = a->seqlen / 64;
   p.dk_div = a->dk_div, p.dk_rcp = a->dk_rcp;
   p.pack = a->pack;
+  if (local) {
+    p.q = (const _Float16*)local->q, p.qc = local->qc, p.A = (_Float16*)local->A, p.gpk = local->gpk;
+    p.sq = local->sq, p.sk = local->sk, p.scale = local->scale;
+  }
   if ((int64_t)(a->seqlen / 64) * a->batch * a->nheads > 0x7fffffff) return LQ_ERR_SHAPE;
   if (big) return a->kdim == 128 ? launch128_decay<128>(p, a->decay, stream) : launch128_decay<64>(p, a->decay, stream);
   dim3 grid((uint32_t)((a->seqlen / 64) * a->batch * a->nheads));
-  return a->kdim == 128 ? launch_decay<128>(p, a->decay, scan, grid, stream) : launch_decay<64>(p, a->decay, scan, grid, stream);
+  if (a->decay != LQ_DECAY_DIAGONAL) return zoo_wy_ns_launch(p, a->decay == LQ_DECAY_SCALAR, a->kdim, scan, grid, stream);
+  return a->kdim == 128 ? launch<128>(p, scan, grid, stream) : launch<64>(p, scan, grid, stream);
 }
 
-extern "C" int lq_zoo_wy_prep(const lq_zoo_wy_prep_args* a, hipStream_t stream) { return zoo_wy_prep_launch(a, false, stream); }
+extern "C" int lq_zoo_wy_prep(const lq_zoo_wy_prep_args* a, hipStream_t stream) { return zoo_wy_prep_launch(a, false, nullptr, stream); }
