@@ -17,7 +17,7 @@
 // chunk's local product and store follow after that one.
 //
 // Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 64 us, KDA B2 T8192 H32 157 +
-// 128 -> 135 us, KDA B1 T2048 H8 41 + 7 -> 36 us.  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
+// 128 -> 135 us, KDA B1 T2048 H8 41 + 7 -> 36 us (25 with 16 columns).  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
 // carry, 300 to issue its requests, 1000 for state read and E, 300 for the update; one workgroup of 32 columns per compute unit
 // at the first two shapes.
 //
@@ -34,22 +34,24 @@ namespace {
 
 using ScanParams = ZooScanParams;
 
-constexpr int BV = 32;  // value columns per workgroup
-
-template <bool DELTA, int K>
+// BV: value columns per workgroup.  32, and 16 where 32 would leave half of the 256 compute units or more without a workgroup: a
+// step is bound by the vector instructions of the two waves of a SIMD, and half the columns are little more than half of them
+// (32 -> 16 columns: no / scalar decay B1 T2048 H8 K = V = 64 21.4 -> 15.9 us, KDA B1 T2048 H8 K = V = 128 36.7 -> 25.2 us).  From
+// more than half of the compute units on, a second workgroup of 16 columns would only repeat what does not depend on the columns.
+template <bool DELTA, int K, int BV>
 struct ChainOps {
   lq_v4i kop[K / 64];                 // key write codes: rows of this wave, 16 token slots of the lane's group
   lq_v4i vop[DELTA ? 1 : BV / 16];    // linear: value write codes
   lq_v4i wop[DELTA ? K / 64 : 1];     // delta: state-read codes of token 16*wave + (lane & 15)
-  lq_v4i uraw;                        // delta: U of token 16*wave + (lane >> 2), columns 8 * (lane & 3) .. + 7
+  typename std::conditional<BV == 32, lq_v4i, lq_v2i>::type uraw;  // delta: U of token 16*wave + (lane >> 2), a quarter of the columns
   float misc;                         // lanes 0..15 fw, 16..31 ev of the wave's tokens (delta), 32.. decay of the carry rows
 };
 
-template <bool DELTA, bool SCALAR, int K>
+template <bool DELTA, bool SCALAR, int K, int BV>
 struct OutOps {
   lq_v4i qop[K / 64];                     // codes of q: token 16*w + (lane & 15)
   lq_v4i aop[2];                          // A (fp16): the same token, columns 32 js + 8 kg ..
-  lq_v4i vop[DELTA ? 1 : BV / 16];        // linear: local value codes of column NJ rl + jj, tokens 8 kg .. and 32 + 8 kg ..
+  lq_v4i vop[DELTA ? 1 : BV / 16];        // linear: local value codes of column NJ rl + jj (NJ = BV / 16), tokens 8 kg .. and 32 + 8 kg ..
   lq_v4f g;                               // scalar decay: cumulative log decay of tokens 16*w + 4 kg ..
 };
 
@@ -78,7 +80,7 @@ LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
 // compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
 constexpr int scan_sets(bool delta) { return delta ? 3 : 5; }
 
-template <bool DELTA, bool SCALAR, int K, bool BF, bool OF32>
+template <bool DELTA, bool SCALAR, int K, int BV, bool BF, bool OF32>
 __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
   constexpr int D = scan_sets(DELTA);
   constexpr int KR = K / 4;        // carry rows per chain wave
@@ -140,7 +142,8 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
         inv_ew_d[jj] = 1.0f / p.svw[h * V + v0 + NJ * rl + jj];
       }
     }
-    using Ops = ChainOps<DELTA, K>;
+    using Ops = ChainOps<DELTA, K, BV>;
+    using URaw = decltype(Ops::uraw);
     // part: 0 = everything, 1 = key codes, decays and per-token factors, 2 = state-read codes and U
     auto load_part = [&](auto part_c, int ct, Ops& o) __attribute__((always_inline)) {
       constexpr int part = decltype(part_c)::value;
@@ -162,7 +165,7 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
 #pragma unroll
         for (int ks = 0; ks < K / 64; ++ks)
           o.wop[ks] = *(const lq_v4i*)(p.wq + cb * 64 * K + ((wave * (K / 64) + ks) * 64 + lane) * 16);
-        o.uraw = *(const lq_v4i*)(p.u + cb * 64 * V + 64 * v0 + (wave * 64 + lane) * 8);  // token lane >> 2, a quarter of the columns
+        o.uraw = *(const URaw*)(p.u + cb * 64 * V + zoo_op_U(16 * wave + (lane >> 2), v0 + BV / 4 * (lane & 3)));
       }
     };
     float hc[KT][VT][4];
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
       unsigned char* hTb = hT + (DELTA ? 0 : (ct & 1) * BV * HS);
       misc_s[lane] = cur.misc;
       if constexpr (DELTA) {
-        *(lq_v4i*)(ue_s + (lane >> 2) * US + 16 * (lane & 3)) = cur.uraw;
+        *(URaw*)(ue_s + (lane >> 2) * US + BV / 2 * (lane & 3)) = cur.uraw;
       }
       // stored copy of the incoming state -> LDS (V-major)
 #pragma unroll
@@ -217,7 +220,8 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const unsigned char* cell = ue_s + (4 * kg + r) * US + 2 * NJ * rl;
-          const uint32_t uw = *(const uint32_t*)cell;
+          uint32_t uw;
+          if constexpr (NJ == 2) uw = *(const uint32_t*)cell; else uw = *(const uint16_t*)cell;
 #pragma unroll
           for (int jj = 0; jj < NJ; ++jj) {
             float ws = (float)aw[jj][r] * sw;
@@ -294,8 +298,8 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
     float ss_o[NJ], svl_o[NJ], inv_el = 0.0f;
 #pragma unroll
     for (int jj = 0; jj < NJ; ++jj) ss_o[jj] = p.ss[h * V + v0 + NJ * rl + jj], svl_o[jj] = p.svl[h * V + v0 + NJ * rl + jj];
-    if constexpr (DELTA) inv_el = 1.0f / p.svl[h * V + v0 + (ot >> 3)];  // E -> local codes: this thread's column
-    using Ops = OutOps<DELTA, SCALAR, K>;
+    if constexpr (DELTA) inv_el = 1.0f / p.svl[h * V + v0 + ot / (256 / BV)];  // E -> local codes: this thread's column
+    using Ops = OutOps<DELTA, SCALAR, K, BV>;
     auto load = [&](int ct, Ops& o) __attribute__((always_inline)) {
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
 #pragma unroll
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
       for (int js = 0; js < 2; ++js) o.aop[js] = *(const lq_v4i*)(p.A + cb * 4096 + ((w * 2 + js) * 64 + lane) * 8);
       if constexpr (!DELTA) {
 #pragma unroll
-        for (int jj = 0; jj < NJ; ++jj) o.vop[jj] = *(const lq_v4i*)(p.vcT + cb * 64 * V + 64 * v0 + (jj * 64 + lane) * 16);
+        for (int jj = 0; jj < NJ; ++jj) o.vop[jj] = *(const lq_v4i*)(p.vcT + cb * 64 * V + zoo_op_values(v0 + NJ * rl + jj, 8 * kg));
       }
       if constexpr (SCALAR) o.g = *(const lq_v4f*)(p.gpk + cb * 64 + 16 * w + 4 * kg);
     };
@@ -360,25 +364,26 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
         for (int jj = 0; jj < NJ; ++jj) res[jj] = of[jj][r] + loc[jj][r] * svl_o[jj];
         if constexpr (OF32) {
           float* op = (float*)p.o + off;
-          *(lq_v2i*)op = lq_v2i{__float_as_int(res[0]), __float_as_int(res[1])};
+          if constexpr (NJ == 2) *(lq_v2i*)op = lq_v2i{__float_as_int(res[0]), __float_as_int(res[1])}; else *op = res[0];
         } else {
           _Float16* op = (_Float16*)p.o + off;
-          *(uint32_t*)op = zoo_enc2(res[0], res[1], bf);
+          if constexpr (NJ == 2) *(uint32_t*)op = zoo_enc2(res[0], res[1], bf); else *(uint16_t*)op = zoo_enc1(res[0], bf);
         }
       }
     };
-    // E of the chunk the chain has just formed -> its local codes (fp16), eight tokens of a column per thread
+    // E of the chunk the chain has just formed -> its local codes (fp16), BV / 4 tokens of a column per thread
     auto convert = [&]() __attribute__((always_inline)) {
-      const int col = ot >> 3;
-      const lq_v4i raw = *(const lq_v4i*)(eB + col * LS + 16 * (ot & 7));
-      lq_v4i o;
+      using Raw = typename std::conditional<BV == 32, lq_v4i, lq_v2i>::type;
+      const int at = ot / (256 / BV) * LS + BV / 2 * (ot % (256 / BV));
+      const Raw raw = *(const Raw*)(eB + at);
+      Raw o;
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
+      for (int d = 0; d < BV / 8; ++d) {
         float e0, e1;
         zoo_dec2((uint32_t)raw[d], bf, e0, e1);
         o[d] = (int)zoo_pack_h2((float)zoo_q8(e0, inv_el, qmax), (float)zoo_q8(e1, inv_el, qmax));
       }
-      *(lq_v4i*)(eL + col * LS + 16 * (ot & 7)) = o;
+      *(Raw*)(eL + at) = o;
     };
     // One step: `cur` holds chunk ct, `prev` chunk ct - 1, into which chunk ct + D - 1 is requested once its last use is past.
     auto do_step = [&](auto first_c, int ct, Ops& cur, Ops& prev) __attribute__((always_inline)) {
@@ -416,23 +421,29 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
   }
 }
 
-template <bool DELTA, bool SCALAR, int K>
+template <bool DELTA, bool SCALAR, int K, int BV>
 int launch(const ScanParams& p, int B, hipStream_t stream) {
   const dim3 grid(p.V / BV, B * p.H), block(512);
   if (DELTA && p.o_is_f32 && p.bf)  // (the linear family reads codes only: the activation dtype is that of the output)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, DELTA, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, DELTA, true>), grid, block, 0, stream, p);
   else if (p.o_is_f32)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, false, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, true>), grid, block, 0, stream, p);
   else if (p.bf)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, true, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, true, false>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, false>), grid, block, 0, stream, p);
   return lq_check_launch();
+}
+
+template <bool DELTA, bool SCALAR, int K>
+int launch_bv(const ScanParams& p, int B, hipStream_t stream) {
+  const bool few = (int64_t)B * p.H * (p.V / 32) <= 128;
+  return few ? launch<DELTA, SCALAR, K, 16>(p, B, stream) : launch<DELTA, SCALAR, K, 32>(p, B, stream);
 }
 
 template <bool DELTA, bool SCALAR>
 int launch_k(const ScanParams& p, int K, int B, hipStream_t stream) {
-  return K == 128 ? launch<DELTA, SCALAR, 128>(p, B, stream) : launch<DELTA, SCALAR, 64>(p, B, stream);
+  return K == 128 ? launch_bv<DELTA, SCALAR, 128>(p, B, stream) : launch_bv<DELTA, SCALAR, 64>(p, B, stream);
 }
 
 }  // namespace
