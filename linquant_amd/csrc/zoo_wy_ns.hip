@@ -39,7 +39,10 @@ LQ_DEV lq_v4f wn_mfma(lq_v4i a, lq_v4i b, lq_v4f c) {
 
 constexpr int kGS = 70;   // floats per row of the G / T tiles: an A-operand read (16 rows, 4 adjacent slots) takes one LDS pass at 2 mod 4
 constexpr int kXP = 36;   // dwords per column of the transposed tiles (32 token pairs + pad)
-constexpr int kCS = 80;   // bytes per channel row of the transposed write codes (64 tokens + pad)
+// byte of the transposed write codes [channel][64 tokens]: 16 bytes of pad after every eight channels, so that the 16 channel
+// groups of a wave's writes fall on different banks (rows of 80 bytes put them on two: Gated DeltaNet B4 T4096 H16 260 -> 256 us,
+// DeltaNet B8 T2048 H8 bf16 101 -> 99 for the whole call)
+LQ_DEV int wn_ct(int ch, int token) { return ch * 64 + (ch >> 3) * 16 + token; }
 
 // dword of the transposed tile [column][token pair]; the pairs are permuted in groups of four (one 16-byte operand piece) so that
 // the writes of a wave (16 groups of eight columns x 4 pairs) fall on 64 different banks
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   constexpr int QS = K == 128 ? 160 : 80;         // bytes per row of the code tiles
   constexpr int kR1 = 64 * FS * 2 > 64 * kGS * 4 ? 64 * FS * 2 : 64 * kGS * 4;            // raw keys, then T
   constexpr int kR2 = 2 * 64 * QS > 128 * kXP * 4 ? 2 * 64 * QS : 128 * kXP * 4;          // codes of q and k, then transposed v
-  constexpr int kR3 = K * kCS > 64 * kGS * 4 ? K * kCS : 64 * kGS * 4;                    // transposed write codes, then G
+  constexpr int kR3 = K * 66 > 64 * kGS * 4 ? K * 66 : 64 * kGS * 4;                    // transposed write codes, then G
   constexpr int kR4 = K * kXP * 4;                                                       // transposed keys
   __shared__ __align__(16) unsigned char lds[kR1 + kR2 + kR3 + kR4];
   _Float16* kF = (_Float16*)lds;
@@ -227,14 +230,14 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
     if constexpr (CODES) {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        *(uint16_t*)(cT + (8 * kc + e) * kCS + 2 * krp) = (uint16_t)__builtin_amdgcn_perm(wc[1][e], wc[0][e], 0x0c0c0400u);
+        *(uint16_t*)(cT + wn_ct(8 * kc + e, 2 * krp)) = (uint16_t)__builtin_amdgcn_perm(wc[1][e], wc[0][e], 0x0c0c0400u);
     }
   }
   __syncthreads();
 
   // ---- the write codes leave as whole rows
   if constexpr (CODES) {
-    if (tid < K * 4) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(cT + (tid >> 2) * kCS + 16 * (tid & 3));
+    if (tid < K * 4) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(cT + wn_ct(tid >> 2, 16 * (tid & 3)));
   }
   // ---- Gram blocks (tasks 0..9) and, MODE_SCAN, A blocks (tasks 10..19): task t belongs to wave t % 8
   // block n of the lower triangle: (0,0) (1,0) (1,1) (2,0) (2,1) (2,2) (3,0) ..
