@@ -441,10 +441,9 @@ typedef struct {
 int lq_zoo_output(const lq_zoo_output_args* args, hipStream_t stream);
 
 /* replaces chunk_simple_gla_int8 as a whole (linquant/kernels/zoo/simple_gla.py:175-212; rotated storage, raw operands):
- * lq_zoo_cumsum (scalar decay only), lq_zoo_write_codes, lq_zoo_state and lq_zoo_output launched back to back on `stream`
- * over one caller-supplied workspace that holds the intermediates (cumulative decay, write codes, per-token factors, stored
- * states, and for chunk sizes above 64 the cross workspace).  Same kernels and bits as the four calls; one foreign call and
- * one allocation per forward, which is what bounds small shapes.  Field meanings as in the per-stage structs. */
+ * what lq_zoo_cumsum (scalar decay only), lq_zoo_write_codes, lq_zoo_state and lq_zoo_output make one after the other, on
+ * `stream` over one caller-supplied workspace that holds the intermediates; the bits of the four calls.  64-token chunks run
+ * as an operand pre-pass and one launch for recurrence and output.  Field meanings as in the per-stage structs. */
 typedef struct {
   const void* q;             /* (B,T,H,K) fp16/bf16 */
   const void* k;             /* (B,T,H,K) */
@@ -466,6 +465,11 @@ typedef struct {
   void* workspace;           /* device memory, 256-byte aligned, lq_zoo_simple_gla_workspace_bytes() bytes; contents undefined
                                 on entry and on return */
   int64_t workspace_bytes;
+  /* Optional, each NULL or set (64-token chunks): q, k, v are rotated and rescaled as they are loaded, as lq_zoo_rotate_quant does */
+  const float* signs_qk;     /* (K,) column signs of R_QK, 16-byte aligned */
+  const float* signs_v;      /* (V,) column signs of R_V, 16-byte aligned (V in {64,128}) */
+  const float* dq;           /* (H,K) D_QK: q is multiplied by it, k divided; with dq_rcp */
+  const float* dq_rcp;       /* (H,K) RN(1 / dq) */
 } lq_zoo_simple_gla_args;
 int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* args, hipStream_t stream);
 /* workspace size for the dims in `args` (pointers are not read), written to *bytes */

@@ -1,10 +1,10 @@
 // One call for the whole no / scalar decay chunk forward: chunk_simple_gla_int8 (linquant/kernels/zoo/simple_gla.py:175-212)
-// as one C entry.  The four stages -- cumsum (scalar decay only), write-operand pre-pass, state recurrence, output -- are
-// the stand-alone entry points, launched back to back on the caller's stream over one caller-supplied workspace that holds
-// what the Python wrapper would otherwise allocate per call (cumulative decay, write codes, per-token factors, stored
-// states).  Same kernels, same arguments, same bits; what it saves is the host: one foreign call and one allocation per
-// forward instead of four calls and nine allocations, which is what bounds small shapes (B1 T2048 H8: the kernels take
-// 30 us, issuing them from Python 50).
+// as one C entry over one caller-supplied workspace that holds what the Python wrapper would otherwise allocate per call.
+// 64-token chunks: two launches, the operand pre-pass (zoo_lin_prep.hip; with it the operand rotations, if asked for) and recurrence
+// with output (zoo_scan.hip).  Longer chunks: the four stand-alone stages (cumsum, write-operand pre-pass, state recurrence,
+// output) back to back.  The bits of the stage entry points in either case.
+#include <initializer_list>
+
 #include "zoo_params.h"
 
 namespace {
@@ -13,8 +13,20 @@ constexpr int64_t kAlign = 256;
 int64_t up(int64_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
-  int64_t gc, kqT, vqT, ev, gam, h_i8, cross, total;
+  int64_t gc, kqT, vqT, vcT, qc, A, gpk, ev, gam, h_i8, cross, total;
 };
+
+// What the launches over 64-token chunks (operand pre-pass, zoo_scan.hip) ask of a call, checked in front of the first of them; the
+// same calls that the stage entry points take
+int check_scan(const void* q, const void* k, const void* v, const void* o, const void* ss, const void* svl, int B, int T, int H, int K,
+               int V, int qmax, int dt) {
+  if ((K != 64 && K != 128) || V % 64 != 0 || qmax < 1 || qmax > 127) return LQ_ERR_SHAPE;
+  if (dt != LQ_DT_F16 && dt != LQ_DT_BF16) return LQ_ERR_SHAPE;
+  for (const void* x : {q, k, v, o, ss, svl})
+    if (!zoo_al(x, 16)) return LQ_ERR_SHAPE;
+  if ((int64_t)B * H > 65535 || T / 64 > 65535 || (int64_t)(T / 64) * B * H > 0x7fffffff) return LQ_ERR_SHAPE;
+  return LQ_OK;
+}
 
 // Offsets of the intermediates for the dims in `a` (64-token chunks; chunk sizes above 64 keep the 64-token layouts)
 int plan(const lq_zoo_simple_gla_args* a, Layout* l) {
@@ -23,14 +35,19 @@ int plan(const lq_zoo_simple_gla_args* a, Layout* l) {
   if (cs != 64 && cs != 128 && cs != 192 && cs != 256) return LQ_ERR_SHAPE;
   if (a->seqlen % cs != 0) return LQ_ERR_SHAPE;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
+  const bool scan = cs == 64;
   int64_t off = 0;
-  l->gc = off, off += up(B * T * H * 4);
   l->kqT = off, off += up(B * NT * H * K * 64);
   l->vqT = off, off += up(B * NT * H * V * 64);
-  l->ev = off, off += up(B * T * H * 4);
   l->gam = off, off += up(B * NT * H * K * 4);
-  l->h_i8 = off, off += up(B * (T / cs) * H * V * K);
-  l->cross = off, off += cs == 64 ? 0 : up(B * T * H * V * 4);
+  l->vcT = off, off += scan ? up(B * NT * H * V * 64) : 0;
+  l->qc = off, off += scan ? up(B * NT * H * K * 64) : 0;
+  l->A = off, off += scan ? up(B * NT * H * 8192) : 0;
+  l->gpk = off, off += scan ? up(B * NT * H * 256) : 0;
+  l->gc = off, off += scan ? 0 : up(B * T * H * 4);
+  l->ev = off, off += scan ? 0 : up(B * T * H * 4);
+  l->h_i8 = off, off += scan ? 0 : up(B * (T / cs) * H * V * K);
+  l->cross = off, off += scan ? 0 : up(B * T * H * V * 4);
   l->total = off;
   return LQ_OK;
 }
@@ -53,8 +70,31 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
   int rc = plan(a, &l);
   if (rc != LQ_OK) return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
+  if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
+  const bool prologue = a->signs_qk || a->signs_v || a->dq;
+  if (prologue && a->chunk_size != 64) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
   const int decay = a->g ? LQ_DECAY_SCALAR : LQ_DECAY_NONE;
+  if (a->chunk_size == 64) {
+    if ((rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
+      return rc;
+    if (!zoo_al(a->signs_qk, 16) || !zoo_al(a->signs_v, 16) || (a->signs_v && a->vdim != 64 && a->vdim != 128)) return LQ_ERR_SHAPE;
+    const bool bf = a->act_dtype == LQ_DT_BF16;
+    ZooLinPrepParams w = {};
+    w.q = (const _Float16*)a->q, w.k = (const _Float16*)a->k, w.v = (const _Float16*)a->v, w.g = a->g;
+    w.signs_qk = a->signs_qk, w.signs_v = a->signs_v, w.dq = a->dq, w.dq_rcp = a->dq_rcp;
+    w.kqT = (int8_t*)(ws + l.kqT), w.vqT = (int8_t*)(ws + l.vqT), w.vcT = (int8_t*)(ws + l.vcT), w.qc = (int8_t*)(ws + l.qc);
+    w.A = (_Float16*)(ws + l.A), w.gam = (float*)(ws + l.gam), w.gpk = (float*)(ws + l.gpk);
+    w.sq = a->sq, w.sk = a->sk, w.skw = a->skw, w.svw = a->svw, w.svl = a->svl, w.eta = a->eta, w.scale = a->scale, w.qmax = a->qmax;
+    w.B = a->batch, w.T = a->seqlen, w.H = a->nheads, w.V = a->vdim, w.NT = a->seqlen / 64;
+    if ((rc = zoo_lin_prep_launch(w, a->kdim, bf, stream)) != LQ_OK) return rc;
+    ZooScanParams s = {};
+    s.kqT = w.kqT, s.vqT = w.vqT, s.vcT = w.vcT, s.gam = w.gam, s.qc = w.qc, s.A = w.A, s.gpk = w.gpk;
+    s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
+    s.skw = a->skw, s.svw = a->svw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
+    s.qmax = a->qmax, s.bf = bf, s.T = w.T, s.H = w.H, s.V = w.V, s.NT = w.NT;
+    return zoo_scan_launch(s, false, a->g != nullptr, a->kdim, a->batch, stream);
+  }
   float* gc = a->g ? (float*)(ws + l.gc) : nullptr;
 
   // every stage validates its own arguments before it launches; the stages share the dims, so what the first accepts the
@@ -164,6 +204,8 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
   if (a->dq && (!delta || !diag || big)) return LQ_ERR_SHAPE;  // D_QK at load: KDA, 64-token chunks
   if (a->rot && !diag) return LQ_ERR_SHAPE;
+  if (l.scan && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
+    return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
   float* gc = a->decay == LQ_DECAY_NONE ? nullptr : (float*)(ws + l.gc);

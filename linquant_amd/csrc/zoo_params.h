@@ -180,3 +180,31 @@ struct ZooWyParams {
 };
 // no / scalar decay; defined in zoo_wy_ns.hip
 int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, dim3 grid, hipStream_t stream);
+
+// Operand pre-pass of the linear family with no / scalar decay for zoo_scan.hip; defined in zoo_lin_prep.hip
+struct ZooLinPrepParams {
+  const _Float16* q;
+  const _Float16* k;
+  const _Float16* v;
+  const float* g;         // (B,T,H) log decay per token (not cumulated), or nullptr
+  const float* signs_qk;  // (K,), (V,) column signs of R_QK, R_V, or nullptr: no rotation
+  const float* signs_v;
+  const float* dq;        // (H,K) D_QK and its reciprocal, or nullptr
+  const float* dq_rcp;
+  int8_t* kqT;            // what zoo_scan.hip reads (ZooScanParams)
+  int8_t* vqT;
+  int8_t* vcT;
+  int8_t* qc;
+  _Float16* A;
+  float* gam;
+  float* gpk;
+  const float* sq;
+  const float* sk;
+  const float* skw;
+  const float* svw;
+  const float* svl;
+  float eta, scale;
+  int qmax;
+  int B, T, H, V, NT;
+};
+int zoo_lin_prep_launch(const ZooLinPrepParams& p, int K, bool bf, hipStream_t stream);

@@ -50,9 +50,9 @@ def chunk_simple_gla_int8(q, k, v, g, scales, *, eta=1.0, scale=None, chunk_size
     qmax = 2 ** (bits - 1) - 1
     decay = C.DECAY_NONE if g is None else C.DECAY_SCALAR
     assert g is None or g.shape == (B, T, H)
-    if prologue is None and unrot is None and _debug is None and not _staged:
-        # the whole forward as one C call over one workspace (same kernels and bits as the stage-by-stage route below)
-        o, ht = _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, output_final_state, out_dtype)
+    if unrot is None and _debug is None and not _staged:
+        # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
+        o, ht = _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, output_final_state, out_dtype, **(prologue or {}))
         return C.cut_values(restore(o), C.cut_keys(ht, K0), V0)
     gg = None
     if g is not None:
@@ -78,8 +78,9 @@ def chunk_simple_gla_int8(q, k, v, g, scales, *, eta=1.0, scale=None, chunk_size
     return C.cut_values(restore(o), C.cut_keys(ht, K0), V0)
 
 
-def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out_dtype):
-    """lq_zoo_simple_gla: cumsum, write-operand pre-pass, state recurrence and output from one foreign call."""
+def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out_dtype, signs_qk=None, signs_v=None,
+              dqk=None):
+    """lq_zoo_simple_gla: the whole forward from one foreign call, 64-token chunks with the operand rotations in it."""
     import ctypes
 
     from ... import _lib
@@ -89,6 +90,8 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "kw", "vw", "vl", "state")}
     svl, ss = _lib.aligned(sc["vl"]), _lib.aligned(sc["state"])
     gf = None if g is None else C.f32(g)
+    dq, dq_rcp = C.dqk_tables(dqk, H, K)
+    sg_qk, sg_v = [None if t is None else _lib.aligned(C.f32(t).reshape(n)) for t, n in ((signs_qk, K), (signs_v, V))]
     key = (B, T, H, K, V, span)
     nbytes = _WS_BYTES.get(key)
     if nbytes is None:
@@ -105,7 +108,8 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
               o_is_f32=int(o.dtype == torch.float32), ht=_lib.ptr(ht), sq=_lib.ptr(sc["q"]), sk=_lib.ptr(sc["k"]),
               skw=_lib.ptr(sc["kw"]), svw=_lib.ptr(sc["vw"]), svl=_lib.ptr(svl), ss=_lib.ptr(ss), eta=float(eta), scale=float(scale),
               qmax=int(qmax), batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span, act_dtype=C.act_code(v),
-              workspace=_lib.ptr(ws), workspace_bytes=nbytes)
+              workspace=_lib.ptr(ws), workspace_bytes=nbytes, signs_qk=_lib.ptr(sg_qk), signs_v=_lib.ptr(sg_v), dq=_lib.ptr(dq),
+              dq_rcp=_lib.ptr(dq_rcp))
     return o, ht
 
 

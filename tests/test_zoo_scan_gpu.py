@@ -43,3 +43,24 @@ def test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell
     torch.cuda.synchronize()
     assert o1.dtype == (out_dtype or dtype) and float(o1.float().abs().max()) > 0
     assert torch.equal(o0, o1) and torch.equal(h0, h1)
+
+
+# row widths that share the workgroup's waves differently, the scalar decay's fp64 running sum, every part of the prologue
+@pytest.mark.parametrize("cell,NT,B,H,K,V,dtype,parts", [
+    ("linear_none", 2, 1, 3, 128, 128, torch.float16, ("signs_qk", "signs_v", "dqk")), ("mamba2", 3, 2, 4, 64, 128, torch.bfloat16, ("signs_v",)),
+    ("mamba2", 1, 1, 1, 128, 64, torch.float16, ("signs_qk", "dqk")), ("linear_none", 4, 2, 2, 64, 64, torch.bfloat16, ("dqk",))])
+def test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts):
+    from linquant_amd.kernels import zoo
+
+    q, k, v, g, _ = [t.to(cuda) if t is not None else None for t in zc.inputs(cell, B=B, T=64 * NT, H=H, K=K, V=V, seed=NT, dtype=dtype)]
+    gen = torch.Generator().manual_seed(NT)
+    r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
+    sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.03), "kw": r(H, K, lo=0.005, hi=0.03), "vw": r(H, V, lo=0.02, hi=0.04),
+          "vl": r(H, V, lo=0.02, hi=0.04), "state": r(H, V, lo=0.02, hi=0.07)}
+    every = {"signs_qk": (r(K, lo=-1, hi=1)).sign(), "signs_v": (r(V, lo=-1, hi=1)).sign(), "dqk": r(H, K, lo=0.5, hi=2.0)}
+    kw = dict(eta=0.75, output_final_state=True, prologue={n: every[n] for n in parts})
+    o1, h1 = zoo.chunk_simple_gla_int8(q, k, v, g, sc, **kw)
+    o0, h0 = zoo.chunk_simple_gla_int8(q, k, v, g, sc, _staged=True, **kw)
+    torch.cuda.synchronize()
+    assert float(o1.float().abs().max()) > 0
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
