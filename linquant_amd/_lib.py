@@ -118,44 +118,23 @@ def current_stream(device):
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_FIELD_NAMES = {}
+
+
 def fill(struct_name: str, **fields):
     """An instance of the named args struct with the given fields set (unknown names raise KeyError)."""
-    st = STRUCTS[struct_name]()
-    known = {n for n, _ in st._fields_}
-    for k, v in fields.items():
-        if k not in known:
-            raise KeyError(f"{struct_name} has no field {k!r}")
-        setattr(st, k, v)
-    return st
+    cls = STRUCTS[struct_name]
+    known = _FIELD_NAMES.get(struct_name)
+    if known is None:
+        known = _FIELD_NAMES[struct_name] = frozenset(n for n, _ in cls._fields_)
+    if not fields.keys() <= known:
+        raise KeyError(f"{struct_name} has no field {next(k for k in fields if k not in known)!r}")
+    return cls(**fields)
 
 
 def launch(fn: str, device, st):
     """Call entry point ``fn`` with an already filled args struct on the current stream of ``device``."""
-    lib = load()
-    import torch
-
-    with torch.cuda.device(device):
-        rc = getattr(lib, fn)(ctypes.byref(st), current_stream(device))
-    if rc != 0:
-        raise LinQuantHipError(f"{fn} failed with code {rc}: {_ERRORS.get(rc, 'unknown error')}")
-
-
-_FIELD_NAMES = {}
-
-
-def call(fn: str, device, **fields):
-    """Fill ``<fn>_args`` from keyword fields and launch on the current stream of ``device``."""
     lib = _lib if _lib is not None else load()
-    sname = _SHARED_ARGS.get(fn, fn + "_args")
-    cls = STRUCTS[sname]
-    known = _FIELD_NAMES.get(sname)
-    if known is None:
-        known = _FIELD_NAMES[sname] = frozenset(n for n, _ in cls._fields_)
-    st = cls()
-    for k, v in fields.items():
-        if k not in known:
-            raise KeyError(f"{fn}_args has no field {k!r}")
-        setattr(st, k, v)
     import torch
 
     # (the device guard costs several microseconds a launch: it is entered only when the tensors' device is not the current one)
@@ -167,3 +146,8 @@ def call(fn: str, device, **fields):
             rc = getattr(lib, fn)(ctypes.byref(st), current_stream(device))
     if rc != 0:
         raise LinQuantHipError(f"{fn} failed with code {rc}: {_ERRORS.get(rc, 'unknown error')}")
+
+
+def call(fn: str, device, **fields):
+    """Fill ``<fn>_args`` from keyword fields and launch on the current stream of ``device``."""
+    launch(fn, device, fill(_SHARED_ARGS.get(fn, fn + "_args"), **fields))

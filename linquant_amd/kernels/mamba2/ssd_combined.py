@@ -7,6 +7,7 @@ allocation; a re-bound stage switches the call to the stage-by-stage path, which
 """
 
 import ctypes
+import functools
 
 import torch
 
@@ -92,15 +93,16 @@ def combined_args(x_fp, q_dt, dt_scale, q_A_log, A_log_scale, q_B, B_scale, q_C,
     dts, als = _as_f32_scalar(dt_scale, dev), _as_f32_scalar(A_log_scale, dev)
     dsc = None if q_D is None else _as_f32_scalar(D_scale, dev)
     keep += [Bs, Cs, scb, dts, als, dsc]
-    f = dict(x=_lib.ptr(x_fp), x_stride_b=x_fp.stride(0), x_stride_l=x_fp.stride(1), x_stride_h=x_fp.stride(2),
-             dt=_lib.ptr(q_dt), dt_dtype=_DT_CODES[q_dt.dtype], dt_stride_b=q_dt.stride(0), dt_stride_l=q_dt.stride(1),
-             dt_stride_h=q_dt.stride(2), dt_scale=_lib.ptr(dts), A_log=_lib.ptr(q_A_log), A_log_stride_h=q_A_log.stride(0),
+    x_st, dt_st, c_st, ss_st = x_fp.stride(), q_dt.stride(), q_C.stride(), sst.stride()
+    f = dict(x=_lib.ptr(x_fp), x_stride_b=x_st[0], x_stride_l=x_st[1], x_stride_h=x_st[2],
+             dt=_lib.ptr(q_dt), dt_dtype=_DT_CODES[q_dt.dtype], dt_stride_b=dt_st[0], dt_stride_l=dt_st[1],
+             dt_stride_h=dt_st[2], dt_scale=_lib.ptr(dts), A_log=_lib.ptr(q_A_log), A_log_stride_h=q_A_log.stride(0),
              A_log_scale=_lib.ptr(als), dt_bias=_lib.ptr(bias), dt_bias_stride_h=0 if bias is None else bias.stride(0),
              dt_softplus=int(bool(dt_softplus)), dt_min=float(dt_limit[0]), dt_max=float(dt_limit[1]),
-             qC=_lib.ptr(q_C), qC_stride_b=q_C.stride(0), qC_stride_l=q_C.stride(1), qC_stride_g=q_C.stride(2),
+             qC=_lib.ptr(q_C), qC_stride_b=c_st[0], qC_stride_l=c_st[1], qC_stride_g=c_st[2],
              B_scale=_lib.ptr(Bs), C_scale=_lib.ptr(Cs), D=_lib.ptr(q_D), D_stride_h=0 if q_D is None else q_D.stride(0),
              D_has_hdim=int(q_D is not None and q_D.dim() == 2), D_scale=_lib.ptr(dsc),
-             state_scale=_lib.ptr(sst), ss_stride_h=sst.stride(0), ss_stride_p=sst.stride(1), cb_scale=_lib.ptr(scb),
+             state_scale=_lib.ptr(sst), ss_stride_h=ss_st[0], ss_stride_p=ss_st[1], cb_scale=_lib.ptr(scb),
              keyside=int(bool(keyside)), gate_shift=_GATE_SHIFT, out=_lib.ptr(out), final_states=_lib.ptr(final_states),
              workspace=_lib.ptr(workspace), workspace_bytes=0 if workspace is None else workspace.numel(),
              batch=batch, seqlen=seqlen, nheads=nheads, headdim=headdim, ngroups=ngroups, dstate=dstate, chunk_size=chunk_size)
@@ -109,7 +111,8 @@ def combined_args(x_fp, q_dt, dt_scale, q_A_log, A_log_scale, q_B, B_scale, q_C,
     if keyside:
         assert b_fp.dtype == torch.float16 and b_fp.stride(3) == 1, "b_fp must be fp16 with unit dstate stride"
         sb = _bgs_strides(bgs)
-        f.update(b_fp=_lib.ptr(b_fp), bfp_stride_b=b_fp.stride(0), bfp_stride_l=b_fp.stride(1), bfp_stride_g=b_fp.stride(2),
+        b_st = b_fp.stride()
+        f.update(b_fp=_lib.ptr(b_fp), bfp_stride_b=b_st[0], bfp_stride_l=b_st[1], bfp_stride_g=b_st[2],
                  x_scale_hp=_lib.ptr(xs), xs_stride_h=xs.stride(0), xs_stride_p=xs.stride(1), b_gate_scale=_lib.ptr(bgs),
                  bgs_stride_b=sb[0], bgs_stride_c=sb[1], bgs_stride_h=sb[2], bgs_stride_n=sb[3])
         if b_rowmax is not None:
@@ -123,6 +126,7 @@ def combined_args(x_fp, q_dt, dt_scale, q_A_log, A_log_scale, q_B, B_scale, q_C,
     return _lib.fill("lq_ssd_combined_args", **f), keep
 
 
+@functools.lru_cache(maxsize=256)
 def workspace_bytes(batch, seqlen, nheads, headdim, ngroups, dstate, chunk_size):
     """Bytes of device workspace lq_ssd_combined needs for these dims."""
     st = _lib.fill("lq_ssd_combined_args", batch=batch, seqlen=seqlen, nheads=nheads, headdim=headdim, ngroups=ngroups,
