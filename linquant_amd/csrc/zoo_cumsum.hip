@@ -178,30 +178,49 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
       code[t] = zoo_q8(x, inv_skw, cc.qmax);
     }
     lq_v4i o;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) o[d] = (int)zoo_pack_codes(code[4 * d], code[4 * d + 1], code[4 * d + 2], code[4 * d + 3]);
-    *(lq_v4i*)(cc.kqT + (cb * K + k) * 64 + 16 * q) = o;
-    // value write codes: channel c = k, k + K, ... of the V value channels
-    const int V = cc.V;
-    for (int c = k; c < V; c += K) {
-      const float inv_svw = 1.0f / cc.svw[h * V + c];
-      uint16_t vraw[16];
-#pragma unroll
-      for (int t = 0; t < 16; ++t) vraw[t] = cc.v[((row0 + 16 * q + t) * H + h) * V + c];
-#pragma unroll
-      for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf) * zoo_exp(cc.eta * le_s[16 * q + t]), inv_svw, cc.qmax);
+    auto pack = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int d = 0; d < 4; ++d) o[d] = (int)zoo_pack_codes(code[4 * d], code[4 * d + 1], code[4 * d + 2], code[4 * d + 3]);
-      *(lq_v4i*)(cc.vqT + (cb * V + c) * 64 + 16 * q) = o;
-      if (cc.vcT) {
-        const float inv_svl = 1.0f / cc.svl[h * V + c];
+    };
+    pack();
+    // The codes leave through the dead envelope tile as whole contiguous pieces, 16 bytes per thread: straight from the registers a
+    // thread's 16 tokens were a quarter of a 64-byte row (and 8-byte halves of the operand-ordered ones), the rest of each line
+    // written by other waves (GLA B4 T4096 H16 K = V = 128: 107 -> 92 us).  K rows of 64 codes per buffer and pass, three buffers.
+    const int nb = K * 64;
+    unsigned char* kb = (unsigned char*)tile;
+    unsigned char *vb = kb + nb, *lb = vb + nb;
+    const int at = 16 * threadIdx.x;
+    __syncthreads();  // the tile has been read
+    *(lq_v4i*)(kb + k * 64 + 16 * q) = o;
+    // value write codes: channel c0 + k of the V value channels
+    const int V = cc.V;
+    for (int c0 = 0; c0 < V; c0 += K) {
+      if (c0) __syncthreads();  // the pass before has been copied out
+      const int c = c0 + k;
+      if (c < V) {
+        const float inv_svw = 1.0f / cc.svw[h * V + c];
+        uint16_t vraw[16];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf), inv_svl, cc.qmax);
+        for (int t = 0; t < 16; ++t) vraw[t] = cc.v[((row0 + 16 * q + t) * H + h) * V + c];
 #pragma unroll
-        for (int d = 0; d < 4; ++d) o[d] = (int)zoo_pack_codes(code[4 * d], code[4 * d + 1], code[4 * d + 2], code[4 * d + 3]);
-        int8_t* dst = cc.vcT + cb * V * 64 + zoo_op_values(c, 16 * q);
-        *(lq_v2i*)dst = lq_v2i{o[0], o[1]};
-        *(lq_v2i*)(dst + 256) = lq_v2i{o[2], o[3]};  // the next group of eight tokens
+        for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf) * zoo_exp(cc.eta * le_s[16 * q + t]), inv_svw, cc.qmax);
+        pack();
+        *(lq_v4i*)(vb + k * 64 + 16 * q) = o;
+        if (cc.vcT) {
+          const float inv_svl = 1.0f / cc.svl[h * V + c];
+#pragma unroll
+          for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf), inv_svl, cc.qmax);
+          pack();
+          unsigned char* dst = lb + zoo_op_values(k, 16 * q);
+          *(lq_v2i*)dst = lq_v2i{o[0], o[1]};
+          *(lq_v2i*)(dst + 256) = lq_v2i{o[2], o[3]};  // the next group of eight tokens
+        }
+      }
+      __syncthreads();
+      if (c0 == 0) *(lq_v4i*)(cc.kqT + cb * nb + at) = *(const lq_v4i*)(kb + at);
+      if (at < min(K, V - c0) * 64) {
+        *(lq_v4i*)(cc.vqT + (cb * V + c0) * 64 + at) = *(const lq_v4i*)(vb + at);
+        if (cc.vcT) *(lq_v4i*)(cc.vcT + (cb * V + c0) * 64 + at) = *(const lq_v4i*)(lb + at);  // (V is a multiple of 64 then, K 64 or 128)
       }
     }
   }
