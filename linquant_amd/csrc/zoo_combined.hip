@@ -1,8 +1,8 @@
 // One call for the whole no / scalar decay chunk forward: chunk_simple_gla_int8 (linquant/kernels/zoo/simple_gla.py:175-212)
 // as one C entry over one caller-supplied workspace that holds what the Python wrapper would otherwise allocate per call.
-// 64-token chunks: two launches, the operand pre-pass (zoo_lin_prep.hip; with it the operand rotations, if asked for) and recurrence
-// with output (zoo_scan.hip).  Longer chunks: the four stand-alone stages (cumsum, write-operand pre-pass, state recurrence,
-// output) back to back.  The bits of the stage entry points in either case.
+// 64-token chunks of many or short chains: two launches, the operand pre-pass (zoo_lin_prep.hip; with it the operand rotations, if asked for) and recurrence
+// with output (zoo_scan.hip).  Otherwise: the four stand-alone stages (cumsum, write-operand pre-pass or rotate-quantize, state
+// recurrence, output) back to back.  The bits of the stage entry points in either case.
 #include <initializer_list>
 
 #include "zoo_params.h"
@@ -13,8 +13,16 @@ constexpr int64_t kAlign = 256;
 int64_t up(int64_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
-  int64_t gc, kqT, vqT, vcT, qc, A, gpk, ev, gam, h_i8, cross, total;
+  int64_t gc, kqT, vqT, vcT, qc, kc, A, gpk, ev, gam, h_i8, cross, total;
+  bool scan;  // operand pre-pass, then recurrence and output in one launch
 };
+
+// Linear family, 64-token chunks: recurrence and output in one launch, or one after the other?  The chain is NT steps in either
+// case; a step that shares its SIMDs with the output takes about twice as long (K = 128: 1.0 us, 0.5 without), while an output launch
+// of its own uses the whole chip whatever the number of chains.  So few long chains keep the two launches (scalar decay B3 T21184 H5 K
+// = V = 128: 319 us, 397 in one), many chains (linear attention B4 T4096 H16: 176 us, 153 in one; GLA 317, 288) and short ones, where
+// launches count (Mamba-2 cell B1 T2048 H8 K = V = 64: 28 us, 24 in one), take the one.
+bool linear_scan(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) { return B * H * (V / 64) >= 64 || T / 64 * K <= 2048; }
 
 // What the launches over 64-token chunks (operand pre-pass, zoo_scan.hip) ask of a call, checked in front of the first of them; the
 // same calls that the stage entry points take
@@ -35,13 +43,14 @@ int plan(const lq_zoo_simple_gla_args* a, Layout* l) {
   if (cs != 64 && cs != 128 && cs != 192 && cs != 256) return LQ_ERR_SHAPE;
   if (a->seqlen % cs != 0) return LQ_ERR_SHAPE;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
-  const bool scan = cs == 64;
+  const bool scan = l->scan = cs == 64 && linear_scan(B, T, H, K, V), codes = cs == 64 && !scan;
   int64_t off = 0;
   l->kqT = off, off += up(B * NT * H * K * 64);
   l->vqT = off, off += up(B * NT * H * V * 64);
   l->gam = off, off += up(B * NT * H * K * 4);
-  l->vcT = off, off += scan ? up(B * NT * H * V * 64) : 0;
-  l->qc = off, off += scan ? up(B * NT * H * K * 64) : 0;
+  l->vcT = off, off += scan || codes ? up(B * NT * H * V * 64) : 0;  // (codes: token-major local codes of q, k, v)
+  l->qc = off, off += scan || codes ? up(B * NT * H * K * 64) : 0;
+  l->kc = off, off += codes ? up(B * NT * H * K * 64) : 0;
   l->A = off, off += scan ? up(B * NT * H * 8192) : 0;
   l->gpk = off, off += scan ? up(B * NT * H * 256) : 0;
   l->gc = off, off += scan ? 0 : up(B * T * H * 4);
@@ -75,9 +84,9 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
   if (prologue && a->chunk_size != 64) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
   const int decay = a->g ? LQ_DECAY_SCALAR : LQ_DECAY_NONE;
-  if (a->chunk_size == 64) {
-    if ((rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
-      return rc;
+  if (a->chunk_size == 64 && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
+    return rc;
+  if (l.scan) {
     if (!zoo_al(a->signs_qk, 16) || !zoo_al(a->signs_v, 16) || (a->signs_v && a->vdim != 64 && a->vdim != 128)) return LQ_ERR_SHAPE;
     const bool bf = a->act_dtype == LQ_DT_BF16;
     ZooLinPrepParams w = {};
@@ -105,7 +114,16 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
     c.g = a->g, c.gc = gc, c.batch = a->batch, c.seqlen = a->seqlen, c.nheads = a->nheads, c.kdim = 0, c.chunk_size = a->chunk_size;
     if ((rc = lq_zoo_cumsum(&c, stream)) != LQ_OK) return rc;
   }
-  {
+  if (prologue) {
+    lq_zoo_rotate_quant_args w = {};
+    w.q = a->q, w.k = a->k, w.v = a->v, w.g = gc, w.qc = (int8_t*)(ws + l.qc), w.kc = (int8_t*)(ws + l.kc), w.vc = (int8_t*)(ws + l.vcT);
+    w.kqT = (int8_t*)(ws + l.kqT), w.vqT = (int8_t*)(ws + l.vqT), w.ev = (float*)(ws + l.ev), w.gam = (float*)(ws + l.gam);
+    w.dq = a->dq, w.dk = a->dq_rcp, w.signs_qk = a->signs_qk, w.signs_v = a->signs_v;
+    w.sq = a->sq, w.sk = a->sk, w.svl = a->svl, w.skw = a->skw, w.svw = a->svw, w.eta = a->eta, w.scale = a->scale, w.qmax = a->qmax;
+    w.batch = a->batch, w.seqlen = a->seqlen, w.nheads = a->nheads, w.kdim = a->kdim, w.vdim = a->vdim, w.chunk_size = 64;
+    w.act_dtype = a->act_dtype;
+    if ((rc = lq_zoo_rotate_quant(&w, stream)) != LQ_OK) return rc;
+  } else {
     lq_zoo_write_codes_args w = {};
     w.key = a->k, w.val = a->v, w.g = gc, w.kqT = (int8_t*)(ws + l.kqT), w.vqT = (int8_t*)(ws + l.vqT);
     w.ev = (float*)(ws + l.ev), w.gam = (float*)(ws + l.gam), w.skw = a->skw, w.svw = a->svw, w.eta = a->eta, w.qmax = a->qmax;
@@ -123,7 +141,9 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
   }
   {
     lq_zoo_output_args o = {};
-    o.q = a->q, o.k = a->k, o.v = a->v, o.h_i8 = (const int8_t*)(ws + l.h_i8), o.g = gc, o.o = a->o, o.o_is_f32 = a->o_is_f32;
+    o.q = a->q, o.k = a->k, o.v = a->v, o.h_i8 = (const int8_t*)(ws + l.h_i8), o.g = gc;
+    if (prologue) o.qc = (const int8_t*)(ws + l.qc), o.kc = (const int8_t*)(ws + l.kc), o.vc = (const int8_t*)(ws + l.vcT);
+    o.o = a->o, o.o_is_f32 = a->o_is_f32;
     o.sq = a->sq, o.sk = a->sk, o.svl = a->svl, o.ss = a->ss, o.scale = a->scale, o.qmax = a->qmax;
     o.batch = a->batch, o.seqlen = a->seqlen, o.nheads = a->nheads, o.kdim = a->kdim, o.vdim = a->vdim, o.chunk_size = a->chunk_size;
     o.decay = decay, o.act_dtype = a->act_dtype, o.cross = a->chunk_size == 64 ? nullptr : (float*)(ws + l.cross);
@@ -135,8 +155,8 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // ---- the other cells: chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry each way round: the stage entry points in
 // the order the Python wrappers issue them, over one workspace.  64-token chunks take the fused pre-passes (the cumsum / WY
-// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks run the
-// recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).
+// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks (GLA: of
+// many or short chains, linear_scan) run the recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).
 namespace {
 
 struct FLayout {
@@ -153,6 +173,7 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   if (a->family == LQ_FAMILY_LINEAR && a->decay != LQ_DECAY_DIAGONAL) return LQ_ERR_SHAPE;  // lq_zoo_simple_gla serves those
   const bool delta = a->family == LQ_FAMILY_DELTA, diag = a->decay == LQ_DECAY_DIAGONAL, big = cs == 128;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
+  l->scan = !big && (delta || linear_scan(B, T, H, K, V));
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
   take(l->gc, a->decay == LQ_DECAY_NONE ? 0 : B * T * H * (diag ? K : 1) * 4);
@@ -167,7 +188,6 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->Ax, diag && big ? B * T * H * 64 * 2 : 0);
   take(l->qg, diag || !big ? B * T * H * K : 0);
   take(l->gpk, a->decay == LQ_DECAY_SCALAR && !big ? B * NT * H * 64 * 4 : 0);
-  l->scan = !big;
   take(l->vcT, l->scan && !delta ? B * NT * H * V * 64 : 0);
   take(l->Hw, delta && (diag || big) ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
@@ -204,7 +224,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
   if (a->dq && (!delta || !diag || big)) return LQ_ERR_SHAPE;  // D_QK at load: KDA, 64-token chunks
   if (a->rot && !diag) return LQ_ERR_SHAPE;
-  if (l.scan && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
+  if (!big && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
     return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;

@@ -88,7 +88,7 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
     B, T, H, K, V = dims
     dev = q.device
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "kw", "vw", "vl", "state")}
-    svl, ss = _lib.aligned(sc["vl"]), _lib.aligned(sc["state"])
+    svl, ss, skw, svw = [_lib.aligned(sc[n]) for n in ("vl", "state", "kw", "vw")]
     gf = None if g is None else C.f32(g)
     dq, dq_rcp = C.dqk_tables(dqk, H, K)
     sg_qk, sg_v = [None if t is None else _lib.aligned(C.f32(t).reshape(n)) for t, n in ((signs_qk, K), (signs_v, V))]
@@ -106,7 +106,7 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
     ht = torch.empty(B, H, K, V, dtype=torch.float32, device=dev) if final_state else None
     _lib.call("lq_zoo_simple_gla", dev, q=_lib.ptr(q), k=_lib.ptr(k), v=_lib.ptr(v), g=_lib.ptr(gf), o=_lib.ptr(o),
               o_is_f32=int(o.dtype == torch.float32), ht=_lib.ptr(ht), sq=_lib.ptr(sc["q"]), sk=_lib.ptr(sc["k"]),
-              skw=_lib.ptr(sc["kw"]), svw=_lib.ptr(sc["vw"]), svl=_lib.ptr(svl), ss=_lib.ptr(ss), eta=float(eta), scale=float(scale),
+              skw=_lib.ptr(skw), svw=_lib.ptr(svw), svl=_lib.ptr(svl), ss=_lib.ptr(ss), eta=float(eta), scale=float(scale),
               qmax=int(qmax), batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span, act_dtype=C.act_code(v),
               workspace=_lib.ptr(ws), workspace_bytes=nbytes, signs_qk=_lib.ptr(sg_qk), signs_v=_lib.ptr(sg_v), dq=_lib.ptr(dq),
               dq_rcp=_lib.ptr(dq_rcp))

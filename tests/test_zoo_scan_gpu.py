@@ -48,7 +48,9 @@ def test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell
 # row widths that share the workgroup's waves differently, the scalar decay's fp64 running sum, every part of the prologue
 @pytest.mark.parametrize("cell,NT,B,H,K,V,dtype,parts", [
     ("linear_none", 2, 1, 3, 128, 128, torch.float16, ("signs_qk", "signs_v", "dqk")), ("mamba2", 3, 2, 4, 64, 128, torch.bfloat16, ("signs_v",)),
-    ("mamba2", 1, 1, 1, 128, 64, torch.float16, ("signs_qk", "dqk")), ("linear_none", 4, 2, 2, 64, 64, torch.bfloat16, ("dqk",))])
+    ("mamba2", 1, 1, 1, 128, 64, torch.float16, ("signs_qk", "dqk")), ("linear_none", 4, 2, 2, 64, 64, torch.bfloat16, ("dqk",)),
+    # few long chains: the stages one after the other behind the same call; many: one launch again
+    ("mamba2", 40, 1, 2, 128, 64, torch.float16, ("signs_qk", "signs_v")), ("linear_none", 40, 4, 8, 128, 128, torch.bfloat16, ("signs_qk", "dqk"))])
 def test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts):
     from linquant_amd.kernels import zoo
 
