@@ -8,10 +8,15 @@
 // Nothing but per-token factors separates the operands of these products from k and v themselves, and a per-token factor is an
 // index of T's columns.  So the half-precision rows stay exact and all arithmetic goes to T:
 //   Gram: k . k^T on the half-precision MFMA (exact products, fp32 accumulation), the factors applied to the 64 x 64 result;
-//   W, U: (T . diag(bs exp(g))) . k and (T . diag(bs)) . v with k and v as they are and only T split: two fp16 pieces of each
-//     row scaled by a power of two to just below fp16's range (so that neither piece of an entry down to 2^-18 of the row's largest
-//     is subnormal), three bf16 pieces for bf16 activations.  Share of W, U entries on the other side of a rounding boundary than
-//     the float64 result (B2 T512, unit keys): 2.5e-4, 3.5e-4 in fp16, 4e-5 in bf16; the fp32 form below 4.5e-4, 5.6e-4 and 1e-4.
+//   W, U: (T . diag(bs exp(g))) . k and (T . diag(bs)) . v with k and v as they are and only T split, in three half-precision
+//     pieces that together hold the 24 bits of an fp32 entry.  bf16 pieces have fp32's range.  fp16 pieces: each row is scaled by a
+//     power of two to just below fp16's range and the third piece by another 2^22, in an accumulator that is scaled back before
+//     the other two are added: what is left of an entry is below 2^-51 of its row's largest (two pieces left 2^-39, which behind a
+//     strong decay and in front of a large value cost half of an entry's bits).
+//     Share of W, U entries on the other side of a rounding boundary than the float64 result (B4 T2048 H16 K = V = 128, unit keys;
+//     two fp16 pieces, and the fp32 form below, in brackets): fp16 2.6e-4, 2.9e-4 (2.9e-4, 3.3e-4; 4.5e-4, 5.4e-4), with scalar decay
+//     1.1e-4, 0.9e-4 (1.2e-4, 1.2e-4; 1.3e-4, 1.6e-4); bf16 5.0e-5, 4.5e-5 (fp32 form 9.5e-5, 8.7e-5).  The third fp16 piece costs 6
+//     us of 256 (Gated DeltaNet B4 T4096 H16, whole call).
 // An fp32 form of the same (operands scaled and staged as fp32, 32 fp32 MFMA steps per Gram block, T and X split in three bf16
 // pieces, six products) took 121 us at B4 T4096 H16 K = V = 128, of which the splitting and the fp32 steps were two thirds.
 //
@@ -54,11 +59,11 @@ LQ_DEV float wn_powb(float b, float e) {
   return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(b));
 }
 
-// T operand of one row block and contraction step: eight values of a row, scaled, as NP pieces
+// T operand of one row block and contraction step: eight values of a row (fp16: scaled) as three pieces (fp16: the third
+// times 2^22)
 template <bool BF>
 struct TPieces {
-  static constexpr int NP = BF ? 3 : 2;
-  lq_v4i p[NP];
+  lq_v4i p[3];
 };
 
 template <bool BF>
@@ -75,9 +80,12 @@ LQ_DEV void wn_split(const float (&x)[8], TPieces<BF>& t) {
       const float q0 = r0 - __uint_as_float(c0 & 0xffff0000u), q1 = r1 - __uint_as_float(c1 & 0xffff0000u);
       t.p[2][d] = (int)__builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
     } else {
-      const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
-      t.p[0][d] = __builtin_bit_cast(int, lq_v2h{h0, h1});
-      t.p[1][d] = (int)zoo_pack_h2(x0 - (float)h0, x1 - (float)h1);
+      const _Float16 b0 = (_Float16)x0, b1 = (_Float16)x1;
+      t.p[0][d] = __builtin_bit_cast(int, lq_v2h{b0, b1});
+      const float r0 = x0 - (float)b0, r1 = x1 - (float)b1;
+      const _Float16 c0 = (_Float16)r0, c1 = (_Float16)r1;
+      t.p[1][d] = __builtin_bit_cast(int, lq_v2h{c0, c1});
+      t.p[2][d] = (int)zoo_pack_h2((r0 - (float)c0) * 0x1p22f, (r1 - (float)c1) * 0x1p22f);
     }
   }
 }
@@ -373,6 +381,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
     float mw = 0.0f, mu = 0.0f;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
+      if (st >= NST) continue;  // (wave-uniform)
       const int m0 = 32 * st + 8 * kg;
       const bool live = m0 < 16 * (I + 1);  // blocks right of the diagonal were never written
 #pragma unroll
@@ -388,7 +397,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
       auto scale_of = [&](float m, float& un) {
         m = fmaxf(m, __shfl_xor(m, 16));
         m = fmaxf(m, __shfl_xor(m, 32));
-        const int e = min(max((int)(__float_as_uint(m) >> 23), 16), 252);  // largest entry 2^(e - 127) .. 2^(e - 126)
+        const int e = min(max((int)(__float_as_uint(m) >> 23), 16), 254);  // largest entry 2^(e - 127) .. 2^(e - 126)
         un = __uint_as_float((uint32_t)(e - 14) << 23);
         return __uint_as_float((uint32_t)(268 - e) << 23);  // 2^(141 - e)
       };
@@ -398,20 +407,36 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xw[st][e] = xw[st][e] * sw_, xu[st][e] = xu[st][e] * su_;
+        for (int e = 0; e < 8; ++e)
+          if (st < NST) xw[st][e] = xw[st][e] * sw_, xu[st][e] = xu[st][e] * su_;
     }
-    wn_split<BF>(xw[0], tw[0]), wn_split<BF>(xw[1], tw[1]);
-    if constexpr (SCALAR) wn_split<BF>(xu[0], tu[0]), wn_split<BF>(xu[1], tu[1]);
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      if (st >= NST) continue;
+      wn_split<BF>(xw[st], tw[st]);
+      if constexpr (SCALAR) wn_split<BF>(xu[st], tu[st]);
+    }
   }
   // D^T tile: lane (rl = token of block I, kg) gets columns 16nt + 4kg + r
   auto tile = [&](const uint32_t* X, const TPieces<BF> (&t)[2], int nt) {
     lq_v4f acc = {0.f, 0.f, 0.f, 0.f};
+    lq_v4i x[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
-      if (st >= NST) continue;  // (wave-uniform)
-      const lq_v4i x = *(const lq_v4i*)(X + wn_xt(16 * nt + rl, 16 * st + 4 * kg));
+      if (st >= NST) continue;
+      x[st] = *(const lq_v4i*)(X + wn_xt(16 * nt + rl, 16 * st + 4 * kg));
 #pragma unroll
-      for (int i = TPieces<BF>::NP - 1; i >= 0; --i) acc = wn_mfma<BF>(x, t[st].p[i], acc);
+      for (int i = 2; i >= (BF ? 0 : 2); --i) acc = wn_mfma<BF>(x[st], t[st].p[i], acc);
+    }
+    if constexpr (!BF) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = acc[r] * 0x1p-22f;
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        if (st >= NST) continue;
+#pragma unroll
+        for (int i = 1; i >= 0; --i) acc = wn_mfma<BF>(x[st], t[st].p[i], acc);
+      }
     }
     return acc;
   };
