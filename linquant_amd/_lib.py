@@ -137,6 +137,8 @@ def launch(fn: str, device, st):
     lib = _lib if _lib is not None else load()
     import torch
 
+    if getattr(device, "type", "cuda") != "cuda":  # host pointers must not reach a kernel
+        raise ValueError(f"{fn}: expected tensors on a GPU, got {device}")
     # (the device guard costs several microseconds a launch: it is entered only when the tensors' device is not the current one)
     idx = device.index if getattr(device, "index", None) is not None else torch.cuda.current_device()
     if idx == torch.cuda.current_device():

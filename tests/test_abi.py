@@ -195,3 +195,29 @@ def test_documented_binding_example_matches_the_library(monkeypatch):
     assert [n for n, _ in st._fields_] == [n for n, _ in _lib.STRUCTS["lq_state_passing_args"]._fields_]
     assert ctypes.sizeof(st) == ctypes.sizeof(_lib.STRUCTS["lq_state_passing_args"])
     assert callable(ns["_fixedpoint_state_passing_fwd"])
+
+
+@pytest.mark.parametrize("how", ["launch", "call"])
+def test_tensors_that_are_not_on_a_gpu_are_refused_before_the_library_is_entered(monkeypatch, how):
+    """A CPU tensor's device (which has no index, like the current GPU's short form) must not be taken for the current device: the
+    kernels would read host addresses."""
+    entered = []
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: entered.append(name) or 0
+
+    class Stream:
+        cuda_stream = 0
+
+    monkeypatch.setattr(_lib, "_lib", Library())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+    with pytest.raises(ValueError):
+        if how == "launch":
+            _lib.launch("lq_ssd_combined", torch.zeros(1).device, _lib.fill("lq_ssd_combined_args"))
+        else:
+            _lib.call("lq_zoo_cumsum", torch.zeros(1).device, batch=1)
+    assert not entered
+    _lib.call("lq_zoo_cumsum", torch.device("cuda"), batch=1)
+    assert entered == ["lq_zoo_cumsum"]
