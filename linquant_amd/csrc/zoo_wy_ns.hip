@@ -204,7 +204,9 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
       for (int d = 0; d < 4; ++d) {
         float x0, x1;
         zoo_dec2((uint32_t)kraw[u][d], bf, x0, x1);
-        hw[d] = (int)zoo_enc2(bw * x0, bw * x1, bf);  // Hw as it would be stored
+        // Hw as it would be stored, rounded to fp32 first (folded into one rounding, a product next to a midpoint went the other
+        // way than the stored Hw in some of the instantiations, and its code with it)
+        hw[d] = (int)zoo_enc2(zoo_mul_rn(bw, x0), zoo_mul_rn(bw, x1), bf);
       }
       if constexpr (!SCAN) *(lq_v4i*)(p.Hw + ((t0 + t) * H + h) * K + 8 * kc) = hw;
       if constexpr (CODES) {
