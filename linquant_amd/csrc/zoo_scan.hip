@@ -26,6 +26,14 @@
 // derives each wait from a count of those issued since, merged over all paths, so a branch around a store or a product made
 // every step wait for the operands it had just requested (seen in its assembly: vmcnt(2) .. vmcnt(4)
 // where vmcnt(27) is meant).
+//
+// The linear family keeps two operand sets and at most 128 registers, so that two workgroups fit a compute unit.  With five sets
+// (199 .. 236 registers, one workgroup) 257 to 511 workgroups took two rounds of the chip, the second nearly empty, and lost to the
+// two launches that this one replaces; the second workgroup hides more than the three further sets did.  Linear attention K = V = 128,
+// us per call with two launches / five sets / two sets: B*H = 80 T1024 54 / 63 / 54, B*H = 192 T1024 112 / 116 / 106, B*H = 96 T2048
+// 112 / 118 / 106, B*H = 64 T4096 (one full round) 151 / 145 / 146.  The delta family's sets hold more per step (three sets, 142 ..
+// 165 registers at K = 128): its step is longer, and with one workgroup per compute unit it was faster than its two launches at every
+// size measured (B*H = 4 .. 256, T = 256 .. 16384: 1.04 to 1.7 times).
 #include <type_traits>
 
 #include "zoo_params.h"
@@ -78,10 +86,10 @@ LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
 // Operand sets in rotation: a set is requested D - 1 steps ahead of its use, and the loop is unrolled by D so that the sets
 // keep their registers.  Its body has no exit in it (what does not fill D steps follows behind): an exit inside merged, in the
 // compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
-constexpr int scan_sets(bool delta) { return delta ? 3 : 5; }
+constexpr int scan_sets(bool delta) { return delta ? 3 : 2; }
 
 template <bool DELTA, bool SCALAR, int K, int BV, bool BF, bool OF32>
-__global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
+__global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams p) {
   constexpr int D = scan_sets(DELTA);
   constexpr int KR = K / 4;        // carry rows per chain wave
   constexpr int KT = K / 64;       // 16-row tiles per chain wave
@@ -148,7 +156,6 @@ __global__ __launch_bounds__(512, 2) void zoo_scan_kernel(ScanParams p) {
     auto load_part = [&](auto part_c, int ct, Ops& o) __attribute__((always_inline)) {
       constexpr int part = decltype(part_c)::value;
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
-      const int64_t t0 = (int64_t)b * T + (int64_t)ct * 64;
       if constexpr (part == 0 || part == 1) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) o.kop[kt] = *(const lq_v4i*)(p.kqT + (cb * K + KR * wave + 16 * kt + rl) * 64 + 16 * kg);
