@@ -101,8 +101,8 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
     s.kqT = w.kqT, s.vqT = w.vqT, s.vcT = w.vcT, s.gam = w.gam, s.qc = w.qc, s.A = w.A, s.gpk = w.gpk;
     s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
     s.skw = a->skw, s.svw = a->svw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
-    s.qmax = a->qmax, s.bf = bf, s.T = w.T, s.H = w.H, s.V = w.V, s.NT = w.NT;
-    return zoo_scan_launch(s, false, a->g != nullptr, a->kdim, a->batch, stream);
+    s.qmax = a->qmax, s.bf = bf, s.B = w.B, s.T = w.T, s.H = w.H, s.V = w.V, s.NT = w.NT;
+    return zoo_scan_launch(s, false, a->g != nullptr, a->kdim, stream);
   }
   float* gc = a->g ? (float*)(ws + l.gc) : nullptr;
 
@@ -292,8 +292,9 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     s.kqT = kqT, s.vqT = vqT, s.vcT = vcT, s.wq = wq, s.u = (const _Float16*)U, s.pack = pack, s.gam = gam;
     s.qc = qg, s.A = (const _Float16*)A, s.gpk = gpk, s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
     s.skw = a->skw, s.svw = a->svw, s.sw = a->sw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
-    s.qmax = a->qmax, s.bf = a->act_dtype == LQ_DT_BF16, s.T = a->seqlen, s.H = a->nheads, s.V = a->vdim, s.NT = a->seqlen / 64;
-    return zoo_scan_launch(s, delta, a->decay == LQ_DECAY_SCALAR, a->kdim, a->batch, stream);
+    s.qmax = a->qmax, s.bf = a->act_dtype == LQ_DT_BF16;
+    s.B = a->batch, s.T = a->seqlen, s.H = a->nheads, s.V = a->vdim, s.NT = a->seqlen / 64;
+    return zoo_scan_launch(s, delta, a->decay == LQ_DECAY_SCALAR, a->kdim, stream);
   }
   {
     lq_zoo_state_args s = {};

@@ -120,9 +120,9 @@ struct ZooScanParams {
   const float* svl;
   int qmax;
   int bf;
-  int T, H, V, NT;
+  int B, T, H, V, NT;
 };
-int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, int batch, hipStream_t stream);
+int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, hipStream_t stream);
 
 // The pre-pass entry points with what zoo_scan.hip wants on top of their public arguments.
 // cumsum (GLA): also the local value codes (zoo_op_values)
