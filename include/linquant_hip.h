@@ -465,7 +465,8 @@ typedef struct {
   void* workspace;           /* device memory, 256-byte aligned, lq_zoo_simple_gla_workspace_bytes() bytes; contents undefined
                                 on entry and on return */
   int64_t workspace_bytes;
-  /* Optional, each NULL or set (64-token chunks): q, k, v are rotated and rescaled as they are loaded, as lq_zoo_rotate_quant does */
+  /* Optional, each NULL or set (64-token chunks): q, k, v are rotated and rescaled as they are loaded, as lq_zoo_rotate_quant
+   * does; with signs_qk and dq alone for every V of this call, and with dq, dq_rcp, skw and svw at any address */
   const float* signs_qk;     /* (K,) column signs of R_QK, 16-byte aligned */
   const float* signs_v;      /* (V,) column signs of R_V, 16-byte aligned (V in {64,128}) */
   const float* dq;           /* (H,K) D_QK: q is multiplied by it, k divided; with dq_rcp */

@@ -36,14 +36,23 @@ int check_scan(const void* q, const void* k, const void* v, const void* o, const
   return LQ_OK;
 }
 
+// Does lq_zoo_rotate_quant, the staged route's operand launch, take this call?  (the one-launch route takes any V that is a multiple
+// of 64, and tables at any address)
+bool staged_prologue(const lq_zoo_simple_gla_args* a) {
+  if (a->vdim != 64 && a->vdim != 128) return false;
+  for (const void* x : {a->dq, a->dq_rcp, a->skw, a->svw})
+    if (!zoo_al(x, 16)) return false;
+  return true;
+}
+
 // Offsets of the intermediates for the dims in `a` (64-token chunks; chunk sizes above 64 keep the 64-token layouts)
-int plan(const lq_zoo_simple_gla_args* a, Layout* l) {
+int plan(const lq_zoo_simple_gla_args* a, Layout* l, bool force_scan) {
   if (a->batch <= 0 || a->seqlen <= 0 || a->nheads <= 0 || a->kdim <= 0 || a->vdim <= 0) return LQ_ERR_SHAPE;
   const int cs = a->chunk_size;
   if (cs != 64 && cs != 128 && cs != 192 && cs != 256) return LQ_ERR_SHAPE;
   if (a->seqlen % cs != 0) return LQ_ERR_SHAPE;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
-  const bool scan = l->scan = cs == 64 && linear_scan(B, T, H, K, V), codes = cs == 64 && !scan;
+  const bool scan = l->scan = cs == 64 && (force_scan || linear_scan(B, T, H, K, V)), codes = cs == 64 && !scan;
   int64_t off = 0;
   l->kqT = off, off += up(B * NT * H * K * 64);
   l->vqT = off, off += up(B * NT * H * V * 64);
@@ -65,29 +74,32 @@ int plan(const lq_zoo_simple_gla_args* a, Layout* l) {
 
 extern "C" int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* a, int64_t* bytes) {
   if (!a || !bytes) return LQ_ERR_NULL;
-  Layout l;
-  const int rc = plan(a, &l);
+  // (64-token chunks: the route of a call with a prologue depends on its pointers, so the size is enough for either)
+  Layout l, s;
+  int rc = plan(a, &l, false);
+  if (rc == LQ_OK) rc = plan(a, &s, true);
   if (rc != LQ_OK) return rc;
-  *bytes = l.total;
+  *bytes = l.total > s.total ? l.total : s.total;
   return LQ_OK;
 }
 
 extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t stream) {
   if (!a || !a->q || !a->k || !a->v || !a->o || !a->workspace) return LQ_ERR_NULL;
   if (!a->sq || !a->sk || !a->skw || !a->svw || !a->svl || !a->ss) return LQ_ERR_NULL;
-  Layout l;
-  int rc = plan(a, &l);
-  if (rc != LQ_OK) return rc;
-  if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
+  // what a call with a prologue may be does not depend on its route: checked here, in front of the first launch of either
   const bool prologue = a->signs_qk || a->signs_v || a->dq;
   if (prologue && a->chunk_size != 64) return LQ_ERR_SHAPE;
+  if (!zoo_al(a->signs_qk, 16) || !zoo_al(a->signs_v, 16) || (a->signs_v && a->vdim != 64 && a->vdim != 128)) return LQ_ERR_SHAPE;
+  Layout l;
+  int rc = plan(a, &l, prologue && !staged_prologue(a));
+  if (rc != LQ_OK) return rc;
+  if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
   const int decay = a->g ? LQ_DECAY_SCALAR : LQ_DECAY_NONE;
   if (a->chunk_size == 64 && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
     return rc;
   if (l.scan) {
-    if (!zoo_al(a->signs_qk, 16) || !zoo_al(a->signs_v, 16) || (a->signs_v && a->vdim != 64 && a->vdim != 128)) return LQ_ERR_SHAPE;
     const bool bf = a->act_dtype == LQ_DT_BF16;
     ZooLinPrepParams w = {};
     w.q = (const _Float16*)a->q, w.k = (const _Float16*)a->k, w.v = (const _Float16*)a->v, w.g = a->g;
