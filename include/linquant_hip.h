@@ -40,7 +40,7 @@ typedef struct ihipStream_t* hipStream_t;
 #define LQ_DT_I8 2
 #define LQ_DT_BF16 3
 
-/* ABI version; bumped whenever a struct layout changes. */
+/* ABI version; bumped whenever a struct layout, or what a call asks of its caller, changes. */
 int lq_abi_version(void);
 /* sizeof() of the named args struct as compiled into the library (negative if unknown); lets a binding
  * check its own struct layout before the first call. */
@@ -473,7 +473,8 @@ typedef struct {
   const float* dq_rcp;       /* (H,K) RN(1 / dq) */
 } lq_zoo_simple_gla_args;
 int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* args, hipStream_t stream);
-/* workspace size for the dims in `args` (pointers are not read), written to *bytes */
+/* workspace size for the dims in `args`, written to *bytes; no pointer is followed, but a call with a prologue needs the size asked
+ * for with its prologue fields (signs_qk, signs_v, dq) set */
 int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* args, int64_t* bytes);
 
 /* replaces chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8 (gated_delta_rule.py:159-203) and

@@ -45,41 +45,54 @@ bool staged_prologue(const lq_zoo_simple_gla_args* a) {
   return true;
 }
 
-// Offsets of the intermediates for the dims in `a` (64-token chunks; chunk sizes above 64 keep the 64-token layouts)
-int plan(const lq_zoo_simple_gla_args* a, Layout* l, bool force_scan) {
+bool has_prologue(const lq_zoo_simple_gla_args* a) { return a->signs_qk || a->signs_v || a->dq; }
+
+int check_dims(const lq_zoo_simple_gla_args* a) {
   if (a->batch <= 0 || a->seqlen <= 0 || a->nheads <= 0 || a->kdim <= 0 || a->vdim <= 0) return LQ_ERR_SHAPE;
   const int cs = a->chunk_size;
   if (cs != 64 && cs != 128 && cs != 192 && cs != 256) return LQ_ERR_SHAPE;
-  if (a->seqlen % cs != 0) return LQ_ERR_SHAPE;
+  return a->seqlen % cs == 0 ? LQ_OK : LQ_ERR_SHAPE;
+}
+
+// Offsets of the intermediates for the dims in `a` (chunk sizes above 64 keep the 64-token layouts)
+Layout plan(const lq_zoo_simple_gla_args* a, bool scan) {
+  Layout l;
+  const int cs = a->chunk_size;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
-  const bool scan = l->scan = cs == 64 && (force_scan || linear_scan(B, T, H, K, V)), codes = cs == 64 && !scan;
+  const bool codes = !scan && has_prologue(a);  // token-major local codes of q, k, v
+  l.scan = scan;
   int64_t off = 0;
-  l->kqT = off, off += up(B * NT * H * K * 64);
-  l->vqT = off, off += up(B * NT * H * V * 64);
-  l->gam = off, off += up(B * NT * H * K * 4);
-  l->vcT = off, off += scan || codes ? up(B * NT * H * V * 64) : 0;  // (codes: token-major local codes of q, k, v)
-  l->qc = off, off += scan || codes ? up(B * NT * H * K * 64) : 0;
-  l->kc = off, off += codes ? up(B * NT * H * K * 64) : 0;
-  l->A = off, off += scan ? up(B * NT * H * 8192) : 0;
-  l->gpk = off, off += scan ? up(B * NT * H * 256) : 0;
-  l->gc = off, off += scan ? 0 : up(B * T * H * 4);
-  l->ev = off, off += scan ? 0 : up(B * T * H * 4);
-  l->h_i8 = off, off += scan ? 0 : up(B * (T / cs) * H * V * K);
-  l->cross = off, off += scan ? 0 : up(B * T * H * V * 4);
-  l->total = off;
-  return LQ_OK;
+  auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
+  take(l.kqT, B * NT * H * K * 64);
+  take(l.vqT, B * NT * H * V * 64);
+  take(l.gam, B * NT * H * K * 4);
+  take(l.vcT, scan || codes ? B * NT * H * V * 64 : 0);
+  take(l.qc, scan || codes ? B * NT * H * K * 64 : 0);
+  take(l.kc, codes ? B * NT * H * K * 64 : 0);
+  take(l.A, scan ? B * NT * H * 8192 : 0);
+  take(l.gpk, scan ? B * NT * H * 256 : 0);
+  take(l.gc, scan ? 0 : B * T * H * 4);
+  take(l.ev, scan ? 0 : B * T * H * 4);
+  take(l.h_i8, scan ? 0 : B * (T / cs) * H * V * K);
+  take(l.cross, cs == 64 ? 0 : B * T * H * V * 4);
+  l.total = off;
+  return l;
+}
+
+bool scan_route(const lq_zoo_simple_gla_args* a) {
+  return a->chunk_size == 64 && linear_scan(a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
 }
 
 }  // namespace
 
 extern "C" int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* a, int64_t* bytes) {
   if (!a || !bytes) return LQ_ERR_NULL;
-  // (64-token chunks: the route of a call with a prologue depends on its pointers, so the size is enough for either)
-  Layout l, s;
-  int rc = plan(a, &l, false);
-  if (rc == LQ_OK) rc = plan(a, &s, true);
-  if (rc != LQ_OK) return rc;
-  *bytes = l.total > s.total ? l.total : s.total;
+  if (const int rc = check_dims(a)) return rc;
+  *bytes = plan(a, scan_route(a)).total;
+  if (a->chunk_size == 64 && has_prologue(a)) {  // its route depends on the tables' addresses too: enough for either
+    const int64_t other = plan(a, !scan_route(a)).total;
+    if (other > *bytes) *bytes = other;
+  }
   return LQ_OK;
 }
 
@@ -88,12 +101,12 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
   if (!a->sq || !a->sk || !a->skw || !a->svw || !a->svl || !a->ss) return LQ_ERR_NULL;
   if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
   // what a call with a prologue may be does not depend on its route: checked here, in front of the first launch of either
-  const bool prologue = a->signs_qk || a->signs_v || a->dq;
+  const bool prologue = has_prologue(a);
   if (prologue && a->chunk_size != 64) return LQ_ERR_SHAPE;
   if (!zoo_al(a->signs_qk, 16) || !zoo_al(a->signs_v, 16) || (a->signs_v && a->vdim != 64 && a->vdim != 128)) return LQ_ERR_SHAPE;
-  Layout l;
-  int rc = plan(a, &l, prologue && !staged_prologue(a));
+  int rc = check_dims(a);
   if (rc != LQ_OK) return rc;
+  const Layout l = plan(a, scan_route(a) || (prologue && !staged_prologue(a)));
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
   const int decay = a->g ? LQ_DECAY_SCALAR : LQ_DECAY_NONE;

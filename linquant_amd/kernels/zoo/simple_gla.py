@@ -92,10 +92,11 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
     gf = None if g is None else C.f32(g)
     dq, dq_rcp = C.dqk_tables(dqk, H, K)
     sg_qk, sg_v = [None if t is None else _lib.aligned(C.f32(t).reshape(n)) for t, n in ((signs_qk, K), (signs_v, V))]
-    key = (B, T, H, K, V, span)
+    rotated = dict(signs_qk=_lib.ptr(sg_qk), signs_v=_lib.ptr(sg_v), dq=_lib.ptr(dq))
+    key = (B, T, H, K, V, span, any(p is not None for p in rotated.values()))
     nbytes = _WS_BYTES.get(key)
     if nbytes is None:
-        st = _lib.fill("lq_zoo_simple_gla_args", batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span)
+        st = _lib.fill("lq_zoo_simple_gla_args", batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span, **rotated)
         n = ctypes.c_int64(0)
         rc = _lib.load().lq_zoo_simple_gla_workspace_bytes(ctypes.byref(st), ctypes.byref(n))
         if rc != 0:
@@ -108,8 +109,7 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
               o_is_f32=int(o.dtype == torch.float32), ht=_lib.ptr(ht), sq=_lib.ptr(sc["q"]), sk=_lib.ptr(sc["k"]),
               skw=_lib.ptr(skw), svw=_lib.ptr(svw), svl=_lib.ptr(svl), ss=_lib.ptr(ss), eta=float(eta), scale=float(scale),
               qmax=int(qmax), batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span, act_dtype=C.act_code(v),
-              workspace=_lib.ptr(ws), workspace_bytes=nbytes, signs_qk=_lib.ptr(sg_qk), signs_v=_lib.ptr(sg_v), dq=_lib.ptr(dq),
-              dq_rcp=_lib.ptr(dq_rcp))
+              workspace=_lib.ptr(ws), workspace_bytes=nbytes, dq_rcp=_lib.ptr(dq_rcp), **rotated)
     return o, ht
 
 

@@ -221,3 +221,23 @@ def test_tensors_that_are_not_on_a_gpu_are_refused_before_the_library_is_entered
     assert not entered
     _lib.call("lq_zoo_cumsum", torch.device("cuda"), batch=1)
     assert entered == ["lq_zoo_cumsum"]
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128)])
+def test_workspace_of_a_call_without_a_prologue_has_no_room_for_one(K, V):
+    """lq_zoo_simple_gla on a few long chains (state and output launches): write codes, chunk decays, cumulative decay and value factors
+    and stored states, each rounded up to 256 bytes, and nothing else; a call with the prologue needs its local codes on top; chunks of
+    128 tokens the fp32 cross workspace."""
+    B, T, H = 1, 64 * 400, 2
+    up = lambda n: -(-n // 256) * 256  # noqa: E731
+
+    def size(chunk=64, **kw):
+        st, n = _lib.fill("lq_zoo_simple_gla_args", batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=chunk, **kw), ctypes.c_int64(0)
+        assert _lib.load().lq_zoo_simple_gla_workspace_bytes(ctypes.byref(st), ctypes.byref(n)) == 0
+        return n.value
+
+    chunks = B * (T // 64) * H
+    bare = up(chunks * K * 64) + up(chunks * V * 64) + up(chunks * K * 4) + 2 * up(B * T * H * 4) + up(chunks * K * V)
+    assert size() == bare
+    assert size(signs_qk=16) >= bare + chunks * 64 * (2 * K + V)
+    assert size(chunk=128) == bare - up(chunks * K * V) + up(chunks // 2 * K * V) + up(B * T * H * V * 4)
