@@ -206,8 +206,8 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->kqT, B * NT * H * K * 64);
   take(l->vqT, delta ? 0 : B * NT * H * V * 64);
   take(l->wq, delta ? B * T * H * K : 0);
-  take(l->ev, B * T * H * 4);
-  take(l->gam, B * NT * H * K * 4);
+  take(l->ev, l->scan ? 0 : B * T * H * 4);
+  take(l->gam, l->scan && delta ? 0 : B * NT * H * K * 4);  // (delta family: zoo_scan.hip reads them and fw from the pack)
   take(l->pack, delta && !big ? B * NT * H * (128 + K) * 4 : 0);
   take(l->A, diag || !big ? B * T * H * 64 * 2 : 0);
   take(l->Ax, diag && big ? B * T * H * 64 * 2 : 0);
@@ -217,7 +217,7 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->Hw, delta && (diag || big) ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
   take(l->U, delta ? B * T * H * V * 2 : 0);
-  take(l->fw, delta ? B * T * H * 4 : 0);
+  take(l->fw, delta && !l->scan ? B * T * H * 4 : 0);
   take(l->e_out, delta && !l->scan ? B * T * H * V * 2 : 0);
   take(l->h_i8, l->scan ? 0 : B * (T / cs) * H * V * K);
   take(l->cross, big ? B * T * H * V * 4 : 0);
@@ -258,14 +258,14 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   int8_t* kqT = (int8_t*)(ws + l.kqT);
   int8_t* vqT = delta ? nullptr : (int8_t*)(ws + l.vqT);
   int8_t* wq = delta ? (int8_t*)(ws + l.wq) : nullptr;
-  float* ev = (float*)(ws + l.ev);
-  float* gam = (float*)(ws + l.gam);
+  float* ev = l.scan ? nullptr : (float*)(ws + l.ev);
+  float* gam = l.scan && delta ? nullptr : (float*)(ws + l.gam);
   float* pack = delta && !big ? (float*)(ws + l.pack) : nullptr;
   void* Hw = delta && (diag || big) ? ws + l.Hw : nullptr;
   void* W = delta && big ? ws + l.W : nullptr;
   void* U = delta ? ws + l.U : nullptr;
-  float* fw = delta ? (float*)(ws + l.fw) : nullptr;
-  void* e_out = delta ? ws + l.e_out : nullptr;
+  float* fw = delta && !l.scan ? (float*)(ws + l.fw) : nullptr;
+  void* e_out = delta && !l.scan ? ws + l.e_out : nullptr;
   int8_t* h_i8 = (int8_t*)(ws + l.h_i8);
   void* A = diag || !big ? ws + l.A : nullptr;
   void* Ax = diag && big ? ws + l.Ax : nullptr;

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* _
 // tile it holds (what lq_zoo_write_codes would make from the stored gc and logenv; same arithmetic, same bits):
 //   kqT[k][t] = q8(key[t][k] * exp(gk_last - gk_t - eta*le_t), 1/skw[k]),  vqT[v][t] = q8(val[t][v] * exp(eta*le_t), 1/svw[v]),
 //   ev[t] = exp(eta*le_t),  gam[k] = exp(gk_last),
-// and, when vcT is set, the local value codes q8(val[t][v], 1/svl[v]) that the output wants (zoo_op_values).
+// and, when vcT is set, the local value codes q8(val[t][v], 1/svl[v]) that the output wants (zoo_op_values; ev may be NULL then).
 struct CumsumCodes {
   const uint16_t* k;
   const uint16_t* v;
@@ -158,7 +158,7 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
         logenv[(row0 + ph * CT + t) * H + h] = m;
         if constexpr (CODES) {
           le_s[t] = m;
-          cc.ev[(row0 + t) * H + h] = zoo_exp(cc.eta * m);
+          if (cc.ev) cc.ev[(row0 + t) * H + h] = zoo_exp(cc.eta * m);
         }
       }
     }
@@ -262,7 +262,7 @@ int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl
     CumsumCodes cc = {};
     const dim3 grid((unsigned)((int64_t)a->batch * NT * a->nheads)), block(4 * a->kdim);
     if (a->kqT) {
-      if (!a->k || !a->v || !a->vqT || !a->ev || !a->gam || !a->skw || !a->svw) return LQ_ERR_NULL;
+      if (!a->k || !a->v || !a->vqT || (!a->ev && !vcT) || !a->gam || !a->skw || !a->svw) return LQ_ERR_NULL;
       if (a->chunk_size != 64 || a->vdim <= 0 || a->qmax < 1 || a->qmax > 127) return LQ_ERR_SHAPE;
       if (a->act_dtype != LQ_DT_F16 && a->act_dtype != LQ_DT_BF16) return LQ_ERR_SHAPE;
       if (!zoo_al(a->kqT, 16) || !zoo_al(a->vqT, 16)) return LQ_ERR_SHAPE;

@@ -304,13 +304,13 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
     dk_s[tid] = p.dk_div[h * K + tid];
     dk_s[128 + tid] = p.dk_rcp[h * K + tid];
   }
-  // ---- per-token factors; fw is written straight out
+  // ---- per-token factors; fw is written straight out (SCAN: only packed, with ev and gam)
   if (tid < 64) {
     const float bt = p.beta[(t0 + tid) * H + h];
     bs_s[tid] = powb(bt, sigma);
     bh_s[tid] = powb(bt, 1.0f - sigma);
     const float fwv = powb(bt, (1.0f - sigma) * (1.0f - tau));
-    p.fw[(t0 + tid) * H + h] = fwv;
+    if (!SCAN) p.fw[(t0 + tid) * H + h] = fwv;
     if constexpr (CODES) {
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + tid] = fwv;
     }
@@ -319,12 +319,12 @@ __global__ __launch_bounds__(256, 4) void zoo_wy_prep_kernel(WyParams p) {
     // per-token value factor and per-channel chunk decay, as lq_zoo_write_codes writes them
     if (tid < 64) {
       const float evv = zoo_exp(p.eta * p.logenv[(t0 + tid) * H + h]);
-      p.ev[(t0 + tid) * H + h] = evv;
+      if (!SCAN) p.ev[(t0 + tid) * H + h] = evv;
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + 64 + tid] = evv;
     }
     if (tid < K) {
       const float gl = p.g[((t0 + 63) * H + h) * K + tid], gm = zoo_exp(gl);
-      p.gam[(((int64_t)b * p.NT + ct) * H + h) * K + tid] = gm;
+      if (!SCAN) p.gam[(((int64_t)b * p.NT + ct) * H + h) * K + tid] = gm;
       if (p.pack) p.pack[(((int64_t)b * p.NT + ct) * H + h) * (128 + K) + 128 + tid] = gm;
       glast_s[tid] = gl;
       iskw_s[tid] = 1.0f / p.skw[h * K + tid];
@@ -861,7 +861,7 @@ int launch(const WyParams& p, bool scan, dim3 grid, hipStream_t stream) {
 
 int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, const ZooWyLocal* local, hipStream_t stream) {
   const bool no_hw = scan && local;  // Hw itself is not wanted
-  if (!a || !a->k || !a->v || !a->beta || (!a->Hw && !no_hw) || !a->U || !a->fw) return LQ_ERR_NULL;
+  if (!a || !a->k || !a->v || !a->beta || (!a->Hw && !no_hw) || !a->U || (!a->fw && !scan)) return LQ_ERR_NULL;
   if (a->decay != LQ_DECAY_NONE && !a->g) return LQ_ERR_NULL;
   const bool codes = a->kqT != nullptr;
   if (scan && (!codes || !a->pack || (local != nullptr) != (a->decay != LQ_DECAY_DIAGONAL))) return LQ_ERR_SHAPE;
@@ -869,7 +869,7 @@ int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, const ZooWyLocal
     return LQ_ERR_NULL;
   if (local && !zoo_al(local->q, 16)) return LQ_ERR_SHAPE;
   if (!codes && !a->W) return LQ_ERR_NULL;
-  if (codes && (!a->wq || !a->ev || !a->gam || !a->skw || !a->sw)) return LQ_ERR_NULL;
+  if (codes && (!a->wq || (!scan && (!a->ev || !a->gam)) || !a->skw || !a->sw)) return LQ_ERR_NULL;
   if (codes && a->decay == LQ_DECAY_DIAGONAL && !a->logenv) return LQ_ERR_NULL;
   if (codes && (a->qmax < 1 || a->qmax > 127)) return LQ_ERR_SHAPE;
   if (codes && (!zoo_al(a->kqT, 16) || !zoo_al(a->wq, 4) || !zoo_al(a->skw, 16))) return LQ_ERR_SHAPE;
