@@ -188,8 +188,8 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     auto do_step = [&](int ct, Ops& cur, Ops& pre) __attribute__((always_inline)) {
       __builtin_amdgcn_sched_barrier(0);  // a request hoisted over the last use of its set would need registers of its own
       unsigned char* hTb = hT + (DELTA ? 0 : (ct & 1) * BV * HS);
-      misc_s[lane] = cur.misc;
       if constexpr (DELTA) {
+        misc_s[lane] = cur.misc;
         *(URaw*)(ue_s + (lane >> 2) * US + BV / 2 * (lane & 3)) = cur.uraw;
       }
       // stored copy of the incoming state -> LDS (V-major)
@@ -249,6 +249,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       }
 
       // write product and carry update
+      if constexpr (!DELTA) misc_s[lane] = cur.misc;  // (no earlier: with one set in flight the step would start with this wait)
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) {
         lq_v4i bop;
