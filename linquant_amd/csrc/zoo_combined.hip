@@ -17,12 +17,40 @@ struct Layout {
   bool scan;  // operand pre-pass, then recurrence and output in one launch
 };
 
-// Linear family, 64-token chunks: recurrence and output in one launch, or one after the other?  The chain is NT steps in either
-// case; a step that shares its SIMDs with the output takes about twice as long (K = 128: 1.0 us, 0.5 without), while an output launch
-// of its own uses the whole chip whatever the number of chains.  So few long chains keep the two launches (scalar decay B3 T21184 H5 K
-// = V = 128: 319 us, 397 in one), many chains (linear attention B4 T4096 H16: 176 us, 153 in one; GLA 317, 288) and short ones, where
-// launches count (Mamba-2 cell B1 T2048 H8 K = V = 64: 28 us, 24 in one), take the one.
-bool linear_scan(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) { return B * H * (V / 64) >= 64 || T / 64 * K <= 2048; }
+// Linear family, 64-token chunks: recurrence and output in one launch (zoo_scan.hip), or state and output one after the other?
+// The chain is NT steps either way, and a step that shares its SIMDs with the output is the longer one; the launch of its own has the
+// whole chip for the output.  What the one launch saves is launches (4 .. 6 us a call, which decides short calls), the stored states
+// (2 K V bytes a chunk and head) and the second reading of raw operands (with a prologue: of their token-major codes), against A
+// (16 KB) and one more set of codes.
+//   bytes saved > 0 (GLA; K = V = 128; with a prologue all but K = V = 64): one launch.
+//   else: one launch for short chains whose operands stay in the last-level cache.
+//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns), and more than 32 steps of a second tile per
+//   compute unit (more than 256) where not even 16 KB are saved: the two launches.
+// Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256:
+//                     T = 256     1024         2048         4096         8192        16384 tokens
+//   GLA K = V = 128   1.11..1.22  1.07..1.23   1.05..1.24   1.01..1.19   1.02..1.18   0.99..1.13
+//   GLA K = V = 64    1.12..1.22  1.04..1.12   1.01..1.15   0.98..1.12   0.97..1.15   0.92..1.08
+//   K = V = 128       1.17..1.60  1.06..1.31   1.03..1.27   0.91..1.27   0.95..1.26   0.87..1.13
+//     with prologue   1.16..1.29  1.05..1.21   1.02..1.25   1.01..1.24   1.00..1.22   0.97..1.14
+//   K 128, V 64       1.09..1.44  0.94..1.24   0.83..1.11   0.85..1.08   0.81..1.03   0.75..0.96
+//     B*H*NT <= 2048              1.00..1.24   1.01..1.11
+//     with prologue   1.18..1.41  1.05..1.30   1.03..1.18   1.01..1.14   0.97..1.08   0.88..1.03
+//   K 64, V 128       1.09..1.53  0.99..1.28   0.84..1.15   0.80..1.10   0.78..1.11   0.79..1.03
+//     B*H*NT <= 4096              1.01..1.28   1.00..1.15   0.99..1.10
+//     with prologue   1.27..1.48  1.12..1.29   1.01..1.27   0.94..1.21   0.89..1.15   0.94..1.09
+//     and B*H <= 64                                         1.09..1.21   0.97..1.15
+//   K = V = 64        1.09..1.39  0.81..1.18   0.72..1.08   0.72..1.00   0.67..0.97   0.65..0.91
+//     B*H*NT <= 1024              1.01..1.18   0.97..1.08
+//     with prologue   1.12..1.30  0.93..1.11   0.89..1.07   0.84..1.04   0.83..1.00   0.79..0.96
+//     B*H*NT <= 2048              0.99..1.11   0.98..1.07
+bool linear_scan(bool diag, bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
+  const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
+  if (NT > 128 && tiles < 128) return false;
+  const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
+  if (diag || saved >= 16384) return true;
+  if (saved > 0) return NT <= 32 || tiles <= 256;
+  return saved == 0 ? NT <= V / 2 && chunks <= 32 * V : NT <= 32 && chunks <= 1024;
+}
 
 // What the launches over 64-token chunks (operand pre-pass, zoo_scan.hip) ask of a call, checked in front of the first of them; the
 // same calls that the stage entry points take
@@ -80,7 +108,7 @@ Layout plan(const lq_zoo_simple_gla_args* a, bool scan) {
 }
 
 bool scan_route(const lq_zoo_simple_gla_args* a) {
-  return a->chunk_size == 64 && linear_scan(a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
+  return a->chunk_size == 64 && linear_scan(false, has_prologue(a), a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
 }
 
 }  // namespace
@@ -198,7 +226,7 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   if (a->family == LQ_FAMILY_LINEAR && a->decay != LQ_DECAY_DIAGONAL) return LQ_ERR_SHAPE;  // lq_zoo_simple_gla serves those
   const bool delta = a->family == LQ_FAMILY_DELTA, diag = a->decay == LQ_DECAY_DIAGONAL, big = cs == 128;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
-  l->scan = !big && (delta || linear_scan(B, T, H, K, V));
+  l->scan = !big && (delta || linear_scan(true, false, B, T, H, K, V));
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
   take(l->gc, a->decay == LQ_DECAY_NONE ? 0 : B * T * H * (diag ? K : 1) * 4);

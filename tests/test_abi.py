@@ -264,3 +264,21 @@ def test_workspace_of_the_recurrence_and_output_launch_holds_what_is_read(cell, 
     if decay == 1:
         want += 2 * up(chunks * 64 * 4)                                                   # cumulative decay, once by chunk and head
     assert n.value == want
+
+
+# both sides of every line of the rule: (B, H, T, K, V, recurrence and output in one launch)
+@pytest.mark.parametrize("B,H,T,K,V,one", [
+    (1, 32, 2048, 64, 64, True), (1, 33, 2048, 64, 64, False), (1, 8, 2112, 64, 64, False), (4, 64, 256, 64, 64, True),
+    (1, 64, 2048, 128, 64, True), (3, 23, 2048, 128, 64, False), (1, 64, 4096, 64, 128, True), (1, 8, 4160, 64, 128, False),
+    (1, 42, 2112, 64, 192, True), (1, 43, 2112, 64, 192, False), (1, 300, 2048, 64, 192, True), (1, 72, 4096, 128, 128, True),
+    (1, 31, 8192, 128, 128, True), (1, 31, 8256, 128, 128, False), (1, 32, 8256, 128, 128, True)])
+def test_route_of_the_linear_family_at_the_lines_of_its_rule(B, H, T, K, V, one):
+    """The workspace tells the route: only the one launch keeps A (8 KB a chunk and head), only the two keep the stored states."""
+    up = lambda n: -(-n // 256) * 256  # noqa: E731
+    chunks = B * H * (T // 64)
+    codes = up(chunks * K * 64) + up(chunks * V * 64) + up(chunks * K * 4)
+    scan = codes + up(chunks * V * 64) + up(chunks * K * 64) + up(chunks * 8192) + up(chunks * 256)
+    staged = codes + 2 * up(chunks * 256) + up(chunks * K * V)
+    st, n = _lib.fill("lq_zoo_simple_gla_args", batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=64), ctypes.c_int64(0)
+    assert _lib.load().lq_zoo_simple_gla_workspace_bytes(ctypes.byref(st), ctypes.byref(n)) == 0
+    assert scan != staged and n.value == (scan if one else staged)
