@@ -5,8 +5,8 @@ seqlen 8192, 80 heads x headdim 64, d_state 128, 1 group, chunk 256, key-side ab
 hot path over one batch resident in HBM: split/rotate/quantize prologue of B and C, rotation of the fp16 B
 used by the key-side chunk state, then cumsum -> chunk state -> INT8 state passing -> C.B^T -> chunk scan.
 
-Prints ONE JSON line: the whole-step throughput, a per-stage breakdown measured with HIP events on the
-launch stream, the roofline of the dominant kernel, and the CPU oracle timed on a bounded sample.  The default run
+Prints ONE JSON line: the whole-step throughput, a per-stage breakdown (headline: HIP events on the launch stream around the stage
+entry points, the same kernels; zoo: the profiler's records of the step's own launches), the roofline of the dominant kernel, and the CPU oracle timed on a bounded sample.  The default run
 also measures every other benchmark configuration (the six zoo cells of the first four configurations and the
 headline shape under weak decay) under the same protocol and reports them in the line's "configs" object.
 """
@@ -29,9 +29,9 @@ INT8_PEAK_TOPS = 5000.0  # published dense INT8 MFMA rate of MI355X; the measure
 STAGE_SOURCES = {
     "c5": {"prologue": "prologue_rotate_quant.hip", "chunk_cumsum": "mamba2_cumsum.hip", "chunk_state": "mamba2_chunk_state.hip",
            "state_passing": "mamba2_state_passing.hip", "bmm_chunk": "mamba2_bmm_chunk.hip", "chunk_scan": "mamba2_chunk_scan.hip"},
-    "zoo": {"prologue": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_prep": "zoo_wy_prep.hip", "gla_A": "zoo_gla_A.hip",
-            "write_codes": "zoo_write_codes.hip", "state": "zoo_state.hip", "output": "zoo_output.hip",
-            "rotate_quant": "zoo_rotate_quant.hip"},
+    "zoo": {"rotate": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_prep": "zoo_wy_prep.hip", "wy_ns": "zoo_wy_ns.hip",
+            "gla_A": "zoo_gla_A.hip", "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
+            "state": "zoo_state.hip", "output": "zoo_output.hip", "rotate_quant": "zoo_rotate_quant.hip"},
 }
 COUNTER_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "hbm_traffic_and_mfma_counters.md")
 
@@ -136,44 +136,50 @@ ZOO_CELLS = {"linear_none": ("linear", "none"), "mamba2": ("linear", "scalar"), 
              "deltanet": ("delta", "none"), "gated_deltanet": ("delta", "scalar"), "kda": ("delta", "diagonal")}
 
 
-def zoo_stage_bytes(fam, dec, B, T, H, K, V):
-    """Algorithmic HBM bytes per zoo stage: every tensor the stage must read or write, counted once."""
+def zoo_launch_bytes(workload):
+    """{launch: HBM bytes} of a zoo workload's call in 64-token chunks: every tensor the launch must read or write, counted once."""
+    cell, B, T, H, K, V, _ = ZOO_WORKLOADS[workload]
+    fam, dec = ZOO_CELLS[cell]
     qk, vv, tok = B * T * H * K * 2, B * T * H * V * 2, B * T * H * 4
-    g = 0 if dec == "none" else (tok if dec == "scalar" else B * T * H * K * 4)
-    h8 = B * (T // 64) * H * K * V
-    A = B * T * H * 64 * 4
-    out = {}
-    if dec != "none":
-        out["cumsum"] = 2 * g + (tok if dec == "diagonal" else 0)
-        if fam == "linear" and dec == "diagonal":  # the launch also reads k, v and writes the state kernel's write operands
-            out["cumsum"] += qk + vv + qk // 2 + vv // 2 + tok
-    if fam == "delta":
-        # k, v, beta, g (and the log envelope) in; Hw, U, fw and the state kernel's write operands (key write codes,
-        # state-read codes of W, value factor) out: W itself never leaves the chip
-        out["wy_prep"] = qk + vv + tok + g + (tok if dec == "diagonal" else 0) + qk + vv + tok + qk // 2 + qk // 2 + tok
+    kc, vc, A = qk // 2, vv // 2, B * T * H * 64 * 2  # INT8 codes of a key- / value-wide operand, the intra-chunk product
+    gam, pack = tok * K // 64, tok * (128 + K) // 64
+    sc = tok if dec == "scalar" else 0
+    out = {"rotate": 2 * qk * 2}
+    if dec == "scalar":
+        out["cumsum"] = 2 * tok
     if dec == "diagonal":
-        out["gla_A"] = 2 * qk + g + A // 2 + qk // 2  # A in fp16, INT8 codes of the decayed query
-    if fam == "linear" and dec != "diagonal":
-        # the state stage of the reference reads the fp16 operands; the split pipeline adds the INT8 code round trip
-        out["write_codes"] = qk + g + vv + (tok if dec == "diagonal" else 0) + qk // 2 + vv // 2
-    out["state"] = qk // 2 + h8 + ((qk // 2 + 2 * tok + 2 * vv) if fam == "delta" else vv // 2)
-    out["output"] = (2 * qk + g if dec != "diagonal" else qk // 2 + A // 2) + vv + h8 + vv
+        g = tok * K
+        out["cumsum"] = 2 * g + tok + (qk + vv + kc + 2 * vc + gam if fam == "linear" else 0)
+        out["wy_prep"] = qk + vv + tok + g + tok + qk + vv + 2 * kc + pack
+        out["gla_A"] = 2 * qk + g + A + kc
+    out["wy_ns"] = 2 * qk + vv + tok + sc + 3 * kc + vv + A + pack + sc
+    out["lin_prep"] = 2 * qk + vv + sc + 2 * kc + 2 * vc + A + gam + sc
+    out["scan"] = 2 * kc + A + sc + vv + (kc + vv + pack if fam == "delta" else 2 * vc + gam)
     return out
 
 
-def zoo_workload_bytes(workload):
-    """{stage: algorithmic bytes} of a zoo benchmark workload as bench_zoo runs it (the linear-attention configuration
-    takes the fused operand launch: q, k, v read once, five code tensors written, the output kernel reads codes)."""
-    cell, B, T, H, K, V, _ = ZOO_WORKLOADS[workload]
-    fam, dec = ZOO_CELLS[cell]
-    nbytes = zoo_stage_bytes(fam, dec, B, T, H, K, V)
-    nbytes["prologue"] = 2 * (B * T * H * K * 2) * 2  # q and k, read and written once
-    if fam == "linear" and dec != "diagonal" and workload != "c1":
-        qk_b, vv_b = B * T * H * K * 2, B * T * H * V * 2
-        nbytes["rotate_quant"] = 2 * qk_b + vv_b + 3 * (qk_b // 2) + 2 * (vv_b // 2)
-        nbytes["output"] = 2 * (qk_b // 2) + vv_b // 2 + B * (T // 64) * H * K * V + vv_b
-        nbytes.pop("write_codes", None)
-    return nbytes
+def launch_times(fn, reps):
+    """{launch: [ms, ...]} of the library's kernels in ``reps`` calls of ``fn``, in the order of their first launch, from the GPU
+    timestamps of the profiler's kernel records (several of these kernels leave one C call: no event of ours fits between them)."""
+    import re
+
+    import torch
+    from torch.autograd import DeviceType
+    from torch.profiler import ProfilerActivity, profile
+
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        for _ in range(reps):
+            fn()
+        torch.cuda.synchronize()
+    out = {}
+    for e in sorted((e for e in prof.events() if e.device_type == DeviceType.CUDA), key=lambda e: e.time_range.start):
+        m = re.search(r"(\w+)_kernel\b", e.name)
+        if m and (m.group(1).startswith("zoo_") or m.group(1).startswith("cumsum_")):
+            label = "cumsum" if m.group(1).startswith("cumsum_") else m.group(1)[4:]
+            out.setdefault(label, []).append(e.time_range.elapsed_us() * 1e-3)
+    return out
 
 
 def copy_probe(dev):
@@ -236,13 +242,12 @@ def timed_steps(step, warmup, steps, ramp_ms=0.0):
 
 
 def measure_zoo(args, workload, cpu_baseline):
-    """One step = the operand prologue + one chunk-forward call (cumsum, WY prep, A, state, output kernels) over inputs
-    resident in HBM.  Returns the JSON line as a dict."""
+    """One step = the operand prologue + one chunk-forward call over inputs resident in HBM; "stages" are the launches of that step.
+    Returns the JSON line as a dict."""
     import torch
 
     from linquant_amd import _lib
     from linquant_amd.kernels import zoo
-    from linquant_amd.kernels.zoo import _common as C
 
     _lib.load()
     dev = torch.device("cuda:0")
@@ -320,54 +325,30 @@ def measure_zoo(args, workload, cpu_baseline):
     ms_per_step, ramp_steps = timed_steps(lambda: call(sc), args.warmup, args.steps, 0.0 if args.no_ramp else RAMP_MS)
     tokens = B * T
 
-    records = {}
-    names = {"cumsum": "cumsum", "run_wy_prep": "wy_prep", "run_gla_A": "gla_A", "write_codes": "write_codes",
-             "rotate_quant": "rotate_quant", "state_kernel": "state", "run_output": "output"}
-    saved = {n: getattr(C, n) for n in names}
-
-    def timed(fn, label):
-        def wrapper(*a, **kw):
-            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            e0.record()
-            r = fn(*a, **kw)
-            e1.record()
-            records.setdefault(label, []).append((e0, e1))
-            return r
-        return wrapper
-
-    try:
-        for n, label in names.items():
-            setattr(C, n, timed(saved[n], label))
-        tp = timed(prologue, "prologue")
-        for _ in range(max(10, args.steps)):
-            if has_prologue:
-                tp()
-            kernels(sc, _staged=True)  # (the stage-by-stage route, where the call would issue its stages from one C call)
-        torch.cuda.synchronize()
-    finally:
-        for n, f in saved.items():
-            setattr(C, n, f)
-    nbytes = zoo_workload_bytes(workload)
+    records = launch_times(lambda: call(sc), max(10, args.steps))
+    nbytes = zoo_launch_bytes(workload) if chunk == 64 else {}  # (the byte model is that of the 64-token chunks)
     del qs, ks
     stages = {}
-    for label, evs in records.items():
-        ts = sorted(a.elapsed_time(b) for a, b in evs)
+    for label, ts in records.items():
+        ts = sorted(ts)
         med = statistics.median(ts)
         stages[label] = {"ms": round(med, 4), "p25": round(ts[len(ts) // 4], 4), "p75": round(ts[(3 * len(ts)) // 4], 4)}
-        if chunk == 64:  # (the byte model below is that of the 64-token route)
+        if label in nbytes:
             stages[label].update({"MB": round(nbytes[label] / 1e6, 1), "GBps": round(nbytes[label] / 1e6 / med, 1),
                                   "hbm_frac": round(nbytes[label] / 1e6 / med / HBM_PEAK_GBS, 4)})
-    dom = max((n for n in stages if n in nbytes), key=lambda n: stages[n]["ms"])
-    avg_dom = statistics.mean(a.elapsed_time(b) for a, b in records[dom])
-    achieved = nbytes[dom] / 1e6 / avg_dom
-    roofline = {"kernel": "zoo_" + dom, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "avg_ms": round(avg_dom, 4),
-                "algorithmic_MB": round(nbytes[dom] / 1e6, 1)}
+    dom = max((n for n in stages if n in nbytes), key=lambda n: stages[n]["ms"], default=None)
+    roofline = None
+    if dom is not None:
+        avg_dom = statistics.mean(records[dom])
+        achieved = nbytes[dom] / 1e6 / avg_dom
+        roofline = {"kernel": "zoo_" + dom, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "avg_ms": round(avg_dom, 4),
+                    "algorithmic_MB": round(nbytes[dom] / 1e6, 1)}
     counters, mfma_peak = measured_counters(workload, "zoo") if chunk == 64 else ({}, None)
     for label, rec in counters.items():
         if label in stages:
             stages[label].update({k: v for k, v in rec.items() if k in ("traffic_MB", "mfma_busy_frac")})
-    if "traffic_MB" in counters.get(dom, {}):
+    if roofline is not None and "traffic_MB" in counters.get(dom, {}):
         roofline["traffic"] = int(counters[dom]["traffic_MB"] * 1e6)
 
     cpu = None
