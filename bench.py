@@ -125,12 +125,12 @@ def stage_bytes(s, keyside):
 
 ZOO_WORKLOADS = {
     # name: (cell, B, T, H, K, V, description) -- shapes of the first four benchmark configurations
-    "c1": ("mamba2", 1, 2048, 8, 64, 64, "configs[0]: Mamba-2 cell (linear family, scalar decay) B=1 T=2048 H=8 K=V=64 chunk 64"),
-    "c2_la": ("linear_none", 4, 4096, 16, 128, 128, "configs[1]: linear attention B=4 T=4096 H=16 K=V=128 chunk 64, q,k pre-rotated"),
-    "c2_gla": ("gla", 4, 4096, 16, 128, 128, "configs[1]: GLA B=4 T=4096 H=16 K=V=128 chunk 64, local R_QK in the A kernel"),
-    "c3_deltanet": ("deltanet", 4, 4096, 16, 128, 128, "configs[2]: DeltaNet B=4 T=4096 H=16 K=V=128 chunk 64, sigma=0.5"),
-    "c3_gdn": ("gated_deltanet", 4, 4096, 16, 128, 128, "configs[2]: Gated DeltaNet B=4 T=4096 H=16 K=V=128 chunk 64, sigma=0.5"),
-    "c4_kda": ("kda", 2, 8192, 32, 128, 128, "configs[3]: KDA B=2 T=8192 H=32 K=V=128 chunk 64, local R_QK in the A kernel"),
+    "c1": ("mamba2", 1, 2048, 8, 64, 64, "Mamba-2 cell (linear family, scalar decay) B=1 T=2048 H=8 K=V=64 chunk 64"),
+    "c2_la": ("linear_none", 4, 4096, 16, 128, 128, "linear attention B=4 T=4096 H=16 K=V=128 chunk 64, q,k pre-rotated"),
+    "c2_gla": ("gla", 4, 4096, 16, 128, 128, "GLA B=4 T=4096 H=16 K=V=128 chunk 64, local R_QK in the A kernel"),
+    "c3_deltanet": ("deltanet", 4, 4096, 16, 128, 128, "DeltaNet B=4 T=4096 H=16 K=V=128 chunk 64, sigma=0.5"),
+    "c3_gdn": ("gated_deltanet", 4, 4096, 16, 128, 128, "Gated DeltaNet B=4 T=4096 H=16 K=V=128 chunk 64, sigma=0.5"),
+    "c4_kda": ("kda", 2, 8192, 32, 128, 128, "KDA B=2 T=8192 H=32 K=V=128 chunk 64, local R_QK in the A kernel"),
 }
 ZOO_CELLS = {"linear_none": ("linear", "none"), "mamba2": ("linear", "scalar"), "gla": ("linear", "diagonal"),
              "deltanet": ("delta", "none"), "gated_deltanet": ("delta", "scalar"), "kda": ("delta", "diagonal")}
@@ -326,6 +326,8 @@ def measure_zoo(args, workload, cpu_baseline):
     tokens = B * T
 
     records = launch_times(lambda: call(sc), max(10, args.steps))
+    if sum(statistics.median(ts) for ts in records.values()) < 0.25 * ms_per_step:
+        records = {}  # (another profiler holds the kernel timestamps: this one's records are not durations then)
     nbytes = zoo_launch_bytes(workload) if chunk == 64 else {}  # (the byte model is that of the 64-token chunks)
     del qs, ks
     stages = {}
@@ -383,8 +385,8 @@ def measure_zoo(args, workload, cpu_baseline):
     graph = None
     if args.graph or workload == "c1":
         # the same step captured once in a HIP graph and replayed: no host work between the launches.  The first
-        # configuration is small enough for the eager step to be bound by the launching thread (about 12 us of Python and
-        # launch per kernel); the replay shows what the kernels themselves take
+        # configuration is small enough for the eager step to be bound by the launching thread; the replay shows what the
+        # kernels themselves take
         gr = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -401,7 +403,7 @@ def measure_zoo(args, workload, cpu_baseline):
         "metric": f"prefill tokens/s per layer at T={T}", "value": round(tokens / ms_per_step * 1e3, 1), "unit": "tokens/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms_per_step, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int8", "data": "synthetic",
-        "config": {"workload": f"{workload} = BASELINE.json {desc}; fp16 activations, static absmax scales"
+        "config": {"workload": f"{workload}: {desc}; fp16 activations, static absmax scales"
                                + ("" if chunk == 64 else f"; run in {chunk}-token chunks instead of the configuration's 64"),
                    "tokens_per_step": tokens, "ramp": ramp_note(ramp_steps),
                    "prologue": "in the timed step: R_QK on q, k" if has_prologue else
@@ -828,7 +830,7 @@ def measure_c5(args, regime, keyside, cpu_baseline, with_graph=False):
         "metric": "prefill tokens/s per layer at T=8192", "value": round(tokens / ms_per_step * 1e3, 1), "unit": "tokens/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms_per_step, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int8", "data": "synthetic",
-        "config": {"workload": "mamba2-2.7b-shape SSD layer INT8 prefill (BASELINE.json configs[4]): B=4 L=8192 H=80 P=64 "
+        "config": {"workload": "mamba2-2.7b-shape SSD layer INT8 prefill: B=4 L=8192 H=80 P=64 "
                                "N=128 G=1 chunk=256, " + ("key-side" if keyside else "value-side") + " absorption, "
                                "prologue + 5 SSD stages", "tokens_per_step": tokens,
                    "ramp": ramp_note(ramp_steps),
@@ -861,7 +863,7 @@ def compact(line, keep_cpu):
 
 def other_configs(args, keyside):
     """Every benchmark configuration other than the headline, measured in the same run under the same protocol (ramp,
-    --warmup untimed steps, --steps timed steps): the six zoo cells of configs[0..3] and the headline's shape under weak
+    --warmup untimed steps, --steps timed steps): the six zoo cells and the headline's shape under weak
     decay, where its data-dependent shortcuts find nothing to leave out.  The first configuration, which the CPU oracle
     finishes in seconds, carries its CPU baseline."""
     import gc

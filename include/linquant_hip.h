@@ -443,7 +443,8 @@ int lq_zoo_output(const lq_zoo_output_args* args, hipStream_t stream);
 /* replaces chunk_simple_gla_int8 as a whole (linquant/kernels/zoo/simple_gla.py:175-212; rotated storage, raw operands):
  * what lq_zoo_cumsum (scalar decay only), lq_zoo_write_codes, lq_zoo_state and lq_zoo_output make one after the other, on
  * `stream` over one caller-supplied workspace that holds the intermediates; the bits of the four calls.  64-token chunks run
- * as an operand pre-pass and one launch for recurrence and output.  Field meanings as in the per-stage structs. */
+ * as an operand pre-pass and one launch for recurrence and output, or as the four launches where those are faster (by the
+ * dims and whether there is a prologue).  Field meanings as in the per-stage structs. */
 typedef struct {
   const void* q;             /* (B,T,H,K) fp16/bf16 */
   const void* k;             /* (B,T,H,K) */
@@ -481,8 +482,8 @@ int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* args, int64_
  * chunk_kda_int8 (kda.py:154-203) as a whole (rotated storage): the stage entry points above in the order the wrappers
  * issue them -- cumsum, WY prep (delta family), write-codes pre-pass (128-token chunks; 64-token chunks make them in the
  * cumsum / WY launch), A kernel (per-channel decay), state recurrence, output -- on `stream` over one caller-supplied
- * workspace that holds every intermediate.  Same kernels and bits as the separate calls; one foreign call and one
- * allocation per forward.  family x decay: linear x diagonal = GLA; delta x none = DeltaNet, delta x scalar = Gated
+ * workspace that holds every intermediate; 64-token chunks (GLA: where it is faster) run recurrence and output as one launch.
+ * The bits of the separate calls; one foreign call and one allocation per forward.  family x decay: linear x diagonal = GLA; delta x none = DeltaNet, delta x scalar = Gated
  * DeltaNet, delta x diagonal = KDA (linear x none / scalar: lq_zoo_simple_gla).  Field meanings as in the per-stage structs. */
 typedef struct {
   const void* q;             /* (B,T,H,K) fp16/bf16 */

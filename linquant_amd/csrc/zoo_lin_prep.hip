@@ -8,8 +8,8 @@
 // One 8-wave workgroup per (chunk, batch*head), two to a compute unit (registers): load (a thread takes four adjacent tokens x 8
 // channels; every row is read once) while one wave forms the cumulative decay | rotate and quantize into LDS | operands
 // out as whole 1 KB tiles and 64-byte rows, blocks of A on the INT8 MFMA.  Linear attention with the rotations, B4 T4096 H16 K = V =
-// 128: 91 us for 201 MB read and 168 MB written (4.1 TB/s), vector instructions 70 us of it; with zoo_scan.hip 153 us for the whole
-// call, 176 as operand, state and output launches.  The Mamba-2 cell B1 T2048 H8 K = V = 64: 28.0 -> 24.3 us.
+// 128: 85 to 93 us for 201 MB read and 168 MB written (4.0 to 4.3 TB/s), vector instructions 70 us of it; with zoo_scan.hip 157 us for
+// the whole call, 176 as operand, state and output launches.  The Mamba-2 cell B1 T2048 H8 K = V = 64: 28.0 -> 23.4 us.
 #include <type_traits>
 
 #include "zoo_params.h"

@@ -16,8 +16,8 @@
 // runs half a step behind: E of a chunk becomes local codes between the chain's second and the next first rendezvous, and the
 // chunk's local product and store follow after that one.
 //
-// Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 64 us, KDA B2 T8192 H32 157 +
-// 128 -> 135 us, KDA B1 T2048 H8 41 + 7 -> 36 us (25 with 16 columns).  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
+// Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 67 us, KDA B2 T8192 H32 157 +
+// 128 -> 137 us, KDA B1 T2048 H8 41 + 7 -> 36 us (25 with 16 columns).  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
 // carry, 300 to issue its requests, 1000 for state read and E, 300 for the update; one workgroup of 32 columns per compute unit
 // at the first two shapes.
 //
@@ -44,7 +44,8 @@ using ScanParams = ZooScanParams;
 
 // BV: value columns per workgroup.  32, and 16 where 32 would leave half of the 256 compute units or more without a workgroup: a
 // step is bound by the vector instructions of the two waves of a SIMD, and half the columns are little more than half of them
-// (32 -> 16 columns: no / scalar decay B1 T2048 H8 K = V = 64 21.4 -> 15.9 us, KDA B1 T2048 H8 K = V = 128 36.7 -> 25.2 us).  From
+// (32 -> 16 columns: scalar decay B1 T2048 H8 K = V = 64 21.4 -> 15.9 us, 14 with two operand sets; KDA B1 T2048 H8 K = V = 128 36.7 ->
+// 25.2 us).  From
 // more than half of the compute units on, a second workgroup of 16 columns would only repeat what does not depend on the columns.
 template <bool DELTA, int K, int BV>
 struct ChainOps {

@@ -18,12 +18,14 @@
 //     1.1e-4, 0.9e-4 (1.2e-4, 1.2e-4; 1.3e-4, 1.6e-4); bf16 5.0e-5, 4.5e-5 (fp32 form 9.5e-5, 8.7e-5).  The third fp16 piece costs 6
 //     us of 256 (Gated DeltaNet B4 T4096 H16, whole call).
 // An fp32 form of the same (operands scaled and staged as fp32, 32 fp32 MFMA steps per Gram block, T and X split in three bf16
-// pieces, six products) took 121 us at B4 T4096 H16 K = V = 128, of which the splitting and the fp32 steps were two thirds.
+// pieces, six products) took 121 us at B4 T4096 H16 K = V = 128, of which the splitting and the fp32 steps were two thirds, and left
+// the codes of q and the product A to the output kernel; this one takes 119 us with them (127 with scalar decay).
 //
 // One 8-wave workgroup per (chunk, batch*head), two to a compute unit (77 KB of LDS): load and quantize (every row is read once)
 // | Gram blocks and, MODE_SCAN, the blocks of the intra-chunk product A (20 blocks over the 8 waves) | G | inverse of the four
-// diagonal blocks by forward substitution | block columns of T, one wave each, in registers | products.  Bound by memory: 97 KB a
-// chunk.
+// diagonal blocks by forward substitution | block columns of T, one wave each, in registers | products.  Bound by
+// no unit alone: with scalar decay 410 MB are 81 us at the rate of a large copy and the vector instructions 82 us, of 127; between the
+// eight barriers two workgroups do not cover each other's waits.
 #include "zoo_params.h"
 
 namespace {

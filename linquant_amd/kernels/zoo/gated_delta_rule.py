@@ -2,7 +2,8 @@
 
 Call surface of linquant/kernels/zoo/gated_delta_rule.py:159-203: WY prep (Gram, triangular inverse,
 W = T.(beta^sigma k * exp(g)), U = T.(beta^sigma v)) -> state kernel with E = (U - W.S) * fw formed inside the
-chunk loop -> the simple_gla output kernel on (q, Hw, E).  The prep is always the native fp32 HIP kernel
+chunk loop -> the simple_gla output kernel on (q, Hw, E).  The prep is always the native HIP kernel: fp32 sums over exact
+half-precision k and v with the 24 bits of T in three half-precision pieces (64-token chunks), fp32 throughout (128)
 (``fla_prep`` is accepted for compatibility and ignored)."""
 
 from __future__ import annotations
@@ -33,7 +34,7 @@ def chunk_delta_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=1.0, s
     assert g is None or g.shape == (B, T, H)
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "w", "kw", "el", "ew", "state")}
     if unrot is None and _debug is None and not _staged:
-        # the whole forward as one C call over one workspace (same kernels and bits as the stage-by-stage route below)
+        # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
         o, ht = C.one_call_forward(C.FAMILY_DELTA, decay, q, k, v, None if g is None else C.f32(g), C.f32(beta), sc, dims, span,
                                    sigma=sigma, tau=tau, eta=eta, scale=scale, qmax=qmax, final_state=output_final_state,
                                    out_dtype=out_dtype)

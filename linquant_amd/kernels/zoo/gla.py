@@ -33,7 +33,7 @@ def chunk_gla_int8(q, k, v, g, scales, *, eta=0.0, scale=None, chunk_size=64, ou
     qmax = 2 ** (bits - 1) - 1
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "kw", "vw", "vl", "state")}
     if unrot is None and _debug is None and not _staged:
-        # the whole forward as one C call over one workspace (same kernels and bits as the stage-by-stage route below)
+        # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
         o, ht = C.one_call_forward(C.FAMILY_LINEAR, C.DECAY_DIAGONAL, q, k, v, C.f32(g), None, sc, dims, span, eta=eta, scale=scale,
                                    qmax=qmax, final_state=output_final_state, out_dtype=out_dtype, rot=R)
         return C.cut_values(restore(o), C.cut_keys(ht, K0), V0)

@@ -47,7 +47,7 @@ def chunk_kda_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=0.0, sca
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "w", "kw", "el", "ew", "state")}
     dq, dq_rcp = C.dqk_tables(dqk, H, K)
     if unrot is None and _debug is None and not _staged:
-        # the whole forward as one C call over one workspace (same kernels and bits as the stage-by-stage route below)
+        # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
         o, ht = C.one_call_forward(C.FAMILY_DELTA, C.DECAY_DIAGONAL, q, k, v, C.f32(g), C.f32(beta), sc, dims, span, sigma=sigma,
                                    tau=tau, eta=eta, scale=scale, qmax=qmax, final_state=output_final_state, out_dtype=out_dtype,
                                    rot=R, dq=dq, dq_rcp=dq_rcp)

@@ -118,9 +118,9 @@ def test_chunk_size_128_linear_family(cuda, cell, eta, rot, K, V, dtype):
                                                        (32, 48, 96, torch.float16, torch.float32), (128, 128, 64, torch.float16, None),
                                                        (256, 64, 128, torch.float16, None)])
 def test_one_call_forward_equals_the_stage_by_stage_route(cuda, cell, chunk, K, V, dtype, out_dtype):
-    """chunk_simple_gla_int8 issues its stages from one C call over one workspace (lq_zoo_simple_gla) unless a caller asks
-    for the intermediates; both routes run the same kernels on the same operands: outputs and final states are equal bit
-    for bit, for every chunk size, with widened widths and an fp32 output."""
+    """chunk_simple_gla_int8 is one C call over one workspace (lq_zoo_simple_gla) unless a caller asks for the intermediates;
+    both routes do the same arithmetic in the same order: outputs and final states are equal bit for bit, for every chunk
+    size, with widened widths and an fp32 output."""
     from linquant_amd.kernels import zoo
 
     T = 4 * max(chunk, 64)
@@ -143,9 +143,9 @@ def test_one_call_forward_equals_the_stage_by_stage_route(cuda, cell, chunk, K, 
                                                               (32, 48, 96, torch.float16, torch.float32, False),
                                                               (128, 128, 64, torch.float16, None, True), (96, 64, 128, torch.float16, None, False)])
 def test_one_call_forward_equals_the_stage_by_stage_route_other_cells(cuda, cell, chunk, K, V, dtype, out_dtype, extras):
-    """chunk_gla_int8, chunk_delta_int8 and chunk_kda_int8 issue their stages from one C call over one workspace
-    (lq_zoo_chunk_forward) unless a caller asks for canonical storage or the intermediates; both routes run the same kernels
-    on the same operands: outputs and final states are equal bit for bit.  ``extras``: the local R_QK (per-channel decay)
+    """chunk_gla_int8, chunk_delta_int8 and chunk_kda_int8 are one C call over one workspace (lq_zoo_chunk_forward) unless a
+    caller asks for canonical storage or the intermediates; both routes do the same arithmetic in the same order: outputs and
+    final states are equal bit for bit.  ``extras``: the local R_QK (per-channel decay)
     and D_QK (KDA) as well."""
     from linquant_amd.kernels import zoo
     from oracle.zoo_reference import signed_hadamard

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("cell", list(zc.CELLS))
-# chunks: fewer than the operand sets in rotation (3 and 5), exactly as many, remainders of one and of all but one; grids that
+# chunks: fewer than the operand sets in rotation (3 and 2), exactly as many, remainders of one and of all but one; grids that
 # do and do not divide over the 8 XCDs; one and several V tiles per head, a V the operand prologue is not built for (192)
 @pytest.mark.parametrize("NT,B,H,K,V,dtype,out_dtype", [
     (1, 1, 1, 128, 64, torch.float16, None), (2, 1, 8, 64, 128, torch.bfloat16, None), (3, 2, 3, 128, 192, torch.float16, None),
@@ -21,7 +21,9 @@ pytestmark = pytest.mark.gpu
     # more workgroups than fit the chip at once in the last two
     (1, 5, 14, 64, 64, torch.float16, None), (2, 3, 23, 128, 64, torch.bfloat16, None), (3, 1, 36, 64, 128, torch.float16, torch.float32),
     (4, 2, 17, 128, 128, torch.bfloat16, None), (5, 5, 13, 64, 64, torch.bfloat16, torch.float32), (6, 3, 11, 128, 128, torch.float16, None),
-    (7, 1, 24, 128, 192, torch.bfloat16, None), (8, 9, 8, 128, 128, torch.float16, torch.float32), (3, 5, 27, 64, 128, torch.bfloat16, None)])
+    (7, 1, 24, 128, 192, torch.bfloat16, None), (8, 9, 8, 128, 128, torch.float16, torch.float32), (3, 5, 27, 64, 128, torch.bfloat16, None),
+    # more than 128 steps of few chains: the linear family's stages one after the other behind the same call, the delta family's one launch
+    (130, 1, 2, 128, 64, torch.bfloat16, None)])
 def test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype):
     from linquant_amd.kernels import zoo
     from oracle.zoo_reference import signed_hadamard
@@ -54,8 +56,10 @@ def test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell
 @pytest.mark.parametrize("cell,NT,B,H,K,V,dtype,parts", [
     ("linear_none", 2, 1, 3, 128, 128, torch.float16, ("signs_qk", "signs_v", "dqk")), ("mamba2", 3, 2, 4, 64, 128, torch.bfloat16, ("signs_v",)),
     ("mamba2", 1, 1, 1, 128, 64, torch.float16, ("signs_qk", "dqk")), ("linear_none", 4, 2, 2, 64, 64, torch.bfloat16, ("dqk",)),
-    # few long chains: the stages one after the other behind the same call; many: one launch again
+    # 40 chunks: one launch for few chains and for many
     ("mamba2", 40, 1, 2, 128, 64, torch.float16, ("signs_qk", "signs_v")), ("linear_none", 40, 4, 8, 128, 128, torch.bfloat16, ("signs_qk", "dqk")),
+    # the stages one after the other behind the same call: few chains of more than 128 steps; K = V = 64 and more than 2048 chunks
+    ("mamba2", 130, 1, 2, 128, 64, torch.float16, ("signs_qk", "signs_v")), ("linear_none", 40, 2, 32, 64, 64, torch.bfloat16, ("signs_qk", "dqk")),
     # 32 value columns per workgroup
     ("mamba2", 3, 5, 8, 128, 128, torch.bfloat16, ("signs_qk",)), ("mamba2", 2, 3, 23, 64, 64, torch.float16, ("signs_v", "dqk"))])
 def test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts):
