@@ -29,8 +29,8 @@ INT8_PEAK_TOPS = 5000.0  # published dense INT8 MFMA rate of MI355X; the measure
 STAGE_SOURCES = {
     "c5": {"prologue": "prologue_rotate_quant.hip", "chunk_cumsum": "mamba2_cumsum.hip", "chunk_state": "mamba2_chunk_state.hip",
            "state_passing": "mamba2_state_passing.hip", "bmm_chunk": "mamba2_bmm_chunk.hip", "chunk_scan": "mamba2_chunk_scan.hip"},
-    "zoo": {"rotate": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_prep": "zoo_wy_prep.hip", "wy_ns": "zoo_wy_ns.hip",
-            "gla_A": "zoo_gla_A.hip", "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
+    "zoo": {"rotate": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_ns": "zoo_wy_ns.hip", "diag_prep": "zoo_diag_prep.h",
+            "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
             "state": "zoo_state.hip", "output": "zoo_output.hip", "rotate_quant": "zoo_rotate_quant.hip"},
 }
 COUNTER_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "hbm_traffic_and_mfma_counters.md")
@@ -149,9 +149,7 @@ def zoo_launch_bytes(workload):
         out["cumsum"] = 2 * tok
     if dec == "diagonal":
         g = tok * K
-        out["cumsum"] = 2 * g + tok + (qk + vv + kc + 2 * vc + gam if fam == "linear" else 0)
-        out["wy_prep"] = qk + vv + tok + g + tok + qk + vv + 2 * kc + pack
-        out["gla_A"] = 2 * qk + g + A + kc
+        out["diag_prep"] = 2 * qk + vv + g + A + 2 * kc + (tok + kc + vv + pack if fam == "delta" else 2 * vc + gam)
     out["wy_ns"] = 2 * qk + vv + tok + sc + 3 * kc + vv + A + pack + sc
     out["lin_prep"] = 2 * qk + vv + sc + 2 * kc + 2 * vc + A + gam + sc
     out["scan"] = 2 * kc + A + sc + vv + (kc + vv + pack if fam == "delta" else 2 * vc + gam)

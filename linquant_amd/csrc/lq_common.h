@@ -93,7 +93,12 @@ LQ_DEV float lq_logf(float y) {
 // The float->int conversion saturates, the caller clamps to the code range.
 LQ_DEV int lq_rha_i32(float y) { return (int)(y + __builtin_copysignf(0.5f, y)); }
 
-LQ_DEV int lq_clampi(int v, int lo, int hi) { return min(max(v, lo), hi); }
+// lo <= hi: the median in one instruction (min and max are two, as the compiler does not know the order of run-time bounds)
+LQ_DEV int lq_clampi(int v, int lo, int hi) {
+  int r;
+  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(lo), "v"(hi));
+  return r;
+}
 
 // clamp(rha(y), -qmax, qmax)
 LQ_DEV int lq_q_rha(float y, int qmax) { return lq_clampi(lq_rha_i32(y), -qmax, qmax); }

@@ -232,6 +232,8 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   l->scan = !big && (delta || linear_scan(true, false, B, T, H, K, V));
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
+  // (per-channel decay, one launch in front of the recurrence: gc, logenv and Hw stay on the chip.  The call's workspace keeps the size
+  // that ABI 20 gives it)
   take(l->gc, a->decay == LQ_DECAY_NONE ? 0 : B * T * H * (diag ? K : 1) * 4);
   take(l->logenv, diag ? B * T * H * 4 : 0);
   take(l->kqT, B * NT * H * K * 64);
@@ -292,7 +294,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   float* ev = l.scan ? nullptr : (float*)(ws + l.ev);
   float* gam = l.scan && delta ? nullptr : (float*)(ws + l.gam);
   float* pack = delta && !big ? (float*)(ws + l.pack) : nullptr;
-  void* Hw = delta && (diag || big) ? ws + l.Hw : nullptr;
+  void* Hw = delta && big ? ws + l.Hw : nullptr;
   void* W = delta && big ? ws + l.W : nullptr;
   void* U = delta ? ws + l.U : nullptr;
   float* fw = delta && !l.scan ? (float*)(ws + l.fw) : nullptr;
@@ -305,8 +307,21 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   int8_t* vcT = l.scan && !delta ? (int8_t*)(ws + l.vcT) : nullptr;
   float* cross = big ? (float*)(ws + l.cross) : nullptr;
 
+  if (diag && l.scan) {  // everything in front of the recurrence in one launch
+    for (const void* x : {(const void*)a->rot, (const void*)a->dq, (const void*)a->dq_rcp, delta ? (const void*)a->skw : nullptr})
+      if (!zoo_al(x, 16)) return LQ_ERR_SHAPE;
+    ZooDiagParams d = {};
+    d.q = (const _Float16*)a->q, d.k = (const _Float16*)a->k, d.v = (const _Float16*)a->v, d.g = a->g, d.beta = a->beta;
+    d.rot = (const _Float16*)a->rot, d.dq = a->dq, d.dk_div = a->dq, d.dk_rcp = a->dq_rcp;
+    d.sq = a->sq, d.sk = a->sk, d.skw = a->skw, d.sw = a->sw, d.svw = a->svw, d.svl = a->svl;
+    d.A = (_Float16*)A, d.qc = qg, d.kqT = kqT, d.wq = wq, d.vqT = vqT, d.vcT = vcT, d.U = (_Float16*)U, d.gam = gam, d.pack = pack;
+    d.sigma = a->sigma, d.tau = a->tau, d.eta = a->eta, d.scale = a->scale, d.qmax = a->qmax, d.bf = a->act_dtype == LQ_DT_BF16;
+    d.B = a->batch, d.T = a->seqlen, d.H = a->nheads, d.V = a->vdim, d.NT = a->seqlen / 64;
+    rc = delta ? zoo_diag_kda_launch(d, a->kdim, stream) : zoo_diag_gla_launch(d, a->kdim, stream);
+    if (rc != LQ_OK) return rc;
+  }
   // (every stage validates its own arguments before it launches: see lq_zoo_simple_gla)
-  if (a->decay != LQ_DECAY_NONE) {
+  if (a->decay != LQ_DECAY_NONE && !(diag && l.scan)) {
     lq_zoo_cumsum_args c = {};
     c.g = a->g, c.gc = gc, c.logenv = logenv, c.batch = a->batch, c.seqlen = a->seqlen, c.nheads = a->nheads;
     c.kdim = diag ? a->kdim : 0, c.chunk_size = a->chunk_size;
@@ -314,9 +329,9 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
       c.k = a->k, c.v = a->v, c.kqT = kqT, c.vqT = vqT, c.ev = ev, c.gam = gam, c.skw = a->skw, c.svw = a->svw;
       c.eta = a->eta, c.qmax = a->qmax, c.vdim = a->vdim, c.act_dtype = a->act_dtype;
     }
-    if ((rc = zoo_cumsum_launch(&c, vcT, a->svl, stream)) != LQ_OK) return rc;
+    if ((rc = lq_zoo_cumsum(&c, stream)) != LQ_OK) return rc;
   }
-  if (delta) {
+  if (delta && !(diag && l.scan)) {
     lq_zoo_wy_prep_args w = {};
     w.k = a->k, w.v = a->v, w.beta = a->beta, w.g = gc, w.Hw = Hw, w.W = W, w.U = U, w.fw = fw, w.sigma = a->sigma, w.tau = a->tau;
     w.batch = a->batch, w.seqlen = a->seqlen, w.nheads = a->nheads, w.kdim = a->kdim, w.vdim = a->vdim, w.chunk_size = a->chunk_size;
@@ -326,7 +341,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
       w.dk_div = a->dq, w.dk_rcp = a->dq_rcp, w.pack = pack;
     }
     const ZooWyLocal local = {a->q, qg, A, gpk, a->sq, a->sk, a->scale};
-    if ((rc = zoo_wy_prep_launch(&w, l.scan, l.scan && !diag ? &local : nullptr, stream)) != LQ_OK) return rc;
+    if ((rc = zoo_wy_prep_launch(&w, l.scan, l.scan ? &local : nullptr, stream)) != LQ_OK) return rc;
   }
   if (big) {
     lq_zoo_write_codes_args w = {};
@@ -336,12 +351,12 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     w.decay = a->decay, w.act_dtype = a->act_dtype;
     if ((rc = lq_zoo_write_codes(&w, stream)) != LQ_OK) return rc;
   }
-  if (diag) {
+  if (diag && !l.scan) {
     lq_zoo_gla_A_args g = {};
     g.q = a->q, g.k = delta ? Hw : a->k, g.g = gc, g.A = A, g.qg = qg, g.rot = a->rot, g.sq = a->sq, g.sk = a->sk, g.scale = a->scale;
     g.qmax = a->qmax, g.batch = a->batch, g.seqlen = a->seqlen, g.nheads = a->nheads, g.kdim = a->kdim, g.chunk_size = a->chunk_size;
     g.act_dtype = a->act_dtype, g.dq = a->dq, g.A_cross = Ax;
-    if ((rc = zoo_gla_A_launch(&g, l.scan, stream)) != LQ_OK) return rc;
+    if ((rc = lq_zoo_gla_A(&g, stream)) != LQ_OK) return rc;
   }
   if (l.scan) {
     ZooScanParams s = {};

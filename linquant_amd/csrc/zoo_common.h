@@ -42,6 +42,17 @@ static inline bool zoo_al(const void* q, int n) { return ((uintptr_t)q % n) == 0
 // Triton kernels.  Large negative arguments give 0, never NaN.
 LQ_DEV float zoo_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f); }
 
+// exp with the argument's rounding made good: x log2(e) = t + lo, 2^t (1 + lo ln 2).  zoo_exp's relative error grows with |x| (x = -12:
+// up to 6e-7, five units in the last place), this one's does not.
+LQ_DEV float zoo_exp_acc(float x) {
+  const float t = x * 1.44269504088896340736f;
+  float lo = __builtin_fmaf(x, 1.44269504088896340736f, -t);
+  lo = __builtin_fmaf(x, 1.9259629911266175e-08f, lo);
+  const float y = __builtin_amdgcn_exp2f(t);
+  const float z = __builtin_fmaf(y, lo * 0.693147180559945309f, y);
+  return z == z ? z : y;  // (x infinite: lo is not a number)
+}
+
 // ---- activation dtype: q, k, v (and the prepared Hw, W, U, E) are fp16 or bf16; `bf` is uniform per launch.
 // Pointers are typed _Float16* for their 2-byte element stride only.
 LQ_DEV void zoo_dec2(uint32_t w, bool bf, float& lo, float& hi) {

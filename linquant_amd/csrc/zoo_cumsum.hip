@@ -49,19 +49,16 @@ __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* _
 // Write operands of the linear family's state kernel under per-channel decay, made by the cumsum launch from the decay
 // tile it holds (what lq_zoo_write_codes would make from the stored gc and logenv; same arithmetic, same bits):
 //   kqT[k][t] = q8(key[t][k] * exp(gk_last - gk_t - eta*le_t), 1/skw[k]),  vqT[v][t] = q8(val[t][v] * exp(eta*le_t), 1/svw[v]),
-//   ev[t] = exp(eta*le_t),  gam[k] = exp(gk_last),
-// and, when vcT is set, the local value codes q8(val[t][v], 1/svl[v]) that the output wants (zoo_op_values; ev may be NULL then).
+//   ev[t] = exp(eta*le_t),  gam[k] = exp(gk_last).
 struct CumsumCodes {
   const uint16_t* k;
   const uint16_t* v;
   int8_t* kqT;
   int8_t* vqT;
-  int8_t* vcT;
   float* ev;
   float* gam;
   const float* skw;
   const float* svw;
-  const float* svl;
   float eta;
   int qmax;
   int V;
@@ -158,7 +155,7 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
         logenv[(row0 + ph * CT + t) * H + h] = m;
         if constexpr (CODES) {
           le_s[t] = m;
-          if (cc.ev) cc.ev[(row0 + t) * H + h] = zoo_exp(cc.eta * m);
+          cc.ev[(row0 + t) * H + h] = zoo_exp(cc.eta * m);
         }
       }
     }
@@ -185,10 +182,10 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
     pack();
     // The codes leave through the dead envelope tile as whole contiguous pieces, 16 bytes per thread: straight from the registers a
     // thread's 16 tokens were a quarter of a 64-byte row (and 8-byte halves of the operand-ordered ones), the rest of each line
-    // written by other waves (GLA B4 T4096 H16 K = V = 128: 107 -> 92 us).  K rows of 64 codes per buffer and pass, three buffers.
+    // written by other waves (GLA B4 T4096 H16 K = V = 128: 107 -> 92 us).  K rows of 64 codes per buffer and pass, two buffers.
     const int nb = K * 64;
     unsigned char* kb = (unsigned char*)tile;
-    unsigned char *vb = kb + nb, *lb = vb + nb;
+    unsigned char* vb = kb + nb;
     const int at = 16 * threadIdx.x;
     __syncthreads();  // the tile has been read
     *(lq_v4i*)(kb + k * 64 + 16 * q) = o;
@@ -206,29 +203,17 @@ __global__ void cumsum_diag_kernel(const float* __restrict__ g, float* __restric
         for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf) * zoo_exp(cc.eta * le_s[16 * q + t]), inv_svw, cc.qmax);
         pack();
         *(lq_v4i*)(vb + k * 64 + 16 * q) = o;
-        if (cc.vcT) {
-          const float inv_svl = 1.0f / cc.svl[h * V + c];
-#pragma unroll
-          for (int t = 0; t < 16; ++t) code[t] = zoo_q8(zoo_dec1(vraw[t], bf), inv_svl, cc.qmax);
-          pack();
-          unsigned char* dst = lb + zoo_op_values(k, 16 * q);
-          *(lq_v2i*)dst = lq_v2i{o[0], o[1]};
-          *(lq_v2i*)(dst + 256) = lq_v2i{o[2], o[3]};  // the next group of eight tokens
-        }
       }
       __syncthreads();
       if (c0 == 0) *(lq_v4i*)(cc.kqT + cb * nb + at) = *(const lq_v4i*)(kb + at);
-      if (at < min(K, V - c0) * 64) {
-        *(lq_v4i*)(cc.vqT + (cb * V + c0) * 64 + at) = *(const lq_v4i*)(vb + at);
-        if (cc.vcT) *(lq_v4i*)(cc.vcT + (cb * V + c0) * 64 + at) = *(const lq_v4i*)(lb + at);  // (V is a multiple of 64 then, K 64 or 128)
-      }
+      if (at < min(K, V - c0) * 64) *(lq_v4i*)(cc.vqT + (cb * V + c0) * 64 + at) = *(const lq_v4i*)(vb + at);
     }
   }
 }
 
 }  // namespace
 
-int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl, hipStream_t stream) {
+extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) {
   if (!a || !a->g || !a->gc) return LQ_ERR_NULL;
   if (a->batch <= 0 || a->seqlen <= 0 || a->nheads <= 0 || a->chunk_size <= 0 || a->kdim < 0) return LQ_ERR_SHAPE;
   if (a->seqlen % a->chunk_size != 0) return LQ_ERR_SHAPE;
@@ -262,13 +247,12 @@ int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl
     CumsumCodes cc = {};
     const dim3 grid((unsigned)((int64_t)a->batch * NT * a->nheads)), block(4 * a->kdim);
     if (a->kqT) {
-      if (!a->k || !a->v || !a->vqT || (!a->ev && !vcT) || !a->gam || !a->skw || !a->svw) return LQ_ERR_NULL;
+      if (!a->k || !a->v || !a->vqT || !a->ev || !a->gam || !a->skw || !a->svw) return LQ_ERR_NULL;
       if (a->chunk_size != 64 || a->vdim <= 0 || a->qmax < 1 || a->qmax > 127) return LQ_ERR_SHAPE;
       if (a->act_dtype != LQ_DT_F16 && a->act_dtype != LQ_DT_BF16) return LQ_ERR_SHAPE;
       if (!zoo_al(a->kqT, 16) || !zoo_al(a->vqT, 16)) return LQ_ERR_SHAPE;
       cc.k = (const uint16_t*)a->k, cc.v = (const uint16_t*)a->v, cc.kqT = a->kqT, cc.vqT = a->vqT, cc.ev = a->ev, cc.gam = a->gam;
       cc.skw = a->skw, cc.svw = a->svw, cc.eta = a->eta, cc.qmax = a->qmax, cc.V = a->vdim, cc.bf = a->act_dtype == LQ_DT_BF16;
-      cc.vcT = vcT, cc.svl = svl;
       hipLaunchKernelGGL(cumsum_diag_kernel<true>, grid, block, lds, stream, a->g, a->gc, a->logenv, a->seqlen, a->nheads,
                          a->kdim, a->chunk_size, cc);
     } else if (big) {
@@ -281,5 +265,3 @@ int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl
   }
   return lq_check_launch();
 }
-
-extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) { return zoo_cumsum_launch(a, nullptr, nullptr, stream); }

@@ -1,0 +1,4 @@
+// The DIAG_A form of the per-channel decay pre-pass (zoo_diag_prep.h)
+#include "zoo_diag_prep.h"
+
+int zoo_diag_a_launch(const ZooDiagParams& p, int K, hipStream_t stream) { return zoo_diag::launch<DIAG_A>(p, K, stream); }

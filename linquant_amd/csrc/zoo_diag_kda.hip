@@ -1,0 +1,4 @@
+// The DIAG_KDA form of the per-channel decay pre-pass (zoo_diag_prep.h)
+#include "zoo_diag_prep.h"
+
+int zoo_diag_kda_launch(const ZooDiagParams& p, int K, hipStream_t stream) { return zoo_diag::launch<DIAG_KDA>(p, K, stream); }

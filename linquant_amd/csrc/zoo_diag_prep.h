@@ -1,0 +1,849 @@
+// Everything in front of the chunk recurrence under per-channel (diagonal) decay, 64-token chunks: cumulative log decay and its
+// envelope, key (and value) write codes, state-read codes of the queries, the intra-chunk product A and, for the delta rule, the
+// WY / UT transform.  One kernel in four forms:
+//   DIAG_GLA, DIAG_KDA  all of it in one launch, from the model's tensors to the operands of zoo_scan.hip
+//   DIAG_A              lq_zoo_gla_A: A and the state-read codes, from the cumulative decay
+//   DIAG_WY             lq_zoo_wy_prep: the transform (and its write codes), from the cumulative decay
+// The stage forms run the code of the fused ones, so one call and the stages one after the other give the same bits.
+// Replaces the torch prep of the reference's wrappers (linquant/kernels/zoo/gla.py:249-251, kda.py:22-53, 168-170) and its kernels
+// _gla_A_inter (gla.py:27-63) and _gla_A_intra (gla.py:66-99).  With g the cumulative log decay, a_J its row 16J:
+//   A   off-diagonal block (I > J):  q8(q_i e^(g_i - a_I) scale . R, 1/sq) . q8(Hw_j e^(a_I - g_j) . R, 1/sk) * (sq sk)
+//       diagonal block:              sum_n q8(q_i scale)[n] q8(Hw_j)[n] e^(g_i - g_j)[n] * (sq sk),  j <= i
+//   G[i][j] = beta_i^sigma beta_j^(1-sigma) sum_n k_i[n] k_j[n] e^(g_i - g_j)[n] for i > j,  T = (I + G)^-1
+//   W = T (beta^sigma k e^g),  U = T (beta^sigma v),  Hw = beta^((1-sigma) tau) k,  fw = beta^((1-sigma)(1-tau))
+//
+// The exponentials are what a separate kernel per product repeats (and what the vector unit issues at a quarter of its rate):
+// here an element takes e+ = e^(g - a_J) and e- = e^(a_J - g), J its own 16-token sub-block, and the key write code's.  A sub-block's
+// key operand for a later one is e- times a factor per channel, e^(a_I - a_J); the state read and W's operand are e+ times e^(a_J).
+// Both e+ and e- are used where the decay inside the sub-block spreads over no more than e^40; otherwise (per wave) the operands
+// take one exponential each and the diagonal blocks one per (i, j, channel).
+//
+// One 4-wave workgroup per (chunk, batch*head), two to a compute unit (80 KB of LDS, 256 registers).  Wave J owns sub-block J; lane
+// (rl, kg) holds its token rl, channels 32ks + 8kg + e, which is the layout of every MFMA operand built from them.
+//   1  running sums in fp64, one channel per thread, into LDS          2  own rows: codes, diagonal blocks, e+ k into LDS
+//   3  key operands of the later sub-blocks, Gram blocks               4  rotation: 9 operands x 32 channels per wave, R in registers
+//   5  INT8 products; inverse of the diagonal blocks                   6  block columns of T          7  W, U on the fp32 MFMA
+//
+// Measured (kernel time): KDA B2 T8192 H32 K = V = 128 with rotation and D_QK: cumsum 81 + WY prep 307 + A kernel 209 us -> 501; GLA
+// B4 T4096 H16 K = V = 128: cumsum with codes 86 + A kernel 118 -> 165; KDA B1 T2048 H8 8 + 21 + 24 -> 27.  Bound by instruction
+// issue: at KDA's shape the vector instructions are 261 us of a SIMD's time (4.7 cycles each) and the fp32 MFMA 152 us, during which
+// its SIMD issues no vector instruction (measured: 33 cycles a 16x16x4, the cycles of the instructions between them on top; the
+// half-precision MFMA costs them only its issue).
+#pragma once
+
+#include <type_traits>
+
+#include "zoo_params.h"
+
+enum { DIAG_A = 0, DIAG_WY = 1, DIAG_GLA = 2, DIAG_KDA = 3 };
+
+namespace zoo_diag {
+
+LQ_DEV lq_v4f mfma_f32(float a, float b, lq_v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+LQ_DEV float powb(float b, float e) {
+  if (e == 0.0f) return 1.0f;
+  if (e == 1.0f) return b;
+  return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(b));
+}
+
+// float index of (token, channel) in the 64 x K tile.  Sub-block J and 32 channels are 2 KB: piece p of four channels of token rl is
+// 16-byte slot 16p + (rl + p) % 16, so that a lane's reads (pieces 2kg, 2kg + 1 of token rl), the running sums' writes (one token, 64
+// channels) and the transposed reads of W's operand (16 channels, tokens 4kg + s) all spread over the banks.
+template <int K>
+LQ_DEV int at(int token, int ch) {
+  const int p = (ch >> 2) & 7;
+  return (((token >> 4) * (K / 32) + (ch >> 5)) * 128 + p * 16 + ((token + p) & 15)) * 4 + (ch & 3);
+}
+
+// byte of the transposed write codes [channel][64 tokens]: 16 bytes of pad after every eight channels
+LQ_DEV int ct_at(int ch, int token) { return ch * 64 + (ch >> 3) * 16 + token; }
+
+// 16 x 16 blocks of T (lower triangle; the diagonal ones hold G first) and of G below the diagonal, rows of 20 floats
+constexpr int kBP = 20;
+constexpr int kBlk = 16 * kBP;
+LQ_DEV int t_blk(int I, int J) { return (I * (I + 1) / 2 + J) * kBlk; }
+LQ_DEV int g_blk(int I, int J) { return I == J ? t_blk(I, I) : (10 + I * (I - 1) / 2 + J) * kBlk; }
+
+// pair (J, I), J < I, of sub-blocks: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
+LQ_DEV int pair_of(int J, int I) { return (J == 0 ? -1 : (J == 1 ? 1 : 2)) + I; }
+
+constexpr int maxi(int a, int b) { return a > b ? a : b; }
+
+template <int K, bool ROT, int MODE, bool DK>
+struct Lds {
+  static constexpr bool DO_A = MODE != DIAG_WY, DELTA = MODE == DIAG_WY || MODE == DIAG_KDA, KQ = MODE != DIAG_A;
+  static constexpr int OP = 16 * K * 2, CD = 16 * K;  // bytes of an fp16 operand and of its codes
+  static constexpr int r1 = 0;                        // decay tile, then e+ k; GLA: value codes; U: v
+  static constexpr int r2 = 64 * K * 4;
+  static constexpr int X = ROT ? OP : CD;             // an operand as its wave leaves it
+  static constexpr int F_bytes = 6 * K * 4, GT_bytes = DELTA ? 16 * kBlk * 4 : 0, KQ_bytes = KQ ? K * 64 + K * 2 : 0;
+  // operands (3 queries, 6 keys) | then their codes, blocks of G and T behind them.  The write codes pass through the key
+  // operands' place, the fp64 totals through the queries'; the channel factors F lie at the end, dead when G is written.
+  static constexpr int kq = r2 + (DO_A ? 3 * X : 0);
+  static constexpr int gt = r2 + (DO_A ? 9 * CD : 0);
+  static constexpr int area = maxi(maxi((DO_A ? maxi(9 * X, 3 * X + KQ_bytes) : KQ_bytes) + F_bytes, gt - r2 + GT_bytes), 4 * K * 8);
+  static constexpr int F = r2 + area - F_bytes;
+  static constexpr int an = r2 + area;                // decay rows 0, 16, 32, 48, 63
+  static constexpr int E = an + 5 * K * 4;            // e^(a_J)
+  static constexpr int iskw = E + 4 * K * 4;
+  static constexpr int dq = iskw + (KQ ? K * 4 : 0);
+  static constexpr int dkd = dq + (DK && DO_A ? K * 4 : 0);
+  static constexpr int dkr = dkd + (DK && DELTA ? K * 4 : 0);
+  static constexpr int bs = dkr + (DK && DELTA ? K * 4 : 0);
+  static constexpr int bytes = bs + 64 * 4;
+};
+
+template <int K, bool ROT, bool BF, int MODE, bool DK>
+__global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) {
+  using L = Lds<K, ROT, MODE, DK>;
+  constexpr bool FUSED = MODE == DIAG_GLA || MODE == DIAG_KDA, DO_A = L::DO_A, DELTA = L::DELTA;
+  constexpr int KS = K / 32;      // steps of 32 channels
+  constexpr int SEG = K / 4;      // tokens per thread where a thread takes one channel
+  __shared__ __align__(16) unsigned char lds[L::bytes];
+  float* const R1 = (float*)(lds + L::r1);
+  float* const F_s = (float*)(lds + L::F);
+  float* const AN = (float*)(lds + L::an);
+  float* const E_s = (float*)(lds + L::E);
+  float* const iskw_s = (float*)(lds + L::iskw);
+  float* const dq_s = (float*)(lds + L::dq);
+  float* const dkd_s = (float*)(lds + L::dkd);
+  float* const dkr_s = (float*)(lds + L::dkr);
+  float* const bs_s = (float*)(lds + L::bs);  // beta^sigma per token; GLA: e^(eta * envelope)
+  float* const GT = (float*)(lds + L::gt);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rl = lane & 15, kg = lane >> 4;
+  // Flat grid: workgroup L = x + 8 m (x = its XCD) takes head m % H of (batch, chunk) number x + 8 (m / H): the workgroups
+  // resident on one XCD cover all heads of a few (batch, chunk)s, so rows and (B, T, H) tensors are fetched and written as whole lines
+  const uint32_t ngroups = (uint32_t)p.B * (uint32_t)p.NT;
+  uint32_t group, hh;
+  if ((ngroups & 7u) == 0) {
+    const uint32_t m = blockIdx.x >> 3;
+    hh = m % (uint32_t)p.H;
+    group = (blockIdx.x & 7u) + 8u * (m / (uint32_t)p.H);
+  } else {
+    hh = blockIdx.x % (uint32_t)p.H;
+    group = blockIdx.x / (uint32_t)p.H;
+  }
+  const int h = (int)hh;
+  const int H = p.H, V = p.V, qmax = p.qmax;
+  const int64_t t0 = (int64_t)group * 64;        // (b * T + chunk * 64: T is a multiple of 64)
+  const int64_t cb = (int64_t)group * H + h;
+  constexpr bool bf = BF;
+  const int J = wave;                            // sub-block of this wave
+  const int tok = 16 * J + rl;                   // token of this lane
+  const int col = tid % K, seg = wave / (K / 64);  // one channel per thread: tokens SEG * seg .. (uniform over the wave)
+
+  // ---- requests of the chunk
+  float gv[FUSED ? SEG : 1];
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) {
+      const float* row = p.g + ((t0 + SEG * seg + t) * H + h) * K;  // (a scalar: the lane adds 32 bits)
+      gv[t] = row[(uint32_t)col];
+    }
+  }
+  const int64_t roff = ((t0 + tok) * H + h) * K + 8 * kg;
+  lq_v4i kraw[KS], qraw[DO_A ? KS : 1];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    kraw[ks] = *(const lq_v4i*)(p.k + roff + 32 * ks);
+    if constexpr (DO_A) qraw[ks] = *(const lq_v4i*)(p.q + roff + 32 * ks);
+  }
+  float bt = 0.0f;
+  if constexpr (DELTA) bt = p.beta[(t0 + tok) * H + h];
+  const bool codes = FUSED || (MODE == DIAG_WY && p.kqT);
+  if (tid < K) {
+    if constexpr (L::KQ) iskw_s[tid] = codes ? 1.0f / p.skw[h * K + tid] : 0.0f;
+    if constexpr (DK && DO_A) dq_s[tid] = p.dq[h * K + tid];
+    if constexpr (DK && DELTA) dkd_s[tid] = p.dk_div[h * K + tid], dkr_s[tid] = p.dk_rcp[h * K + tid];
+  }
+
+  // ---- 1: cumulative log decay of the chunk into LDS
+  if constexpr (FUSED) {
+    double* part = (double*)(lds + L::r2);  // totals of the four 16-token quarters [4][K]
+    double pre[SEG];
+#pragma unroll
+    for (int qq = 0; qq < SEG / 16; ++qq) {
+      double run = 0.0;
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        run += (double)gv[16 * qq + t];
+        pre[16 * qq + t] = run;
+      }
+      part[(seg * (SEG / 16) + qq) * K + col] = run;
+    }
+    __syncthreads();
+    double off = 0.0;
+    float last = 0.0f;
+#pragma unroll
+    for (int Q = 0; Q < 4; ++Q) {
+      if (Q / (SEG / 16) == seg) {
+        const int qq = Q % (SEG / 16);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          const float x = (float)(off + pre[16 * qq + t]);
+          R1[at<K>(16 * Q + t, col)] = x;
+          if (t == 0) AN[Q * K + col] = x;
+          last = x;
+        }
+      }
+      off += part[Q * K + col];
+    }
+    if (seg == 64 / SEG - 1) {
+      AN[4 * K + col] = last;
+      const float gm = zoo_exp(last);
+      if constexpr (DELTA) p.pack[cb * (128 + K) + 128 + col] = gm; else p.gam[cb * K + col] = gm;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < K / 16; ++i) {
+      const int it = tid + 256 * i, t = it / (K / 4), n = 4 * (it % (K / 4));
+      const lq_v4f x = *(const lq_v4f*)(p.g + ((t0 + t) * H + h) * K + n);
+      *(lq_v4f*)(R1 + at<K>(t, n)) = x;
+      if ((t & 15) == 0) *(lq_v4f*)(AN + (t >> 4) * K + n) = x;
+      if (t == 63) {
+        *(lq_v4f*)(AN + 4 * K + n) = x;
+        if constexpr (DELTA) {
+          if (codes) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float gm = zoo_exp(x[e]);
+              p.gam[cb * K + n + e] = gm;
+              if (p.pack) p.pack[cb * (128 + K) + 128 + n + e] = gm;
+            }
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- 2: own rows.  gem: the decay of the lane's elements, later e-
+  const float* const an_s = AN + J * K;
+  float gem[KS][8];
+  float spread = 0.0f, le = -__builtin_inff();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int e4 = 0; e4 < 2; ++e4) {
+      const int n = 32 * ks + 8 * kg + 4 * e4;
+      const lq_v4f g4 = *(const lq_v4f*)(R1 + at<K>(tok, n)), a4 = *(const lq_v4f*)(an_s + n);
+      lq_v4f l4;
+      if constexpr (FUSED) l4 = *(const lq_v4f*)(AN + 4 * K + n);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        gem[ks][4 * e4 + e] = g4[e];
+        spread = fmaxf(spread, __builtin_fabsf(g4[e] - a4[e]));
+        if constexpr (FUSED) le = fmaxf(le, l4[e] - g4[e]);
+      }
+    }
+  const bool slow = __any(spread > 40.0f);  // (uniform over the wave)
+  float bs = 1.0f, bh = 1.0f, bw = 1.0f, el = 0.0f;
+  if constexpr (FUSED) {
+    le = fmaxf(le, __shfl_xor(le, 16));
+    le = fmaxf(le, __shfl_xor(le, 32));
+    el = p.eta * le;
+  } else if constexpr (MODE == DIAG_WY) {
+    if (codes) el = p.eta * p.logenv[(t0 + tok) * H + h];
+  }
+  if constexpr (DELTA) {
+    bs = powb(bt, p.sigma);
+    bh = powb(bt, 1.0f - p.sigma);
+    bw = powb(bt, (1.0f - p.sigma) * p.tau);
+    if (kg == 0) {
+      const float fwv = powb(bt, (1.0f - p.sigma) * (1.0f - p.tau)), evv = zoo_exp(el);
+      bs_s[tok] = bs;
+      if constexpr (!FUSED) {
+        p.fw[(t0 + tok) * H + h] = fwv;
+        if (codes) p.ev[(t0 + tok) * H + h] = evv;
+      }
+      if (codes && p.pack) p.pack[cb * (128 + K) + tok] = fwv, p.pack[cb * (128 + K) + 64 + tok] = evv;
+    }
+  } else if constexpr (MODE == DIAG_GLA) {
+    if (kg == 0) bs_s[tok] = zoo_exp(el);
+  }
+  // channel factors of this sub-block: e^(a_J), and e^(a_I - a_J) for the later ones (slow: a_I itself)
+  for (int n = lane; n < K; n += 64) {
+    const float a = an_s[n];
+    E_s[J * K + n] = zoo_exp(a);
+    for (int I = J + 1; I < 4; ++I) F_s[pair_of(J, I) * K + n] = slow ? AN[I * K + n] : zoo_exp(AN[I * K + n] - a);
+  }
+  __builtin_amdgcn_wave_barrier();
+
+  float sq = 0.0f, sk = 0.0f, inv_sq = 0.0f, inv_sk = 0.0f;
+  if constexpr (DO_A) sq = p.sq[h], sk = p.sk[h], inv_sq = 1.0f / sq, inv_sk = 1.0f / sk;
+  // eight channels of a key row: the caller's k, rescaled by D_QK
+  auto load_k = [&](lq_v4i raw, int n, float (&o)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)raw[d], bf, o[2 * d], o[2 * d + 1]);
+    if constexpr (DK && DELTA) {
+      const lq_v4f d0 = *(const lq_v4f*)(dkd_s + n), d1 = *(const lq_v4f*)(dkd_s + n + 4);
+      const lq_v4f r0 = *(const lq_v4f*)(dkr_s + n), r1 = *(const lq_v4f*)(dkr_s + n + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = zoo_round_act(zoo_div_rn(o[e], e < 4 ? d0[e & 3] : d1[e & 3], e < 4 ? r0[e & 3] : r1[e & 3]), bf);
+    }
+  };
+  auto load_q = [&](lq_v4i raw, int n, float (&o)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)raw[d], bf, o[2 * d], o[2 * d + 1]);
+    if constexpr (DK) {
+      const lq_v4f d0 = *(const lq_v4f*)(dq_s + n), d1 = *(const lq_v4f*)(dq_s + n + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = zoo_round_act(zoo_mul_rn(o[e], e < 4 ? d0[e & 3] : d1[e & 3]), bf);
+    }
+  };
+  // Hw = beta^((1-sigma) tau) k as it would be stored
+  auto hw_of = [&](const float (&k)[8], float w, float (&o)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = k[e];
+    if constexpr (DELTA) {
+      if (w != 1.0f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = zoo_round_act(zoo_mul_rn(w, k[e]), bf);
+      }
+    }
+  };
+
+  // diagonal blocks: A transposed (lane: row rl, columns 4kg + r), G (lane: column rl, rows 4kg + r)
+  lq_v4f dacc = {0.f, 0.f, 0.f, 0.f}, gacc = {0.f, 0.f, 0.f, 0.f};
+  lq_v4f dslow = dacc, gslow = gacc;
+  if (slow) {  // every (i, j, channel) weight on its own, masked before use
+#pragma unroll 1
+    for (int n = 0; n < K; n += 8) {
+      float ko[8], qo[8], go[8];
+      load_k(*(const lq_v4i*)(p.k + ((t0 + tok) * H + h) * K + n), n, ko);
+      if constexpr (DO_A) load_q(*(const lq_v4i*)(p.q + ((t0 + tok) * H + h) * K + n), n, qo);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) go[e] = R1[at<K>(tok, n + e)];
+#pragma unroll 1
+      for (int r = 0; r < 4; ++r) {
+        const int o = 4 * kg + r;  // the other token of the pair
+        float kj[8], hj[8];
+        load_k(*(const lq_v4i*)(p.k + ((t0 + 16 * J + o) * H + h) * K + n), n, kj);
+        float w = 1.0f;
+        if constexpr (DELTA) w = powb(p.beta[(t0 + 16 * J + o) * H + h], (1.0f - p.sigma) * p.tau);
+        hw_of(kj, w, hj);
+        float sd = 0.0f, sg = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float gj = R1[at<K>(16 * J + o, n + e)];
+          if constexpr (DO_A) {
+            const float wd = o <= rl ? zoo_exp(go[e] - gj) : 0.0f;
+            sd += ((float)zoo_q8(qo[e] * p.scale, inv_sq, qmax) * (float)zoo_q8(hj[e], inv_sk, qmax)) * wd;
+          }
+          if constexpr (DELTA) {
+            const float wg = o > rl ? zoo_exp(gj - go[e]) : 0.0f;
+            sg += (kj[e] * ko[e]) * wg;
+          }
+        }
+#pragma unroll
+        for (int r2 = 0; r2 < 4; ++r2)
+          if (r2 == r) dslow[r2] += sd, gslow[r2] += sg;
+      }
+    }
+  }
+
+  unsigned char* const xq = lds + L::r2 + L::X * (J - 1);  // this sub-block's query operand (none for the first)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int n = 32 * ks + 8 * kg;
+    float kf[8], qf[8], hf[8];
+    load_k(kraw[ks], n, kf);
+    if constexpr (DO_A) load_q(qraw[ks], n, qf);
+    if constexpr (DK && DELTA) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) kraw[ks][d] = (int)zoo_enc2(kf[2 * d], kf[2 * d + 1], bf);
+    }
+    hw_of(kf, bw, hf);
+    if constexpr (MODE == DIAG_WY) {
+      lq_v4i o;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) o[d] = (int)zoo_enc2(hf[2 * d], hf[2 * d + 1], bf);
+      *(lq_v4i*)(p.Hw + roff + 32 * ks) = o;
+    }
+    int ck[8], cs[8], cx[8];
+    float ge[8];
+    lq_v8h x;
+    lq_v4f kp[2];
+#pragma unroll
+    for (int e4 = 0; e4 < 2; ++e4) {
+      const lq_v4f a4 = *(const lq_v4f*)(an_s + n + 4 * e4);
+      lq_v4f l4, is4, E4;
+      if constexpr (L::KQ) l4 = *(const lq_v4f*)(AN + 4 * K + n + 4 * e4), is4 = *(const lq_v4f*)(iskw_s + n + 4 * e4);
+      if constexpr (DO_A) E4 = *(const lq_v4f*)(E_s + J * K + n + 4 * e4);
+#pragma unroll
+      for (int e_ = 0; e_ < 4; ++e_) {
+        const int e = 4 * e4 + e_;
+        const float g = gem[ks][e], d = g - a4[e_];
+        const float dl = d * 1.44269504088896340736f;
+        const float ep = __builtin_amdgcn_exp2f(dl), em = __builtin_amdgcn_exp2f(-dl);
+        if constexpr (DELTA) {
+          kp[e4][e_] = kf[e] * ep;
+          gacc = mfma_f32(kp[e4][e_], kf[e] * em, gacc);
+        }
+        if constexpr (DO_A) {
+          const float cq = (float)zoo_q8(qf[e] * p.scale, inv_sq, qmax), chw = (float)zoo_q8(hf[e], inv_sk, qmax);
+          dacc = mfma_f32(chw * em, cq * ep, dacc);
+          const float xv = zoo_mul_rn(qf[e] * ep, p.scale);
+          if constexpr (ROT) x[e] = (_Float16)xv; else cx[e] = zoo_q8(xv, inv_sq, qmax);
+          cs[e] = zoo_q8(xv * E4[e_], inv_sq, qmax);
+        }
+        if constexpr (L::KQ) ck[e] = zoo_q8(hf[e] * zoo_exp(l4[e_] - g - el), is4[e_], qmax);
+        ge[e] = em;
+      }
+    }
+    if (!slow) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) gem[ks][e] = ge[e];
+    }
+    if constexpr (DELTA) {
+      *(lq_v4f*)(R1 + at<K>(tok, n)) = kp[0];
+      *(lq_v4f*)(R1 + at<K>(tok, n + 4)) = kp[1];
+      asm volatile("" : "+v"(gacc));
+    }
+    if constexpr (DO_A) {
+      if (FUSED || p.qc) {
+        const lq_v2i o = {(int)zoo_pack_codes(cs[0], cs[1], cs[2], cs[3]), (int)zoo_pack_codes(cs[4], cs[5], cs[6], cs[7])};
+        *(lq_v2i*)(FUSED ? p.qc + cb * 64 * K + zoo_op_codes(tok, n, K) : p.qc + roff + 32 * ks) = o;
+      }
+      if (J > 0) {
+        if constexpr (ROT)
+          *(lq_v8h*)(xq + (ks * 64 + lane) * 16) = x;
+        else
+          *(lq_v2i*)(xq + (ks >> 1) * 1024 + lane * 16 + 8 * (ks & 1)) =
+              lq_v2i{(int)zoo_pack_codes(cx[0], cx[1], cx[2], cx[3]), (int)zoo_pack_codes(cx[4], cx[5], cx[6], cx[7])};
+      }
+      asm volatile("" : "+v"(dacc));
+    }
+    if constexpr (L::KQ) {
+      if (codes) {
+        // four adjacent lanes hold tokens 4Q .. 4Q+3 of the same eight channels: bytes are transposed among them, lane j of the
+        // four keeps channels j and 4 + j, four tokens each
+        uint32_t w[2] = {zoo_pack_codes(ck[0], ck[1], ck[2], ck[3]), zoo_pack_codes(ck[4], ck[5], ck[6], ck[7])};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const uint32_t o1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[i], 0xB1, 0xf, 0xf, true);  // lane ^ 1
+          // even lane: channels 0, 2 of (own, other); odd lane: channels 1, 3 of (other, own)
+          const uint32_t m = __builtin_amdgcn_perm(rl & 1 ? w[i] : o1, rl & 1 ? o1 : w[i], rl & 1 ? 0x07030501u : 0x06020400u);
+          const uint32_t o2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+          w[i] = __builtin_amdgcn_perm(rl & 2 ? m : o2, rl & 2 ? o2 : m, rl & 2 ? 0x07060302u : 0x05040100u);
+        }
+        unsigned char* dst = lds + L::kq;
+        *(uint32_t*)(dst + ct_at(n + (rl & 3), 16 * J + (rl & 12))) = w[0];
+        *(uint32_t*)(dst + ct_at(n + 4 + (rl & 3), 16 * J + (rl & 12))) = w[1];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one step after the other
+  }
+  const float sqk = sq * sk;
+  // element (row, column) of A
+  auto a_store = [&](int row, int c, lq_v4f v) __attribute__((always_inline)) {
+    _Float16* dst = FUSED ? p.A + cb * 4096 + zoo_op_A(row, c) : p.A + ((t0 + row) * H + h) * 64 + c;
+    *(lq_v2i*)dst = lq_v2i{(int)zoo_pack_h2(v[0], v[1]), (int)zoo_pack_h2(v[2], v[3])};
+  };
+  if constexpr (DO_A) {
+    lq_v4f o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r <= rl ? zoo_mul_rn(slow ? dslow[r] : dacc[r], sqk) : 0.0f;
+    a_store(tok, 16 * J + 4 * kg, o);
+  }
+  // R in MFMA operand order: this wave rotates into channels 32 strip .., tile t takes the even / odd ones of them (a lane then
+  // ends up with eight adjacent channels)
+  constexpr int NS = K / 32, WPS = 4 / NS;
+  const int strip = wave % NS, part_of = wave / NS;
+  lq_v4i rop[ROT ? 2 : 1][KS];
+  if constexpr (ROT) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      uint32_t w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(p.rot + (32 * ks + 8 * kg + e) * K + 32 * strip + 2 * rl);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        rop[0][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x05040100u);
+        rop[1][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x07060302u);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- the write codes leave as whole rows
+  if constexpr (L::KQ) {
+    if (codes) {
+      lq_v4i o[K / 64];
+#pragma unroll
+      for (int i = 0; i < K / 64; ++i) {
+        const int it = tid + 256 * i;
+        o[i] = *(const lq_v4i*)(lds + L::kq + ct_at(it >> 2, 16 * (it & 3)));
+      }
+#pragma unroll
+      for (int i = 0; i < K / 64; ++i) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * (tid + 256 * i)) = o[i];
+    }
+    if constexpr (DO_A) __syncthreads();  // the key operands take their place
+  }
+
+  // ---- 3: key rows of this sub-block anchored at the first row of each later one: Gram blocks, operands of A
+  lq_v4f goff[3];
+#pragma unroll
+  for (int di = 0; di < 3; ++di) {
+    goff[di] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+    const int I = J + 1 + di;
+    if (I > 3) continue;  // (wave-uniform)
+    const int pr = pair_of(J, I);
+    unsigned char* const xk = lds + L::r2 + L::X * (3 + pr);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int n = 32 * ks + 8 * kg;
+      float kf[8], hf[8];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)kraw[ks][d], bf, kf[2 * d], kf[2 * d + 1]);
+      if constexpr (DO_A) hw_of(kf, bw, hf);
+      lq_v8h x;
+      int cx[8];
+      float we[8];
+      {
+        const lq_v4f f0 = *(const lq_v4f*)(F_s + pr * K + n), f1 = *(const lq_v4f*)(F_s + pr * K + n + 4);
+        if (!slow) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) we[e] = gem[ks][e] * (e < 4 ? f0[e & 3] : f1[e & 3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            we[e] = zoo_exp((e < 4 ? f0[e & 3] : f1[e & 3]) - gem[ks][e]);
+            asm volatile("" : "+v"(we[e]));  // (a branch, not a selection: the exponentials are not evaluated in vain)
+          }
+        }
+      }
+#pragma unroll
+      for (int e4 = 0; e4 < 2; ++e4) {
+        lq_v4f ki;
+        if constexpr (DELTA) ki = *(const lq_v4f*)(R1 + at<K>(16 * I + rl, n + 4 * e4));
+#pragma unroll
+        for (int e_ = 0; e_ < 4; ++e_) {
+          const int e = 4 * e4 + e_;
+          const float w = we[e];
+          if constexpr (DELTA) goff[di] = mfma_f32(ki[e_], kf[e] * w, goff[di]);
+          if constexpr (DO_A) {
+            const float xv = zoo_mul_rn(hf[e], w);
+            if constexpr (ROT) x[e] = (_Float16)xv; else cx[e] = zoo_q8(xv, inv_sk, qmax);
+          }
+        }
+      }
+      if constexpr (DO_A) {
+        if constexpr (ROT)
+          *(lq_v8h*)(xk + (ks * 64 + lane) * 16) = x;
+        else
+          *(lq_v2i*)(xk + (ks >> 1) * 1024 + lane * 16 + 8 * (ks & 1)) =
+              lq_v2i{(int)zoo_pack_codes(cx[0], cx[1], cx[2], cx[3]), (int)zoo_pack_codes(cx[4], cx[5], cx[6], cx[7])};
+      }
+      if constexpr (DELTA) asm volatile("" : "+v"(goff[di]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // GLA: value codes, one channel per thread, through the dead decay tile; K channels at a time
+  auto value_codes = [&](int c0) __attribute__((always_inline)) {
+    const int c = c0 + col;
+    if (c >= V) return;
+    uint16_t vr[SEG];
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) vr[t] = *(const uint16_t*)(p.v + ((t0 + SEG * seg + t) * H + h) * V + c);
+    const float inv_svw = 1.0f / p.svw[h * V + c], inv_svl = 1.0f / p.svl[h * V + c];
+    unsigned char* const vb = lds + L::r1;
+    unsigned char* const lb = vb + K * 64;
+#pragma unroll
+    for (int t8 = 0; t8 < SEG; t8 += 8) {
+      int cw[8], cl[8];
+#pragma unroll
+      for (int e4 = 0; e4 < 2; ++e4) {
+        const lq_v4f ev4 = *(const lq_v4f*)(bs_s + SEG * seg + t8 + 4 * e4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = zoo_dec1(vr[t8 + 4 * e4 + e], bf);
+          cw[4 * e4 + e] = zoo_q8(x * ev4[e], inv_svw, qmax), cl[4 * e4 + e] = zoo_q8(x, inv_svl, qmax);
+        }
+      }
+      *(lq_v2i*)(vb + col * 64 + SEG * seg + t8) = lq_v2i{(int)zoo_pack_codes(cw[0], cw[1], cw[2], cw[3]), (int)zoo_pack_codes(cw[4], cw[5], cw[6], cw[7])};
+      *(lq_v2i*)(lb + zoo_op_values(col, SEG * seg + t8)) = lq_v2i{(int)zoo_pack_codes(cl[0], cl[1], cl[2], cl[3]), (int)zoo_pack_codes(cl[4], cl[5], cl[6], cl[7])};
+    }
+  };
+  auto value_copy = [&](int c0) __attribute__((always_inline)) {
+    const int nb = min(K, V - c0) * 64;
+#pragma unroll
+    for (int i = 0; i < K / 64; ++i) {
+      const int o = 16 * (tid + 256 * i);
+      if (o >= nb) continue;
+      *(lq_v4i*)(p.vqT + (cb * V + c0) * 64 + o) = *(const lq_v4i*)(lds + L::r1 + o);
+      *(lq_v4i*)(p.vcT + (cb * V + c0) * 64 + o) = *(const lq_v4i*)(lds + L::r1 + K * 64 + o);
+    }
+  };
+  if constexpr (MODE == DIAG_GLA) value_codes(0);
+  __syncthreads();
+  if constexpr (MODE == DIAG_GLA) value_copy(0);
+
+  // ---- 4: rotation of the nine operands into this wave's 32 channels, codes
+  if constexpr (DO_A && ROT) {
+    constexpr int NO = (9 + WPS - 1) / WPS;
+    lq_v2i cd[NO];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const int o = part_of + WPS * i;
+      if (o >= 9) continue;
+      lq_v4f r[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const lq_v8h x = *(const lq_v8h*)(lds + L::r2 + L::X * o + (ks * 64 + lane) * 16);
+        r[0] = lq_mfma_f16(__builtin_bit_cast(lq_v8h, rop[0][ks]), x, r[0]);
+        r[1] = lq_mfma_f16(__builtin_bit_cast(lq_v8h, rop[1][ks]), x, r[1]);
+      }
+      const float inv = o < 3 ? inv_sq : inv_sk;
+      int c[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) c[q] = zoo_q8(r[q & 1][q >> 1], inv, qmax);
+      cd[i] = lq_v2i{(int)zoo_pack_codes(c[0], c[1], c[2], c[3]), (int)zoo_pack_codes(c[4], c[5], c[6], c[7])};
+    }
+    __syncthreads();  // the operands have been read
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const int o = part_of + WPS * i;
+      if (o >= 9) continue;
+      *(lq_v2i*)(lds + L::r2 + L::CD * o + (strip >> 1) * 1024 + lane * 16 + 8 * (strip & 1)) = cd[i];
+    }
+  }
+  // G, with the factors of its rows and columns
+  if constexpr (DELTA) {
+#pragma unroll
+    for (int di = -1; di < 3; ++di) {
+      const int I = J + 1 + di;
+      if (I > 3) continue;
+      const lq_v4f b4 = *(const lq_v4f*)(bs_s + 16 * I + 4 * kg);
+      float* G = GT + g_blk(I, J) + rl;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = di < 0 ? (slow ? gslow[r] : gacc[r]) : goff[di < 0 ? 0 : di][r];
+        G[(4 * kg + r) * kBP] = di >= 0 || 4 * kg + r > rl ? (b4[r] * bh) * v : 0.0f;
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- 5: INT8 products of the six off-diagonal blocks (transposed: lane: row rl of I, columns 4kg + r of J), zeros above
+  if constexpr (DO_A) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int pr = wave + 4 * s;
+      if (pr >= 6) continue;
+      const int Jp = pr < 3 ? 0 : (pr < 5 ? 1 : 2), Ip = pr < 3 ? pr + 1 : (pr < 5 ? pr - 1 : 3);
+      lq_v4i acc = {0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < K / 64; ++ks)
+        acc = lq_mfma_i8(*(const lq_v4i*)(lds + L::r2 + L::CD * (3 + pr) + ks * 1024 + lane * 16),
+                         *(const lq_v4i*)(lds + L::r2 + L::CD * (Ip - 1) + ks * 1024 + lane * 16), acc);
+      lq_v4f o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = zoo_mul_rn((float)acc[r], sqk);
+      a_store(16 * Ip + rl, 16 * Jp + 4 * kg, o);
+      a_store(16 * Jp + rl, 16 * Ip + 4 * kg, lq_v4f{0.f, 0.f, 0.f, 0.f});
+    }
+  }
+  if constexpr (MODE == DIAG_GLA) {
+    for (int c0 = K; c0 < V; c0 += K) {  // further value channels
+      __syncthreads();
+      value_codes(c0);
+      __syncthreads();
+      value_copy(c0);
+    }
+  }
+  if constexpr (DELTA) {
+    // first v columns, requested ahead of the inverse
+    lq_v4i vraw[KS];
+    auto request_v = [&](int vb) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const int it = tid + 256 * i, t = it / (K / 8), c = vb + 8 * (it % (K / 8));
+        vraw[i] = *(const lq_v4i*)(p.v + ((t0 + t) * H + h) * V + (c < V ? c : 0));
+      }
+    };
+    request_v(0);
+    // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w, lane c < 16 holds column c of block w)
+    if (lane < 16) {
+      float* B = GT + t_blk(wave, wave);
+      float tc[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float a = (i == lane) ? 1.0f : 0.0f;
+#pragma unroll
+        for (int j = 0; j < i; ++j) a = fmaf(-B[i * kBP + j], tc[j], a);
+        tc[i] = a;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) B[i * kBP + lane] = tc[i];
+    }
+    __syncthreads();
+    // ---- 6: block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes
+    // out of the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product)
+    if (wave < 3) {
+      lq_v4f tcol[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) tcol[0][s] = GT[t_blk(J, J) + (4 * kg + s) * kBP + rl];
+#pragma unroll
+      for (int di = 1; di < 4; ++di) {
+        const int I = J + di;
+        if (I > 3) break;
+        lq_v4f sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dm = 0; dm < di; ++dm) {
+          const lq_v4f g4 = *(const lq_v4f*)(GT + g_blk(I, J + dm) + rl * kBP + 4 * kg);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) sacc = mfma_f32(g4[s], tcol[dm][s], sacc);
+        }
+        const lq_v4f t4 = *(const lq_v4f*)(GT + t_blk(I, I) + rl * kBP + 4 * kg);
+        lq_v4f tacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) tacc = mfma_f32(t4[s], sacc[s], tacc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          tcol[di][r] = -tacc[r];
+          GT[t_blk(I, J) + (4 * kg + r) * kBP + rl] = -tacc[r];
+        }
+      }
+    }
+    __syncthreads();
+
+    // ---- 7: W = T' (k e^g), U = T' v with T' = T diag(beta^sigma), transposed on the fp32 MFMA: lane: token 16I + rl, channels
+    // 16nt + 4kg + r; contraction slot (s, kg) is token 16M + 4kg + s
+    lq_v4f tt[10];
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+      for (int M = 0; M <= I; ++M) {
+        const lq_v4f t4 = *(const lq_v4f*)(GT + t_blk(I, M) + rl * kBP + 4 * kg), b4 = *(const lq_v4f*)(bs_s + 16 * M + 4 * kg);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) tt[I * (I + 1) / 2 + M][s] = t4[s] * b4[s];
+      }
+    auto product = [&](const float (&x)[4][4], lq_v4f (&acc)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int I = 0; I < 4; ++I) acc[I] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int M = 0; M < 4; ++M)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int I = M; I < 4; ++I) acc[I] = mfma_f32(x[M][s], tt[I * (I + 1) / 2 + M][s], acc[I]);
+    };
+    // places of tokens 4kg + s (of sub-block 0) of column 16nt + rl in the tile
+    auto column = [&](int nt, int (&xi)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) xi[s] = at<K>(4 * kg + s, 16 * nt + rl);
+    };
+    const float inv_sw = codes ? 1.0f / p.sw[h] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < K / 64; ++q) {
+      const int nt = wave * (K / 64) + q, n = 16 * nt + rl;
+      int xi[4];
+      column(nt, xi);
+      float x[4][4];
+#pragma unroll
+      for (int M = 0; M < 4; ++M) {
+        const float E = E_s[M * K + n];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)] * E;
+      }
+      lq_v4f acc[4];
+      product(x, acc);
+#pragma unroll
+      for (int I = 0; I < 4; ++I) {
+        lq_v2i o;
+        o[0] = (int)zoo_enc2(acc[I][0], acc[I][1], bf);
+        o[1] = (int)zoo_enc2(acc[I][2], acc[I][3], bf);
+        const int64_t woff = FUSED ? cb * 64 * K + zoo_op_codes(16 * I + rl, 16 * nt + 4 * kg, K)
+                                   : ((t0 + 16 * I + rl) * H + h) * K + 16 * nt + 4 * kg;
+        if constexpr (!FUSED) {
+          if (p.W) *(lq_v2i*)(p.W + woff) = o;
+        }
+        if (codes) {  // state-read codes of the rounded W
+          float w0, w1, w2, w3;
+          zoo_dec2((uint32_t)o[0], bf, w0, w1);
+          zoo_dec2((uint32_t)o[1], bf, w2, w3);
+          *(uint32_t*)(p.wq + woff) = zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax),
+                                                     zoo_q8(w3, inv_sw, qmax));
+        }
+      }
+    }
+#pragma unroll 1
+    for (int vb = 0; vb < V; vb += K) {
+      if (vb > 0) request_v(vb);
+      __syncthreads();  // the tile has been read
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const int it = tid + 256 * i, t = it / (K / 8), c = 8 * (it % (K / 8));
+        float x[8];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)vraw[i][d], bf, x[2 * d], x[2 * d + 1]);
+        *(lq_v4f*)(R1 + at<K>(t, c)) = lq_v4f{x[0], x[1], x[2], x[3]};
+        *(lq_v4f*)(R1 + at<K>(t, c + 4)) = lq_v4f{x[4], x[5], x[6], x[7]};
+      }
+      __syncthreads();
+      const int tiles = min(V - vb, K) / 64;  // column tiles per wave
+#pragma unroll 1
+      for (int q = 0; q < tiles; ++q) {
+        const int nt = wave * tiles + q;
+        int xi[4];
+        column(nt, xi);
+        float x[4][4];
+#pragma unroll
+        for (int M = 0; M < 4; ++M)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)];
+        lq_v4f acc[4];
+        product(x, acc);
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+          lq_v2i o;
+          o[0] = (int)zoo_enc2(acc[I][0], acc[I][1], bf);
+          o[1] = (int)zoo_enc2(acc[I][2], acc[I][3], bf);
+          *(lq_v2i*)(FUSED ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vb + 16 * nt + 4 * kg)
+                           : p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
+        }
+      }
+    }
+  }
+}
+
+template <int K, bool ROT, bool BF, int MODE, bool DK>
+int launch_one(const ZooDiagParams& p, hipStream_t stream) {
+  const dim3 grid((uint32_t)((int64_t)p.B * p.NT * p.H));
+  hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK>), grid, dim3(256), 0, stream, p);
+  return lq_check_launch();
+}
+
+template <int K, bool ROT, int MODE, bool DK>
+int launch_bf(const ZooDiagParams& p, hipStream_t stream) {
+  return p.bf ? launch_one<K, ROT, true, MODE, DK>(p, stream) : launch_one<K, ROT, false, MODE, DK>(p, stream);
+}
+
+template <int K, int MODE, bool DK>
+int launch_rot(const ZooDiagParams& p, hipStream_t stream) {
+  if constexpr (MODE != DIAG_WY) {
+    if (p.rot) return launch_bf<K, true, MODE, DK>(p, stream);
+  }
+  return launch_bf<K, false, MODE, DK>(p, stream);
+}
+
+template <int K, int MODE>
+int launch_dk(const ZooDiagParams& p, hipStream_t stream) {
+  if constexpr (MODE != DIAG_GLA) {
+    if (MODE == DIAG_WY ? p.dk_div != nullptr : p.dq != nullptr) return launch_rot<K, MODE, true>(p, stream);
+  }
+  return launch_rot<K, MODE, false>(p, stream);
+}
+
+template <int MODE>
+int launch(const ZooDiagParams& p, int K, hipStream_t stream) {
+  return K == 128 ? launch_dk<128, MODE>(p, stream) : launch_dk<64, MODE>(p, stream);
+}
+
+}  // namespace zoo_diag

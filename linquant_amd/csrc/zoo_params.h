@@ -124,13 +124,7 @@ struct ZooScanParams {
 };
 int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, hipStream_t stream);
 
-// The pre-pass entry points with what zoo_scan.hip wants on top of their public arguments.
-// cumsum (GLA): also the local value codes (zoo_op_values)
-int zoo_cumsum_launch(const lq_zoo_cumsum_args* a, int8_t* vcT, const float* svl, hipStream_t stream);
-// A kernel: A and qg in operand order (scan = true)
-int zoo_gla_A_launch(const lq_zoo_gla_A_args* a, bool scan, hipStream_t stream);
-// WY prep.  scan (with the write codes): wq and U in operand order; no / scalar decay also the codes of q and A (`local`), and Hw is
-// not stored then
+// WY prep, no / scalar decay.  scan (with the write codes and `local`): wq and U in operand order, the codes of q and A, no Hw
 struct ZooWyLocal {
   const void* q;
   int8_t* qc;   // zoo_op_codes
@@ -180,6 +174,48 @@ struct ZooWyParams {
 };
 // no / scalar decay; defined in zoo_wy_ns.hip
 int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, dim3 grid, hipStream_t stream);
+
+// Per-channel decay, 64-token chunks (zoo_diag_prep.h); defined in zoo_diag_{a,wy,gla,kda}.hip
+struct ZooDiagParams {
+  const _Float16* q;
+  const _Float16* k;      // DIAG_A: Hw
+  const _Float16* v;
+  const float* g;         // DIAG_GLA, DIAG_KDA: log decay per token; DIAG_A, DIAG_WY: cumulated over the chunk
+  const float* beta;
+  const float* logenv;    // DIAG_WY with write codes
+  const _Float16* rot;    // (K,K) local R_QK, or nullptr
+  const float* dq;        // (H,K) D_QK for q, and for k with its reciprocal, or nullptr
+  const float* dk_div;
+  const float* dk_rcp;
+  const float* sq;
+  const float* sk;
+  const float* skw;
+  const float* sw;
+  const float* svw;       // DIAG_GLA
+  const float* svl;
+  // fused forms: operand order (above); stage forms: token-major
+  _Float16* A;
+  int8_t* qc;
+  int8_t* kqT;
+  int8_t* wq;
+  int8_t* vqT;
+  int8_t* vcT;
+  _Float16* Hw;           // DIAG_WY
+  _Float16* W;            // DIAG_WY, may be nullptr
+  _Float16* U;
+  float* fw;              // DIAG_WY
+  float* ev;              // DIAG_WY with write codes
+  float* gam;             // DIAG_WY with write codes, DIAG_GLA
+  float* pack;            // fw | ev | gam per (batch, chunk, head); DIAG_WY: may be nullptr
+  float sigma, tau, eta, scale;
+  int qmax;
+  int bf;
+  int B, T, H, V, NT;
+};
+int zoo_diag_a_launch(const ZooDiagParams& p, int K, hipStream_t stream);
+int zoo_diag_wy_launch(const ZooDiagParams& p, int K, hipStream_t stream);
+int zoo_diag_gla_launch(const ZooDiagParams& p, int K, hipStream_t stream);
+int zoo_diag_kda_launch(const ZooDiagParams& p, int K, hipStream_t stream);
 
 // Operand pre-pass of the linear family with no / scalar decay for zoo_scan.hip; defined in zoo_lin_prep.hip
 struct ZooLinPrepParams {

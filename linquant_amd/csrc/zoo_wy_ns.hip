@@ -160,7 +160,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
     bh_s[tid] = wn_powb(bt, 1.0f - p.sigma);
     bw_s[tid] = wn_powb(bt, (1.0f - p.sigma) * p.tau);
     gs_s[tid] = gv;
-    fW_s[tid] = SCALAR ? bs * zoo_exp(gv) : bs;
+    fW_s[tid] = SCALAR ? bs * zoo_exp_acc(gv) : bs;
     el_s[tid] = SCALAR ? zoo_exp((1.0f - p.eta) * (gl - gv)) : 1.0f;
     float* pk = p.pack ? p.pack + cb * (128 + K) : nullptr;
     if (!SCAN) p.fw[(t0 + tid) * H + h] = fwv;

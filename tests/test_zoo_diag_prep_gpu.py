@@ -1,0 +1,47 @@
+"""GPU test of the launch in front of the recurrence under per-channel decay (zoo_diag_prep.h) at the edges of its branches: sub-blocks
+whose decay is factorized and sub-blocks that take one exponential per product in one chunk, grids that do and do not divide over the
+8 XCDs, both key widths, value widths of one pass, several and a partial last one, with and without rotation and D_QK.  Its fused forms
+run the code of the stage entry points, which the float64 oracle pins in test_zoo_gpu.py (strong decay included), so outputs and final
+states are equal bit for bit."""
+
+import pytest
+import torch
+
+from tests import zoo_cases as zc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cell", ["gla", "kda"])
+@pytest.mark.parametrize("B,NT,H,K,V,dtype,rot,dqk,sigma", [
+    (1, 1, 1, 64, 64, torch.float16, False, False, 1.0), (2, 4, 3, 128, 128, torch.bfloat16, True, True, 0.5),
+    (1, 3, 5, 128, 64, torch.float16, True, False, 1.0), (2, 2, 4, 64, 192, torch.bfloat16, True, True, 0.0),
+    (3, 8, 2, 128, 192, torch.float16, False, True, 0.5), (1, 2, 3, 64, 128, torch.float16, True, False, 0.5),
+    (1, 5, 1, 128, 320, torch.bfloat16, False, False, 1.0)])
+def test_one_launch_equals_the_stages_in_every_branch(cuda, cell, B, NT, H, K, V, dtype, rot, dqk, sigma):
+    from linquant_amd.kernels import zoo
+    from oracle.zoo_reference import signed_hadamard
+
+    T = 64 * NT
+    q, k, v, g, beta = zc.inputs(cell, B=B, T=T, H=H, K=K, V=V, seed=NT, dtype=dtype)
+    gen = torch.Generator().manual_seed(H)
+    # sub-blocks of 16 tokens: a third as drawn, a third near the factorization's limit, a third far beyond it in some channels
+    kind = torch.randint(0, 3, (B, T // 16, H, 1), generator=gen).repeat_interleave(16, dim=1)
+    far = torch.where(torch.rand(B, T, H, K, generator=gen) < 0.1, 60.0, 1.0)
+    g = (g * torch.where(kind == 0, torch.ones(()), torch.where(kind == 1, torch.tensor(4.0), far))).contiguous()
+    q, k, v, g = q.to(cuda), k.to(cuda), v.to(cuda), g.to(cuda)
+    r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
+    sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.01), "w": r(H, lo=0.02, hi=0.04), "kw": r(H, K, lo=0.005, hi=0.015),
+          "vw": r(H, V, lo=0.02, hi=0.04), "vl": r(H, V, lo=0.02, hi=0.04), "el": r(H, V, lo=0.04, hi=0.06),
+          "ew": r(H, V, lo=0.04, hi=0.06), "state": r(H, V, lo=0.02, hi=0.07)}
+    kw = dict(eta=0.25, output_final_state=True, rot=signed_hadamard(K, 2).float().to(cuda) if rot else None)
+    if cell == "kda":
+        kw.update(sigma=sigma, tau=0.5, dqk=r(H, K, lo=0.25, hi=1.75) if dqk else None)
+        call = lambda **x: zoo.chunk_kda_int8(q, k, v, g, beta.to(cuda), sc, **kw, **x)  # noqa: E731
+    else:
+        call = lambda **x: zoo.chunk_gla_int8(q, k, v, g, sc, **kw, **x)  # noqa: E731
+    o1, h1 = call()
+    o0, h0 = call(_debug={})
+    torch.cuda.synchronize()
+    assert torch.isfinite(o1.float()).all() and float(o1.float().abs().max()) > 0
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
