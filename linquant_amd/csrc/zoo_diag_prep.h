@@ -65,6 +65,28 @@ constexpr int kBlk = 16 * kBP;
 LQ_DEV int t_blk(int I, int J) { return (I * (I + 1) / 2 + J) * kBlk; }
 LQ_DEV int g_blk(int I, int J) { return I == J ? t_blk(I, I) : (10 + I * (I - 1) / 2 + J) * kBlk; }
 
+// T' = T diag(beta^sigma) as three bf16 pieces in the order of the bf16 MFMA's operand: step (I, st) is row block I, tokens 32st .. (what
+// lies right of the diagonal block is zero, steps that are zero altogether are left out); its slot 8kg + 4m + s is token 32st + 16m +
+// 4kg + s, so that the other operand is what a lane reads of one column
+constexpr int kSteps = 6;
+LQ_DEV int t_step(int I, int st) { return I < 2 ? I : 2 * (I - 1) + st; }
+
+// two fp32 values -> one dword each of their upper, middle and lower 8 bits as bf16 (first value in the low half)
+LQ_DEV void split3(float x0, float x1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+  hi = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+  const float r0 = x0 - __uint_as_float(b0 & 0xffff0000u), r1 = x1 - __uint_as_float(b1 & 0xffff0000u);  // exact
+  const uint32_t c0 = __float_as_uint(r0), c1 = __float_as_uint(r1);
+  mid = __builtin_amdgcn_perm(c1, c0, 0x07060302u);
+  const float q0 = r0 - __uint_as_float(c0 & 0xffff0000u), q1 = r1 - __uint_as_float(c1 & 0xffff0000u);  // exact
+  lo = __builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
+}
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+LQ_DEV lq_v4f mfma_bf16(lq_v4i a, lq_v4i b, lq_v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
 // pair (J, I), J < I, of sub-blocks: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
 LQ_DEV int pair_of(int J, int I) { return (J == 0 ? -1 : (J == 1 ? 1 : 2)) + I; }
 
@@ -78,10 +100,11 @@ struct Lds {
   static constexpr int r2 = 64 * K * 4;
   static constexpr int X = ROT ? OP : CD;             // an operand as its wave leaves it
   static constexpr int F_bytes = 6 * K * 4, GT_bytes = DELTA ? 16 * kBlk * 4 : 0, KQ_bytes = KQ ? K * 64 + K * 2 : 0;
-  // operands (3 queries, 6 keys) | then their codes, blocks of G and T behind them.  The write codes pass through the key
+  // operands (3 queries, 6 keys) | then their codes, then the pieces of T'; blocks of G and T behind them.  The write codes pass through the key
   // operands' place, the fp64 totals through the queries'; the channel factors F lie at the end, dead when G is written.
   static constexpr int kq = r2 + (DO_A ? 3 * X : 0);
-  static constexpr int gt = r2 + (DO_A ? 9 * CD : 0);
+  static constexpr int TP_bytes = DELTA ? 3 * kSteps * 1024 : 0;
+  static constexpr int gt = r2 + maxi(DO_A ? 9 * CD : 0, TP_bytes);  // (the pieces of T' take the codes' place)
   static constexpr int area = maxi(maxi((DO_A ? maxi(9 * X, 3 * X + KQ_bytes) : KQ_bytes) + F_bytes, gt - r2 + GT_bytes), 4 * K * 8);
   static constexpr int F = r2 + area - F_bytes;
   static constexpr int an = r2 + area;                // decay rows 0, 16, 32, 48, 63
@@ -111,6 +134,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   float* const dkr_s = (float*)(lds + L::dkr);
   float* const bs_s = (float*)(lds + L::bs);  // beta^sigma per token; GLA: e^(eta * envelope)
   float* const GT = (float*)(lds + L::gt);
+  uint16_t* const TP = (uint16_t*)(lds + L::r2);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -684,11 +708,27 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     }
     __syncthreads();
     // ---- 6: block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes
-    // out of the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product)
-    if (wave < 3) {
+    // out of the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product); T' leaves in pieces
+    {
+      const float bsj = bs_s[16 * J + rl];
+      uint16_t* const tp = TP + ((rl >> 2) * 16 + 4 * kg) * 8 + 4 * (J & 1) + (rl & 3);
+      auto t_out = [&](int I, lq_v4f t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          uint32_t pc[3];
+          split3(t[r] * bsj, t[r + 1] * bsj, pc[0], pc[1], pc[2]);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            uint16_t* const dst = tp + (i * kSteps + t_step(I, J >> 1)) * 512 + r * 8;
+            dst[0] = (uint16_t)pc[i], dst[8] = (uint16_t)(pc[i] >> 16);
+          }
+        }
+      };
       lq_v4f tcol[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) tcol[0][s] = GT[t_blk(J, J) + (4 * kg + s) * kBP + rl];
+      t_out(J, tcol[0]);
+      if (J & 1) t_out(J - 1, lq_v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
       for (int di = 1; di < 4; ++di) {
         const int I = J + di;
@@ -705,34 +745,44 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
         for (int s = 0; s < 4; ++s) tacc = mfma_f32(t4[s], sacc[s], tacc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          tcol[di][r] = -tacc[r];
-          GT[t_blk(I, J) + (4 * kg + r) * kBP + rl] = -tacc[r];
-        }
+        for (int r = 0; r < 4; ++r) tcol[di][r] = -tacc[r];
+        t_out(I, tcol[di]);
       }
     }
     __syncthreads();
 
-    // ---- 7: W = T' (k e^g), U = T' v with T' = T diag(beta^sigma), transposed on the fp32 MFMA: lane: token 16I + rl, channels
-    // 16nt + 4kg + r; contraction slot (s, kg) is token 16M + 4kg + s
-    lq_v4f tt[10];
+    // ---- 7: W = T' (k e^g), U = T' v, transposed: lane: token 16I + rl, channels 16nt + 4kg + r
+    lq_v4i tt[3][kSteps];
 #pragma unroll
-    for (int I = 0; I < 4; ++I)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int M = 0; M <= I; ++M) {
-        const lq_v4f t4 = *(const lq_v4f*)(GT + t_blk(I, M) + rl * kBP + 4 * kg), b4 = *(const lq_v4f*)(bs_s + 16 * M + 4 * kg);
+      for (int q = 0; q < kSteps; ++q) tt[i][q] = *(const lq_v4i*)(TP + (i * kSteps + q) * 512 + lane * 8);
+    // x: tokens 16M + 4kg + s of the lane's column in NP pieces; the products below the last kept one are 2^-21 of the leading one
+    // at most (NP = 3) or none (the column has 16 significant bits: NP = 2, 8: NP = 1)
+    auto product = [&](auto np, const float (&x)[4][4], lq_v4f (&acc)[4]) __attribute__((always_inline)) {
+      constexpr int NP = decltype(np)::value;
+      lq_v4i xp[3][2];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) tt[I * (I + 1) / 2 + M][s] = t4[s] * b4[s];
-      }
-    auto product = [&](const float (&x)[4][4], lq_v4f (&acc)[4]) __attribute__((always_inline)) {
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          uint32_t pc[3];
+          split3(x[2 * st + (d >> 1)][2 * (d & 1)], x[2 * st + (d >> 1)][2 * (d & 1) + 1], pc[0], pc[1], pc[2]);
+#pragma unroll
+          for (int i = 0; i < NP; ++i) xp[i][st][d] = (int)pc[i];
+        }
 #pragma unroll
       for (int I = 0; I < 4; ++I) acc[I] = lq_v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int M = 0; M < 4; ++M)
+      for (int sum = NP == 3 ? 2 : NP + 1; sum >= 0; --sum)  // smallest products first
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int i = 0; i < NP; ++i) {
+          if (sum - i < 0 || sum - i > 2) continue;
 #pragma unroll
-          for (int I = M; I < 4; ++I) acc[I] = mfma_f32(x[M][s], tt[I * (I + 1) / 2 + M][s], acc[I]);
+          for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int I = 2 * st; I < 4; ++I) acc[I] = mfma_bf16(xp[i][st], tt[sum - i][t_step(I, st)], acc[I]);
+        }
     };
     // places of tokens 4kg + s (of sub-block 0) of column 16nt + rl in the tile
     auto column = [&](int nt, int (&xi)[4]) __attribute__((always_inline)) {
@@ -753,7 +803,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
         for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)] * E;
       }
       lq_v4f acc[4];
-      product(x, acc);
+      product(std::integral_constant<int, 3>{}, x, acc);
 #pragma unroll
       for (int I = 0; I < 4; ++I) {
         lq_v2i o;
@@ -799,7 +849,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
           for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)];
         lq_v4f acc[4];
-        product(x, acc);
+        product(std::integral_constant<int, BF ? 1 : 2>{}, x, acc);
 #pragma unroll
         for (int I = 0; I < 4; ++I) {
           lq_v2i o;
