@@ -48,12 +48,12 @@ LQ_DEV float powb(float b, float e) {
 }
 
 // float index of (token, channel) in the 64 x K tile.  Sub-block J and 32 channels are 2 KB: piece p of four channels of token rl is
-// 16-byte slot 16p + (rl + p) % 16, so that a lane's reads (pieces 2kg, 2kg + 1 of token rl), the running sums' writes (one token, 64
+// 16-byte slot 16p + (rl xor p), so that a lane's reads (pieces 2kg, 2kg + 1 of token rl), the running sums' writes (one token, 64
 // channels) and the transposed reads of W's operand (16 channels, tokens 4kg + s) all spread over the banks.
 template <int K>
 LQ_DEV int at(int token, int ch) {
   const int p = (ch >> 2) & 7;
-  return (((token >> 4) * (K / 32) + (ch >> 5)) * 128 + p * 16 + ((token + p) & 15)) * 4 + (ch & 3);
+  return (((token >> 4) * (K / 32) + (ch >> 5)) * 128 + p * 16 + ((token & 15) ^ p)) * 4 + (ch & 3);
 }
 
 // byte of the transposed write codes [channel][64 tokens]: 16 bytes of pad after every eight channels
@@ -65,7 +65,7 @@ constexpr int kBlk = 16 * kBP;
 LQ_DEV int t_blk(int I, int J) { return (I * (I + 1) / 2 + J) * kBlk; }
 LQ_DEV int g_blk(int I, int J) { return I == J ? t_blk(I, I) : (10 + I * (I - 1) / 2 + J) * kBlk; }
 
-// T' = T diag(beta^sigma) as three bf16 pieces in the order of the bf16 MFMA's operand: step (I, st) is row block I, tokens 32st .. (what
+// T as three bf16 pieces in the order of the bf16 MFMA's operand: step (I, st) is row block I, tokens 32st .. (what
 // lies right of the diagonal block is zero, steps that are zero altogether are left out); its slot 8kg + 4m + s is token 32st + 16m +
 // 4kg + s, so that the other operand is what a lane reads of one column
 constexpr int kSteps = 6;
@@ -87,6 +87,25 @@ LQ_DEV lq_v4f mfma_bf16(lq_v4i a, lq_v4i b, lq_v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
+// rows I .. 15 of a 16 x 16 unit lower triangular inverse, column rl: t_i = e_i - sum_{j < i} G_ij t_j, G_ij held by lane j of the 16
+template <int I, int JJ>
+LQ_DEV void subst_terms(float g, const float (&tc)[16], float& a) {
+  if constexpr (JJ < I) {
+    const float gij = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(g), 0x150 + JJ, 0xf, 0xf, true));  // row_newbcast
+    a = fmaf(-gij, tc[JJ], a);
+    subst_terms<I, JJ + 1>(g, tc, a);
+  }
+}
+template <int I>
+LQ_DEV void subst_rows(const float (&gr)[16], float (&tc)[16], int rl) {
+  if constexpr (I < 16) {
+    float a = rl == I ? 1.0f : 0.0f;
+    subst_terms<I, 0>(gr[I], tc, a);
+    tc[I] = a;
+    subst_rows<I + 1>(gr, tc, rl);
+  }
+}
+
 // pair (J, I), J < I, of sub-blocks: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
 LQ_DEV int pair_of(int J, int I) { return (J == 0 ? -1 : (J == 1 ? 1 : 2)) + I; }
 
@@ -98,31 +117,34 @@ struct Lds {
   static constexpr int OP = 16 * K * 2, CD = 16 * K;  // bytes of an fp16 operand and of its codes
   static constexpr int r1 = 0;                        // decay tile, then e+ k; GLA: value codes; U: v
   static constexpr int r2 = 64 * K * 4;
-  static constexpr int X = ROT ? OP : CD;             // an operand as its wave leaves it
+  static constexpr int X = ROT ? OP : CD;             // an operand as its waves leave it
   static constexpr int F_bytes = 6 * K * 4, GT_bytes = DELTA ? 16 * kBlk * 4 : 0, KQ_bytes = KQ ? K * 64 + K * 2 : 0;
-  // operands (3 queries, 6 keys) | then their codes, then the pieces of T'; blocks of G and T behind them.  The write codes pass through the key
-  // operands' place, the fp64 totals through the queries'; the channel factors F lie at the end, dead when G is written.
+  // operands (3 queries, 6 keys) | then their codes, then the pieces of T; blocks of G and T behind them.  The write codes pass
+  // through the key operands' place, the fp64 totals through the queries'; the channel factors F lie at the end, dead when G is written.
   static constexpr int kq = r2 + (DO_A ? 3 * X : 0);
   static constexpr int TP_bytes = DELTA ? 3 * kSteps * 1024 : 0;
-  static constexpr int gt = r2 + maxi(DO_A ? 9 * CD : 0, TP_bytes);  // (the pieces of T' take the codes' place)
+  static constexpr int gt = r2 + maxi(DO_A ? 9 * CD : 0, TP_bytes);
   static constexpr int area = maxi(maxi((DO_A ? maxi(9 * X, 3 * X + KQ_bytes) : KQ_bytes) + F_bytes, gt - r2 + GT_bytes), 4 * K * 8);
   static constexpr int F = r2 + area - F_bytes;
-  static constexpr int an = r2 + area;                // decay rows 0, 16, 32, 48, 63
-  static constexpr int E = an + 5 * K * 4;            // e^(a_J)
-  static constexpr int iskw = E + 4 * K * 4;
+  static constexpr int E = r2 + area;                 // e^(a_J)
+  static constexpr int bs = E + 4 * K * 4;
+  static constexpr int le = bs + 64 * 4;              // envelope over either half of the channels
+  // tables of phase 2, then the second half's share of the diagonal blocks of A
+  static constexpr int an = le + 2 * 64 * 4;          // decay rows 0, 16, 32, 48, 63
+  static constexpr int iskw = an + 5 * K * 4;
   static constexpr int dq = iskw + (KQ ? K * 4 : 0);
   static constexpr int dkd = dq + (DK && DO_A ? K * 4 : 0);
   static constexpr int dkr = dkd + (DK && DELTA ? K * 4 : 0);
-  static constexpr int bs = dkr + (DK && DELTA ? K * 4 : 0);
-  static constexpr int bytes = bs + 64 * 4;
+  static constexpr int bytes = maxi(dkr + (DK && DELTA ? K * 4 : 0), an + (DO_A ? 4 * 64 * 16 : 0));
 };
 
 template <int K, bool ROT, bool BF, int MODE, bool DK>
-__global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) {
+__global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) {
   using L = Lds<K, ROT, MODE, DK>;
   constexpr bool FUSED = MODE == DIAG_GLA || MODE == DIAG_KDA, DO_A = L::DO_A, DELTA = L::DELTA;
   constexpr int KS = K / 32;      // steps of 32 channels
-  constexpr int SEG = K / 4;      // tokens per thread where a thread takes one channel
+  constexpr int KW = KS / 2;      // of one wave
+  constexpr int SEG = K / 8;      // tokens per thread where all threads take one value channel
   __shared__ __align__(16) unsigned char lds[L::bytes];
   float* const R1 = (float*)(lds + L::r1);
   float* const F_s = (float*)(lds + L::F);
@@ -133,6 +155,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   float* const dkd_s = (float*)(lds + L::dkd);
   float* const dkr_s = (float*)(lds + L::dkr);
   float* const bs_s = (float*)(lds + L::bs);  // beta^sigma per token; GLA: e^(eta * envelope)
+  float* const le_s = (float*)(lds + L::le);
   float* const GT = (float*)(lds + L::gt);
   uint16_t* const TP = (uint16_t*)(lds + L::r2);
 
@@ -156,25 +179,31 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   const int64_t t0 = (int64_t)group * 64;        // (b * T + chunk * 64: T is a multiple of 64)
   const int64_t cb = (int64_t)group * H + h;
   constexpr bool bf = BF;
-  const int J = wave;                            // sub-block of this wave
+  // sub-block and half of the channels of this wave (the two waves of a SIMD, w and w + 4, share the work of sub-blocks J and 3 - J:
+  // the earlier a sub-block, the more later ones take its keys)
+  const int half = wave >> 2, J = half ? 7 - wave : wave;
   const int tok = 16 * J + rl;                   // token of this lane
-  const int col = tid % K, seg = wave / (K / 64);  // one channel per thread: tokens SEG * seg .. (uniform over the wave)
+  const int ks0 = KW * half, n0 = 32 * ks0 + 8 * kg;  // first step, first channel of this lane
 
   // ---- requests of the chunk
-  float gv[FUSED ? SEG : 1];
+  const int col = tid % K, seg = wave / (K / 64);  // running sums: one channel, 16 tokens (seg: uniform over the wave)
+  const bool scans = K == 128 || wave < 4;
+  float gv[FUSED ? 16 : 1];
   if constexpr (FUSED) {
+    if (scans) {
 #pragma unroll
-    for (int t = 0; t < SEG; ++t) {
-      const float* row = p.g + ((t0 + SEG * seg + t) * H + h) * K;  // (a scalar: the lane adds 32 bits)
-      gv[t] = row[(uint32_t)col];
+      for (int t = 0; t < 16; ++t) {
+        const float* row = p.g + ((t0 + 16 * seg + t) * H + h) * K;  // (a scalar: the lane adds 32 bits)
+        gv[t] = row[(uint32_t)col];
+      }
     }
   }
-  const int64_t roff = ((t0 + tok) * H + h) * K + 8 * kg;
-  lq_v4i kraw[KS], qraw[DO_A ? KS : 1];
+  const int64_t roff = ((t0 + tok) * H + h) * K + n0;
+  lq_v4i kraw[KW], qraw[DO_A ? KW : 1];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    kraw[ks] = *(const lq_v4i*)(p.k + roff + 32 * ks);
-    if constexpr (DO_A) qraw[ks] = *(const lq_v4i*)(p.q + roff + 32 * ks);
+  for (int i = 0; i < KW; ++i) {
+    kraw[i] = *(const lq_v4i*)(p.k + roff + 32 * i);
+    if constexpr (DO_A) qraw[i] = *(const lq_v4i*)(p.q + roff + 32 * i);
   }
   float bt = 0.0f;
   if constexpr (DELTA) bt = p.beta[(t0 + tok) * H + h];
@@ -188,43 +217,39 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   // ---- 1: cumulative log decay of the chunk into LDS
   if constexpr (FUSED) {
     double* part = (double*)(lds + L::r2);  // totals of the four 16-token quarters [4][K]
-    double pre[SEG];
-#pragma unroll
-    for (int qq = 0; qq < SEG / 16; ++qq) {
+    double pre[16];
+    if (scans) {
       double run = 0.0;
 #pragma unroll
       for (int t = 0; t < 16; ++t) {
-        run += (double)gv[16 * qq + t];
-        pre[16 * qq + t] = run;
+        run += (double)gv[t];
+        pre[t] = run;
       }
-      part[(seg * (SEG / 16) + qq) * K + col] = run;
+      part[seg * K + col] = run;
     }
     __syncthreads();
-    double off = 0.0;
-    float last = 0.0f;
+    if (scans) {
+      double off = 0.0;
+      for (int Q = 0; Q < seg; ++Q) off += part[Q * K + col];
+      float x = 0.0f;
+      float* const dst = R1 + at<K>(16 * seg, col);
+      const int p4 = 4 * ((col >> 2) & 7);  // (slot t xor p of the piece's sixteen)
 #pragma unroll
-    for (int Q = 0; Q < 4; ++Q) {
-      if (Q / (SEG / 16) == seg) {
-        const int qq = Q % (SEG / 16);
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          const float x = (float)(off + pre[16 * qq + t]);
-          R1[at<K>(16 * Q + t, col)] = x;
-          if (t == 0) AN[Q * K + col] = x;
-          last = x;
-        }
+      for (int t = 0; t < 16; ++t) {
+        x = (float)(off + pre[t]);
+        dst[((4 * t) ^ p4) - p4] = x;
+        if (t == 0) AN[seg * K + col] = x;
       }
-      off += part[Q * K + col];
-    }
-    if (seg == 64 / SEG - 1) {
-      AN[4 * K + col] = last;
-      const float gm = zoo_exp(last);
-      if constexpr (DELTA) p.pack[cb * (128 + K) + 128 + col] = gm; else p.gam[cb * K + col] = gm;
+      if (seg == 3) {
+        AN[4 * K + col] = x;
+        const float gm = zoo_exp(x);
+        if constexpr (DELTA) p.pack[cb * (128 + K) + 128 + col] = gm; else p.gam[cb * K + col] = gm;
+      }
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < K / 16; ++i) {
-      const int it = tid + 256 * i, t = it / (K / 4), n = 4 * (it % (K / 4));
+    for (int i = 0; i < K / 32; ++i) {
+      const int it = tid + 512 * i, t = it / (K / 4), n = 4 * (it % (K / 4));
       const lq_v4f x = *(const lq_v4f*)(p.g + ((t0 + t) * H + h) * K + n);
       *(lq_v4f*)(R1 + at<K>(t, n)) = x;
       if ((t & 15) == 0) *(lq_v4f*)(AN + (t >> 4) * K + n) = x;
@@ -247,37 +272,51 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 
   // ---- 2: own rows.  gem: the decay of the lane's elements, later e-
   const float* const an_s = AN + J * K;
-  float gem[KS][8];
+  float gem[KW][8];
   float spread = 0.0f, le = -__builtin_inff();
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
+  for (int i = 0; i < KW; ++i)
 #pragma unroll
     for (int e4 = 0; e4 < 2; ++e4) {
-      const int n = 32 * ks + 8 * kg + 4 * e4;
+      const int n = n0 + 32 * i + 4 * e4;
       const lq_v4f g4 = *(const lq_v4f*)(R1 + at<K>(tok, n)), a4 = *(const lq_v4f*)(an_s + n);
       lq_v4f l4;
       if constexpr (FUSED) l4 = *(const lq_v4f*)(AN + 4 * K + n);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        gem[ks][4 * e4 + e] = g4[e];
+        gem[i][4 * e4 + e] = g4[e];
         spread = fmaxf(spread, __builtin_fabsf(g4[e] - a4[e]));
         if constexpr (FUSED) le = fmaxf(le, l4[e] - g4[e]);
       }
     }
-  const bool slow = __any(spread > 40.0f);  // (uniform over the wave)
-  float bs = 1.0f, bh = 1.0f, bw = 1.0f, el = 0.0f;
+  const bool slow = __any(spread > 40.0f);  // (uniform over the wave: a sub-block's halves decide for themselves)
   if constexpr (FUSED) {
     le = fmaxf(le, __shfl_xor(le, 16));
     le = fmaxf(le, __shfl_xor(le, 32));
-    el = p.eta * le;
-  } else if constexpr (MODE == DIAG_WY) {
-    if (codes) el = p.eta * p.logenv[(t0 + tok) * H + h];
+    if (kg == 0) le_s[64 * half + tok] = le;
   }
+  // channel factors of this sub-block: e^(a_J), and e^(a_I - a_J) for the later ones (slow: a_I itself)
+  if (lane < K / 2) {
+    const int n = K / 2 * half + lane;
+    const float a = an_s[n];
+    E_s[J * K + n] = zoo_exp(a);
+    for (int I = J + 1; I < 4; ++I) F_s[pair_of(J, I) * K + n] = slow ? AN[I * K + n] : zoo_exp(AN[I * K + n] - a);
+  }
+  float bs = 1.0f, bh = 1.0f, bw = 1.0f, el = 0.0f;
   if constexpr (DELTA) {
     bs = powb(bt, p.sigma);
     bh = powb(bt, 1.0f - p.sigma);
     bw = powb(bt, (1.0f - p.sigma) * p.tau);
-    if (kg == 0) {
+  }
+  if constexpr (FUSED) {
+    __syncthreads();
+    el = p.eta * fmaxf(le, le_s[64 * (1 - half) + tok]);
+  } else if constexpr (MODE == DIAG_WY) {
+    if (codes) el = p.eta * p.logenv[(t0 + tok) * H + h];
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (half == 0 && kg == 0) {
+    if constexpr (DELTA) {
       const float fwv = powb(bt, (1.0f - p.sigma) * (1.0f - p.tau)), evv = zoo_exp(el);
       bs_s[tok] = bs;
       if constexpr (!FUSED) {
@@ -285,17 +324,10 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
         if (codes) p.ev[(t0 + tok) * H + h] = evv;
       }
       if (codes && p.pack) p.pack[cb * (128 + K) + tok] = fwv, p.pack[cb * (128 + K) + 64 + tok] = evv;
+    } else if constexpr (MODE == DIAG_GLA) {
+      bs_s[tok] = zoo_exp(el);
     }
-  } else if constexpr (MODE == DIAG_GLA) {
-    if (kg == 0) bs_s[tok] = zoo_exp(el);
   }
-  // channel factors of this sub-block: e^(a_J), and e^(a_I - a_J) for the later ones (slow: a_I itself)
-  for (int n = lane; n < K; n += 64) {
-    const float a = an_s[n];
-    E_s[J * K + n] = zoo_exp(a);
-    for (int I = J + 1; I < 4; ++I) F_s[pair_of(J, I) * K + n] = slow ? AN[I * K + n] : zoo_exp(AN[I * K + n] - a);
-  }
-  __builtin_amdgcn_wave_barrier();
 
   float sq = 0.0f, sk = 0.0f, inv_sq = 0.0f, inv_sk = 0.0f;
   if constexpr (DO_A) sq = p.sq[h], sk = p.sk[h], inv_sq = 1.0f / sq, inv_sk = 1.0f / sk;
@@ -331,12 +363,12 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     }
   };
 
-  // diagonal blocks: A transposed (lane: row rl, columns 4kg + r), G (lane: column rl, rows 4kg + r)
+  // diagonal blocks, this half's channels: A transposed (lane: row rl, columns 4kg + r), G (lane: column rl, rows 4kg + r)
   lq_v4f dacc = {0.f, 0.f, 0.f, 0.f}, gacc = {0.f, 0.f, 0.f, 0.f};
   lq_v4f dslow = dacc, gslow = gacc;
   if (slow) {  // every (i, j, channel) weight on its own, masked before use
 #pragma unroll 1
-    for (int n = 0; n < K; n += 8) {
+    for (int n = K / 2 * half; n < K / 2 * (half + 1); n += 8) {
       float ko[8], qo[8], go[8];
       load_k(*(const lq_v4i*)(p.k + ((t0 + tok) * H + h) * K + n), n, ko);
       if constexpr (DO_A) load_q(*(const lq_v4i*)(p.q + ((t0 + tok) * H + h) * K + n), n, qo);
@@ -372,21 +404,21 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 
   unsigned char* const xq = lds + L::r2 + L::X * (J - 1);  // this sub-block's query operand (none for the first)
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int n = 32 * ks + 8 * kg;
+  for (int i = 0; i < KW; ++i) {
+    const int ks = ks0 + i, n = n0 + 32 * i;
     float kf[8], qf[8], hf[8];
-    load_k(kraw[ks], n, kf);
-    if constexpr (DO_A) load_q(qraw[ks], n, qf);
+    load_k(kraw[i], n, kf);
+    if constexpr (DO_A) load_q(qraw[i], n, qf);
     if constexpr (DK && DELTA) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) kraw[ks][d] = (int)zoo_enc2(kf[2 * d], kf[2 * d + 1], bf);
+      for (int d = 0; d < 4; ++d) kraw[i][d] = (int)zoo_enc2(kf[2 * d], kf[2 * d + 1], bf);
     }
     hw_of(kf, bw, hf);
     if constexpr (MODE == DIAG_WY) {
       lq_v4i o;
 #pragma unroll
       for (int d = 0; d < 4; ++d) o[d] = (int)zoo_enc2(hf[2 * d], hf[2 * d + 1], bf);
-      *(lq_v4i*)(p.Hw + roff + 32 * ks) = o;
+      *(lq_v4i*)(p.Hw + roff + 32 * i) = o;
     }
     int ck[8], cs[8], cx[8];
     float ge[8];
@@ -401,7 +433,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
       for (int e_ = 0; e_ < 4; ++e_) {
         const int e = 4 * e4 + e_;
-        const float g = gem[ks][e], d = g - a4[e_];
+        const float g = gem[i][e], d = g - a4[e_];
         const float dl = d * 1.44269504088896340736f;
         const float ep = __builtin_amdgcn_exp2f(dl), em = __builtin_amdgcn_exp2f(-dl);
         if constexpr (DELTA) {
@@ -421,7 +453,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     }
     if (!slow) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) gem[ks][e] = ge[e];
+      for (int e = 0; e < 8; ++e) gem[i][e] = ge[e];
     }
     if constexpr (DELTA) {
       *(lq_v4f*)(R1 + at<K>(tok, n)) = kp[0];
@@ -431,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     if constexpr (DO_A) {
       if (FUSED || p.qc) {
         const lq_v2i o = {(int)zoo_pack_codes(cs[0], cs[1], cs[2], cs[3]), (int)zoo_pack_codes(cs[4], cs[5], cs[6], cs[7])};
-        *(lq_v2i*)(FUSED ? p.qc + cb * 64 * K + zoo_op_codes(tok, n, K) : p.qc + roff + 32 * ks) = o;
+        *(lq_v2i*)(FUSED ? p.qc + cb * 64 * K + zoo_op_codes(tok, n, K) : p.qc + roff + 32 * i) = o;
       }
       if (J > 0) {
         if constexpr (ROT)
@@ -448,12 +480,12 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
         // four keeps channels j and 4 + j, four tokens each
         uint32_t w[2] = {zoo_pack_codes(ck[0], ck[1], ck[2], ck[3]), zoo_pack_codes(ck[4], ck[5], ck[6], ck[7])};
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const uint32_t o1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[i], 0xB1, 0xf, 0xf, true);  // lane ^ 1
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t o1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[q], 0xB1, 0xf, 0xf, true);  // lane ^ 1
           // even lane: channels 0, 2 of (own, other); odd lane: channels 1, 3 of (other, own)
-          const uint32_t m = __builtin_amdgcn_perm(rl & 1 ? w[i] : o1, rl & 1 ? o1 : w[i], rl & 1 ? 0x07030501u : 0x06020400u);
+          const uint32_t m = __builtin_amdgcn_perm(rl & 1 ? w[q] : o1, rl & 1 ? o1 : w[q], rl & 1 ? 0x07030501u : 0x06020400u);
           const uint32_t o2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);  // lane ^ 2
-          w[i] = __builtin_amdgcn_perm(rl & 2 ? m : o2, rl & 2 ? o2 : m, rl & 2 ? 0x07060302u : 0x05040100u);
+          w[q] = __builtin_amdgcn_perm(rl & 2 ? m : o2, rl & 2 ? o2 : m, rl & 2 ? 0x07060302u : 0x05040100u);
         }
         unsigned char* dst = lds + L::kq;
         *(uint32_t*)(dst + ct_at(n + (rl & 3), 16 * J + (rl & 12))) = w[0];
@@ -462,21 +494,16 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     }
     __builtin_amdgcn_sched_barrier(0);  // one step after the other
   }
+  if (slow) dacc = dslow, gacc = gslow;
   const float sqk = sq * sk;
   // element (row, column) of A
   auto a_store = [&](int row, int c, lq_v4f v) __attribute__((always_inline)) {
     _Float16* dst = FUSED ? p.A + cb * 4096 + zoo_op_A(row, c) : p.A + ((t0 + row) * H + h) * 64 + c;
     *(lq_v2i*)dst = lq_v2i{(int)zoo_pack_h2(v[0], v[1]), (int)zoo_pack_h2(v[2], v[3])};
   };
-  if constexpr (DO_A) {
-    lq_v4f o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r <= rl ? zoo_mul_rn(slow ? dslow[r] : dacc[r], sqk) : 0.0f;
-    a_store(tok, 16 * J + 4 * kg, o);
-  }
   // R in MFMA operand order: this wave rotates into channels 32 strip .., tile t takes the even / odd ones of them (a lane then
   // ends up with eight adjacent channels)
-  constexpr int NS = K / 32, WPS = 4 / NS;
+  constexpr int NS = K / 32, WPS = 8 / NS;
   const int strip = wave % NS, part_of = wave / NS;
   lq_v4i rop[ROT ? 2 : 1][KS];
   if constexpr (ROT) {
@@ -494,18 +521,13 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
   __syncthreads();
 
-  // ---- the write codes leave as whole rows
+  // ---- the write codes leave as whole rows; the second half's share of the diagonal blocks of A passes through the dead tables
+  lq_v4f* const dg = (lq_v4f*)(lds + L::an) + J * 64 + lane;
+  if constexpr (DO_A) {
+    if (half) *dg = dacc;
+  }
   if constexpr (L::KQ) {
-    if (codes) {
-      lq_v4i o[K / 64];
-#pragma unroll
-      for (int i = 0; i < K / 64; ++i) {
-        const int it = tid + 256 * i;
-        o[i] = *(const lq_v4i*)(lds + L::kq + ct_at(it >> 2, 16 * (it & 3)));
-      }
-#pragma unroll
-      for (int i = 0; i < K / 64; ++i) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * (tid + 256 * i)) = o[i];
-    }
+    if (codes && tid < 4 * K) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(lds + L::kq + ct_at(tid >> 2, 16 * (tid & 3)));
     if constexpr (DO_A) __syncthreads();  // the key operands take their place
   }
 
@@ -519,11 +541,11 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
     const int pr = pair_of(J, I);
     unsigned char* const xk = lds + L::r2 + L::X * (3 + pr);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int n = 32 * ks + 8 * kg;
+    for (int i = 0; i < KW; ++i) {
+      const int ks = ks0 + i, n = n0 + 32 * i;
       float kf[8], hf[8];
 #pragma unroll
-      for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)kraw[ks][d], bf, kf[2 * d], kf[2 * d + 1]);
+      for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)kraw[i][d], bf, kf[2 * d], kf[2 * d + 1]);
       if constexpr (DO_A) hw_of(kf, bw, hf);
       lq_v8h x;
       int cx[8];
@@ -532,11 +554,11 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
         const lq_v4f f0 = *(const lq_v4f*)(F_s + pr * K + n), f1 = *(const lq_v4f*)(F_s + pr * K + n + 4);
         if (!slow) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) we[e] = gem[ks][e] * (e < 4 ? f0[e & 3] : f1[e & 3]);
+          for (int e = 0; e < 8; ++e) we[e] = gem[i][e] * (e < 4 ? f0[e & 3] : f1[e & 3]);
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            we[e] = zoo_exp((e < 4 ? f0[e & 3] : f1[e & 3]) - gem[ks][e]);
+            we[e] = zoo_exp((e < 4 ? f0[e & 3] : f1[e & 3]) - gem[i][e]);
             asm volatile("" : "+v"(we[e]));  // (a branch, not a selection: the exponentials are not evaluated in vain)
           }
         }
@@ -548,10 +570,9 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
         for (int e_ = 0; e_ < 4; ++e_) {
           const int e = 4 * e4 + e_;
-          const float w = we[e];
-          if constexpr (DELTA) goff[di] = mfma_f32(ki[e_], kf[e] * w, goff[di]);
+          if constexpr (DELTA) goff[di] = mfma_f32(ki[e_], kf[e] * we[e], goff[di]);
           if constexpr (DO_A) {
-            const float xv = zoo_mul_rn(hf[e], w);
+            const float xv = zoo_mul_rn(hf[e], we[e]);
             if constexpr (ROT) x[e] = (_Float16)xv; else cx[e] = zoo_q8(xv, inv_sk, qmax);
           }
         }
@@ -570,11 +591,11 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 
   // GLA: value codes, one channel per thread, through the dead decay tile; K channels at a time
   auto value_codes = [&](int c0) __attribute__((always_inline)) {
-    const int c = c0 + col;
+    const int c = c0 + col, vt = SEG * seg;
     if (c >= V) return;
     uint16_t vr[SEG];
 #pragma unroll
-    for (int t = 0; t < SEG; ++t) vr[t] = *(const uint16_t*)(p.v + ((t0 + SEG * seg + t) * H + h) * V + c);
+    for (int t = 0; t < SEG; ++t) vr[t] = *(const uint16_t*)(p.v + ((t0 + vt + t) * H + h) * V + c);
     const float inv_svw = 1.0f / p.svw[h * V + c], inv_svl = 1.0f / p.svl[h * V + c];
     unsigned char* const vb = lds + L::r1;
     unsigned char* const lb = vb + K * 64;
@@ -583,23 +604,20 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
       int cw[8], cl[8];
 #pragma unroll
       for (int e4 = 0; e4 < 2; ++e4) {
-        const lq_v4f ev4 = *(const lq_v4f*)(bs_s + SEG * seg + t8 + 4 * e4);
+        const lq_v4f ev4 = *(const lq_v4f*)(bs_s + vt + t8 + 4 * e4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float x = zoo_dec1(vr[t8 + 4 * e4 + e], bf);
           cw[4 * e4 + e] = zoo_q8(x * ev4[e], inv_svw, qmax), cl[4 * e4 + e] = zoo_q8(x, inv_svl, qmax);
         }
       }
-      *(lq_v2i*)(vb + col * 64 + SEG * seg + t8) = lq_v2i{(int)zoo_pack_codes(cw[0], cw[1], cw[2], cw[3]), (int)zoo_pack_codes(cw[4], cw[5], cw[6], cw[7])};
-      *(lq_v2i*)(lb + zoo_op_values(col, SEG * seg + t8)) = lq_v2i{(int)zoo_pack_codes(cl[0], cl[1], cl[2], cl[3]), (int)zoo_pack_codes(cl[4], cl[5], cl[6], cl[7])};
+      *(lq_v2i*)(vb + col * 64 + vt + t8) = lq_v2i{(int)zoo_pack_codes(cw[0], cw[1], cw[2], cw[3]), (int)zoo_pack_codes(cw[4], cw[5], cw[6], cw[7])};
+      *(lq_v2i*)(lb + zoo_op_values(col, vt + t8)) = lq_v2i{(int)zoo_pack_codes(cl[0], cl[1], cl[2], cl[3]), (int)zoo_pack_codes(cl[4], cl[5], cl[6], cl[7])};
     }
   };
   auto value_copy = [&](int c0) __attribute__((always_inline)) {
-    const int nb = min(K, V - c0) * 64;
-#pragma unroll
-    for (int i = 0; i < K / 64; ++i) {
-      const int o = 16 * (tid + 256 * i);
-      if (o >= nb) continue;
+    const int o = 16 * tid;
+    if (o < min(K, V - c0) * 64) {
       *(lq_v4i*)(p.vqT + (cb * V + c0) * 64 + o) = *(const lq_v4i*)(lds + L::r1 + o);
       *(lq_v4i*)(p.vcT + (cb * V + c0) * 64 + o) = *(const lq_v4i*)(lds + L::r1 + K * 64 + o);
     }
@@ -607,6 +625,15 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   if constexpr (MODE == DIAG_GLA) value_codes(0);
   __syncthreads();
   if constexpr (MODE == DIAG_GLA) value_copy(0);
+  if constexpr (DO_A) {
+    if (half == 0) {
+      const lq_v4f d1 = *dg;
+      lq_v4f o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r <= rl ? zoo_mul_rn(dacc[r] + d1[r], sqk) : 0.0f;
+      a_store(tok, 16 * J + 4 * kg, o);
+    }
+  }
 
   // ---- 4: rotation of the nine operands into this wave's 32 channels, codes
   if constexpr (DO_A && ROT) {
@@ -637,29 +664,44 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
       *(lq_v2i*)(lds + L::r2 + L::CD * o + (strip >> 1) * 1024 + lane * 16 + 8 * (strip & 1)) = cd[i];
     }
   }
-  // G, with the factors of its rows and columns
+  // G: the second half's share, then the sum with the factors of its rows and columns
   if constexpr (DELTA) {
+    if (half) {
 #pragma unroll
-    for (int di = -1; di < 3; ++di) {
-      const int I = J + 1 + di;
-      if (I > 3) continue;
-      const lq_v4f b4 = *(const lq_v4f*)(bs_s + 16 * I + 4 * kg);
-      float* G = GT + g_blk(I, J) + rl;
+      for (int di = -1; di < 3; ++di) {
+        const int I = J + 1 + di;
+        if (I > 3) continue;
+        float* G = GT + g_blk(I, J) + rl;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = di < 0 ? (slow ? gslow[r] : gacc[r]) : goff[di < 0 ? 0 : di][r];
-        G[(4 * kg + r) * kBP] = di >= 0 || 4 * kg + r > rl ? (b4[r] * bh) * v : 0.0f;
+        for (int r = 0; r < 4; ++r) G[(4 * kg + r) * kBP] = di < 0 ? gacc[r] : goff[di < 0 ? 0 : di][r];
       }
     }
   }
   __syncthreads();
 
   // ---- 5: INT8 products of the six off-diagonal blocks (transposed: lane: row rl of I, columns 4kg + r of J), zeros above
-  if constexpr (DO_A) {
+  if constexpr (DELTA) {
+    if (half == 0) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int pr = wave + 4 * s;
-      if (pr >= 6) continue;
+      for (int di = -1; di < 3; ++di) {
+        const int I = J + 1 + di;
+        if (I > 3) continue;
+        const lq_v4f b4 = *(const lq_v4f*)(bs_s + 16 * I + 4 * kg);
+        float* G = GT + g_blk(I, J) + rl;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float v = (di < 0 ? gacc[r] : goff[di < 0 ? 0 : di][r]) + G[(4 * kg + r) * kBP];
+          G[(4 * kg + r) * kBP] = di >= 0 || 4 * kg + r > rl ? (b4[r] * bh) * v : 0.0f;
+        }
+      }
+    }
+  }
+  if constexpr (DO_A) {
+    // GLA: one to a wave; KDA: the first half's waves are busy with G, the others take one or two
+#pragma unroll
+    for (int s = 0; s < (DELTA ? 2 : 1); ++s) {
+      const int pr = DELTA ? wave - 4 + 4 * s : wave;
+      if (pr < 0 || pr >= 6 || (DELTA && wave < 4)) continue;
       const int Jp = pr < 3 ? 0 : (pr < 5 ? 1 : 2), Ip = pr < 3 ? pr + 1 : (pr < 5 ? pr - 1 : 3);
       lq_v4i acc = {0, 0, 0, 0};
 #pragma unroll
@@ -683,52 +725,36 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
   if constexpr (DELTA) {
     // first v columns, requested ahead of the inverse
-    lq_v4i vraw[KS];
+    constexpr int VP = K / 64;  // 16-byte pieces of a pass per thread
+    lq_v4i vraw[VP];
     auto request_v = [&](int vb) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < KS; ++i) {
-        const int it = tid + 256 * i, t = it / (K / 8), c = vb + 8 * (it % (K / 8));
+      for (int i = 0; i < VP; ++i) {
+        const int it = tid + 512 * i, t = it / (K / 8), c = vb + 8 * (it % (K / 8));
         vraw[i] = *(const lq_v4i*)(p.v + ((t0 + t) * H + h) * V + (c < V ? c : 0));
       }
     };
     request_v(0);
-    // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w, lane c < 16 holds column c of block w)
-    if (lane < 16) {
-      float* B = GT + t_blk(wave, wave);
-      float tc[16];
+    // ---- T = (I + G)^-1: diagonal block J by forward substitution in the wave that has just written it (lane c of every 16 holds
+    // column c; an entry of G reaches the lanes of its row of 16 by a lane broadcast)
+    if (half == 0) {
+      float* B = GT + t_blk(J, J);
+      float gr[16], tc[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float a = (i == lane) ? 1.0f : 0.0f;
+      for (int i = 1; i < 16; ++i) gr[i] = B[i * kBP + rl];
+      tc[0] = rl == 0 ? 1.0f : 0.0f;
+      subst_rows<1>(gr, tc, rl);
 #pragma unroll
-        for (int j = 0; j < i; ++j) a = fmaf(-B[i * kBP + j], tc[j], a);
-        tc[i] = a;
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) B[i * kBP + lane] = tc[i];
+      for (int i = 0; i < 16; ++i)
+        if (kg == (i >> 2)) B[i * kBP + rl] = tc[i];
     }
     __syncthreads();
     // ---- 6: block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes
-    // out of the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product); T' leaves in pieces
-    {
-      const float bsj = bs_s[16 * J + rl];
-      uint16_t* const tp = TP + ((rl >> 2) * 16 + 4 * kg) * 8 + 4 * (J & 1) + (rl & 3);
-      auto t_out = [&](int I, lq_v4f t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < 4; r += 2) {
-          uint32_t pc[3];
-          split3(t[r] * bsj, t[r + 1] * bsj, pc[0], pc[1], pc[2]);
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            uint16_t* const dst = tp + (i * kSteps + t_step(I, J >> 1)) * 512 + r * 8;
-            dst[0] = (uint16_t)pc[i], dst[8] = (uint16_t)(pc[i] >> 16);
-          }
-        }
-      };
+    // out of the MFMA (rows 4kg + s of column rl is the contraction slot 4kg + s of the next product)
+    if (wave < 3) {
       lq_v4f tcol[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) tcol[0][s] = GT[t_blk(J, J) + (4 * kg + s) * kBP + rl];
-      t_out(J, tcol[0]);
-      if (J & 1) t_out(J - 1, lq_v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
       for (int di = 1; di < 4; ++di) {
         const int I = J + di;
@@ -745,23 +771,33 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
         for (int s = 0; s < 4; ++s) tacc = mfma_f32(t4[s], sacc[s], tacc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tcol[di][r] = -tacc[r];
-        t_out(I, tcol[di]);
+        for (int r = 0; r < 4; ++r) {
+          tcol[di][r] = -tacc[r];
+          GT[t_blk(I, J) + (4 * kg + r) * kBP + rl] = -tacc[r];
+        }
       }
     }
     __syncthreads();
+    // T in pieces: twelve blocks of 16 columns (two of them zero) over the waves
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int n = wave + 8 * q;  // (step, M parity): steps (0,0) (1,0) (2,0) (2,1) (3,0) (3,1)
+      if (n >= 2 * kSteps) continue;
+      const int step = n >> 1, I = step < 2 ? step : 1 + (step >> 1), M = (step < 2 ? 0 : 2 * (step & 1)) + (n & 1);
+      lq_v4f t = {0.f, 0.f, 0.f, 0.f};
+      if (M <= I) t = *(const lq_v4f*)(GT + t_blk(I, M) + rl * kBP + 4 * kg);
+      uint32_t pc[2][3];
+      split3(t[0], t[1], pc[0][0], pc[0][1], pc[0][2]);
+      split3(t[2], t[3], pc[1][0], pc[1][1], pc[1][2]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *(lq_v2i*)(TP + (i * kSteps + step) * 512 + lane * 8 + 4 * (n & 1)) = lq_v2i{(int)pc[0][i], (int)pc[1][i]};
+    }
+    __syncthreads();
 
-    // ---- 7: W = T' (k e^g), U = T' v, transposed: lane: token 16I + rl, channels 16nt + 4kg + r
-    lq_v4i tt[3][kSteps];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int q = 0; q < kSteps; ++q) tt[i][q] = *(const lq_v4i*)(TP + (i * kSteps + q) * 512 + lane * 8);
-    // x: tokens 16M + 4kg + s of the lane's column in NP pieces; the products below the last kept one are 2^-21 of the leading one
-    // at most (NP = 3) or none (the column has 16 significant bits: NP = 2, 8: NP = 1)
-    auto product = [&](auto np, const float (&x)[4][4], lq_v4f (&acc)[4]) __attribute__((always_inline)) {
-      constexpr int NP = decltype(np)::value;
-      lq_v4i xp[3][2];
+    // ---- 7: W = T (beta^sigma k e^g), U = T (beta^sigma v), transposed: lane: token 16I + rl, channels 16nt + 4kg + r.  Row blocks
+    // 0, 3 and then 1, 2 (three steps each) of a column tile to a wave, or, where there are fewer tiles than waves, either to one of two
+    // x: tokens 16M + 4kg + s of the lane's column
+    auto split_x = [&](const float (&x)[4][4], lq_v4i (&xp)[3][2]) __attribute__((always_inline)) {
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -769,19 +805,21 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
           uint32_t pc[3];
           split3(x[2 * st + (d >> 1)][2 * (d & 1)], x[2 * st + (d >> 1)][2 * (d & 1) + 1], pc[0], pc[1], pc[2]);
 #pragma unroll
-          for (int i = 0; i < NP; ++i) xp[i][st][d] = (int)pc[i];
+          for (int i = 0; i < 3; ++i) xp[i][st][d] = (int)pc[i];
         }
+    };
+    // row blocks u and 3 - u; six of the nine products of pieces: the others are 2^-21 of the leading one at most
+    auto product = [&](int u, const lq_v4i (&xp)[3][2], lq_v4f (&acc)[2]) __attribute__((always_inline)) {
+      acc[0] = acc[1] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+      const uint16_t* const t_at = TP + lane * 8;
 #pragma unroll
-      for (int I = 0; I < 4; ++I) acc[I] = lq_v4f{0.f, 0.f, 0.f, 0.f};
+      for (int sum = 2; sum >= 0; --sum)  // smallest first
 #pragma unroll
-      for (int sum = NP == 3 ? 2 : NP + 1; sum >= 0; --sum)  // smallest products first
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-          if (sum - i < 0 || sum - i > 2) continue;
-#pragma unroll
-          for (int st = 0; st < 2; ++st)
-#pragma unroll
-            for (int I = 2 * st; I < 4; ++I) acc[I] = mfma_bf16(xp[i][st], tt[sum - i][t_step(I, st)], acc[I]);
+        for (int i = 0; i <= sum; ++i) {
+          const uint16_t* const tq = t_at + (sum - i) * (kSteps * 512);
+          acc[0] = mfma_bf16(xp[i][0], *(const lq_v4i*)(tq + u * 512), acc[0]);
+          acc[1] = mfma_bf16(xp[i][0], *(const lq_v4i*)(tq + (u ? 2 : 4) * 512), acc[1]);
+          acc[1] = mfma_bf16(xp[i][1], *(const lq_v4i*)(tq + (u ? 3 : 5) * 512), acc[1]);
         }
     };
     // places of tokens 4kg + s (of sub-block 0) of column 16nt + rl in the tile
@@ -789,37 +827,45 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
       for (int s = 0; s < 4; ++s) xi[s] = at<K>(4 * kg + s, 16 * nt + rl);
     };
+    constexpr bool SPLIT = K == 64;  // four column tiles: two waves to each
+    const int ntile = SPLIT ? wave & 3 : wave;
     const float inv_sw = codes ? 1.0f / p.sw[h] : 0.0f;
-#pragma unroll
-    for (int q = 0; q < K / 64; ++q) {
-      const int nt = wave * (K / 64) + q, n = 16 * nt + rl;
+    {
       int xi[4];
-      column(nt, xi);
+      column(ntile, xi);
       float x[4][4];
 #pragma unroll
       for (int M = 0; M < 4; ++M) {
-        const float E = E_s[M * K + n];
+        const float E = E_s[M * K + 16 * ntile + rl];
+        const lq_v4f b4 = *(const lq_v4f*)(bs_s + 16 * M + 4 * kg);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)] * E;
+        for (int s = 0; s < 4; ++s) x[M][s] = (R1[xi[s] + M * (KS * 512)] * E) * b4[s];
       }
-      lq_v4f acc[4];
-      product(std::integral_constant<int, 3>{}, x, acc);
+      lq_v4i xp[3][2];
+      split_x(x, xp);
 #pragma unroll
-      for (int I = 0; I < 4; ++I) {
-        lq_v2i o;
-        o[0] = (int)zoo_enc2(acc[I][0], acc[I][1], bf);
-        o[1] = (int)zoo_enc2(acc[I][2], acc[I][3], bf);
-        const int64_t woff = FUSED ? cb * 64 * K + zoo_op_codes(16 * I + rl, 16 * nt + 4 * kg, K)
-                                   : ((t0 + 16 * I + rl) * H + h) * K + 16 * nt + 4 * kg;
-        if constexpr (!FUSED) {
-          if (p.W) *(lq_v2i*)(p.W + woff) = o;
-        }
-        if (codes) {  // state-read codes of the rounded W
-          float w0, w1, w2, w3;
-          zoo_dec2((uint32_t)o[0], bf, w0, w1);
-          zoo_dec2((uint32_t)o[1], bf, w2, w3);
-          *(uint32_t*)(p.wq + woff) = zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax),
-                                                     zoo_q8(w3, inv_sw, qmax));
+      for (int q = 0; q < (SPLIT ? 1 : 2); ++q) {
+        const int u = SPLIT ? half : q;
+        lq_v4f acc[2];
+        product(u, xp, acc);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int I = i ? 3 - u : u;
+          lq_v2i o;
+          o[0] = (int)zoo_enc2(acc[i][0], acc[i][1], bf);
+          o[1] = (int)zoo_enc2(acc[i][2], acc[i][3], bf);
+          const int64_t woff = FUSED ? cb * 64 * K + zoo_op_codes(16 * I + rl, 16 * ntile + 4 * kg, K)
+                                     : ((t0 + 16 * I + rl) * H + h) * K + 16 * ntile + 4 * kg;
+          if constexpr (!FUSED) {
+            if (p.W) *(lq_v2i*)(p.W + woff) = o;
+          }
+          if (codes) {  // state-read codes of the rounded W
+            float w0, w1, w2, w3;
+            zoo_dec2((uint32_t)o[0], bf, w0, w1);
+            zoo_dec2((uint32_t)o[1], bf, w2, w3);
+            *(uint32_t*)(p.wq + woff) = zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax),
+                                                       zoo_q8(w3, inv_sw, qmax));
+          }
         }
       }
     }
@@ -828,33 +874,40 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
       if (vb > 0) request_v(vb);
       __syncthreads();  // the tile has been read
 #pragma unroll
-      for (int i = 0; i < KS; ++i) {
-        const int it = tid + 256 * i, t = it / (K / 8), c = 8 * (it % (K / 8));
+      for (int i = 0; i < VP; ++i) {
+        const int it = tid + 512 * i, t = it / (K / 8), c = 8 * (it % (K / 8));
         float x[8];
 #pragma unroll
         for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)vraw[i][d], bf, x[2 * d], x[2 * d + 1]);
+        const float bt_ = bs_s[t];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = bt_ * x[e];
         *(lq_v4f*)(R1 + at<K>(t, c)) = lq_v4f{x[0], x[1], x[2], x[3]};
         *(lq_v4f*)(R1 + at<K>(t, c + 4)) = lq_v4f{x[4], x[5], x[6], x[7]};
       }
       __syncthreads();
-      const int tiles = min(V - vb, K) / 64;  // column tiles per wave
+      // a pass of K columns as above; of 64 out of 128: two waves to a tile
+      const bool pairs = SPLIT || V - vb < 128;
+      const int nt = pairs ? wave & 3 : wave;
+      int xi[4];
+      column(nt, xi);
+      float x[4][4];
+#pragma unroll
+      for (int M = 0; M < 4; ++M)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)];
+      lq_v4i xp[3][2];
+      split_x(x, xp);
 #pragma unroll 1
-      for (int q = 0; q < tiles; ++q) {
-        const int nt = wave * tiles + q;
-        int xi[4];
-        column(nt, xi);
-        float x[4][4];
+      for (int u = pairs ? half : 0; u < (pairs ? half + 1 : 2); ++u) {
+        lq_v4f acc[2];
+        product(u, xp, acc);
 #pragma unroll
-        for (int M = 0; M < 4; ++M)
-#pragma unroll
-          for (int s = 0; s < 4; ++s) x[M][s] = R1[xi[s] + M * (KS * 512)];
-        lq_v4f acc[4];
-        product(std::integral_constant<int, BF ? 1 : 2>{}, x, acc);
-#pragma unroll
-        for (int I = 0; I < 4; ++I) {
+        for (int i = 0; i < 2; ++i) {
+          const int I = i ? 3 - u : u;
           lq_v2i o;
-          o[0] = (int)zoo_enc2(acc[I][0], acc[I][1], bf);
-          o[1] = (int)zoo_enc2(acc[I][2], acc[I][3], bf);
+          o[0] = (int)zoo_enc2(acc[i][0], acc[i][1], bf);
+          o[1] = (int)zoo_enc2(acc[i][2], acc[i][3], bf);
           *(lq_v2i*)(FUSED ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vb + 16 * nt + 4 * kg)
                            : p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
         }
@@ -866,7 +919,7 @@ __global__ __launch_bounds__(256, 2) void zoo_diag_prep_kernel(ZooDiagParams p) 
 template <int K, bool ROT, bool BF, int MODE, bool DK>
 int launch_one(const ZooDiagParams& p, hipStream_t stream) {
   const dim3 grid((uint32_t)((int64_t)p.B * p.NT * p.H));
-  hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK>), grid, dim3(256), 0, stream, p);
+  hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK>), grid, dim3(512), 0, stream, p);
   return lq_check_launch();
 }
 
