@@ -87,24 +87,38 @@ LQ_DEV lq_v4f mfma_bf16(lq_v4i a, lq_v4i b, lq_v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
-// rows I .. 15 of a 16 x 16 unit lower triangular inverse, column rl: t_i = e_i - sum_{j < i} G_ij t_j, G_ij held by lane j of the 16
-template <int I, int JJ>
-LQ_DEV void subst_terms(float g, const float (&tc)[16], float& a) {
-  if constexpr (JJ < I) {
-    const float gij = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(g), 0x150 + JJ, 0xf, 0xf, true));  // row_newbcast
-    a = fmaf(-gij, tc[JJ], a);
-    subst_terms<I, JJ + 1>(g, tc, a);
-  }
+// One term of the substitution below: t_i -= G_ij t_j, with G_ij broadcast from lane j of every 16
+#define LQ_SUBST(OP, JJ) "v_fmac_f32_dpp %0, -%1, %" #OP " row_newbcast:" #JJ " row_mask:0xf bank_mask:0xf\n"
+#define LQ_SUBST4 LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) LQ_SUBST(5, 3)
+#define LQ_SUBST8 LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) LQ_SUBST(9, 7)
+#define LQ_SUBST12 LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) LQ_SUBST(13, 11)
+
+// Inverse of a 16 x 16 unit lower triangular matrix by forward substitution: lane c of every 16 computes column c; g[i] is row i of the
+// matrix, one entry a lane.  One instruction a term: with the entries from LDS, broadcast reads a row, it took 2200 cycles, with a lane
+// move and a multiply-add a term 4000.  (The no-ops: a lane broadcast must not follow the write of its source at once.)
+LQ_DEV void substitute(const float (&g)[16], float (&t)[16], int rl) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t[i] = rl == i ? 1.0f : 0.0f;
+  asm("s_nop 1\n" LQ_SUBST(2, 0) : "+v"(t[1]) : "v"(g[1]), "v"(t[0]));
+  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) : "+v"(t[2]) : "v"(g[2]), "v"(t[0]), "v"(t[1]));
+  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) : "+v"(t[3]) : "v"(g[3]), "v"(t[0]), "v"(t[1]), "v"(t[2]));
+  asm("s_nop 1\n" LQ_SUBST4 : "+v"(t[4]) : "v"(g[4]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) : "+v"(t[5]) : "v"(g[5]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) : "+v"(t[6]) : "v"(g[6]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) : "+v"(t[7]) : "v"(g[7]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]));
+  asm("s_nop 1\n" LQ_SUBST8 : "+v"(t[8]) : "v"(g[8]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) : "+v"(t[9]) : "v"(g[9]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) : "+v"(t[10]) : "v"(g[10]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) : "+v"(t[11]) : "v"(g[11]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]));
+  asm("s_nop 1\n" LQ_SUBST12 : "+v"(t[12]) : "v"(g[12]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) : "+v"(t[13]) : "v"(g[13]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) : "+v"(t[14]) : "v"(g[14]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) LQ_SUBST(16, 14) : "+v"(t[15]) : "v"(g[15]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]), "v"(t[14]));
 }
-template <int I>
-LQ_DEV void subst_rows(const float (&gr)[16], float (&tc)[16], int rl) {
-  if constexpr (I < 16) {
-    float a = rl == I ? 1.0f : 0.0f;
-    subst_terms<I, 0>(gr[I], tc, a);
-    tc[I] = a;
-    subst_rows<I + 1>(gr, tc, rl);
-  }
-}
+#undef LQ_SUBST12
+#undef LQ_SUBST8
+#undef LQ_SUBST4
+#undef LQ_SUBST
 
 // pair (J, I), J < I, of sub-blocks: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
 LQ_DEV int pair_of(int J, int I) { return (J == 0 ? -1 : (J == 1 ? 1 : 2)) + I; }
@@ -501,24 +515,6 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
     _Float16* dst = FUSED ? p.A + cb * 4096 + zoo_op_A(row, c) : p.A + ((t0 + row) * H + h) * 64 + c;
     *(lq_v2i*)dst = lq_v2i{(int)zoo_pack_h2(v[0], v[1]), (int)zoo_pack_h2(v[2], v[3])};
   };
-  // R in MFMA operand order: this wave rotates into channels 32 strip .., tile t takes the even / odd ones of them (a lane then
-  // ends up with eight adjacent channels)
-  constexpr int NS = K / 32, WPS = 8 / NS;
-  const int strip = wave % NS, part_of = wave / NS;
-  lq_v4i rop[ROT ? 2 : 1][KS];
-  if constexpr (ROT) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      uint32_t w[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(p.rot + (32 * ks + 8 * kg + e) * K + 32 * strip + 2 * rl);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        rop[0][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x05040100u);
-        rop[1][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x07060302u);
-      }
-    }
-  }
   __syncthreads();
 
   // ---- the write codes leave as whole rows; the second half's share of the diagonal blocks of A passes through the dead tables
@@ -540,9 +536,18 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
     if (I > 3) continue;  // (wave-uniform)
     const int pr = pair_of(J, I);
     unsigned char* const xk = lds + L::r2 + L::X * (3 + pr);
+    lq_v4f fr[KW][2], ki[KW][2];  // all of the pair's reads ahead of its products
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+#pragma unroll
+      for (int e4 = 0; e4 < 2; ++e4) {
+        const int n = n0 + 32 * i + 4 * e4;
+        fr[i][e4] = *(const lq_v4f*)(F_s + pr * K + n);
+        if constexpr (DELTA) ki[i][e4] = *(const lq_v4f*)(R1 + at<K>(16 * I + rl, n));
+      }
 #pragma unroll
     for (int i = 0; i < KW; ++i) {
-      const int ks = ks0 + i, n = n0 + 32 * i;
+      const int ks = ks0 + i;
       float kf[8], hf[8];
 #pragma unroll
       for (int d = 0; d < 4; ++d) zoo_dec2((uint32_t)kraw[i][d], bf, kf[2 * d], kf[2 * d + 1]);
@@ -551,7 +556,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       int cx[8];
       float we[8];
       {
-        const lq_v4f f0 = *(const lq_v4f*)(F_s + pr * K + n), f1 = *(const lq_v4f*)(F_s + pr * K + n + 4);
+        const lq_v4f f0 = fr[i][0], f1 = fr[i][1];
         if (!slow) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) we[e] = gem[i][e] * (e < 4 ? f0[e & 3] : f1[e & 3]);
@@ -565,12 +570,10 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       }
 #pragma unroll
       for (int e4 = 0; e4 < 2; ++e4) {
-        lq_v4f ki;
-        if constexpr (DELTA) ki = *(const lq_v4f*)(R1 + at<K>(16 * I + rl, n + 4 * e4));
 #pragma unroll
         for (int e_ = 0; e_ < 4; ++e_) {
           const int e = 4 * e4 + e_;
-          if constexpr (DELTA) goff[di] = mfma_f32(ki[e_], kf[e] * we[e], goff[di]);
+          if constexpr (DELTA) goff[di] = mfma_f32(ki[i][e4][e_], kf[e] * we[e], goff[di]);
           if constexpr (DO_A) {
             const float xv = zoo_mul_rn(hf[e], we[e]);
             if constexpr (ROT) x[e] = (_Float16)xv; else cx[e] = zoo_q8(xv, inv_sk, qmax);
@@ -584,9 +587,8 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
           *(lq_v2i*)(xk + (ks >> 1) * 1024 + lane * 16 + 8 * (ks & 1)) =
               lq_v2i{(int)zoo_pack_codes(cx[0], cx[1], cx[2], cx[3]), (int)zoo_pack_codes(cx[4], cx[5], cx[6], cx[7])};
       }
-      if constexpr (DELTA) asm volatile("" : "+v"(goff[di]));
-      __builtin_amdgcn_sched_barrier(0);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // GLA: value codes, one channel per thread, through the dead decay tile; K channels at a time
@@ -622,6 +624,24 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       *(lq_v4i*)(p.vcT + (cb * V + c0) * 64 + o) = *(const lq_v4i*)(lds + L::r1 + K * 64 + o);
     }
   };
+  // R in MFMA operand order: this wave rotates into channels 32 strip .., tile t takes the even / odd ones of them (a lane then
+  // ends up with eight adjacent channels)
+  constexpr int NS = K / 32, WPS = 8 / NS;
+  const int strip = wave % NS, part_of = wave / NS;
+  lq_v4i rop[ROT ? 2 : 1][KS];
+  if constexpr (ROT) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      uint32_t w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(p.rot + (32 * ks + 8 * kg + e) * K + 32 * strip + 2 * rl);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        rop[0][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x05040100u);
+        rop[1][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x07060302u);
+      }
+    }
+  }
   if constexpr (MODE == DIAG_GLA) value_codes(0);
   __syncthreads();
   if constexpr (MODE == DIAG_GLA) value_copy(0);
@@ -735,18 +755,18 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       }
     };
     request_v(0);
-    // ---- T = (I + G)^-1: diagonal block J by forward substitution in the wave that has just written it (lane c of every 16 holds
-    // column c; an entry of G reaches the lanes of its row of 16 by a lane broadcast)
+    // ---- T = (I + G)^-1: diagonal block J in the wave that has just written it
     if (half == 0) {
       float* B = GT + t_blk(J, J);
       float gr[16], tc[16];
 #pragma unroll
-      for (int i = 1; i < 16; ++i) gr[i] = B[i * kBP + rl];
-      tc[0] = rl == 0 ? 1.0f : 0.0f;
-      subst_rows<1>(gr, tc, rl);
+      for (int i = 0; i < 16; ++i) gr[i] = B[i * kBP + rl];
+      substitute(gr, tc, rl);
+      if (lane < 16) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (kg == (i >> 2)) B[i * kBP + rl] = tc[i];
+        for (int i = 1; i < 16; ++i) B[i * kBP + lane] = tc[i];
+        B[lane] = tc[0];
+      }
     }
     __syncthreads();
     // ---- 6: block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes
