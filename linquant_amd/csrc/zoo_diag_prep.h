@@ -152,7 +152,8 @@ struct Lds {
   static constexpr int bytes = maxi(dkr + (DK && DELTA ? K * 4 : 0), an + (DO_A ? 4 * 64 * 16 : 0));
 };
 
-template <int K, bool ROT, bool BF, int MODE, bool DK>
+// GATE (delta rule): beta^((1-sigma) tau) is not one for every token (otherwise Hw is k)
+template <int K, bool ROT, bool BF, int MODE, bool DK, bool GATE>
 __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) {
   using L = Lds<K, ROT, MODE, DK>;
   constexpr bool FUSED = MODE == DIAG_GLA || MODE == DIAG_KDA, DO_A = L::DO_A, DELTA = L::DELTA;
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   if constexpr (DELTA) {
     bs = powb(bt, p.sigma);
     bh = powb(bt, 1.0f - p.sigma);
-    bw = powb(bt, (1.0f - p.sigma) * p.tau);
+    if constexpr (GATE) bw = powb(bt, (1.0f - p.sigma) * p.tau);
   }
   if constexpr (FUSED) {
     __syncthreads();
@@ -369,11 +370,9 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   auto hw_of = [&](const float (&k)[8], float w, float (&o)[8]) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = k[e];
-    if constexpr (DELTA) {
-      if (w != 1.0f) {
+    if constexpr (GATE) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = zoo_round_act(zoo_mul_rn(w, k[e]), bf);
-      }
+      for (int e = 0; e < 8; ++e) o[e] = zoo_round_act(zoo_mul_rn(w, k[e]), bf);
     }
   };
 
@@ -394,7 +393,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
         float kj[8], hj[8];
         load_k(*(const lq_v4i*)(p.k + ((t0 + 16 * J + o) * H + h) * K + n), n, kj);
         float w = 1.0f;
-        if constexpr (DELTA) w = powb(p.beta[(t0 + 16 * J + o) * H + h], (1.0f - p.sigma) * p.tau);
+        if constexpr (GATE) w = powb(p.beta[(t0 + 16 * J + o) * H + h], (1.0f - p.sigma) * p.tau);
         hw_of(kj, w, hj);
         float sd = 0.0f, sg = 0.0f;
 #pragma unroll
@@ -573,9 +572,10 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
         for (int e_ = 0; e_ < 4; ++e_) {
           const int e = 4 * e4 + e_;
-          if constexpr (DELTA) goff[di] = mfma_f32(ki[i][e4][e_], kf[e] * we[e], goff[di]);
+          const float kv = zoo_mul_rn(kf[e], we[e]);
+          if constexpr (DELTA) goff[di] = mfma_f32(ki[i][e4][e_], kv, goff[di]);
           if constexpr (DO_A) {
-            const float xv = zoo_mul_rn(hf[e], we[e]);
+            const float xv = GATE ? zoo_mul_rn(hf[e], we[e]) : kv;
             if constexpr (ROT) x[e] = (_Float16)xv; else cx[e] = zoo_q8(xv, inv_sk, qmax);
           }
         }
@@ -936,16 +936,20 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
 }
 
-template <int K, bool ROT, bool BF, int MODE, bool DK>
+template <int K, bool ROT, bool BF, int MODE, bool DK, bool GATE>
 int launch_one(const ZooDiagParams& p, hipStream_t stream) {
   const dim3 grid((uint32_t)((int64_t)p.B * p.NT * p.H));
-  hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK>), grid, dim3(512), 0, stream, p);
+  hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK, GATE>), grid, dim3(512), 0, stream, p);
   return lq_check_launch();
 }
 
 template <int K, bool ROT, int MODE, bool DK>
 int launch_bf(const ZooDiagParams& p, hipStream_t stream) {
-  return p.bf ? launch_one<K, ROT, true, MODE, DK>(p, stream) : launch_one<K, ROT, false, MODE, DK>(p, stream);
+  if constexpr (MODE == DIAG_WY || MODE == DIAG_KDA) {
+    if ((1.0f - p.sigma) * p.tau != 0.0f)
+      return p.bf ? launch_one<K, ROT, true, MODE, DK, true>(p, stream) : launch_one<K, ROT, false, MODE, DK, true>(p, stream);
+  }
+  return p.bf ? launch_one<K, ROT, true, MODE, DK, false>(p, stream) : launch_one<K, ROT, false, MODE, DK, false>(p, stream);
 }
 
 template <int K, int MODE, bool DK>
