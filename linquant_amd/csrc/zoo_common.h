@@ -154,3 +154,36 @@ LQ_DEV void zoo_fwht(float (&v)[8], int sub) {
   zoo_fwht_stage<4>(v, sub);
   if constexpr (LPR == 16) zoo_fwht_stage<8>(v, sub);
 }
+
+// One term of the substitution below: t_i -= G_ij t_j, with G_ij broadcast from lane j of every 16
+#define LQ_SUBST(OP, JJ) "v_fmac_f32_dpp %0, -%1, %" #OP " row_newbcast:" #JJ " row_mask:0xf bank_mask:0xf\n"
+#define LQ_SUBST4 LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) LQ_SUBST(5, 3)
+#define LQ_SUBST8 LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) LQ_SUBST(9, 7)
+#define LQ_SUBST12 LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) LQ_SUBST(13, 11)
+
+// Inverse of a 16 x 16 unit lower triangular matrix by forward substitution: lane c of every 16 computes column c; g[i] is row i of the
+// matrix, one entry a lane.  One instruction a term: with the entries from LDS, broadcast reads a row, it took 2200 cycles, with a lane
+// move and a multiply-add a term 4000.  (The no-ops: a lane broadcast must not follow the write of its source at once.)
+LQ_DEV void zoo_substitute(const float (&g)[16], float (&t)[16], int rl) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t[i] = rl == i ? 1.0f : 0.0f;
+  asm("s_nop 1\n" LQ_SUBST(2, 0) : "+v"(t[1]) : "v"(g[1]), "v"(t[0]));
+  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) : "+v"(t[2]) : "v"(g[2]), "v"(t[0]), "v"(t[1]));
+  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) : "+v"(t[3]) : "v"(g[3]), "v"(t[0]), "v"(t[1]), "v"(t[2]));
+  asm("s_nop 1\n" LQ_SUBST4 : "+v"(t[4]) : "v"(g[4]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) : "+v"(t[5]) : "v"(g[5]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) : "+v"(t[6]) : "v"(g[6]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]));
+  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) : "+v"(t[7]) : "v"(g[7]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]));
+  asm("s_nop 1\n" LQ_SUBST8 : "+v"(t[8]) : "v"(g[8]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) : "+v"(t[9]) : "v"(g[9]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) : "+v"(t[10]) : "v"(g[10]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]));
+  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) : "+v"(t[11]) : "v"(g[11]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]));
+  asm("s_nop 1\n" LQ_SUBST12 : "+v"(t[12]) : "v"(g[12]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) : "+v"(t[13]) : "v"(g[13]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) : "+v"(t[14]) : "v"(g[14]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]));
+  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) LQ_SUBST(16, 14) : "+v"(t[15]) : "v"(g[15]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]), "v"(t[14]));
+}
+#undef LQ_SUBST12
+#undef LQ_SUBST8
+#undef LQ_SUBST4
+#undef LQ_SUBST

@@ -87,39 +87,6 @@ LQ_DEV lq_v4f mfma_bf16(lq_v4i a, lq_v4i b, lq_v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
-// One term of the substitution below: t_i -= G_ij t_j, with G_ij broadcast from lane j of every 16
-#define LQ_SUBST(OP, JJ) "v_fmac_f32_dpp %0, -%1, %" #OP " row_newbcast:" #JJ " row_mask:0xf bank_mask:0xf\n"
-#define LQ_SUBST4 LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) LQ_SUBST(5, 3)
-#define LQ_SUBST8 LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) LQ_SUBST(9, 7)
-#define LQ_SUBST12 LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) LQ_SUBST(13, 11)
-
-// Inverse of a 16 x 16 unit lower triangular matrix by forward substitution: lane c of every 16 computes column c; g[i] is row i of the
-// matrix, one entry a lane.  One instruction a term: with the entries from LDS, broadcast reads a row, it took 2200 cycles, with a lane
-// move and a multiply-add a term 4000.  (The no-ops: a lane broadcast must not follow the write of its source at once.)
-LQ_DEV void substitute(const float (&g)[16], float (&t)[16], int rl) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) t[i] = rl == i ? 1.0f : 0.0f;
-  asm("s_nop 1\n" LQ_SUBST(2, 0) : "+v"(t[1]) : "v"(g[1]), "v"(t[0]));
-  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) : "+v"(t[2]) : "v"(g[2]), "v"(t[0]), "v"(t[1]));
-  asm("s_nop 1\n" LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) : "+v"(t[3]) : "v"(g[3]), "v"(t[0]), "v"(t[1]), "v"(t[2]));
-  asm("s_nop 1\n" LQ_SUBST4 : "+v"(t[4]) : "v"(g[4]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]));
-  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) : "+v"(t[5]) : "v"(g[5]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]));
-  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) : "+v"(t[6]) : "v"(g[6]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]));
-  asm("s_nop 1\n" LQ_SUBST4 LQ_SUBST(6, 4) LQ_SUBST(7, 5) LQ_SUBST(8, 6) : "+v"(t[7]) : "v"(g[7]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]));
-  asm("s_nop 1\n" LQ_SUBST8 : "+v"(t[8]) : "v"(g[8]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]));
-  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) : "+v"(t[9]) : "v"(g[9]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]));
-  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) : "+v"(t[10]) : "v"(g[10]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]));
-  asm("s_nop 1\n" LQ_SUBST8 LQ_SUBST(10, 8) LQ_SUBST(11, 9) LQ_SUBST(12, 10) : "+v"(t[11]) : "v"(g[11]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]));
-  asm("s_nop 1\n" LQ_SUBST12 : "+v"(t[12]) : "v"(g[12]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]));
-  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) : "+v"(t[13]) : "v"(g[13]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]));
-  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) : "+v"(t[14]) : "v"(g[14]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]));
-  asm("s_nop 1\n" LQ_SUBST12 LQ_SUBST(14, 12) LQ_SUBST(15, 13) LQ_SUBST(16, 14) : "+v"(t[15]) : "v"(g[15]), "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9]), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]), "v"(t[14]));
-}
-#undef LQ_SUBST12
-#undef LQ_SUBST8
-#undef LQ_SUBST4
-#undef LQ_SUBST
-
 // pair (J, I), J < I, of sub-blocks: (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
 LQ_DEV int pair_of(int J, int I) { return (J == 0 ? -1 : (J == 1 ? 1 : 2)) + I; }
 
@@ -514,6 +481,19 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
     _Float16* dst = FUSED ? p.A + cb * 4096 + zoo_op_A(row, c) : p.A + ((t0 + row) * H + h) * 64 + c;
     *(lq_v2i*)dst = lq_v2i{(int)zoo_pack_h2(v[0], v[1]), (int)zoo_pack_h2(v[2], v[3])};
   };
+  // GLA: value rows, requested a phase ahead of their codes
+  uint16_t vr[MODE == DIAG_GLA ? SEG : 1];
+  auto request_values = [&](int c0) __attribute__((always_inline)) {
+    if constexpr (MODE == DIAG_GLA) {
+      const uint32_t c = (uint32_t)min(c0 + col, V - 1);
+#pragma unroll
+      for (int t = 0; t < SEG; ++t) {
+        const uint16_t* row = (const uint16_t*)p.v + ((t0 + SEG * seg + t) * H + h) * V;
+        vr[t] = row[c];
+      }
+    }
+  };
+  request_values(0);
   __syncthreads();
 
   // ---- the write codes leave as whole rows; the second half's share of the diagonal blocks of A passes through the dead tables
@@ -595,9 +575,6 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   auto value_codes = [&](int c0) __attribute__((always_inline)) {
     const int c = c0 + col, vt = SEG * seg;
     if (c >= V) return;
-    uint16_t vr[SEG];
-#pragma unroll
-    for (int t = 0; t < SEG; ++t) vr[t] = *(const uint16_t*)(p.v + ((t0 + vt + t) * H + h) * V + c);
     const float inv_svw = 1.0f / p.svw[h * V + c], inv_svl = 1.0f / p.svl[h * V + c];
     unsigned char* const vb = lds + L::r1;
     unsigned char* const lb = vb + K * 64;
@@ -737,6 +714,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
   if constexpr (MODE == DIAG_GLA) {
     for (int c0 = K; c0 < V; c0 += K) {  // further value channels
+      request_values(c0);
       __syncthreads();
       value_codes(c0);
       __syncthreads();
@@ -761,7 +739,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       float gr[16], tc[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) gr[i] = B[i * kBP + rl];
-      substitute(gr, tc, rl);
+      zoo_substitute(gr, tc, rl);
       if (lane < 16) {
 #pragma unroll
         for (int i = 1; i < 16; ++i) B[i * kBP + lane] = tc[i];

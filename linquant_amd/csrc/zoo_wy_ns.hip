@@ -331,19 +331,17 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   stage_v();
   __syncthreads();
 
-  // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w < 4, lane c < 16 holds column c of block w)
-  if (wave < 4 && lane < 16) {
+  // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w < 4, lane c of every 16 holds column c of block w)
+  if (wave < 4) {
     const int o = 16 * wave;
-    float tc[16];
+    float gr[16], tc[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float a = (i == lane) ? 1.0f : 0.0f;
+    for (int i = 0; i < 16; ++i) gr[i] = G_s[(o + i) * kGS + o + rl];
+    zoo_substitute(gr, tc, rl);
+    if (lane < 16) {
 #pragma unroll
-      for (int j = 0; j < i; ++j) a = fmaf(-G_s[(o + i) * kGS + o + j], tc[j], a);
-      tc[i] = a;
+      for (int i = 0; i < 16; ++i) T_s[(o + i) * kGS + o + lane] = tc[i];
     }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) T_s[(o + i) * kGS + o + lane] = tc[i];
   }
   __syncthreads();
   // block column J of T by wave J: T_IJ = -T_II . sum_{J <= M < I} G_IM . T_MJ.  A block of the column is used as it comes out of
