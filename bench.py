@@ -27,8 +27,8 @@ INT8_PEAK_TOPS = 5000.0  # published dense INT8 MFMA rate of MI355X; the measure
 # source file of each stage's kernel: a counter figure from profiles/ is attached to a stage only while that file (and the
 # shared headers) still hash to what the profile was taken on
 STAGE_SOURCES = {
-    "c5": {"prologue": "prologue_rotate_quant.hip", "chunk_cumsum": "mamba2_cumsum.hip", "chunk_state": "mamba2_chunk_state.hip",
-           "state_passing": "mamba2_state_passing.hip", "bmm_chunk": "mamba2_bmm_chunk.hip", "chunk_scan": "mamba2_chunk_scan.hip"},
+    "c5": {"prologue": "prologue_rotate_quant.hip", "chunk_cumsum": "mamba2_cumsum.h", "chunk_state": "mamba2_chunk_state.hip",
+           "state_passing": "mamba2_state_passing.hip", "bmm_chunk": "mamba2_bmm_chunk.h", "chunk_scan": "mamba2_chunk_scan.hip"},
     "zoo": {"rotate": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_ns": "zoo_wy_ns.hip", "diag_prep": "zoo_diag_prep.h",
             "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
             "state": "zoo_state.hip", "output": "zoo_output.hip", "rotate_quant": "zoo_rotate_quant.hip"},

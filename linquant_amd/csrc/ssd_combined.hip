@@ -1,4 +1,4 @@
-// The Mamba-2 INT8 SSD forward as one C call: cumsum -> chunk state -> state passing -> C.B^T -> chunk scan launched
+// The Mamba-2 INT8 SSD forward as one C call: cumsum and C.B^T -> chunk state -> state passing -> chunk scan launched
 // back to back on the caller's stream.  Replaces the orchestration of linquant/kernels/mamba2/ssd_combined.py:58-131;
 // the intermediates that function allocates per call live in one workspace: caller-supplied (lq_ssd_combined) or a
 // device array that is part of the library image (lq_ssd_combined_static, for callers that cannot allocate).
@@ -6,6 +6,8 @@
 
 #include "lq_common.h"
 #include "../../include/linquant_hip.h"
+
+int lq_cumsum_bmm(const lq_chunk_cumsum_args* cs, const lq_bmm_chunk_args* bm, hipStream_t stream);  // mamba2_cumsum_bmm.hip
 
 namespace {
 
@@ -57,7 +59,18 @@ int run(const lq_ssd_combined_args* a, char* ws, const Layout& l, hipStream_t st
   cs.dt_out = dt, cs.dA_cumsum = dA;
   cs.batch = a->batch, cs.seqlen = a->seqlen, cs.nheads = a->nheads, cs.chunk_size = Q;
   cs.dt_softplus = a->dt_softplus, cs.dt_min = a->dt_min, cs.dt_max = a->dt_max;
-  if ((rc = lq_chunk_cumsum(&cs, stream)) != LQ_OK) return rc;
+  lq_bmm_chunk_args bm = {};
+  bm.a = a->qC, bm.a_stride_b = a->qC_stride_b, bm.a_stride_l = a->qC_stride_l, bm.a_stride_g = a->qC_stride_g;
+  if (a->keyside) {
+    bm.b = a->b_fp, bm.b_stride_b = a->bfp_stride_b, bm.b_stride_l = a->bfp_stride_l, bm.b_stride_g = a->bfp_stride_g;
+  } else {
+    bm.b = a->qB, bm.b_stride_b = a->qB_stride_b, bm.b_stride_l = a->qB_stride_l, bm.b_stride_g = a->qB_stride_g;
+  }
+  bm.a_scale = a->C_scale, bm.b_scale = a->B_scale, bm.cb_scale = a->cb_scale;
+  bm.out = cb;
+  bm.batch = a->batch, bm.seqlen = a->seqlen, bm.ngroups = a->ngroups, bm.dstate = a->dstate, bm.chunk_size = Q;
+  bm.b_is_fp = a->keyside ? 1 : 0;
+  if ((rc = lq_cumsum_bmm(&cs, &bm, stream)) != LQ_OK) return rc;
 
   if (a->keyside) {
     lq_chunk_state_key_args k = {};
@@ -106,19 +119,6 @@ int run(const lq_ssd_combined_args* a, char* ws, const Layout& l, hipStream_t st
   sp.gate_shift = a->gate_shift, sp.vec_hint = 0, sp.in_place = 1;
   if (dim > 0x7fffffffLL) return LQ_ERR_SHAPE;
   if ((rc = lq_state_passing(&sp, stream)) != LQ_OK) return rc;
-
-  lq_bmm_chunk_args bm = {};
-  bm.a = a->qC, bm.a_stride_b = a->qC_stride_b, bm.a_stride_l = a->qC_stride_l, bm.a_stride_g = a->qC_stride_g;
-  if (a->keyside) {
-    bm.b = a->b_fp, bm.b_stride_b = a->bfp_stride_b, bm.b_stride_l = a->bfp_stride_l, bm.b_stride_g = a->bfp_stride_g;
-  } else {
-    bm.b = a->qB, bm.b_stride_b = a->qB_stride_b, bm.b_stride_l = a->qB_stride_l, bm.b_stride_g = a->qB_stride_g;
-  }
-  bm.a_scale = a->C_scale, bm.b_scale = a->B_scale, bm.cb_scale = a->cb_scale;
-  bm.out = cb;
-  bm.batch = a->batch, bm.seqlen = a->seqlen, bm.ngroups = a->ngroups, bm.dstate = a->dstate, bm.chunk_size = Q;
-  bm.b_is_fp = a->keyside ? 1 : 0;
-  if ((rc = lq_bmm_chunk(&bm, stream)) != LQ_OK) return rc;
 
   lq_chunk_scan_args sc = {};
   sc.cb = cb;
