@@ -144,19 +144,9 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rl = lane & 15, kg = lane >> 4;
-  // Flat grid: workgroup L = x + 8 m (x = its XCD) takes head m % H of (batch, chunk) number x + 8 (m / H): the workgroups
-  // resident on one XCD cover all heads of a few (batch, chunk)s, so rows and (B, T, H) tensors are fetched and written as whole lines
-  const uint32_t ngroups = (uint32_t)p.B * (uint32_t)p.NT;
-  uint32_t group, hh;
-  if ((ngroups & 7u) == 0) {
-    const uint32_t m = blockIdx.x >> 3;
-    hh = m % (uint32_t)p.H;
-    group = (blockIdx.x & 7u) + 8u * (m / (uint32_t)p.H);
-  } else {
-    hh = blockIdx.x % (uint32_t)p.H;
-    group = blockIdx.x / (uint32_t)p.H;
-  }
-  const int h = (int)hh;
+  int h;
+  uint32_t group;
+  if (!zoo_unit((uint32_t)p.B * (uint32_t)p.NT, h, group)) return;
   const int H = p.H, V = p.V, qmax = p.qmax;
   const int64_t t0 = (int64_t)group * 64;        // (b * T + chunk * 64: T is a multiple of 64)
   const int64_t cb = (int64_t)group * H + h;
@@ -916,7 +906,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
 
 template <int K, bool ROT, bool BF, int MODE, bool DK, bool GATE>
 int launch_one(const ZooDiagParams& p, hipStream_t stream) {
-  const dim3 grid((uint32_t)((int64_t)p.B * p.NT * p.H));
+  const dim3 grid = zoo_unit_grid((int64_t)p.B * p.NT, p.H);
   hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK, GATE>), grid, dim3(512), 0, stream, p);
   return lq_check_launch();
 }

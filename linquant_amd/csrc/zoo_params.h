@@ -77,6 +77,24 @@ int zoo_gla_A_cross_launch(const ZooACrossParams& p, int K, hipStream_t stream);
 int zoo_state_unrot_launch(const ZooStateParams& p, bool delta, int K, int batch, bool pair, hipStream_t stream);
 int zoo_output_unrot_launch(const ZooOutParams& p, int decay, int K, hipStream_t stream);
 
+// ---- Grid of the per-channel decay pre-pass: one workgroup per (batch, chunk) and head.  Workgroups are dealt to the 8 XCDs round-robin in launch
+// order (x first): x = XCD + 8 head, y counts (batch, chunk)s by eights.  The workgroups resident on one XCD at a time then cover all heads
+// of a few (batch, chunk)s, so rows and (B, T, H) tensors (a head's values 4 H bytes apart) are fetched and written as whole lines, and
+// the eight XCDs work on neighbouring chunks.  Two dimensions and not one: no division stands
+// in front of a workgroup's first request (GLA B4 T4096 H16 141 -> 136.5 us; KDA even; the no / scalar decay pre-passes were 1 % slower).
+static inline dim3 zoo_unit_grid(int64_t groups, int H) {
+  const int64_t n = groups % 8 ? groups : groups / 8, y = n < 32768 ? n : 32768;
+  return dim3((uint32_t)(groups % 8 ? H : 8 * H), (uint32_t)y, (uint32_t)((n + y - 1) / y));
+}
+// false: beyond the last (batch, chunk) (uniform over the workgroup)
+LQ_DEV bool zoo_unit(uint32_t groups, int& h, uint32_t& group) {
+  const uint32_t y = blockIdx.y + gridDim.y * blockIdx.z;
+  const bool by8 = (groups & 7u) == 0;
+  h = (int)(by8 ? blockIdx.x >> 3 : blockIdx.x);
+  group = by8 ? (blockIdx.x & 7u) + 8u * y : y;
+  return group < groups;
+}
+
 // ---- Operand order: the layouts in which the pre-pass kernels leave the operands of zoo_scan.hip.  Tiles of one (batch, chunk,
 // head) are contiguous, and inside a tile the 16 bytes that lane l of a wave wants as its MFMA operand (row l & 15, contraction
 // group l >> 4) lie at 16 l: a wave's request is 1 KB of whole cache lines.  From token-major rows (16 rows of 64 bytes, H * K
