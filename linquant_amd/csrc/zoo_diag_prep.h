@@ -144,12 +144,12 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rl = lane & 15, kg = lane >> 4;
-  int h;
-  uint32_t group;
-  if (!zoo_unit((uint32_t)p.B * (uint32_t)p.NT, h, group)) return;
-  const int H = p.H, V = p.V, qmax = p.qmax;
-  const int64_t t0 = (int64_t)group * 64;        // (b * T + chunk * 64: T is a multiple of 64)
-  const int64_t cb = (int64_t)group * H + h;
+  ZooUnit unit;
+  if (!zoo_unit(p.B, p.NT, p.H, unit)) return;
+  const int h = unit.h, H = p.H, V = p.V, qmax = p.qmax;
+  const int64_t group = (int64_t)unit.b * p.NT + unit.ct;
+  const int64_t t0 = group * 64;                 // (b * T + chunk * 64: T is a multiple of 64)
+  const int64_t cb = group * H + h;
   constexpr bool bf = BF;
   // sub-block and half of the channels of this wave (the two waves of a SIMD, w and w + 4, share the work of sub-blocks J and 3 - J:
   // the earlier a sub-block, the more later ones take its keys)
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
 
 template <int K, bool ROT, bool BF, int MODE, bool DK, bool GATE>
 int launch_one(const ZooDiagParams& p, hipStream_t stream) {
-  const dim3 grid = zoo_unit_grid((int64_t)p.B * p.NT, p.H);
+  const dim3 grid = zoo_unit_grid(p.B, p.NT, p.H);
   hipLaunchKernelGGL((zoo_diag_prep_kernel<K, ROT, BF, MODE, DK, GATE>), grid, dim3(512), 0, stream, p);
   return lq_check_launch();
 }

@@ -80,20 +80,9 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rl = lane & 15, kg = lane >> 4;
-  // flat grid: the workgroups resident on one XCD cover all heads of a few (batch, chunk)s, so that the (B, T, H) tensors are
-  // fetched as whole lines (workgroups are dealt to the 8 XCDs round-robin)
-  const uint32_t ngroups = (uint32_t)p.B * (uint32_t)p.NT;
-  uint32_t group, hh;
-  if ((ngroups & 7u) == 0) {
-    const uint32_t m = blockIdx.x >> 3;
-    hh = m % (uint32_t)p.H;
-    group = (blockIdx.x & 7u) + 8u * (m / (uint32_t)p.H);
-  } else {
-    hh = blockIdx.x % (uint32_t)p.H;
-    group = blockIdx.x / (uint32_t)p.H;
-  }
-  const int h = (int)hh;
-  const int ct = (int)(group % (uint32_t)p.NT), b = (int)(group / (uint32_t)p.NT);
+  ZooUnit unit;
+  if (!zoo_unit(p.B, p.NT, p.H, unit)) return;
+  const int h = unit.h, b = unit.b, ct = unit.ct;
   const int H = p.H, V = p.V, qmax = p.qmax;
   const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
   const int64_t cb = ((int64_t)b * p.NT + ct) * H + h;
@@ -283,7 +272,7 @@ void launch(const ZooLinPrepParams& p, bool bf, dim3 grid, hipStream_t stream) {
 }  // namespace
 
 int zoo_lin_prep_launch(const ZooLinPrepParams& p, int K, bool bf, hipStream_t stream) {
-  const dim3 grid((unsigned)((int64_t)p.NT * p.B * p.H));
+  const dim3 grid = zoo_unit_grid(p.B, p.NT, p.H);
   if (p.g) {
     if (K == 128) launch<true, 128>(p, bf, grid, stream); else launch<true, 64>(p, bf, grid, stream);
   } else {

@@ -16,8 +16,8 @@
 // runs half a step behind: E of a chunk becomes local codes between the chain's second and the next first rendezvous, and the
 // chunk's local product and store follow after that one.
 //
-// Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 67 us, KDA B2 T8192 H32 157 +
-// 128 -> 137 us, KDA B1 T2048 H8 41 + 7 -> 36 us (25 with 16 columns).  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
+// Measured (kernel time; before = zoo_state + zoo_output): GLA B4 T4096 H16 K = V = 128 47 + 66 -> 67 us (63 since the launch in front
+// of it takes the last chunks first: zoo_params.h), KDA B2 T8192 H32 157 + 128 -> 135 us, KDA B1 T2048 H8 41 + 7 -> 36 us (24 with 16 columns).  A step (1.0 us at KDA) is now the chain's own: about 900 cycles to quantize the
 // carry, 300 to issue its requests, 1000 for state read and E, 300 for the update; one workgroup of 32 columns per compute unit
 // at the first two shapes.
 //

@@ -115,20 +115,9 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rl = lane & 15, kg = lane >> 4;
-  // Flat grid: workgroup L = x + 8 m (x = its XCD) takes head m % H of (batch, chunk) number x + 8 (m / H): the workgroups
-  // resident on one XCD cover all heads of a few (batch, chunk)s, so the (B, T, H) tensors are fetched and written as whole lines
-  const uint32_t ngroups = (uint32_t)p.B * (uint32_t)p.NT;
-  uint32_t group, hh;
-  if ((ngroups & 7u) == 0) {
-    const uint32_t m = blockIdx.x >> 3;
-    hh = m % (uint32_t)p.H;
-    group = (blockIdx.x & 7u) + 8u * (m / (uint32_t)p.H);
-  } else {
-    hh = blockIdx.x % (uint32_t)p.H;
-    group = blockIdx.x / (uint32_t)p.H;
-  }
-  const int h = (int)hh;
-  const int ct = (int)(group % (uint32_t)p.NT), b = (int)(group / (uint32_t)p.NT);
+  ZooUnit unit;
+  if (!zoo_unit(p.B, p.NT, p.H, unit)) return;
+  const int h = unit.h, b = unit.b, ct = unit.ct;
   const int H = p.H, V = p.V, qmax = p.qmax;
   const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
   const int64_t cb = ((int64_t)b * p.NT + ct) * H + h;
@@ -502,7 +491,8 @@ void launch_bf(const ZooWyParams& p, bool scan, dim3 grid, hipStream_t stream) {
 
 }  // namespace
 
-int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, dim3 grid, hipStream_t stream) {
+int zoo_wy_ns_launch(const ZooWyParams& p, bool scalar, int K, bool scan, hipStream_t stream) {
+  const dim3 grid = zoo_unit_grid(p.B, p.NT, p.H);
   if (scalar) {
     if (K == 128) launch_bf<true, 128>(p, scan, grid, stream); else launch_bf<true, 64>(p, scan, grid, stream);
   } else {

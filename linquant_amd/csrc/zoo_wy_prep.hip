@@ -372,8 +372,7 @@ int zoo_wy_prep_launch(const lq_zoo_wy_prep_args* a, bool scan, const ZooWyLocal
   }
   if ((int64_t)(a->seqlen / 64) * a->batch * a->nheads > 0x7fffffff) return LQ_ERR_SHAPE;
   if (big) return a->kdim == 128 ? launch128_decay<128>(p, a->decay, stream) : launch128_decay<64>(p, a->decay, stream);
-  dim3 grid((uint32_t)((a->seqlen / 64) * a->batch * a->nheads));
-  if (a->decay != LQ_DECAY_DIAGONAL) return zoo_wy_ns_launch(p, a->decay == LQ_DECAY_SCALAR, a->kdim, scan, grid, stream);
+  if (a->decay != LQ_DECAY_DIAGONAL) return zoo_wy_ns_launch(p, a->decay == LQ_DECAY_SCALAR, a->kdim, scan, stream);
   ZooDiagParams d = {};
   d.k = p.k, d.v = p.v, d.beta = p.beta, d.g = p.g, d.logenv = p.logenv, d.dk_div = p.dk_div, d.dk_rcp = p.dk_rcp;
   d.skw = p.skw, d.sw = p.sw, d.kqT = p.kqT, d.wq = p.wq, d.Hw = p.Hw, d.W = p.W, d.U = p.U, d.fw = p.fw, d.ev = p.ev, d.gam = p.gam;
