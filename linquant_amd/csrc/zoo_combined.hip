@@ -17,19 +17,17 @@ struct Layout {
   bool scan;  // operand pre-pass, then recurrence and output in one launch
 };
 
-// Linear family, 64-token chunks: recurrence and output in one launch (zoo_scan.hip), or state and output one after the other?
+// No / scalar decay, linear family, 64-token chunks: recurrence and output in one launch (zoo_scan.hip), or state and output one after the other?
 // The chain is NT steps either way, and a step that shares its SIMDs with the output is the longer one; the launch of its own has the
 // whole chip for the output.  What the one launch saves is launches (4 .. 6 us a call, which decides short calls), the stored states
 // (2 K V bytes a chunk and head) and the second reading of raw operands (with a prologue: of their token-major codes), against A
 // (16 KB) and one more set of codes.
-//   bytes saved > 0 (GLA; K = V = 128; with a prologue all but K = V = 64): one launch.
+//   bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch.
 //   else: one launch for short chains whose operands stay in the last-level cache.
 //   more than 128 steps on less than half of the compute units (128 tiles of 32 columns), and more than 32 steps of a second tile per
 //   compute unit (more than 256) where not even 16 KB are saved: the two launches.
 // Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256:
 //                     T = 256     1024         2048         4096         8192        16384 tokens
-//   GLA K = V = 128   1.11..1.22  1.07..1.23   1.05..1.24   1.01..1.19   1.02..1.18   0.99..1.13
-//   GLA K = V = 64    1.12..1.22  1.04..1.12   1.01..1.15   0.98..1.12   0.97..1.15   0.92..1.08
 //   K = V = 128       1.17..1.60  1.06..1.31   1.03..1.27   0.91..1.27   0.95..1.26   0.87..1.13
 //     with prologue   1.16..1.29  1.05..1.21   1.02..1.25   1.01..1.24   1.00..1.22   0.97..1.14
 //   K 128, V 64       1.09..1.44  0.94..1.24   0.83..1.11   0.85..1.08   0.81..1.03   0.75..0.96
@@ -43,11 +41,11 @@ struct Layout {
 //     B*H*NT <= 1024              1.01..1.18   0.97..1.08
 //     with prologue   1.12..1.30  0.93..1.11   0.89..1.07   0.84..1.04   0.83..1.00   0.79..0.96
 //     B*H*NT <= 2048              0.99..1.11   0.98..1.07
-bool linear_scan(bool diag, bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
+bool linear_scan(bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
   if (NT > 128 && tiles < 128) return false;
   const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
-  if (diag || saved >= 16384) return true;
+  if (saved >= 16384) return true;
   if (saved > 0) return NT <= 32 || tiles <= 256;
   return saved == 0 ? NT <= V / 2 && chunks <= 32 * V : NT <= 32 && chunks <= 1024;
 }
@@ -108,7 +106,7 @@ Layout plan(const lq_zoo_simple_gla_args* a, bool scan) {
 }
 
 bool scan_route(const lq_zoo_simple_gla_args* a) {
-  return a->chunk_size == 64 && linear_scan(false, has_prologue(a), a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
+  return a->chunk_size == 64 && linear_scan(has_prologue(a), a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
 }
 
 }  // namespace
@@ -208,16 +206,17 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // ---- the other cells: chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry each way round: the stage entry points in
 // the order the Python wrappers issue them, over one workspace.  64-token chunks take the fused pre-passes (the cumsum / WY
-// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks (GLA: where linear_scan says
-// so) run the recurrence and the output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory).  The delta
-// family needs no rule: its step is two rendezvous and two dependent products with or without the output beside it, and the one launch
-// was the faster at every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0 to 1.7 times with scalar decay and
-// without, 1.0 to 1.56 with per-channel decay; the most on few long chains).
+// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks run the recurrence and the
+// output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory), per-channel decay with one launch in front of it
+// (zoo_diag_prep.h).  Neither family needs a rule.  Delta: its step is two rendezvous and two dependent products with or without the
+// output beside it, and the one launch was the faster at every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0
+// to 1.7 times with scalar decay and without, 1.0 to 1.56 with per-channel decay; the most on few long chains).  GLA: more than 128 steps
+// on less than half of the compute units took four launches while the pre-pass was two of them; against all four the two launches are,
+// at T = 16384, K = V = 128, H = 4 / 12 / 28: 164 -> 152, 308 -> 229, 558 -> 389 us, K = V = 64, H = 4 / B2 H16: 115 -> 113, 326 -> 300.
 namespace {
 
 struct FLayout {
   int64_t gc, logenv, kqT, vqT, vcT, wq, ev, gam, pack, gpk, A, Ax, qg, Hw, W, U, fw, e_out, h_i8, cross, total;
-  bool scan;  // recurrence and output in one launch
 };
 
 int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
@@ -229,7 +228,6 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   if (a->family == LQ_FAMILY_LINEAR && a->decay != LQ_DECAY_DIAGONAL) return LQ_ERR_SHAPE;  // lq_zoo_simple_gla serves those
   const bool delta = a->family == LQ_FAMILY_DELTA, diag = a->decay == LQ_DECAY_DIAGONAL, big = cs == 128;
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
-  l->scan = !big && (delta || linear_scan(true, false, B, T, H, K, V));
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
   // (per-channel decay, one launch in front of the recurrence: gc, logenv and Hw stay on the chip.  The call's workspace keeps the size
@@ -239,20 +237,20 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->kqT, B * NT * H * K * 64);
   take(l->vqT, delta ? 0 : B * NT * H * V * 64);
   take(l->wq, delta ? B * T * H * K : 0);
-  take(l->ev, l->scan ? 0 : B * T * H * 4);
-  take(l->gam, l->scan && delta ? 0 : B * NT * H * K * 4);  // (delta family: zoo_scan.hip reads them and fw from the pack)
+  take(l->ev, big ? B * T * H * 4 : 0);
+  take(l->gam, !big && delta ? 0 : B * NT * H * K * 4);  // (delta family: zoo_scan.hip reads them and fw from the pack)
   take(l->pack, delta && !big ? B * NT * H * (128 + K) * 4 : 0);
   take(l->A, diag || !big ? B * T * H * 64 * 2 : 0);
   take(l->Ax, diag && big ? B * T * H * 64 * 2 : 0);
   take(l->qg, diag || !big ? B * T * H * K : 0);
   take(l->gpk, a->decay == LQ_DECAY_SCALAR && !big ? B * NT * H * 64 * 4 : 0);
-  take(l->vcT, l->scan && !delta ? B * NT * H * V * 64 : 0);
+  take(l->vcT, !big && !delta ? B * NT * H * V * 64 : 0);
   take(l->Hw, delta && (diag || big) ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
   take(l->U, delta ? B * T * H * V * 2 : 0);
-  take(l->fw, delta && !l->scan ? B * T * H * 4 : 0);
-  take(l->e_out, delta && !l->scan ? B * T * H * V * 2 : 0);
-  take(l->h_i8, l->scan ? 0 : B * (T / cs) * H * V * K);
+  take(l->fw, delta && big ? B * T * H * 4 : 0);
+  take(l->e_out, delta && big ? B * T * H * V * 2 : 0);
+  take(l->h_i8, big ? B * (T / cs) * H * V * K : 0);
   take(l->cross, big ? B * T * H * V * 4 : 0);
   l->total = off;
   return LQ_OK;
@@ -291,23 +289,23 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   int8_t* kqT = (int8_t*)(ws + l.kqT);
   int8_t* vqT = delta ? nullptr : (int8_t*)(ws + l.vqT);
   int8_t* wq = delta ? (int8_t*)(ws + l.wq) : nullptr;
-  float* ev = l.scan ? nullptr : (float*)(ws + l.ev);
-  float* gam = l.scan && delta ? nullptr : (float*)(ws + l.gam);
+  float* ev = big ? (float*)(ws + l.ev) : nullptr;
+  float* gam = !big && delta ? nullptr : (float*)(ws + l.gam);
   float* pack = delta && !big ? (float*)(ws + l.pack) : nullptr;
   void* Hw = delta && big ? ws + l.Hw : nullptr;
   void* W = delta && big ? ws + l.W : nullptr;
   void* U = delta ? ws + l.U : nullptr;
-  float* fw = delta && !l.scan ? (float*)(ws + l.fw) : nullptr;
-  void* e_out = delta && !l.scan ? ws + l.e_out : nullptr;
+  float* fw = delta && big ? (float*)(ws + l.fw) : nullptr;
+  void* e_out = delta && big ? ws + l.e_out : nullptr;
   int8_t* h_i8 = (int8_t*)(ws + l.h_i8);
   void* A = diag || !big ? ws + l.A : nullptr;
   void* Ax = diag && big ? ws + l.Ax : nullptr;
   int8_t* qg = diag || !big ? (int8_t*)(ws + l.qg) : nullptr;
   float* gpk = a->decay == LQ_DECAY_SCALAR && !big ? (float*)(ws + l.gpk) : nullptr;
-  int8_t* vcT = l.scan && !delta ? (int8_t*)(ws + l.vcT) : nullptr;
+  int8_t* vcT = !big && !delta ? (int8_t*)(ws + l.vcT) : nullptr;
   float* cross = big ? (float*)(ws + l.cross) : nullptr;
 
-  if (diag && l.scan) {  // everything in front of the recurrence in one launch
+  if (diag && !big) {  // everything in front of the recurrence in one launch
     for (const void* x : {(const void*)a->rot, (const void*)a->dq, (const void*)a->dq_rcp, delta ? (const void*)a->skw : nullptr})
       if (!zoo_al(x, 16)) return LQ_ERR_SHAPE;
     ZooDiagParams d = {};
@@ -321,27 +319,22 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     if (rc != LQ_OK) return rc;
   }
   // (every stage validates its own arguments before it launches: see lq_zoo_simple_gla)
-  if (a->decay != LQ_DECAY_NONE && !(diag && l.scan)) {
+  if (a->decay != LQ_DECAY_NONE && (big || !diag)) {
     lq_zoo_cumsum_args c = {};
     c.g = a->g, c.gc = gc, c.logenv = logenv, c.batch = a->batch, c.seqlen = a->seqlen, c.nheads = a->nheads;
     c.kdim = diag ? a->kdim : 0, c.chunk_size = a->chunk_size;
-    if (!delta && !big) {  // GLA, 64-token chunks: the write operands come with the cumsum
-      c.k = a->k, c.v = a->v, c.kqT = kqT, c.vqT = vqT, c.ev = ev, c.gam = gam, c.skw = a->skw, c.svw = a->svw;
-      c.eta = a->eta, c.qmax = a->qmax, c.vdim = a->vdim, c.act_dtype = a->act_dtype;
-    }
     if ((rc = lq_zoo_cumsum(&c, stream)) != LQ_OK) return rc;
   }
-  if (delta && !(diag && l.scan)) {
+  if (delta && (big || !diag)) {
     lq_zoo_wy_prep_args w = {};
     w.k = a->k, w.v = a->v, w.beta = a->beta, w.g = gc, w.Hw = Hw, w.W = W, w.U = U, w.fw = fw, w.sigma = a->sigma, w.tau = a->tau;
     w.batch = a->batch, w.seqlen = a->seqlen, w.nheads = a->nheads, w.kdim = a->kdim, w.vdim = a->vdim, w.chunk_size = a->chunk_size;
     w.decay = a->decay, w.act_dtype = a->act_dtype;
     if (!big) {  // the write operands come with the transform
-      w.kqT = kqT, w.wq = wq, w.ev = ev, w.gam = gam, w.logenv = logenv, w.skw = a->skw, w.sw = a->sw, w.eta = a->eta, w.qmax = a->qmax;
-      w.dk_div = a->dq, w.dk_rcp = a->dq_rcp, w.pack = pack;
+      w.kqT = kqT, w.wq = wq, w.ev = ev, w.gam = gam, w.skw = a->skw, w.sw = a->sw, w.eta = a->eta, w.qmax = a->qmax, w.pack = pack;
     }
     const ZooWyLocal local = {a->q, qg, A, gpk, a->sq, a->sk, a->scale};
-    if ((rc = zoo_wy_prep_launch(&w, l.scan, l.scan ? &local : nullptr, stream)) != LQ_OK) return rc;
+    if ((rc = zoo_wy_prep_launch(&w, !big, big ? nullptr : &local, stream)) != LQ_OK) return rc;
   }
   if (big) {
     lq_zoo_write_codes_args w = {};
@@ -351,14 +344,14 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     w.decay = a->decay, w.act_dtype = a->act_dtype;
     if ((rc = lq_zoo_write_codes(&w, stream)) != LQ_OK) return rc;
   }
-  if (diag && !l.scan) {
+  if (diag && big) {
     lq_zoo_gla_A_args g = {};
     g.q = a->q, g.k = delta ? Hw : a->k, g.g = gc, g.A = A, g.qg = qg, g.rot = a->rot, g.sq = a->sq, g.sk = a->sk, g.scale = a->scale;
     g.qmax = a->qmax, g.batch = a->batch, g.seqlen = a->seqlen, g.nheads = a->nheads, g.kdim = a->kdim, g.chunk_size = a->chunk_size;
     g.act_dtype = a->act_dtype, g.dq = a->dq, g.A_cross = Ax;
     if ((rc = lq_zoo_gla_A(&g, stream)) != LQ_OK) return rc;
   }
-  if (l.scan) {
+  if (!big) {
     ZooScanParams s = {};
     s.kqT = kqT, s.vqT = vqT, s.vcT = vcT, s.wq = wq, s.u = (const _Float16*)U, s.pack = pack, s.gam = gam;
     s.qc = qg, s.A = (const _Float16*)A, s.gpk = gpk, s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     (1, 1, 1, 64, 64, torch.float16, False, False, 1.0), (2, 4, 3, 128, 128, torch.bfloat16, True, True, 0.5),
     (1, 3, 5, 128, 64, torch.float16, True, False, 1.0), (2, 2, 4, 64, 192, torch.bfloat16, True, True, 0.0),
     (3, 8, 2, 128, 192, torch.float16, False, True, 0.5), (1, 2, 3, 64, 128, torch.float16, True, False, 0.5),
-    (1, 5, 1, 128, 320, torch.bfloat16, False, False, 1.0)])
+    (1, 5, 1, 128, 320, torch.bfloat16, False, False, 1.0), (1, 130, 1, 64, 64, torch.float16, True, False, 1.0)])
 def test_one_launch_equals_the_stages_in_every_branch(cuda, cell, B, NT, H, K, V, dtype, rot, dqk, sigma):
     from linquant_amd.kernels import zoo
     from oracle.zoo_reference import signed_hadamard
