@@ -24,8 +24,8 @@ struct Layout {
 // (16 KB) and one more set of codes.
 //   bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch.
 //   else: one launch for short chains whose operands stay in the last-level cache.
-//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns), and more than 32 steps of a second tile per
-//   compute unit (more than 256) where not even 16 KB are saved: the two launches.
+//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns; K = V = 128 with a prologue: 40), and more than 32
+//   steps of a second tile per compute unit (more than 256) where not even 16 KB are saved: the two launches.
 // Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256:
 //                     T = 256     1024         2048         4096         8192        16384 tokens
 //   K = V = 128       1.17..1.60  1.06..1.31   1.03..1.27   0.91..1.27   0.95..1.26   0.87..1.13
@@ -41,9 +41,13 @@ struct Layout {
 //     B*H*NT <= 1024              1.01..1.18   0.97..1.08
 //     with prologue   1.12..1.30  0.93..1.11   0.89..1.07   0.84..1.04   0.83..1.00   0.79..0.96
 //     B*H*NT <= 2048              0.99..1.11   0.98..1.07
+// K = V = 128 with a prologue past 128 steps, since the operand pre-pass takes the last chunks first (zoo_params.h), one set of inputs, no
+// and scalar decay, T = 16384: 40 tiles 1.06 1.04, 56 1.09 1.02, 72 1.10 1.04, 96 1.15 1.10; T = 12288, 64 tiles 1.05.  K 128, V 64 with
+// a prologue, 80 tiles: 0.99 0.94.
 bool linear_scan(bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
-  if (NT > 128 && tiles < 128) return false;
+  const int64_t few = prologue && K == 128 && V >= 128 ? 40 : 128;
+  if (NT > 128 && tiles < few) return false;
   const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
   if (saved >= 16384) return true;
   if (saved > 0) return NT <= 32 || tiles <= 256;

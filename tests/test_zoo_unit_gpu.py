@@ -57,3 +57,25 @@ def test_more_chunks_than_the_grid_holds_in_one_dimension(cuda):
     for s in (slice(0, 64 * 5), slice(64 * 32764, T)):
         for name, a, b in zip(("Hw", "W", "U", "fw"), whole, prep(s)):
             assert torch.equal(a[:, s], b), (name, s)
+
+
+@pytest.mark.parametrize("cell", ["linear_none", "mamba2"])
+@pytest.mark.parametrize("H,prologue", [(31, False), (32, False), (9, True), (10, True)])
+def test_long_chains_on_either_side_of_the_rule(cuda, cell, H, prologue):
+    """More than 128 chunk steps, K = V = 128: one launch or two by the number of workgroups, the same bits as the stages."""
+    from linquant_amd.kernels import zoo
+    from linquant_amd.kernels.zoo.prologue import rotation_signs
+    from oracle.zoo_reference import signed_hadamard
+
+    K = V = 128
+    q, k, v, g, _ = (None if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=64 * 129, H=H, K=K, V=V, seed=H, dtype=torch.float16))
+    gen = torch.Generator().manual_seed(H)
+    r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
+    sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.01), "kw": r(H, K, lo=0.005, hi=0.015), "vw": r(H, V, lo=0.02, hi=0.04),
+          "vl": r(H, V, lo=0.02, hi=0.04), "state": r(H, V, lo=0.02, hi=0.07)}
+    kw = dict(output_final_state=True)
+    if prologue:
+        kw["prologue"] = dict(signs_qk=rotation_signs(signed_hadamard(K, 2)).to(cuda))
+    o1, h1 = zoo.chunk_simple_gla_int8(q, k, v, g, sc, **kw)
+    o0, h0 = zoo.chunk_simple_gla_int8(q, k, v, g, sc, _debug={}, **kw)
+    assert torch.equal(o0, o1) and torch.equal(h0, h1) and float(o1.float().abs().max()) > 0
