@@ -15,20 +15,24 @@
 // The exponentials are what a separate kernel per product repeats (and what the vector unit issues at a quarter of its rate):
 // here an element takes e+ = e^(g - a_J) and e- = e^(a_J - g), J its own 16-token sub-block, and the key write code's.  A sub-block's
 // key operand for a later one is e- times a factor per channel, e^(a_I - a_J); the state read and W's operand are e+ times e^(a_J).
-// Both e+ and e- are used where the decay inside the sub-block spreads over no more than e^40; otherwise (per wave) the operands
-// take one exponential each and the diagonal blocks one per (i, j, channel).
+// Both e+ and e- are used where the decay inside the sub-block spreads over no more than e^40; otherwise (each wave for its sub-block and
+// half of the channels) the operands take one exponential each and the diagonal blocks one per (i, j, channel).
 //
-// One 4-wave workgroup per (chunk, batch*head), two to a compute unit (80 KB of LDS, 256 registers).  Wave J owns sub-block J; lane
-// (rl, kg) holds its token rl, channels 32ks + 8kg + e, which is the layout of every MFMA operand built from them.
-//   1  running sums in fp64, one channel per thread, into LDS          2  own rows: codes, diagonal blocks, e+ k into LDS
-//   3  key operands of the later sub-blocks, Gram blocks               4  rotation: 9 operands x 32 channels per wave, R in registers
-//   5  INT8 products; inverse of the diagonal blocks                   6  block columns of T          7  W, U on the fp32 MFMA
+// One 8-wave workgroup per (chunk, batch*head), two to a compute unit (80 KB of LDS, 128 registers).  Two waves own sub-block J, half of
+// the channels each; lane (rl, kg) holds its token rl, channels 32ks + 8kg + e, which is the layout of every MFMA operand built from them.
+//   1  running sums in fp64, 16 tokens of a channel per thread, into LDS
+//   2  own rows: codes, diagonal blocks, e+ k into LDS          3  key operands of the later sub-blocks, Gram blocks
+//   4  rotation: 9 operands x 32 channels per wave, R in registers   5  INT8 products; inverse of the diagonal blocks
+//   6  block columns of T                                       7  W, U: T and the rows in three bf16 pieces, six products
 //
-// Measured (kernel time): KDA B2 T8192 H32 K = V = 128 with rotation and D_QK: cumsum 81 + WY prep 307 + A kernel 209 us -> 501; GLA
-// B4 T4096 H16 K = V = 128: cumsum with codes 86 + A kernel 118 -> 165; KDA B1 T2048 H8 8 + 21 + 24 -> 27.  Bound by instruction
-// issue: at KDA's shape the vector instructions are 261 us of a SIMD's time (4.7 cycles each) and the fp32 MFMA 152 us, during which
-// its SIMD issues no vector instruction (measured: 33 cycles a 16x16x4, the cycles of the instructions between them on top; the
-// half-precision MFMA costs them only its issue).
+// Measured (kernel time, against a kernel each for cumsum, WY prep and A): KDA B2 T8192 H32 K = V = 128 with rotation and D_QK 81 + 307 +
+// 209 -> 400 us; GLA B4 T4096 H16 K = V = 128: cumsum with codes 86 + 118 -> 139; KDA B1 T2048 H8 8 + 21 + 24 -> 22.  On the way, KDA / GLA:
+// 4 waves of 256 registers with W and U on the fp32 MFMA 501 / 165; on the bf16 MFMA 475; eight waves 467 / 148; the inverse one instruction
+// a term, the key operands read ahead of their products 443; no gate arithmetic where Hw is k, bf16 rounded by the conversion 409 / 141.  Bound by instruction
+// issue between its rendezvous (two workgroups cover part of each other's waits): the exponentials, the quantizations and the products of
+// phases 2 and 3, which stay on the fp32 MFMA: 33 cycles a 16x16x4, during which its SIMD issues no vector instruction (the half-precision
+// MFMA costs them only its issue), yet splitting their operands in three would cost more.  Persistent workgroups with the next chunk's
+// requests ahead spilled (KDA 714), three workgroups a compute unit for GLA too (194).
 #pragma once
 
 #include <type_traits>
