@@ -13,10 +13,12 @@
 //   W = T (beta^sigma k e^g),  U = T (beta^sigma v),  Hw = beta^((1-sigma) tau) k,  fw = beta^((1-sigma)(1-tau))
 //
 // The exponentials are what a separate kernel per product repeats (and what the vector unit issues at a quarter of its rate):
-// here an element takes e+ = e^(g - a_J) and e- = e^(a_J - g), J its own 16-token sub-block, and the key write code's.  A sub-block's
-// key operand for a later one is e- times a factor per channel, e^(a_I - a_J); the state read and W's operand are e+ times e^(a_J).
-// Both e+ and e- are used where the decay inside the sub-block spreads over no more than e^40; otherwise (each wave for its sub-block and
-// half of the channels) the operands take one exponential each and the diagonal blocks one per (i, j, channel).
+// here an element takes e+ = e^(g - a_J) and e- = e^(a_J - g), J its own 16-token sub-block, the key write code's, and e^(a_I - g) for each
+// later sub-block I.  (e- times a factor per channel, e^(a_I - a_J), in the latter's place took 390 us where this takes 381, and put two
+// to five times as many entries of A beside the fp16 of their float64 value: its operands are rounded next.)  The state read and W's
+// operand are e+ times e^(a_J), the latter with the rounding of its argument made good.  The diagonal blocks are products of e+ and e- where the decay inside
+// the sub-block spreads over no more than e^40 (each wave decides for its half of the channels), otherwise they take one exponential per
+// (i, j, channel).
 //
 // One 8-wave workgroup per (chunk, batch*head), two to a compute unit (80 KB of LDS, 128 registers).  Two waves own sub-block J, half of
 // the channels each; lane (rl, kg) holds its token rl, channels 32ks + 8kg + e, which is the layout of every MFMA operand built from them.
@@ -25,8 +27,9 @@
 //   4  rotation: 9 operands x 32 channels per wave, R in registers   5  INT8 products; inverse of the diagonal blocks
 //   6  block columns of T                                       7  W, U: T and the rows in three bf16 pieces, six products
 //
-// Measured (kernel time, against a kernel each for cumsum, WY prep and A): KDA B2 T8192 H32 K = V = 128 with rotation and D_QK 81 + 307 +
-// 209 -> 400 us; GLA B4 T4096 H16 K = V = 128: cumsum with codes 86 + 118 -> 139; KDA B1 T2048 H8 8 + 21 + 24 -> 22.  On the way, KDA / GLA:
+// Measured (kernel time, against a kernel each for cumsum, WY prep and A): KDA B2 T8192 H32 K = V = 128 fp16, sigma = 1, with rotation and
+// D_QK 82 + 303 + 208 -> 381 us; GLA B4 T4096 H16 K = V = 128 fp16: cumsum with codes 87 + 117 -> 139; KDA B1 T2048 H8 bf16 8 + 21 + 24 ->
+// 23.  On the way, KDA / GLA:
 // 4 waves of 256 registers with W and U on the fp32 MFMA 501 / 165; on the bf16 MFMA 475; eight waves 467 / 148; the inverse one instruction
 // a term, the key operands read ahead of their products 443; no gate arithmetic where Hw is k, bf16 rounded by the conversion 409 / 141.  Bound by instruction
 // issue between its rendezvous (two workgroups cover part of each other's waits): the exponentials, the quantizations and the products of
@@ -103,9 +106,9 @@ struct Lds {
   static constexpr int r1 = 0;                        // decay tile, then e+ k; GLA: value codes; U: v
   static constexpr int r2 = 64 * K * 4;
   static constexpr int X = ROT ? OP : CD;             // an operand as its waves leave it
-  static constexpr int F_bytes = 6 * K * 4, GT_bytes = DELTA ? 16 * kBlk * 4 : 0, KQ_bytes = KQ ? K * 64 + K * 2 : 0;
+  static constexpr int F_bytes = 3 * K * 4, GT_bytes = DELTA ? 16 * kBlk * 4 : 0, KQ_bytes = KQ ? K * 64 + K * 2 : 0;
   // operands (3 queries, 6 keys) | then their codes, then the pieces of T; blocks of G and T behind them.  The write codes pass
-  // through the key operands' place, the fp64 totals through the queries'; the channel factors F lie at the end, dead when G is written.
+  // through the key operands' place, the fp64 totals through the queries'; the rows a_1 .. a_3 (F) lie at the end, dead when G is written.
   static constexpr int kq = r2 + (DO_A ? 3 * X : 0);
   static constexpr int TP_bytes = DELTA ? 3 * kSteps * 1024 : 0;
   static constexpr int gt = r2 + maxi(DO_A ? 9 * CD : 0, TP_bytes);
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
   __syncthreads();
 
-  // ---- 2: own rows.  gem: the decay of the lane's elements, later e-
+  // ---- 2: own rows.  gem: the decay of the lane's elements
   const float* const an_s = AN + J * K;
   float gem[KW][8];
   float spread = 0.0f, le = -__builtin_inff();
@@ -271,12 +274,12 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
     le = fmaxf(le, __shfl_xor(le, 32));
     if (kg == 0) le_s[64 * half + tok] = le;
   }
-  // channel factors of this sub-block: e^(a_J), and e^(a_I - a_J) for the later ones (slow: a_I itself)
+  // e^(a_J) of this sub-block, and a_J for the earlier ones (the tables that hold it are overwritten behind this phase)
   if (lane < K / 2) {
     const int n = K / 2 * half + lane;
     const float a = an_s[n];
-    E_s[J * K + n] = zoo_exp(a);
-    for (int I = J + 1; I < 4; ++I) F_s[pair_of(J, I) * K + n] = slow ? AN[I * K + n] : zoo_exp(AN[I * K + n] - a);
+    E_s[J * K + n] = zoo_exp_acc(a);
+    if (J > 0) F_s[(J - 1) * K + n] = a;
   }
   float bs = 1.0f, bh = 1.0f, bw = 1.0f, el = 0.0f;
   if constexpr (DELTA) {
@@ -395,7 +398,6 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       *(lq_v4i*)(p.Hw + roff + 32 * i) = o;
     }
     int ck[8], cs[8], cx[8];
-    float ge[8];
     lq_v8h x;
     lq_v4f kp[2];
 #pragma unroll
@@ -422,12 +424,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
           cs[e] = zoo_q8(xv * E4[e_], inv_sq, qmax);
         }
         if constexpr (L::KQ) ck[e] = zoo_q8(hf[e] * zoo_exp(l4[e_] - g - el), is4[e_], qmax);
-        ge[e] = em;
       }
-    }
-    if (!slow) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) gem[i][e] = ge[e];
     }
     if constexpr (DELTA) {
       *(lq_v4f*)(R1 + at<K>(tok, n)) = kp[0];
@@ -515,7 +512,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
 #pragma unroll
       for (int e4 = 0; e4 < 2; ++e4) {
         const int n = n0 + 32 * i + 4 * e4;
-        fr[i][e4] = *(const lq_v4f*)(F_s + pr * K + n);
+        fr[i][e4] = *(const lq_v4f*)(F_s + (I - 1) * K + n);
         if constexpr (DELTA) ki[i][e4] = *(const lq_v4f*)(R1 + at<K>(16 * I + rl, n));
       }
 #pragma unroll
@@ -528,19 +525,8 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       lq_v8h x;
       int cx[8];
       float we[8];
-      {
-        const lq_v4f f0 = fr[i][0], f1 = fr[i][1];
-        if (!slow) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) we[e] = gem[i][e] * (e < 4 ? f0[e & 3] : f1[e & 3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            we[e] = zoo_exp((e < 4 ? f0[e & 3] : f1[e & 3]) - gem[i][e]);
-            asm volatile("" : "+v"(we[e]));  // (a branch, not a selection: the exponentials are not evaluated in vain)
-          }
-        }
-      }
+      for (int e = 0; e < 8; ++e) we[e] = zoo_exp(fr[i][e >> 2][e & 3] - gem[i][e]);
 #pragma unroll
       for (int e4 = 0; e4 < 2; ++e4) {
 #pragma unroll
