@@ -100,6 +100,13 @@ LQ_DEV float zoo_mul_rn(float a, float b) {
   return p;
 }
 
+// fp16 of a0 * b and of a1 * b, each rounded once
+LQ_DEV uint32_t zoo_mul_h2(float a0, float a1, float b) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0" : "=&v"(r) : "v"(a0), "v"(a1), "v"(b));
+  return r;
+}
+
 // x / d rounded once to fp32 (the IEEE quotient) from r = RN(1 / d): q0 = RN(x r), rem = x - q0 d (exact in the fused
 // multiply-add), q = RN(q0 + rem r).  Correct for finite d > 0 and half-precision x (checked over every fp16 and bf16
 // value on the CPU); three instructions instead of the division sequence.

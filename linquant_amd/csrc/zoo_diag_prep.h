@@ -467,10 +467,10 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   }
   if (slow) dacc = dslow, gacc = gslow;
   const float sqk = sq * sk;
-  // element (row, column) of A
+  // elements (row, column ..) of A: sums of products of codes, scaled as they are rounded
   auto a_store = [&](int row, int c, lq_v4f v) __attribute__((always_inline)) {
     _Float16* dst = FUSED ? p.A + cb * 4096 + zoo_op_A(row, c) : p.A + ((t0 + row) * H + h) * 64 + c;
-    *(lq_v2i*)dst = lq_v2i{(int)zoo_pack_h2(v[0], v[1]), (int)zoo_pack_h2(v[2], v[3])};
+    *(lq_v2i*)dst = lq_v2i{(int)zoo_mul_h2(v[0], v[1], sqk), (int)zoo_mul_h2(v[2], v[3], sqk)};
   };
   // GLA: value rows, requested a phase ahead of their codes
   uint16_t vr[MODE == DIAG_GLA ? SEG : 1];
@@ -607,7 +607,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
       const lq_v4f d1 = *dg;
       lq_v4f o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r <= rl ? zoo_mul_rn(dacc[r] + d1[r], sqk) : 0.0f;
+      for (int r = 0; r < 4; ++r) o[r] = 4 * kg + r <= rl ? dacc[r] + d1[r] : 0.0f;
       a_store(tok, 16 * J + 4 * kg, o);
     }
   }
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
                          *(const lq_v4i*)(lds + L::r2 + L::CD * (Ip - 1) + ks * 1024 + lane * 16), acc);
       lq_v4f o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = zoo_mul_rn((float)acc[r], sqk);
+      for (int r = 0; r < 4; ++r) o[r] = (float)acc[r];
       a_store(16 * Ip + rl, 16 * Jp + 4 * kg, o);
       a_store(16 * Jp + rl, 16 * Ip + 4 * kg, lq_v4f{0.f, 0.f, 0.f, 0.f});
     }

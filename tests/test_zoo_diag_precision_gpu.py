@@ -2,6 +2,7 @@
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -64,3 +65,23 @@ def test_off_diagonal_blocks_are_no_further_from_float64_than_their_fp32_form(cu
     print(f"K {K} {dtype} rotate {rotate} gscale {gscale}: {off} entries, fp32 form {off32}")
     assert float(ref[..., below].float().abs().max()) > 0
     assert off <= 1.25 * off32 + 64, (off, off32)
+
+
+@pytest.mark.parametrize("K", [64, 128])
+def test_entries_of_A_are_rounded_once(cuda, K):
+    """Without decay every entry is a whole number times the fp32 product of the two scales: it is stored as the fp16 nearest to that
+    exact product, not to its fp32 rounding."""
+    from linquant_amd.kernels.zoo import _common as C
+
+    B, T, H = 2, 1024, 8
+    gen = torch.Generator().manual_seed(K)
+    cq, ck = (torch.randint(-127, 128, (B, T, H, K), generator=gen) for _ in range(2))
+    sq, sk = (torch.rand(H, generator=gen) * 0.01 + 0.005 for _ in range(2))
+    q, k = ((c * s[None, None, :, None]).half() for c, s in ((cq, sq), (ck, sk)))  # (fp16: within 0.07 of the code's middle)
+    A, _ = C.run_gla_A(q.cuda(), k.cuda(), torch.zeros(B, T, H, K, device="cuda"), sq.cuda(), sk.cuda(), 1.0, 127, (B, T, H, K, K))
+    dots = (_chunks(cq.double(), H) @ _chunks(ck.double(), H).transpose(-1, -2)).tril().numpy()
+    sqk = (sq * sk).view(1, 1, H, 1, 1).numpy()
+    once = (dots * sqk.astype(np.float64)).astype(np.float16)  # (the product is exact in 53 bits)
+    twice = (dots.astype(np.float32) * sqk).astype(np.float16)
+    assert (once != twice).sum() > 8
+    assert np.array_equal(_chunks(A.cpu(), H).numpy(), once)
