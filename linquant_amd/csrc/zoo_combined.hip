@@ -234,10 +234,9 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
-  // (per-channel decay, one launch in front of the recurrence: gc, logenv and Hw stay on the chip.  The call's workspace keeps the size
-  // that ABI 20 gives it)
-  take(l->gc, a->decay == LQ_DECAY_NONE ? 0 : B * T * H * (diag ? K : 1) * 4);
-  take(l->logenv, diag ? B * T * H * 4 : 0);
+  // (per-channel decay, one launch in front of the recurrence: gc, logenv and Hw stay on the chip)
+  take(l->gc, a->decay == LQ_DECAY_NONE || (diag && !big) ? 0 : B * T * H * (diag ? K : 1) * 4);
+  take(l->logenv, diag && big ? B * T * H * 4 : 0);
   take(l->kqT, B * NT * H * K * 64);
   take(l->vqT, delta ? 0 : B * NT * H * V * 64);
   take(l->wq, delta ? B * T * H * K : 0);
@@ -249,7 +248,7 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   take(l->qg, diag || !big ? B * T * H * K : 0);
   take(l->gpk, a->decay == LQ_DECAY_SCALAR && !big ? B * NT * H * 64 * 4 : 0);
   take(l->vcT, !big && !delta ? B * NT * H * V * 64 : 0);
-  take(l->Hw, delta && (diag || big) ? B * T * H * K * 2 : 0);
+  take(l->Hw, delta && big ? B * T * H * K * 2 : 0);
   take(l->W, delta && big ? B * T * H * K * 2 : 0);
   take(l->U, delta ? B * T * H * V * 2 : 0);
   take(l->fw, delta && big ? B * T * H * 4 : 0);
@@ -288,8 +287,8 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
-  float* gc = a->decay == LQ_DECAY_NONE ? nullptr : (float*)(ws + l.gc);
-  float* logenv = diag ? (float*)(ws + l.logenv) : nullptr;
+  float* gc = a->decay == LQ_DECAY_NONE || (diag && !big) ? nullptr : (float*)(ws + l.gc);
+  float* logenv = diag && big ? (float*)(ws + l.logenv) : nullptr;
   int8_t* kqT = (int8_t*)(ws + l.kqT);
   int8_t* vqT = delta ? nullptr : (int8_t*)(ws + l.vqT);
   int8_t* wq = delta ? (int8_t*)(ws + l.wq) : nullptr;

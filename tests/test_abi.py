@@ -246,7 +246,8 @@ def test_workspace_of_a_call_without_a_prologue_has_no_room_for_one(K, V):
 @pytest.mark.parametrize("cell,family,decay", [("gla", 0, 2), ("deltanet", 1, 0), ("gated_deltanet", 1, 1), ("kda", 1, 2)])
 def test_workspace_of_the_recurrence_and_output_launch_holds_what_is_read(cell, family, decay):
     """lq_zoo_chunk_forward, 64-token chunks of many chains: the operands of zoo_scan.hip and what its pre-passes hand to each other,
-    each rounded up to 256 bytes; per-token factors and chunk decays of the delta family only in their packed form."""
+    each rounded up to 256 bytes; per-token factors and chunk decays of the delta family only in their packed form.  Per-channel decay:
+    one launch makes all of them, so the cumulative decay, its envelope and Hw have no place here."""
     B, T, H, K, V = 2, 640, 32, 128, 64
     up = lambda n: -(-n // 256) * 256  # noqa: E731
     chunks = B * (T // 64) * H
@@ -258,9 +259,6 @@ def test_workspace_of_the_recurrence_and_output_launch_holds_what_is_read(cell, 
         want += 2 * up(chunks * V * 64) + up(chunks * K * 4)                              # value codes (write, local), chunk decays
     else:
         want += up(chunks * 64 * K) + up(chunks * (128 + K) * 4) + up(chunks * 64 * V * 2)  # codes of W, packed factors, U
-    if decay == 2:
-        want += up(chunks * 64 * K * 4) + up(chunks * 64 * 4)                             # cumulative decay, envelope
-        want += up(chunks * 64 * K * 2) if family else 0                                  # Hw
     if decay == 1:
         want += 2 * up(chunks * 64 * 4)                                                   # cumulative decay, once by chunk and head
     assert n.value == want
