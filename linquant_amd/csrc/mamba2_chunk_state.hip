@@ -152,11 +152,12 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(Params p) {
   const float bs_t = KEYSIDE ? 0.0f : p.bscale_g[(int64_t)g * p.sbs_g];
 
   // fixed thread -> work mapping of the quantize phase: x slab = 16 token quads x 16 groups of 4 channels (all 256
-  // threads), B slab = 16 token quads x NT/8 groups of 8 channels (threads without a B item load a clamped address)
+  // threads), B slab = 16 token quads x NT/8 groups of 8 channels (64 columns: threads 128 .. repeat the requests of threads 0 ..;
+  // 64 tokens further on, as tid / kBItems goes, would lie behind the end of B at the last slab of the last sequence)
   const int kqx = tid >> 4, c4x = tid & 15;
   constexpr int kBItems = NT / 8;
   const bool has_b = (NT == 128) || (tid < 16 * kBItems);
-  const int kqb = (NT == 128) ? (tid >> 4) : (tid / kBItems);
+  const int kqb = (NT == 128) ? (tid >> 4) : ((tid / kBItems) & 15);
   const int cb8 = (NT == 128) ? (tid & 15) : (tid % kBItems);
 
   const int pr = p0 + 16 * wave + rl;

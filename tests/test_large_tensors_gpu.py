@@ -206,3 +206,42 @@ def test_long_sequences(cuda):
     assert torch.equal(o[0], o[2]) and torch.equal(ht[0], ht[2]), "batch rows with the same data differ"
     o_s, _ = zoo.chunk_kda_int8(q[:1, :4096], k[:1, :4096], v[:1, :4096], g[:1, :4096], beta[:1, :4096], zs, sigma=0.5, eta=0.0)
     assert torch.equal(o[:1, :4096], o_s), "causal prefix differs from the launch on the prefix"
+
+
+@pytest.mark.parametrize("keyside", [True, False])
+def test_keys_that_end_where_their_allocation_ends(cuda, keyside):
+    """64 state columns, whole chunks, B as many whole 2 MiB pages: nothing may be requested behind its last row (threads of the chunk
+    state kernel that have no piece of a 64-column tile to load once asked for rows of a slab further on).  The last sequence equals
+    its own launch, bit for bit."""
+    from linquant_amd.calibration import Mamba2Shape, calibrate_mamba2, mamba2_params
+    from linquant_amd.kernels.mamba2 import ssd_combined as M
+    from linquant_amd.kernels.mamba2.fused_split_rotate_xBC import fused_split_rotate_quant_xBC
+
+    B, L = 8, 4096
+    s = Mamba2Shape(batch=B, seqlen=L, nheads=16, headdim=64, dstate=64, ngroups=8, chunk=256)
+    page = 2 << 20
+    assert B * L * s.ngroups * s.dstate % page == 0
+    p = mamba2_params(s, 42, cuda)
+    gen = torch.Generator(device=cuda).manual_seed(0)
+    xBC = torch.randn(B, L, s.xbc_dim, generator=gen, device=cuda, dtype=torch.float16)
+    dt_raw = (torch.randn(B, L, s.nheads, generator=gen, device=cuda) * 0.5 - 4.5).half()
+    cal = Mamba2Shape(batch=1, seqlen=2048, nheads=16, headdim=64, dstate=64, ngroups=8, chunk=256)
+    sc = calibrate_mamba2(cal, xBC[:1, :2048], dt_raw[:1, :2048], p)
+    torch.cuda.empty_cache()
+
+    def forward(xb, dtb):
+        args = (xb, p["r_signs"], s.nheads, s.ngroups, s.dstate, s.headdim, sc["B_inv_scale"], sc["C_inv_scale"])
+        kw = {}
+        if keyside:
+            x, qB, qC, b_fp = fused_split_rotate_quant_xBC(*args, return_b_fp=True)
+            kw = dict(keyside=True, x_scale_hp=sc["x_scale_hp"], b_fp=b_fp, b_gate_scale=sc["b_gate_scale"])
+        else:
+            x, qB, qC = fused_split_rotate_quant_xBC(*args)
+        return M._quant_mamba_chunk_scan_combined_fwd(
+            x, dtb, p["dt_scale"], p["A_log"], p["A_log_scale"], qB, sc["B_scale"], qC, sc["C_scale"], s.chunk, p["D"],
+            p["D_scale"], dt_bias=p["dt_bias"], dt_softplus=True, static_state_scale=sc["static_state_scale"],
+            static_cb_scale=sc["static_cb_scale"], alpha_hp=sc["alpha_hp"], bscale_g=sc["bscale_g"], **kw)[0]
+
+    full, one = forward(xBC, dt_raw), forward(xBC[-1:], dt_raw[-1:])
+    torch.cuda.synchronize()
+    assert torch.equal(full[-1:], one) and float(one.float().abs().max()) > 0
