@@ -24,9 +24,11 @@ struct Layout {
 // (16 KB) and one more set of codes.
 //   bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch.
 //   else: one launch for short chains whose operands stay in the last-level cache.
-//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns; K = V = 128 with a prologue: 40), and more than 32
-//   steps of a second tile per compute unit (more than 256) where not even 16 KB are saved: the two launches.
-// Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256:
+//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns; K = V = 128 with a prologue: below), and more than
+//   32 steps of a second tile per compute unit (more than 256) where not even 16 KB are saved: the two launches.
+// Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256
+// (before the operand pre-pass took the last chunks first, zoo_params.h, by which the one launch gains.  K = V = 128 without a prologue past
+// 128 steps: T = 16384, 96 tiles is 287 us by the two launches of this rule and 255 by the one; its line has not been moved):
 //                     T = 256     1024         2048         4096         8192        16384 tokens
 //   K = V = 128       1.17..1.60  1.06..1.31   1.03..1.27   0.91..1.27   0.95..1.26   0.87..1.13
 //     with prologue   1.16..1.29  1.05..1.21   1.02..1.25   1.01..1.24   1.00..1.22   0.97..1.14
@@ -41,13 +43,26 @@ struct Layout {
 //     B*H*NT <= 1024              1.01..1.18   0.97..1.08
 //     with prologue   1.12..1.30  0.93..1.11   0.89..1.07   0.84..1.04   0.83..1.00   0.79..0.96
 //     B*H*NT <= 2048              0.99..1.11   0.98..1.07
-// K = V = 128 with a prologue past 128 steps, since the operand pre-pass takes the last chunks first (zoo_params.h), one set of inputs, no
-// and scalar decay, T = 16384: 40 tiles 1.06 1.04, 56 1.09 1.02, 72 1.10 1.04, 96 1.15 1.10; T = 12288, 64 tiles 1.05.  K 128, V 64 with
-// a prologue, 80 tiles: 0.99 0.94.
-bool linear_scan(bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
+// K = V = 128 with a prologue past 128 steps, two or three sets of inputs in turn, no decay | scalar decay:
+//   steps       129         192         256         384         512         768         1024        1536
+//   32 tiles    1.04 1.04   1.01 1.01   1.01 1.00   1.00 0.97   1.05 1.00   0.97 0.93   0.95 0.89
+//   40          1.07 1.09   1.06 1.05   1.05 1.02   1.04 0.99   0.99 0.95   0.96 0.92   0.93 0.89
+//   48          1.03 1.04   1.03 1.01   1.03 0.99   1.02 0.98   1.02 0.98   0.99 0.94   0.97 0.93
+//   56          1.12 1.10   1.10 1.06   1.11 1.05   1.08 1.01   1.06 0.99   1.04 0.96   1.02 0.94   1.00 0.92
+//   64          1.07 1.07   1.07 1.03   1.16 1.10   1.09 1.03   1.08 1.02   1.06 1.00   1.05 0.99   1.04 0.98
+//   72                                                          1.08 1.01   1.07 0.99               1.05 0.97
+//   80          1.05 1.04   1.10 1.05   1.09 1.05   1.07 1.03   1.05 1.01   1.04 0.99   1.03 0.98
+//   88                                                                      1.09 1.01   1.09 1.01
+//   96          1.11 1.09   1.15 1.10   1.14 1.10   1.12 1.06   1.10 1.05   1.09 1.03   1.08 1.02   1.09 1.03
+//   112         1.16 1.14   1.17 1.12   1.16 1.10   1.14 1.09   1.13 1.08   1.12 1.06   1.14 1.07
+// Few tiles are bound by the chain, whose step is the shorter one in a launch without the output, with scalar decay by more; the launch
+// saved counts for less the longer the chain.
+bool linear_scan(bool prologue, bool scalar, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
-  const int64_t few = prologue && K == 128 && V >= 128 ? 40 : 128;
-  if (NT > 128 && tiles < few) return false;
+  int64_t most = 128;
+  if (prologue && K >= 128 && V >= 128 && tiles >= 40)
+    most = scalar ? (tiles < 56 ? 256 : (tiles < 64 ? 384 : (tiles < 88 ? 512 : NT))) : (tiles < 48 ? 384 : (tiles < 56 ? 512 : (tiles < 64 ? 1024 : NT)));
+  if (NT > most && tiles < 128) return false;
   const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
   if (saved >= 16384) return true;
   if (saved > 0) return NT <= 32 || tiles <= 256;
@@ -110,7 +125,7 @@ Layout plan(const lq_zoo_simple_gla_args* a, bool scan) {
 }
 
 bool scan_route(const lq_zoo_simple_gla_args* a) {
-  return a->chunk_size == 64 && linear_scan(has_prologue(a), a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
+  return a->chunk_size == 64 && linear_scan(has_prologue(a), a->g != nullptr, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
 }
 
 }  // namespace
@@ -119,7 +134,7 @@ extern "C" int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* a
   if (!a || !bytes) return LQ_ERR_NULL;
   if (const int rc = check_dims(a)) return rc;
   *bytes = plan(a, scan_route(a)).total;
-  if (a->chunk_size == 64 && has_prologue(a)) {  // its route depends on the tables' addresses too: enough for either
+  if (a->chunk_size == 64 && has_prologue(a)) {  // its route depends on the decay and on the tables' addresses too: enough for either
     const int64_t other = plan(a, !scan_route(a)).total;
     if (other > *bytes) *bytes = other;
   }
@@ -216,7 +231,9 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // output beside it, and the one launch was the faster at every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0
 // to 1.7 times with scalar decay and without, 1.0 to 1.56 with per-channel decay; the most on few long chains).  GLA: more than 128 steps
 // on less than half of the compute units took four launches while the pre-pass was two of them; against all four the two launches are,
-// at T = 16384, K = V = 128, H = 4 / 12 / 28: 164 -> 152, 308 -> 229, 558 -> 389 us, K = V = 64, H = 4 / B2 H16: 115 -> 113, 326 -> 300.
+// at T = 16384, K = V = 128, H = 4 / 12 / 28: 164 -> 152, 308 -> 229, 558 -> 389 us, K = V = 64, H = 4 / B2 H16: 115 -> 113, 326 -> 300; at
+// T = 65536, K = V = 128, H = 1 / 4: 452 -> 445, 678 -> 655.  The slower ones are those of one or two heads of 64 key channels from 512
+// steps on, by 2 to 7 % (T = 65536, V = 64, H = 1 / 2 / 4: 338 -> 362, 361 -> 382, 423 -> 423).
 namespace {
 
 struct FLayout {

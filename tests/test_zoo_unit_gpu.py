@@ -60,15 +60,16 @@ def test_more_chunks_than_the_grid_holds_in_one_dimension(cuda):
 
 
 @pytest.mark.parametrize("cell", ["linear_none", "mamba2"])
-@pytest.mark.parametrize("H,prologue", [(31, False), (32, False), (9, True), (10, True)])
-def test_long_chains_on_either_side_of_the_rule(cuda, cell, H, prologue):
-    """More than 128 chunk steps, K = V = 128: one launch or two by the number of workgroups, the same bits as the stages."""
+@pytest.mark.parametrize("H,NT,prologue", [(31, 129, False), (32, 129, False), (9, 129, True), (10, 129, True), (10, 256, True), (10, 257, True),
+                                           (10, 385, True), (13, 513, True), (14, 385, True), (16, 513, True), (22, 513, True)])
+def test_long_chains_on_either_side_of_the_rule(cuda, cell, H, NT, prologue):
+    """More than 128 chunk steps, K = V = 128: one launch or two by the numbers of workgroups and steps and the decay, the same bits as the stages."""
     from linquant_amd.kernels import zoo
     from linquant_amd.kernels.zoo.prologue import rotation_signs
     from oracle.zoo_reference import signed_hadamard
 
     K = V = 128
-    q, k, v, g, _ = (None if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=64 * 129, H=H, K=K, V=V, seed=H, dtype=torch.float16))
+    q, k, v, g, _ = (None if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=64 * NT, H=H, K=K, V=V, seed=H, dtype=torch.float16))
     gen = torch.Generator().manual_seed(H)
     r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
     sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.01), "kw": r(H, K, lo=0.005, hi=0.015), "vw": r(H, V, lo=0.02, hi=0.04),
