@@ -1,6 +1,7 @@
 """GPU test of the launch that runs the cumulative sum and C.B^T side by side (mamba2_cumsum_bmm.hip): the one-call forward equals the
-stages one after the other bit for bit at the edges of its dispatch: every chunk size, units that do and do not divide over the 8 XCDs,
-one tile to a workgroup up to eight, a ragged last chunk, heads off the 16-head tile, groups, and a d_state it leaves to two launches."""
+stages one after the other bit for bit at the edges of its dispatch: every chunk size that the other stages take, units that
+do and do not divide over the 8 XCDs, either with one tile to a workgroup and with several and a partial last workgroup, a ragged last
+chunk, heads off the 16-head tile, groups, and a d_state it leaves to two launches."""
 
 import pytest
 import torch
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("keyside", [True, False])
 @pytest.mark.parametrize("B,L,H,G,N,Q", [
     (1, 64, 1, 1, 64, 64), (2, 1000, 6, 2, 128, 128), (8, 256, 16, 1, 128, 256), (3, 700, 17, 1, 64, 256), (2, 1024, 4, 1, 128, 512),
-    (4, 2560, 32, 4, 64, 256), (8, 4096, 80, 1, 128, 256), (1, 300, 4, 1, 256, 256)])
+    (4, 2560, 32, 4, 64, 256), (8, 4096, 80, 1, 128, 256), (3, 5000, 80, 1, 128, 256), (1, 6300, 80, 2, 64, 256), (1, 300, 4, 1, 256, 256)])
 def test_one_call_equals_the_stages(cuda, B, L, H, G, N, Q, keyside):
     from linquant_amd.kernels.hadamard import kronecker_hadamard_fwd
     from linquant_amd.kernels.mamba2 import ssd_combined as M

@@ -1,8 +1,8 @@
 """GPU test of the launch in front of the recurrence under per-channel decay (zoo_diag_prep.h) at the edges of its branches: sub-blocks
 whose decay is factorized and sub-blocks that take one exponential per product in one chunk, grids that do and do not divide over the
 8 XCDs, both key widths, value widths of one pass, several and a partial last one, with and without rotation and D_QK.  Its fused forms
-run the code of the stage entry points, which the float64 oracle pins in test_zoo_gpu.py (strong decay included), so outputs and final
-states are equal bit for bit."""
+run the code of the stage entry points, so outputs and final states are equal bit for bit: that comparison pins the forms to each other,
+the last test here and test_zoo_gpu.py pin them to the float64 oracle."""
 
 import pytest
 import torch
@@ -45,3 +45,30 @@ def test_one_launch_equals_the_stages_in_every_branch(cuda, cell, B, NT, H, K, V
     torch.cuda.synchronize()
     assert torch.isfinite(o1.float()).all() and float(o1.float().abs().max()) > 0
     assert torch.equal(o0, o1) and torch.equal(h0, h1)
+
+
+@pytest.mark.parametrize("cell", ["gla", "kda"])
+@pytest.mark.parametrize("K,rot", [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("staged", [False, True])
+def test_halves_of_a_sub_block_that_decide_apart_match_the_oracle(cuda, cell, K, rot, staged):
+    """The two waves of a 16-token sub-block, half of the channels each, decide for themselves whether its decay is factorized: here the
+    lower, the upper, both or neither half of the channels decays by far more than e^40 in it, every order of the four in a chunk."""
+    from oracle.zoo_reference import signed_hadamard
+
+    B, T, H, V = 1, 64 * 6, 4, 64
+    q, k, v, g, beta = zc.inputs(cell, B=B, T=T, H=H, K=K, V=V, seed=K)
+    gen = torch.Generator().manual_seed(3)
+    order = torch.stack([torch.randperm(4, generator=gen) for _ in range(T // 64 * H)]).view(T // 64, H, 4).permute(0, 2, 1)
+    kind = order.reshape(T // 16, H).repeat_interleave(16, dim=0)  # bit 0: the lower half of the channels, bit 1: the upper
+    far = torch.stack([kind & 1, kind >> 1], dim=-1).repeat_interleave(K // 2, dim=-1).bool()
+    some = torch.rand(T, H, K, generator=gen) < 0.2  # (in one channel of five, so that the others still carry the output)
+    g = torch.where(far & some, g * 60.0, g).contiguous()
+    rise = g.view(B, T // 16, 16, H, 2, K // 2)[:, :, 1:].sum(2).amin(-1)  # spread of each half over its sub-block
+    wide = (rise < -40.0).view(B, T // 16, H, 2)
+    assert ((wide[..., 0] == far.view(1, T // 16, 16, H, K)[:, :, 0, :, 0]) & (wide[..., 1] == far.view(1, T // 16, 16, H, K)[:, :, 0, :, -1])).float().mean() > 0.9
+    tensors = (q, k, v, g, beta)
+    R = signed_hadamard(K, 3) if rot else None
+    qz, run = zc.calibrated(cell, tensors, eta=0.0, rot_qk=R)
+    scales = qz.kernel_scales(0, H, K, V, delta=cell == "kda")
+    out = zc.run_kernel(cell, tensors, scales, eta=0.0, rot=R, debug={} if staged else None)[0]
+    zc.check(out, run, qz, f"{cell} K={K} rot={rot} staged={staged}")
