@@ -223,11 +223,10 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 }
 
 // ---- the other cells: chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8
-// (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry each way round: the stage entry points in
-// the order the Python wrappers issue them, over one workspace.  64-token chunks take the fused pre-passes (the cumsum / WY
-// launch also makes the write codes), 128-token chunks the separate write-codes launch.  64-token chunks run the recurrence and the
-// output as one launch (zoo_scan.hip: the same bits, no stored states, no E in memory), per-channel decay with one launch in front of it
-// (zoo_diag_prep.h).  Neither family needs a rule.  Delta: its step is two rendezvous and two dependent products with or without the
+// (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry over one workspace.  128-token chunks: the stage
+// entry points in the order the Python wrappers issue them.  64-token chunks: recurrence and output in one launch (zoo_scan.hip: the bits
+// of the stages, no stored states, no E in memory); in front of it under per-channel decay one launch for everything (zoo_diag_prep.h),
+// otherwise cumsum (scalar decay) and WY prep, which also makes the write codes.  Neither family needs a rule.  Delta: its step is two rendezvous and two dependent products with or without the
 // output beside it, and the one launch was the faster at every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0
 // to 1.7 times with scalar decay and without, 1.0 to 1.56 with per-channel decay; the most on few long chains).  GLA: more than 128 steps
 // on less than half of the compute units took four launches while the pre-pass was two of them; against all four the two launches are,

@@ -27,15 +27,23 @@
 //   4  rotation: 9 operands x 32 channels per wave, R in registers   5  INT8 products; inverse of the diagonal blocks
 //   6  block columns of T                                       7  W, U: T and the rows in three bf16 pieces, six products
 //
-// Measured (kernel time, against a kernel each for cumsum, WY prep and A): KDA B2 T8192 H32 K = V = 128 fp16, sigma = 1, with rotation and
-// D_QK 82 + 303 + 208 -> 381 us; GLA B4 T4096 H16 K = V = 128 fp16: cumsum with codes 87 + 117 -> 139; KDA B1 T2048 H8 bf16 8 + 21 + 24 ->
-// 23.  On the way, KDA / GLA:
-// 4 waves of 256 registers with W and U on the fp32 MFMA 501 / 165; on the bf16 MFMA 475; eight waves 467 / 148; the inverse one instruction
-// a term, the key operands read ahead of their products 443; no gate arithmetic where Hw is k, bf16 rounded by the conversion 409 / 141.  Bound by instruction
-// issue between its rendezvous (two workgroups cover part of each other's waits): the exponentials, the quantizations and the products of
-// phases 2 and 3, which stay on the fp32 MFMA: 33 cycles a 16x16x4, during which its SIMD issues no vector instruction (the half-precision
-// MFMA costs them only its issue), yet splitting their operands in three would cost more.  Persistent workgroups with the next chunk's
-// requests ahead spilled (KDA 714), three workgroups a compute unit for GLA too (194).
+// Measured (kernel us, against a kernel each for cumsum, WY prep and A), fp16 unless said, with rotation: KDA B2 T8192 H32 K = V = 128,
+// sigma = 1, 82 + 266 + 208 -> 380 (with D_QK 82 + 303 + 208 -> 381, bf16 377); sigma = 0.5, 82 + 268 + 208 -> 454 (with D_QK 82 + 303
+// + 208 -> 451, bf16 81 + 276 + 203 -> 454); GLA B4 T4096 H16 K = V = 128 cumsum with codes 87 + 117 -> 139; KDA B1 T2048 H8 bf16
+// 8 + 21 + 24 -> 23.
+// On the way, KDA / GLA: 4 waves of 256 registers with W and U on the fp32 MFMA 501 / 165; on the bf16 MFMA 475; eight waves 467 / 148;
+// the inverse one instruction a term, the key operands read ahead of their products 443; no gate arithmetic where Hw is k, bf16 rounded
+// by the conversion 409 / 141; one exponential for a key operand (above).
+// Bound by vector issue and the waits at its rendezvous, of which two workgroups cover part of each other's.  By counters, KDA B2 T8192 /
+// GLA B4 T4096: vector unit busy 74 / 73 % of the time, matrix unit 26 / 11 %, waves waiting 38 % of theirs, LDS conflicts 2.5 / 3.5 %,
+// memory 1093 / 507 MB at 2.9 / 3.6 TB/s; KDA B1 T2048, one workgroup to a compute unit: 31, 12, 24 %.  The vector work is the
+// exponentials, the quantizations and what the products of phases 2 and 3 hold up: these stay on the fp32 MFMA, 33 cycles a 16x16x4,
+// during which its SIMD issues no vector instruction (the half-precision MFMA costs them only its issue), yet splitting their operands in
+// three would cost more.  Persistent workgroups with the next chunk's requests ahead spilled (KDA 714), three workgroups a compute unit for
+// GLA too (194).
+// Spilled registers: DIAG_KDA at K = 128 with the gate (sigma < 1, tau > 0) keeps Hw beside k over the key operands and spills 13 to 19
+// of its 128 in fp16 and up to 15 in bf16 (56 to 80 and up to 64 bytes a lane; about 300 of the 972 MB read and of the 730 MB written at
+// sigma = 0.5 above); without the gate at most one (bf16 with D_QK); the other forms and K = 64 none.
 #pragma once
 
 #include <type_traits>
