@@ -226,9 +226,10 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry over one workspace.  128-token chunks: the stage
 // entry points in the order the Python wrappers issue them.  64-token chunks: recurrence and output in one launch (zoo_scan.hip: the bits
 // of the stages, no stored states, no E in memory); in front of it under per-channel decay one launch for everything (zoo_diag_prep.h),
-// otherwise cumsum (scalar decay) and WY prep, which also makes the write codes.  Neither family needs a rule.  Delta: its step is two rendezvous and two dependent products with or without the
-// output beside it, and the one launch was the faster at every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0
-// to 1.7 times with scalar decay and without, 1.0 to 1.56 with per-channel decay; the most on few long chains).  GLA: more than 128 steps
+// otherwise cumsum (scalar decay) and WY prep, which also makes the write codes.  Neither family needs a rule.
+// Delta: its step is two rendezvous and two dependent products with or without the output beside it, and the one launch was the faster at
+// every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0 to 1.7 times with scalar decay and without, 1.0 to 1.56
+// with per-channel decay; the most on few long chains).  GLA: more than 128 steps
 // on less than half of the compute units took four launches while the pre-pass was two of them; against all four the two launches are,
 // at T = 16384, K = V = 128, H = 4 / 12 / 28: 164 -> 152, 308 -> 229, 558 -> 389 us, K = V = 64, H = 4 / B2 H16: 115 -> 113, 326 -> 300; at
 // T = 65536, K = V = 128, H = 1 / 4: 452 -> 445, 678 -> 655.  The slower ones are those of one or two heads of 64 key channels from 512
