@@ -22,47 +22,35 @@ struct Layout {
 // whole chip for the output.  What the one launch saves is launches (4 .. 6 us a call, which decides short calls), the stored states
 // (2 K V bytes a chunk and head) and the second reading of raw operands (with a prologue: of their token-major codes), against A
 // (16 KB) and one more set of codes.
-//   bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch.
-//   else: one launch for short chains whose operands stay in the last-level cache.
-//   more than 128 steps on less than half of the compute units (128 tiles of 32 columns; K = V = 128 with a prologue: below), and more than
-//   32 steps of a second tile per compute unit (more than 256) where not even 16 KB are saved: the two launches.
-// Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, B*H = 4 .. 256
-// (before the operand pre-pass took the last chunks first, zoo_params.h, by which the one launch gains.  K = V = 128 without a prologue past
-// 128 steps: T = 16384, 96 tiles is 287 us by the two launches of this rule and 255 by the one; its line has not been moved):
-//                     T = 256     1024         2048         4096         8192        16384 tokens
-//   K = V = 128       1.17..1.60  1.06..1.31   1.03..1.27   0.91..1.27   0.95..1.26   0.87..1.13
-//     with prologue   1.16..1.29  1.05..1.21   1.02..1.25   1.01..1.24   1.00..1.22   0.97..1.14
-//   K 128, V 64       1.09..1.44  0.94..1.24   0.83..1.11   0.85..1.08   0.81..1.03   0.75..0.96
-//     B*H*NT <= 2048              1.00..1.24   1.01..1.11
-//     with prologue   1.18..1.41  1.05..1.30   1.03..1.18   1.01..1.14   0.97..1.08   0.88..1.03
-//   K 64, V 128       1.09..1.53  0.99..1.28   0.84..1.15   0.80..1.10   0.78..1.11   0.79..1.03
-//     B*H*NT <= 4096              1.01..1.28   1.00..1.15   0.99..1.10
-//     with prologue   1.27..1.48  1.12..1.29   1.01..1.27   0.94..1.21   0.89..1.15   0.94..1.09
-//     and B*H <= 64                                         1.09..1.21   0.97..1.15
-//   K = V = 64        1.09..1.39  0.81..1.18   0.72..1.08   0.72..1.00   0.67..0.97   0.65..0.91
-//     B*H*NT <= 1024              1.01..1.18   0.97..1.08
-//     with prologue   1.12..1.30  0.93..1.11   0.89..1.07   0.84..1.04   0.83..1.00   0.79..0.96
-//     B*H*NT <= 2048              0.99..1.11   0.98..1.07
-// K = V = 128 with a prologue past 128 steps, two or three sets of inputs in turn, no decay | scalar decay:
-//   steps       129         192         256         384         512         768         1024        1536
-//   32 tiles    1.04 1.04   1.01 1.01   1.01 1.00   1.00 0.97   1.05 1.00   0.97 0.93   0.95 0.89
-//   40          1.07 1.09   1.06 1.05   1.05 1.02   1.04 0.99   0.99 0.95   0.96 0.92   0.93 0.89
-//   48          1.03 1.04   1.03 1.01   1.03 0.99   1.02 0.98   1.02 0.98   0.99 0.94   0.97 0.93
-//   56          1.12 1.10   1.10 1.06   1.11 1.05   1.08 1.01   1.06 0.99   1.04 0.96   1.02 0.94   1.00 0.92
-//   64          1.07 1.07   1.07 1.03   1.16 1.10   1.09 1.03   1.08 1.02   1.06 1.00   1.05 0.99   1.04 0.98
-//   72                                                          1.08 1.01   1.07 0.99               1.05 0.97
-//   80          1.05 1.04   1.10 1.05   1.09 1.05   1.07 1.03   1.05 1.01   1.04 0.99   1.03 0.98
-//   88                                                                      1.09 1.01   1.09 1.01
-//   96          1.11 1.09   1.15 1.10   1.14 1.10   1.12 1.06   1.10 1.05   1.09 1.03   1.08 1.02   1.09 1.03
-//   112         1.16 1.14   1.17 1.12   1.16 1.10   1.14 1.09   1.13 1.08   1.12 1.06   1.14 1.07
-// Few tiles are bound by the chain, whose step is the shorter one in a launch without the output, with scalar decay by more; the launch
-// saved counts for less the longer the chain.
-bool linear_scan(bool prologue, bool scalar, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
+// Up to 128 tiles of 32 columns the one launch runs a chain in segments side by side (zoo_scan.hip), and is the faster but for K = V = 64
+// on more than half of the compute units' worth of tiles, where the chain is long.  GPU time of the two launches over that of the one, no
+// decay .. scalar decay (B = 1; graph replays of two sets of inputs in turn):
+//                                T = 2048      4096          8192          32768
+//   K = V = 128, 16 tiles        1.50 .. 1.63  1.45 .. 1.60  1.65 .. 1.76  1.75 .. 1.79
+//     48 .. 128 tiles            1.11 .. 1.39  1.09 .. 1.29  1.08 .. 1.29  1.12 .. 1.35
+//     with prologue              1.14 .. 1.54  1.15 .. 1.55  1.10 .. 1.73  1.12 .. 1.77
+//   K 128, V 64                  1.00 .. 1.49  0.97 .. 1.51  0.98 .. 1.59  1.01 .. 1.63
+//     with prologue              1.16 .. 1.64  1.07 .. 1.65  1.05 .. 1.65  1.05 .. 1.66
+//   K 64, V 128                  1.08 .. 1.57  1.09 .. 1.66  1.05 .. 1.67  1.04 .. 1.86
+//     with prologue              1.27 .. 1.72  1.26 .. 1.80  1.19 .. 1.82  1.01 .. 1.94
+//   K = V = 64, 16 tiles         1.27 .. 1.41  1.34 .. 1.38  1.50 .. 1.51  1.42 .. 1.57
+//     48                         1.04 .. 1.14  1.05 .. 1.08  1.05 .. 1.07  1.04
+//     64                         1.02 .. 1.06  1.03 .. 1.10  0.90 .. 0.99  0.96 .. 1.09
+//     80                         1.05 .. 1.06  0.98 .. 1.06  0.91 .. 0.94  0.90 .. 0.97
+//     96                         0.99 .. 1.02  0.91 .. 0.99  0.80 .. 0.84  0.85 .. 0.94
+//     128                        0.96 .. 1.00  0.82 .. 0.87  0.74 .. 0.83  0.95 .. 1.11
+//     with prologue, to 80       1.09 .. 1.44  1.08 .. 1.43  1.00 .. 1.55  1.02 .. 1.61
+//     96 .. 128                  1.05 .. 1.11  0.98 .. 1.05  0.91 .. 1.01  0.97 .. 1.19
+// More tiles: bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch, while 16 KB are saved or there is no second
+// tile per compute unit (more than 256) or no more than 32 steps; else: one launch for short chains whose operands stay in the last-level
+// cache.  Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, before the
+// operand pre-pass took the last chunks first (zoo_params.h), by which the one launch gains: T = 2048 .. 8192, B*H = 4 .. 256 (where fewer
+// tiles ran their chains in one piece): K = V = 128 0.91 .. 1.27, with prologue 1.00 .. 1.25; K 128, V 64 0.81 .. 1.11, with prologue
+// 0.97 .. 1.18; K 64, V 128 0.78 .. 1.15 (B*H*NT <= 4096 0.99 .. 1.15), with prologue 0.89 .. 1.27; K = V = 64 0.67 .. 1.08, with
+// prologue 0.83 .. 1.07 (B*H*NT <= 2048 0.98 .. 1.07).
+bool linear_scan(bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
-  int64_t most = 128;
-  if (prologue && K >= 128 && V >= 128 && tiles >= 40)
-    most = scalar ? (tiles < 56 ? 256 : (tiles < 64 ? 384 : (tiles < 88 ? 512 : NT))) : (tiles < 48 ? 384 : (tiles < 56 ? 512 : (tiles < 64 ? 1024 : NT)));
-  if (NT > most && tiles < 128) return false;
+  if (tiles <= 128) return K + V > 128 || (prologue ? NT <= 64 || tiles <= 80 : tiles <= 52 || NT <= (tiles <= 64 ? 64 : (tiles <= 96 ? 32 : 16)));
   const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
   if (saved >= 16384) return true;
   if (saved > 0) return NT <= 32 || tiles <= 256;
@@ -125,7 +113,7 @@ Layout plan(const lq_zoo_simple_gla_args* a, bool scan) {
 }
 
 bool scan_route(const lq_zoo_simple_gla_args* a) {
-  return a->chunk_size == 64 && linear_scan(has_prologue(a), a->g != nullptr, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
+  return a->chunk_size == 64 && linear_scan(has_prologue(a), a->batch, a->seqlen, a->nheads, a->kdim, a->vdim);
 }
 
 }  // namespace
@@ -134,7 +122,7 @@ extern "C" int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* a
   if (!a || !bytes) return LQ_ERR_NULL;
   if (const int rc = check_dims(a)) return rc;
   *bytes = plan(a, scan_route(a)).total;
-  if (a->chunk_size == 64 && has_prologue(a)) {  // its route depends on the decay and on the tables' addresses too: enough for either
+  if (a->chunk_size == 64 && has_prologue(a)) {  // its route depends on the tables' addresses too: enough for either
     const int64_t other = plan(a, !scan_route(a)).total;
     if (other > *bytes) *bytes = other;
   }

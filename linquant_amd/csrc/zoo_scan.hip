@@ -34,6 +34,7 @@
 // 112 / 118 / 106, B*H = 64 T4096 (one full round) 151 / 145 / 146.  The delta family's sets hold more per step (three sets, 142 ..
 // 165 registers at K = 128): its step is longer, and with one workgroup per compute unit it was faster than its two launches at every
 // size measured (B*H = 4 .. 256, T = 256 .. 16384: 1.04 to 1.7 times).
+#include <algorithm>
 #include <type_traits>
 
 #include "zoo_params.h"
@@ -42,11 +43,33 @@ namespace {
 
 using ScanParams = ZooScanParams;
 
+// ---- Segments (linear family).  Its carry reads neither the stored copy nor anything else of a step but the write codes and the
+// decay, so a workgroup can start in the middle of a chain: it first runs the updates of the chunks in front (one MFMA a tile and five
+// vector instructions a value, no rendezvous, three or four operand sets in rotation), with the order and the arithmetic of the whole
+// chain and so with its bits, and then its own steps.  An update takes about 0.3 of a step; segments that shrink by that share, first to
+// last, end together.  One workgroup per compute unit: as many segments as keep all of them at 256 or fewer (a second workgroup per
+// compute unit repeats updates faster than it hides waits: B4 T4096 H16 K = V = 128, 256 tiles, one / two segments 150 / 156 us).
+// GPU time of the whole call, one segment or two launches (zoo_combined.hip), whichever was taken before -> segments: linear attention
+// with R_QK, K = V = 128, H4 T4096 / T16384 49.3 -> 30.3 / 132 -> 75.5 us, H16 60.3 -> 49.9 / 231 -> 187; K = V = 64 H8 T2048 / T16384
+// 24.2 -> 16.6 / 110 -> 67.4; GLA K = V = 128 H4 T16384 162 -> 90, H5 T8192 96.3 -> 59.4.  Decay of the segments' lengths by 0.2 or 0.4
+// in the place of 0.3: at most 4 % slower.
+constexpr int scan_update_sets(int K, int BV) { return K == 128 && BV == 32 ? 3 : 4; }  // (four spill there)
+constexpr int kMaxCuts = 16;
+struct ScanCuts {
+  int n;                 // segments of a chain (1 for the delta family)
+  int at[kMaxCuts + 1];  // first chunk of each (multiples of scan_update_sets), then NT
+};
+
 // BV: value columns per workgroup.  32, and 16 where 32 would leave half of the 256 compute units or more without a workgroup: a
 // step is bound by the vector instructions of the two waves of a SIMD, and half the columns are little more than half of them
 // (32 -> 16 columns: scalar decay B1 T2048 H8 K = V = 64 21.4 -> 15.9 us, 14 with two operand sets; KDA B1 T2048 H8 K = V = 128 36.7 ->
 // 25.2 us).  From
 // more than half of the compute units on, a second workgroup of 16 columns would only repeat what does not depend on the columns.
+// The linear family, whose chains come in segments (below), takes 16 columns for up to 42 tiles of 32, and for more where the chain is
+// too short for segments that make up for it.  GPU us of the whole call with 16 / 32 columns, both in segments, scalar decay: K = V =
+// 128 with R_QK, T = 2048 / 8192 / 32768: 32 tiles 24.1 / 26.2, 61.8 / 68.5, 234 / 252; 44 tiles 32.1 / 32.4, 80.9 / 79.8, 365 / 312; 60
+// tiles 31.3 / 32.1, 95.1 / 96.3, 430 / 380; K = V = 64: 34 tiles 27.7 / 28.5, 63.5 / 61.8, 284 / 254; 48 tiles 28.2 / 26.9, 85.5 / 76.1,
+// 401 / 334; K = V = 128, 96 tiles, T = 512 / 1024 / 2048 / 8192: 17.4 / 17.7, 27.3 / 27.4, 38.9 / 37.2, 131 / 121.
 template <bool DELTA, int K, int BV>
 struct ChainOps {
   lq_v4i kop[K / 64];                 // key write codes: rows of this wave, 16 token slots of the lane's group
@@ -90,8 +113,8 @@ LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
 constexpr int scan_sets(bool delta) { return delta ? 3 : 2; }
 
 template <bool DELTA, bool SCALAR, int K, int BV, bool BF, bool OF32>
-__global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams p) {
-  constexpr int D = scan_sets(DELTA);
+__global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams p, ScanCuts cuts) {
+  constexpr int D = scan_sets(DELTA), DU = scan_update_sets(K, BV);
   constexpr int KR = K / 4;        // carry rows per chain wave
   constexpr int KT = K / 64;       // 16-row tiles per chain wave
   constexpr int VT = BV / 16;      // 16-column tiles
@@ -112,19 +135,23 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rl = lane & 15, kg = lane >> 4;
   // The V tiles of one (batch, head) read the same key, query, state-read and decay operands at the same time: all of them run on one
-  // XCD (workgroups are dealt to the 8 XCDs round-robin, blockIdx.x counts to 8 times the V tiles), and the (batch, head)s are dealt to
-  // the XCDs as evenly as they go; blockIdx.y counts to the most that one XCD has.  (When only grids that divide evenly were
-  // renumbered, the operands of the others were fetched by up to eight L2s: T4096 H28 K = V = 128, DeltaNet 145 -> 107 us, KDA 226 ->
-  // 187.)
-  const uint32_t xcd = blockIdx.x & 7u, mine = blockIdx.y;
-  const uint32_t nbh = (uint32_t)p.B * (uint32_t)p.H, each = nbh >> 3, extra = nbh & 7u;
+  // XCD (workgroups are dealt to the 8 XCDs round-robin, blockIdx.x counts to 8 times the V tiles), and the (batch, head)s, each with
+  // its segments, are dealt to the XCDs as evenly as they go; blockIdx.y counts to the most that one XCD has.  (When only grids that
+  // divide evenly were renumbered, the operands of the others were fetched by up to eight L2s: T4096 H28 K = V = 128, DeltaNet 145 ->
+  // 107 us, KDA 226 -> 187.  Four heads of sixteen tiles with all segments of a head on one XCD left four XCDs idle: T16384 115 us.)
+  const uint32_t xcd = blockIdx.x & 7u, mine = blockIdx.y, nseg = DELTA ? 1u : (uint32_t)cuts.n;
+  const uint32_t units = (uint32_t)p.B * (uint32_t)p.H * nseg, each = units >> 3, extra = units & 7u;
   if (mine >= each + (xcd < extra ? 1u : 0u)) return;  // (uniform over the workgroup)
-  const int vtile = (int)(blockIdx.x >> 3), bh = (int)(xcd * each + min(xcd, extra) + mine);
+  const uint32_t unit = xcd * each + min(xcd, extra) + mine;
+  const int vtile = (int)(blockIdx.x >> 3), bh = (int)(DELTA ? unit : unit / nseg);
   const int v0 = vtile * BV;
   const int b = bh / p.H, h = bh % p.H;
   const int H = p.H, V = p.V, T = p.T, NT = p.NT;
   const int qmax = p.qmax;
   constexpr bool bf = BF;
+  // linear family: chunks c0 .. c1 - 1 of this workgroup's segment
+  const int seg = DELTA ? 0 : (int)(unit - (uint32_t)bh * nseg);
+  const int c0 = DELTA ? 0 : cuts.at[seg], c1 = DELTA ? NT : cuts.at[seg + 1];
 
   if (wv < 4) {
     // ------------------------------------------------------------------------------------------------------- chain
@@ -184,6 +211,30 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     float* misc_s = misc_lds + 64 * wave;
     unsigned char* ue_s = ue_lds + wave * 16 * US;
 
+    // write product and carry update
+    auto update = [&](const Ops& cur) __attribute__((always_inline)) {
+      if constexpr (!DELTA) misc_s[lane] = cur.misc;  // (no earlier: with one set in flight the step would start with this wait)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        lq_v4i bop;
+        if constexpr (DELTA)
+          bop = *(const lq_v4i*)(eT + (16 * vt + rl) * ES + 16 * kg);
+        else
+          bop = cur.vop[vt];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const lq_v4i a = lq_mfma_i8(cur.kop[kt], bop, lq_v4i{0, 0, 0, 0});
+          const lq_v4f gam4 = *(const lq_v4f*)(misc_s + 32 + 16 * kt + 4 * kg);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float prod = (float)a[r] * skw_r[kt][r];
+            prod = prod * svw_c[vt];
+            hc[kt][vt][r] = hc[kt][vt][r] * gam4[r] + prod;
+          }
+        }
+      }
+    };
+
     // one chunk step; the operands of chunk ct + D - 1 are requested into `pre` (unconditionally: the last chunks re-request the
     // final one, so that the compiler's count of outstanding requests does not depend on the path)
     auto do_step = [&](int ct, Ops& cur, Ops& pre) __attribute__((always_inline)) {
@@ -203,7 +254,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
           for (int r = 0; r < 4; ++r) cd[r] = zoo_q8(hc[kt][vt][r], inv_ss_c[vt], 127);
           *(uint32_t*)(hTb + (16 * vt + rl) * HS + KR * wave + 16 * kt + 4 * kg) = zoo_pack_codes(cd[0], cd[1], cd[2], cd[3]);
         }
-      const int ctn = min(ct + D - 1, NT - 1);
+      const int ctn = min(ct + D - 1, c1 - 1);
       load_part(std::integral_constant<int, 1>{}, ctn, pre);
       __syncthreads();
 
@@ -249,46 +300,45 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
         __syncthreads();
       }
 
-      // write product and carry update
-      if constexpr (!DELTA) misc_s[lane] = cur.misc;  // (no earlier: with one set in flight the step would start with this wait)
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        lq_v4i bop;
-        if constexpr (DELTA)
-          bop = *(const lq_v4i*)(eT + (16 * vt + rl) * ES + 16 * kg);
-        else
-          bop = cur.vop[vt];
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-          const lq_v4i a = lq_mfma_i8(cur.kop[kt], bop, lq_v4i{0, 0, 0, 0});
-          const lq_v4f gam4 = *(const lq_v4f*)(misc_s + 32 + 16 * kt + 4 * kg);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float prod = (float)a[r] * skw_r[kt][r];
-            prod = prod * svw_c[vt];
-            hc[kt][vt][r] = hc[kt][vt][r] * gam4[r] + prod;
-          }
-        }
-      }
+      update(cur);
     };
 
-    Ops st[D];
-    load_part(std::integral_constant<int, 0>{}, 0, st[0]);
-    scan_for<D - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
-    scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load_part(std::integral_constant<int, 0>{}, min(i + 1, NT - 1), st[i + 1]); });
-    // everything requested so far is waited for once, in front of the loop (a load still outstanding at loop entry would make
+    // everything requested so far is waited for once, in front of a loop (a load still outstanding at loop entry would make
     // every iteration wait until almost nothing is in flight)
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    asm volatile("" ::: "memory");
-    int ct = 0;
-    for (; ct + D <= NT; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(ct + i, st[i], st[(i + D - 1) % D]); });
+    auto arrive = [&]() __attribute__((always_inline)) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      asm volatile("" ::: "memory");
+    };
+    Ops st[DELTA ? D : DU];
+    load_part(std::integral_constant<int, 0>{}, 0, st[0]);
+    scan_for<(DELTA ? D : DU) - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
+    if constexpr (!DELTA) {
+      // the carry that enters the segment: the updates of all chunks in front of it, in their order and with their arithmetic (so
+      // with their bits).  No rendezvous: a wave updates its own rows.  The sets hold DU - 1 chunks in flight, and as cuts are
+      // multiples of DU, chunk c0 ends up in the first.
+      if (c0 > 0) {
+        scan_for<DU - 2>([&](auto i) __attribute__((always_inline)) { load_part(std::integral_constant<int, 0>{}, i + 1, st[i + 1]); });
+        arrive();
+        for (int cu = 0; cu < c0; cu += DU)
+          scan_for<DU>([&](auto i) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_part(std::integral_constant<int, 0>{}, min(cu + i + DU - 1, c0), st[(i + DU - 1) % DU]);
+            update(st[i]);
+          });
+      }
+    } else {
+      scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load_part(std::integral_constant<int, 0>{}, min(i + 1, NT - 1), st[i + 1]); });
+    }
+    arrive();
+    int ct = c0;
+    for (; ct + D <= c1; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(ct + i, st[i], st[(i + D - 1) % D]); });
     scan_for<D - 1>([&](auto i) __attribute__((always_inline)) {
-      if (ct + i < NT) do_step(ct + i, st[i], st[(i + D - 1) % D]);
+      if (ct + i < c1) do_step(ct + i, st[i], st[(i + D - 1) % D]);
     });
     if constexpr (DELTA) __syncthreads();  // the output's last local codes (its rendezvous below)
 
-    if (p.ht) {
+    if (p.ht && c1 == NT) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -397,7 +447,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();  // the stored copy of chunk ct is in LDS
       if constexpr (DELTA && !decltype(first_c)::value) finish(ct - 1, prev);
-      load(min(ct + D - 1, NT - 1), prev);
+      load(min(ct + D - 1, c1 - 1), prev);
       read_state(ct, cur);
       if constexpr (DELTA) {
         __syncthreads();  // E of chunk ct is in LDS
@@ -407,17 +457,17 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       }
     };
     Ops st[D];
-    load(0, st[0]);
+    load(c0, st[0]);
     scan_for<D - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
-    scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load(min(i + 1, NT - 1), st[i + 1]); });
+    scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load(min(c0 + i + 1, c1 - 1), st[i + 1]); });
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
     asm volatile("" ::: "memory");
-    do_step(std::true_type{}, 0, st[0], st[D - 1]);
-    int ct = 1;
-    for (; ct + D <= NT; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]); });
+    do_step(std::true_type{}, c0, st[0], st[D - 1]);
+    int ct = c0 + 1;
+    for (; ct + D <= c1; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]); });
     scan_for<D - 1>([&](auto i) __attribute__((always_inline)) {
-      if (ct + i < NT) do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]);
+      if (ct + i < c1) do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]);
     });
     if constexpr (DELTA) {
       __syncthreads();  // the local codes of the last chunk, written by all four output waves
@@ -428,23 +478,43 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
   }
 }
 
+// Segments of a chain of NT chunks where `tiles` workgroups of them would run side by side, cut at multiples of `step`
+ScanCuts scan_cuts(int64_t tiles, int NT, int step) {
+  const int n = (int)std::min((int64_t)kMaxCuts, 256 / tiles);
+  ScanCuts c = {};
+  double len = 1.0, all = 0.0, at = 0.0;
+  for (int s = 0; s < n; ++s) all += len, len *= 0.7;
+  len = NT / all;
+  for (int s = 1; s < n; ++s) {
+    at += len, len *= 0.7;
+    const int cut = (int)(at / step + 0.5) * step;
+    if (cut > c.at[c.n] && cut < NT) c.at[++c.n] = cut;
+  }
+  c.at[++c.n] = NT;
+  return c;
+}
+
 template <bool DELTA, bool SCALAR, int K, int BV>
 int launch(const ScanParams& p, hipStream_t stream) {
-  const dim3 grid(8 * (p.V / BV), (p.B * p.H + 7) / 8), block(512);
+  const int64_t tiles = (int64_t)p.B * p.H * (p.V / BV);
+  const ScanCuts cuts = DELTA || tiles > 128 ? ScanCuts{1, {0, p.NT}} : scan_cuts(tiles, p.NT, scan_update_sets(K, BV));
+  const dim3 grid(8 * (p.V / BV), (p.B * p.H * cuts.n + 7) / 8), block(512);
   if (DELTA && p.o_is_f32 && p.bf)  // (the linear family reads codes only: the activation dtype is that of the output)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, DELTA, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, DELTA, true>), grid, block, 0, stream, p, cuts);
   else if (p.o_is_f32)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, true>), grid, block, 0, stream, p, cuts);
   else if (p.bf)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, true, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, true, false>), grid, block, 0, stream, p, cuts);
   else
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, false>), grid, block, 0, stream, p, cuts);
   return lq_check_launch();
 }
 
 template <bool DELTA, bool SCALAR, int K>
 int launch_bv(const ScanParams& p, hipStream_t stream) {
-  const bool few = (int64_t)p.B * p.H * (p.V / 32) <= 128;
+  const int64_t tiles = (int64_t)p.B * p.H * (p.V / 32);
+  // linear family: a tile of 32 columns in more segments is the better use of the same compute units once the chain is long
+  const bool few = tiles <= (DELTA || p.NT <= 12 ? 128 : (p.NT <= 32 ? 64 : (p.NT <= 256 ? 42 : 32)));
   return few ? launch<DELTA, SCALAR, K, 16>(p, stream) : launch<DELTA, SCALAR, K, 32>(p, stream);
 }
 

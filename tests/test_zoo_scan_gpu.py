@@ -77,3 +77,17 @@ def test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda
     torch.cuda.synchronize()
     assert float(o1.float().abs().max()) > 0
     assert torch.equal(o0, o1) and torch.equal(h0, h1)
+
+
+# chains in segments: cuts at multiples of four (three: K = 128, 32 value columns), as many as the chain has room for (16 segments of
+# at least one cut step, fewer), one that starts in the last chunk; the lines between 16 and 32 columns (12, 32 and 256 steps; 42 and 64
+# tiles of 32), the last grid with two segments and the first with one
+@pytest.mark.parametrize("cell", ["linear_none", "mamba2", "gla"])
+@pytest.mark.parametrize("NT,B,H,K,V,dtype,out_dtype", [
+    (4, 1, 1, 64, 64, torch.float16, None), (5, 1, 1, 128, 64, torch.bfloat16, None), (13, 1, 2, 64, 64, torch.float16, torch.float32),
+    (64, 1, 1, 64, 64, torch.bfloat16, None), (65, 2, 1, 128, 128, torch.float16, None), (30, 3, 1, 128, 192, torch.float16, None),
+    (33, 1, 11, 128, 128, torch.bfloat16, None), (34, 2, 11, 64, 64, torch.float16, torch.float32), (32, 1, 16, 128, 128, torch.float16, None),
+    (12, 1, 17, 128, 128, torch.float16, None), (13, 1, 17, 128, 128, torch.float16, None), (14, 1, 32, 64, 128, torch.bfloat16, None),
+    (13, 3, 11, 128, 128, torch.float16, torch.float32), (257, 1, 9, 64, 128, torch.float16, None), (258, 1, 17, 128, 64, torch.bfloat16, None)])
+def test_a_chain_in_segments_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype):
+    test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype)
