@@ -22,35 +22,29 @@ struct Layout {
 // whole chip for the output.  What the one launch saves is launches (4 .. 6 us a call, which decides short calls), the stored states
 // (2 K V bytes a chunk and head) and the second reading of raw operands (with a prologue: of their token-major codes), against A
 // (16 KB) and one more set of codes.
-// Up to 128 tiles of 32 columns the one launch runs a chain in segments side by side (zoo_scan.hip), and is the faster but for K = V = 64
-// on more than half of the compute units' worth of tiles, where the chain is long.  GPU time of the two launches over that of the one, no
-// decay .. scalar decay (B = 1; graph replays of two sets of inputs in turn):
+// With a prologue, up to 128 tiles of 32 columns: there the one launch runs a chain in segments side by side (zoo_scan.hip), and is the
+// faster but for K = V = 64 on more than 80 tiles, where the chain is long.  GPU time of the two launches over that of the one, no decay ..
+// scalar decay (B = 1, 16 to 128 tiles; graph replays of two sets of inputs in turn):
 //                                T = 2048      4096          8192          32768
-//   K = V = 128, 16 tiles        1.50 .. 1.63  1.45 .. 1.60  1.65 .. 1.76  1.75 .. 1.79
-//     48 .. 128 tiles            1.11 .. 1.39  1.09 .. 1.29  1.08 .. 1.29  1.12 .. 1.35
-//     with prologue              1.14 .. 1.54  1.15 .. 1.55  1.10 .. 1.73  1.12 .. 1.77
-//   K 128, V 64                  1.00 .. 1.49  0.97 .. 1.51  0.98 .. 1.59  1.01 .. 1.63
-//     with prologue              1.16 .. 1.64  1.07 .. 1.65  1.05 .. 1.65  1.05 .. 1.66
-//   K 64, V 128                  1.08 .. 1.57  1.09 .. 1.66  1.05 .. 1.67  1.04 .. 1.86
-//     with prologue              1.27 .. 1.72  1.26 .. 1.80  1.19 .. 1.82  1.01 .. 1.94
-//   K = V = 64, 16 tiles         1.27 .. 1.41  1.34 .. 1.38  1.50 .. 1.51  1.42 .. 1.57
-//     48                         1.04 .. 1.14  1.05 .. 1.08  1.05 .. 1.07  1.04
-//     64                         1.02 .. 1.06  1.03 .. 1.10  0.90 .. 0.99  0.96 .. 1.09
-//     80                         1.05 .. 1.06  0.98 .. 1.06  0.91 .. 0.94  0.90 .. 0.97
-//     96                         0.99 .. 1.02  0.91 .. 0.99  0.80 .. 0.84  0.85 .. 0.94
-//     128                        0.96 .. 1.00  0.82 .. 0.87  0.74 .. 0.83  0.95 .. 1.11
-//     with prologue, to 80       1.09 .. 1.44  1.08 .. 1.43  1.00 .. 1.55  1.02 .. 1.61
+//   K = V = 128                  1.14 .. 1.54  1.15 .. 1.55  1.10 .. 1.73  1.12 .. 1.77
+//   K 128, V 64                  1.16 .. 1.64  1.07 .. 1.65  1.05 .. 1.65  1.05 .. 1.66
+//   K 64, V 128                  1.27 .. 1.72  1.26 .. 1.80  1.19 .. 1.82  1.01 .. 1.94
+//   K = V = 64, to 80 tiles      1.09 .. 1.44  1.08 .. 1.43  1.00 .. 1.55  1.02 .. 1.61
 //     96 .. 128                  1.05 .. 1.11  0.98 .. 1.05  0.91 .. 1.01  0.97 .. 1.19
-// More tiles: bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch, while 16 KB are saved or there is no second
+// Otherwise, bytes saved > 0 (K = V = 128; with a prologue all but K = V = 64): one launch, while 16 KB are saved or there is no second
 // tile per compute unit (more than 256) or no more than 32 steps; else: one launch for short chains whose operands stay in the last-level
 // cache.  Time of the two launches over that of the one, three sets of inputs in turn, geometric mean over no and scalar decay, before the
 // operand pre-pass took the last chunks first (zoo_params.h), by which the one launch gains: T = 2048 .. 8192, B*H = 4 .. 256 (where fewer
 // tiles ran their chains in one piece): K = V = 128 0.91 .. 1.27, with prologue 1.00 .. 1.25; K 128, V 64 0.81 .. 1.11, with prologue
 // 0.97 .. 1.18; K 64, V 128 0.78 .. 1.15 (B*H*NT <= 4096 0.99 .. 1.15), with prologue 0.89 .. 1.27; K = V = 64 0.67 .. 1.08, with
 // prologue 0.83 .. 1.07 (B*H*NT <= 2048 0.98 .. 1.07).
+// Without a prologue the lines of few tiles are still those of chains in one piece, also where segments have moved them (two launches over
+// the one, measured as in the table above, K = V = 128, 128 tiles or fewer, past 128 steps 1.08 .. 1.79): the workspace that a caller asks
+// for follows the route (lq_zoo_simple_gla_workspace_bytes), and that of few long chains grows by the one launch's operands.
 bool linear_scan(bool prologue, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V) {
   const int64_t NT = T / 64, chunks = B * H * NT, tiles = B * H * (V / 32);
-  if (tiles <= 128) return K + V > 128 || (prologue ? NT <= 64 || tiles <= 80 : tiles <= 52 || NT <= (tiles <= 64 ? 64 : (tiles <= 96 ? 32 : 16)));
+  if (prologue && tiles <= 128) return K + V > 128 || NT <= 64 || tiles <= 80;
+  if (NT > 128 && tiles < 128) return false;
   const int64_t saved = 2 * K * V - 16384 + (prologue ? 128 * K : 0);  // bytes a chunk and head
   if (saved >= 16384) return true;
   if (saved > 0) return NT <= 32 || tiles <= 256;

@@ -91,3 +91,13 @@ def test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda
     (13, 3, 11, 128, 128, torch.float16, torch.float32), (257, 1, 9, 64, 128, torch.float16, None), (258, 1, 17, 128, 64, torch.bfloat16, None)])
 def test_a_chain_in_segments_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype):
     test_recurrence_and_output_in_one_launch_equal_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, out_dtype)
+
+
+# the same with the operand prologue, whose route differs: chains of more than 128 steps in segments, and on the other side of its line
+# (K = V = 64, more than 80 tiles, more than 64 steps) the stages behind the same call
+@pytest.mark.parametrize("cell", ["linear_none", "mamba2"])
+@pytest.mark.parametrize("NT,B,H,K,V,dtype,parts", [
+    (257, 1, 9, 64, 128, torch.float16, ("signs_qk",)), (258, 1, 17, 128, 64, torch.bfloat16, ("signs_qk", "signs_v")),
+    (131, 1, 3, 128, 128, torch.float16, ("dqk",)), (64, 1, 41, 64, 64, torch.float16, ("signs_qk",)), (65, 1, 41, 64, 64, torch.float16, ("signs_qk",))])
+def test_a_chain_in_segments_behind_the_prologue_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts):
+    test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts)
