@@ -19,13 +19,16 @@
 //     us of 256 (Gated DeltaNet B4 T4096 H16, whole call).
 // An fp32 form of the same (operands scaled and staged as fp32, 32 fp32 MFMA steps per Gram block, T and X split in three bf16
 // pieces, six products) took 121 us at B4 T4096 H16 K = V = 128, of which the splitting and the fp32 steps were two thirds, and left
-// the codes of q and the product A to the output kernel; this one takes 119 us with them (127 with scalar decay).
+// the codes of q and the product A to the output kernel; this one takes 117 us with them and with scalar decay.
 //
-// One 8-wave workgroup per (chunk, batch*head), two to a compute unit (77 KB of LDS): load and quantize (every row is read once)
-// | Gram blocks and, MODE_SCAN, the blocks of the intra-chunk product A (20 blocks over the 8 waves) | G | inverse of the four
-// diagonal blocks by forward substitution | block columns of T, one wave each, in registers | products.  Bound by
-// no unit alone: with scalar decay 410 MB are 81 us at the rate of a large copy and the vector instructions 82 us, of 127; between the
-// eight barriers two workgroups do not cover each other's waits.
+// One 8-wave workgroup per (chunk, batch*head), three to a compute unit (49 KB of LDS, 80 registers): load and quantize | Gram blocks and,
+// MODE_SCAN, the blocks of the intra-chunk product A (20 blocks over the 8 waves) | G; keys transposed | inverse of the four diagonal
+// blocks by forward substitution | block columns of T, one wave each, in registers | W | values transposed | U.  Keys and then values
+// pass through one transposed tile, the rows waiting in registers (every row is read once), and G and T lie in 16 blocks in the place of
+// the raw keys and codes.  With a tile each for keys and values and square G and T (77 KB) two workgroups fitted, which did not cover each
+// other's waits between eight barriers: 128.8 -> 117.4 us at B4 T4096 H16 with scalar decay (fp16), 59.3 -> 57.7 at B8 T2048 H8 without
+// (bf16; 2.7 rounds of the chip for four), whole calls 260.9 -> 248.7 and 94.7 -> 89.8, although there are two barriers more.  Bound by no
+// unit alone: 410 MB are 81 us at the rate of a large copy and the vector instructions 82 us.
 #include "zoo_params.h"
 
 namespace {
@@ -44,7 +47,11 @@ LQ_DEV lq_v4f wn_mfma(lq_v4i a, lq_v4i b, lq_v4f c) {
   return lq_mfma_f16(__builtin_bit_cast(lq_v8h, a), __builtin_bit_cast(lq_v8h, b), c);
 }
 
-constexpr int kGS = 70;   // floats per row of the G / T tiles: an A-operand read (16 rows, 4 adjacent slots) takes one LDS pass at 2 mod 4
+// 16 x 16 blocks of T (lower triangle; the diagonal ones hold G first) and of G below the diagonal, rows of 20 floats
+constexpr int kBP = 20;
+constexpr int kBlk = 16 * kBP;
+LQ_DEV int wn_t(int I, int J) { return (I * (I + 1) / 2 + J) * kBlk; }
+LQ_DEV int wn_g(int I, int J) { return I == J ? wn_t(I, I) : (10 + I * (I - 1) / 2 + J) * kBlk; }
 constexpr int kXP = 36;   // dwords per column of the transposed tiles (32 token pairs + pad)
 // byte of the transposed write codes [channel][64 tokens]: 16 bytes of pad after every eight channels, so that the 16 channel
 // groups of a wave's writes fall on different banks (rows of 80 bytes put them on two: Gated DeltaNet B4 T4096 H16 260 -> 256 us,
@@ -93,23 +100,20 @@ LQ_DEV void wn_split(const float (&x)[8], TPieces<BF>& t) {
 }
 
 template <bool SCALAR, int K, bool BF, int MODE>
-__global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
+__global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
   constexpr bool CODES = MODE != MODE_PLAIN, SCAN = MODE == MODE_SCAN;
   constexpr int FS = K + 16;                      // halves per row of the raw key tile (72 or 40 dwords: two-pass operand reads)
   constexpr int QS = K == 128 ? 160 : 80;         // bytes per row of the code tiles
-  constexpr int kR1 = 64 * FS * 2 > 64 * kGS * 4 ? 64 * FS * 2 : 64 * kGS * 4;            // raw keys, then T
-  constexpr int kR2 = 2 * 64 * QS > 128 * kXP * 4 ? 2 * 64 * QS : 128 * kXP * 4;          // codes of q and k, then transposed v
-  constexpr int kR3 = K * 66 > 64 * kGS * 4 ? K * 66 : 64 * kGS * 4;                    // transposed write codes, then G
-  constexpr int kR4 = K * kXP * 4;                                                       // transposed keys
-  __shared__ __align__(16) unsigned char lds[kR1 + kR2 + kR3 + kR4];
+  constexpr int kF_bytes = 64 * FS * 2, kQ_bytes = 2 * 64 * QS;                 // raw keys, codes of q and k, and behind them the transposed
+  constexpr int kP1 = kF_bytes + kQ_bytes + (CODES ? K * 66 : 0);               // write codes; then
+  constexpr int kGT = 16 * kBlk * 4, kP2 = kGT + 128 * kXP * 4;                 // G and T, and keys, then values, transposed
+  __shared__ __align__(16) unsigned char lds[kP1 > kP2 ? kP1 : kP2];
   _Float16* kF = (_Float16*)lds;
-  float* T_s = (float*)lds;
-  unsigned char* qI = lds + kR1;
-  unsigned char* kI = lds + kR1 + 64 * QS;
-  uint32_t* Xv = (uint32_t*)(lds + kR1);
-  unsigned char* cT = lds + kR1 + kR2;
-  float* G_s = (float*)(lds + kR1 + kR2);
-  uint32_t* Xk = (uint32_t*)(lds + kR1 + kR2 + kR3);
+  unsigned char* qI = lds + kF_bytes;
+  unsigned char* kI = qI + 64 * QS;
+  unsigned char* cT = lds + kF_bytes + kQ_bytes;
+  float* GT = (float*)lds;
+  uint32_t* X = (uint32_t*)(lds + kGT);
   __shared__ float bs_s[64], bh_s[64], bw_s[64], el_s[64], fW_s[64], gs_s[64], iskw_s[CODES ? K : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   }
   __syncthreads();
 
-  // ---- rows into LDS: raw keys by token (Gram) and by channel (W), codes of q and Hw, transposed write codes
+  // ---- rows into LDS: raw keys by token (Gram), codes of q and Hw, transposed write codes
   if (kact) {
     if (p.dk_div) {  // D_QK at load: k' = act(k / D), the quotient rounded once (uniform over the launch)
 #pragma unroll
@@ -222,11 +226,6 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
           *(lq_v2i*)(qI + t * QS + 8 * kc) = oq;
         }
       }
-    }
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      Xk[wn_xt(8 * kc + 2 * d, krp)] = __builtin_amdgcn_perm((uint32_t)kraw[1][d], (uint32_t)kraw[0][d], 0x05040100u);
-      Xk[wn_xt(8 * kc + 2 * d + 1, krp)] = __builtin_amdgcn_perm((uint32_t)kraw[1][d], (uint32_t)kraw[0][d], 0x07060302u);
     }
     if constexpr (CODES) {
 #pragma unroll
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   }
   __syncthreads();  // raw keys, codes and transposed codes are dead
 
-  // ---- G, with the factors of its rows and columns; v transposed
+  // ---- G, with the factors of its rows and columns; k transposed
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const int n = wave + 8 * s;
@@ -305,31 +304,30 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
       const int i = 16 * blk_i(n) + 4 * kg + r;
       float x = (bs_s[i] * bh) * gacc[s][r];
       if (SCALAR) x = x * zoo_exp(gs_s[i] - gj);
-      G_s[i * kGS + j] = i > j ? x : 0.0f;
+      GT[wn_g(blk_i(n), blk_j(n)) + (4 * kg + r) * kBP + rl] = i > j ? x : 0.0f;
     }
   }
-  auto stage_v = [&]() {
-    if (vact) {
+  // two rows of eight channels -> transposed tile
+  auto stage = [&](const lq_v4i (&raw)[2], int c8, int pair) __attribute__((always_inline)) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        Xv[wn_xt(8 * vc8 + 2 * d, vrp)] = __builtin_amdgcn_perm((uint32_t)vraw[1][d], (uint32_t)vraw[0][d], 0x05040100u);
-        Xv[wn_xt(8 * vc8 + 2 * d + 1, vrp)] = __builtin_amdgcn_perm((uint32_t)vraw[1][d], (uint32_t)vraw[0][d], 0x07060302u);
-      }
+    for (int d = 0; d < 4; ++d) {
+      X[wn_xt(8 * c8 + 2 * d, pair)] = __builtin_amdgcn_perm((uint32_t)raw[1][d], (uint32_t)raw[0][d], 0x05040100u);
+      X[wn_xt(8 * c8 + 2 * d + 1, pair)] = __builtin_amdgcn_perm((uint32_t)raw[1][d], (uint32_t)raw[0][d], 0x07060302u);
     }
   };
-  stage_v();
+  if (kact) stage(kraw, kc, krp);
   __syncthreads();
 
   // ---- T = (I + G)^-1: diagonal blocks by forward substitution (wave w < 4, lane c of every 16 holds column c of block w)
   if (wave < 4) {
-    const int o = 16 * wave;
+    float* B = GT + wn_t(wave, wave);
     float gr[16], tc[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) gr[i] = G_s[(o + i) * kGS + o + rl];
+    for (int i = 0; i < 16; ++i) gr[i] = B[i * kBP + rl];
     zoo_substitute(gr, tc, rl);
     if (lane < 16) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) T_s[(o + i) * kGS + o + lane] = tc[i];
+      for (int i = 0; i < 16; ++i) B[i * kBP + lane] = tc[i];
     }
   }
   __syncthreads();
@@ -339,23 +337,26 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
     const int J = wave;
     lq_v4f tcol[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) tcol[0][s] = T_s[(16 * J + 4 * kg + s) * kGS + 16 * J + rl];
+    for (int s = 0; s < 4; ++s) tcol[0][s] = GT[wn_t(J, J) + (4 * kg + s) * kBP + rl];
 #pragma unroll
     for (int di = 1; di < 4; ++di) {
       const int I = J + di;
       if (I > 3) break;
       lq_v4f sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int dm = 0; dm < di; ++dm)
+      for (int dm = 0; dm < di; ++dm) {
+        const lq_v4f g4 = *(const lq_v4f*)(GT + wn_g(I, J + dm) + rl * kBP + 4 * kg);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) sacc = wn_mfma_f32(G_s[(16 * I + rl) * kGS + 16 * (J + dm) + 4 * kg + s], tcol[dm][s], sacc);
+        for (int s = 0; s < 4; ++s) sacc = wn_mfma_f32(g4[s], tcol[dm][s], sacc);
+      }
+      const lq_v4f t4 = *(const lq_v4f*)(GT + wn_t(I, I) + rl * kBP + 4 * kg);
       lq_v4f tacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < 4; ++s) tacc = wn_mfma_f32(T_s[(16 * I + rl) * kGS + 16 * I + 4 * kg + s], sacc[s], tacc);
+      for (int s = 0; s < 4; ++s) tacc = wn_mfma_f32(t4[s], sacc[s], tacc);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         tcol[di][r] = -tacc[r];
-        T_s[(16 * I + 4 * kg + r) * kGS + 16 * J + rl] = -tacc[r];
+        GT[wn_t(I, J) + (4 * kg + r) * kBP + rl] = -tacc[r];
       }
     }
   }
@@ -365,51 +366,49 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
   // the column tiles of both
   const int I = wave < 4 ? wave : 7 - wave, half = wave >> 2;
   const int NST = (I >> 1) + 1;  // 32-token contraction steps that are not zero
-  TPieces<BF> tw[2], tu[2];  // (no decay: W and U share T . diag(bs), tu is not used)
-  float unw = 1.0f, unu = 1.0f;
-  {
-    float xw[2][8], xu[2][8];
-    float mw = 0.0f, mu = 0.0f;
+  // T . diag(f) for this row block in pieces; un: what the sums are to be multiplied by
+  auto t_pieces = [&](const float* f, TPieces<BF> (&t)[2], float& un) __attribute__((always_inline)) {
+    float x[2][8];
+    float m = 0.0f;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       if (st >= NST) continue;  // (wave-uniform)
-      const int m0 = 32 * st + 8 * kg;
-      const bool live = m0 < 16 * (I + 1);  // blocks right of the diagonal were never written
+      const int m0 = 32 * st + 8 * kg, M = 2 * st + (kg >> 1);
+      const bool live = M <= I;  // blocks right of the diagonal were never written
+      const float* row = GT + wn_t(I, live ? M : I) + rl * kBP + 8 * (kg & 1);
+      const lq_v4f lo = *(const lq_v4f*)row, hi = *(const lq_v4f*)(row + 4);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float t = live ? T_s[(16 * I + rl) * kGS + m0 + e] : 0.0f;
-        xw[st][e] = t * fW_s[m0 + e];
-        xu[st][e] = t * bs_s[m0 + e];
-        mw = fmaxf(mw, __builtin_fabsf(xw[st][e])), mu = fmaxf(mu, __builtin_fabsf(xu[st][e]));
+        const float v = live ? (e < 4 ? lo[e & 3] : hi[e & 3]) : 0.0f;
+        x[st][e] = v * f[m0 + e];
+        m = fmaxf(m, __builtin_fabsf(x[st][e]));
       }
     }
+    un = 1.0f;
     if constexpr (!BF) {
       // each row scaled so that its largest entry lies in [2^14, 2^15)
-      auto scale_of = [&](float m, float& un) {
-        m = fmaxf(m, __shfl_xor(m, 16));
-        m = fmaxf(m, __shfl_xor(m, 32));
-        const int e = min(max((int)(__float_as_uint(m) >> 23), 16), 254);  // largest entry 2^(e - 127) .. 2^(e - 126)
-        un = __uint_as_float((uint32_t)(e - 14) << 23);
-        return __uint_as_float((uint32_t)(268 - e) << 23);  // 2^(141 - e)
-      };
-      const float sw_ = scale_of(mw, unw);
-      float su_ = sw_;
-      if (SCALAR) su_ = scale_of(mu, unu); else unu = unw;
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+      const int e = min(max((int)(__float_as_uint(m) >> 23), 16), 254);  // largest entry 2^(e - 127) .. 2^(e - 126)
+      un = __uint_as_float((uint32_t)(e - 14) << 23);
+      const float s = __uint_as_float((uint32_t)(268 - e) << 23);  // 2^(141 - e)
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          if (st < NST) xw[st][e] = xw[st][e] * sw_, xu[st][e] = xu[st][e] * su_;
+          if (st < NST) x[st][e] = x[st][e] * s;
     }
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       if (st >= NST) continue;
-      wn_split<BF>(xw[st], tw[st]);
-      if constexpr (SCALAR) wn_split<BF>(xu[st], tu[st]);
+      wn_split<BF>(x[st], t[st]);
     }
-  }
+  };
+  TPieces<BF> t[2];
+  float un;
+  t_pieces(fW_s, t, un);
   // D^T tile: lane (rl = token of block I, kg) gets columns 16nt + 4kg + r
-  auto tile = [&](const uint32_t* X, const TPieces<BF> (&t)[2], int nt) {
+  auto tile = [&](int nt) __attribute__((always_inline)) {
     lq_v4f acc = {0.f, 0.f, 0.f, 0.f};
     lq_v4i x[2];
 #pragma unroll
@@ -435,10 +434,10 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
 #pragma unroll
   for (int q = 0; q < K / 32; ++q) {
     const int nt = half * (K / 32) + q;
-    const lq_v4f a = tile(Xk, tw, nt);
+    const lq_v4f a = tile(nt);
     lq_v2i o;
-    o[0] = (int)zoo_enc2(a[0] * unw, a[1] * unw, bf);
-    o[1] = (int)zoo_enc2(a[2] * unw, a[3] * unw, bf);
+    o[0] = (int)zoo_enc2(a[0] * un, a[1] * un, bf);
+    o[1] = (int)zoo_enc2(a[2] * un, a[3] * un, bf);
     const int64_t woff = ((t0 + 16 * I + rl) * H + h) * K + 16 * nt + 4 * kg;
     if (!SCAN && (!CODES || p.W)) *(lq_v2i*)(p.W + woff) = o;
     if constexpr (CODES) {  // state-read codes of the rounded W
@@ -449,25 +448,22 @@ __global__ __launch_bounds__(512, 4) void zoo_wy_ns_kernel(ZooWyParams p) {
           zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax), zoo_q8(w3, inv_sw, qmax));
     }
   }
-  for (int vb = 0; vb < V; vb += 128) {
-    if (vb > 0) {  // further passes of up to 128 value columns
-      __syncthreads();
-      const int rest = min(V - vb, 128) / 8;
-      if (vact && vc8 < rest) {
+  if constexpr (SCALAR) t_pieces(bs_s, t, un);  // (no decay: W and U share T . diag(bs))
+  for (int vb = 0; vb < V; vb += 128) {  // passes of up to 128 value columns
+    if (vb > 0 && vact && vc8 < min(V - vb, 128) / 8) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * vrp + u) * H + h) * V + vb + 8 * vc8);
-        stage_v();
-      }
-      __syncthreads();
+      for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * vrp + u) * H + h) * V + vb + 8 * vc8);
     }
+    __syncthreads();  // the tile has been read
+    if (vact && vc8 < min(V - vb, 128) / 8) stage(vraw, vc8, vrp);
+    __syncthreads();
     const int ntiles = min(V - vb, 128) / 32;  // column tiles per half
     for (int q = 0; q < ntiles; ++q) {
       const int nt = half * ntiles + q;
-      lq_v4f a;
-      if constexpr (SCALAR) a = tile(Xv, tu, nt); else a = tile(Xv, tw, nt);
+      const lq_v4f a = tile(nt);
       lq_v2i o;
-      o[0] = (int)zoo_enc2(a[0] * unu, a[1] * unu, bf);
-      o[1] = (int)zoo_enc2(a[2] * unu, a[3] * unu, bf);
+      o[0] = (int)zoo_enc2(a[0] * un, a[1] * un, bf);
+      o[1] = (int)zoo_enc2(a[2] * un, a[3] * un, bf);
       *(lq_v2i*)(SCAN ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vb + 16 * nt + 4 * kg)
                       : p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
     }
