@@ -481,7 +481,7 @@ int lq_zoo_simple_gla_workspace_bytes(const lq_zoo_simple_gla_args* args, int64_
 /* replaces chunk_gla_int8 (linquant/kernels/zoo/gla.py:235-279), chunk_delta_int8 (gated_delta_rule.py:159-203) and
  * chunk_kda_int8 (kda.py:154-203) as a whole (rotated storage), on `stream` over one caller-supplied workspace that holds
  * every intermediate.  64-token chunks: under per-channel decay one launch in front (cumulative decay, write codes, A and,
- * KDA, the WY transform), otherwise cumsum (scalar decay) and WY prep with the write codes; then recurrence and output as
+ * KDA, the WY transform), otherwise the WY prep with cumsum (scalar decay) and write codes; then recurrence and output as
  * one launch.  128-token chunks: the stage entry points above in the order the wrappers issue them -- cumsum, WY prep
  * (delta family), write-codes pre-pass, A kernel (per-channel decay), state recurrence, output.
  * The bits of the separate calls; one foreign call and one allocation per forward.  family x decay: linear x diagonal = GLA; delta x none = DeltaNet, delta x scalar = Gated

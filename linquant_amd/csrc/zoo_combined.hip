@@ -208,7 +208,7 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
 // (gated_delta_rule.py:159-203) and chunk_kda_int8 (kda.py:154-203) as one C entry over one workspace.  128-token chunks: the stage
 // entry points in the order the Python wrappers issue them.  64-token chunks: recurrence and output in one launch (zoo_scan.hip: the bits
 // of the stages, no stored states, no E in memory); in front of it under per-channel decay one launch for everything (zoo_diag_prep.h),
-// otherwise cumsum (scalar decay) and WY prep, which also makes the write codes.  Neither family needs a rule.
+// otherwise the WY prep, which also cumulates a scalar decay and makes the write codes.  Neither family needs a rule.
 // Delta: its step is two rendezvous and two dependent products with or without the output beside it, and the one launch was the faster at
 // every size measured (B*H = 4 .. 256, T = 256 .. 16384, K = V = 64 and 128: 1.0 to 1.7 times with scalar decay and without, 1.0 to 1.56
 // with per-channel decay; the most on few long chains).  GLA: more than 128 steps
@@ -233,7 +233,8 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   const int64_t B = a->batch, T = a->seqlen, H = a->nheads, K = a->kdim, V = a->vdim, NT = T / 64;
   int64_t off = 0;
   auto take = [&](int64_t& slot, int64_t n) { slot = off, off += up(n); };
-  // (per-channel decay, one launch in front of the recurrence: gc, logenv and Hw stay on the chip)
+  // (one launch in front of the recurrence: gc, logenv and Hw stay on the chip.  Scalar decay keeps gc's place, 4 bytes a token and
+  // head, all the same: the size of a caller's workspace is part of the interface)
   take(l->gc, a->decay == LQ_DECAY_NONE || (diag && !big) ? 0 : B * T * H * (diag ? K : 1) * 4);
   take(l->logenv, diag && big ? B * T * H * 4 : 0);
   take(l->kqT, B * NT * H * K * 64);
@@ -286,7 +287,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
   char* ws = (char*)a->workspace;
-  float* gc = a->decay == LQ_DECAY_NONE || (diag && !big) ? nullptr : (float*)(ws + l.gc);
+  float* gc = a->decay != LQ_DECAY_NONE && big ? (float*)(ws + l.gc) : nullptr;
   float* logenv = diag && big ? (float*)(ws + l.logenv) : nullptr;
   int8_t* kqT = (int8_t*)(ws + l.kqT);
   int8_t* vqT = delta ? nullptr : (int8_t*)(ws + l.vqT);
@@ -321,7 +322,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     if (rc != LQ_OK) return rc;
   }
   // (every stage validates its own arguments before it launches: see lq_zoo_simple_gla)
-  if (a->decay != LQ_DECAY_NONE && (big || !diag)) {
+  if (a->decay != LQ_DECAY_NONE && big) {
     lq_zoo_cumsum_args c = {};
     c.g = a->g, c.gc = gc, c.logenv = logenv, c.batch = a->batch, c.seqlen = a->seqlen, c.nheads = a->nheads;
     c.kdim = diag ? a->kdim : 0, c.chunk_size = a->chunk_size;
@@ -329,7 +330,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   }
   if (delta && (big || !diag)) {
     lq_zoo_wy_prep_args w = {};
-    w.k = a->k, w.v = a->v, w.beta = a->beta, w.g = gc, w.Hw = Hw, w.W = W, w.U = U, w.fw = fw, w.sigma = a->sigma, w.tau = a->tau;
+    w.k = a->k, w.v = a->v, w.beta = a->beta, w.g = big ? gc : a->g, w.Hw = Hw, w.W = W, w.U = U, w.fw = fw, w.sigma = a->sigma, w.tau = a->tau;
     w.batch = a->batch, w.seqlen = a->seqlen, w.nheads = a->nheads, w.kdim = a->kdim, w.vdim = a->vdim, w.chunk_size = a->chunk_size;
     w.decay = a->decay, w.act_dtype = a->act_dtype;
     if (!big) {  // the write operands come with the transform

@@ -162,6 +162,49 @@ LQ_DEV void zoo_fwht(float (&v)[8], int sub) {
   if constexpr (LPR == 16) zoo_fwht_stage<8>(v, sub);
 }
 
+// ---- Cumulative log decay of 64 tokens in fp64, as every kernel forms it: inside each 16 tokens by sums over the last 1, 2, 4, 8 values,
+// then the totals of the 16s before.  Lane t holds token t.  (One after the other, 64 dependent additions and lane reads of one wave took
+// about 2000 cycles, for which the others of its workgroup wait: Gated DeltaNet B4 T4096 H16, WY prep 128.6 us; this way 117.)
+template <int CTRL, int ROWS>
+LQ_DEV double zoo_dpp_add(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, true);
+  return x + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);  // (lanes without a source add zero)
+}
+LQ_DEV float zoo_cumsum64(float g) {
+  double x = (double)g;
+  x = zoo_dpp_add<0x111, 0xf>(x);  // row_shr:1 (a row: 16 lanes)
+  x = zoo_dpp_add<0x112, 0xf>(x);
+  x = zoo_dpp_add<0x114, 0xf>(x);
+  x = zoo_dpp_add<0x118, 0xf>(x);
+  x = zoo_dpp_add<0x142, 0xa>(x);  // row_bcast:15: the last lane of rows 0 and 2 into rows 1 and 3
+  x = zoo_dpp_add<0x143, 0xc>(x);  // row_bcast:31: the last lane of row 1 into rows 2 and 3
+  return (float)x;
+}
+// the same sums of one thread that holds all 64 tokens
+LQ_DEV void zoo_cumsum64(const float (&g)[64], float (&o)[64]) {
+  double last[2] = {0.0, 0.0};  // the sum that rows 0, 1 end with, and the total of row 2
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    double x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) x[t] = (double)g[16 * r + t];
+#pragma unroll
+    for (int s = 1; s < 16; s <<= 1)
+#pragma unroll
+      for (int t = 15; t >= s; --t) x[t] += x[t - s];
+    const double total = x[15];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      if (r == 3) x[t] += last[1];
+      if (r > 0) x[t] += last[0];
+      o[16 * r + t] = (float)x[t];
+    }
+    if (r < 2) last[0] = x[15]; else last[1] = total;
+  }
+}
+
 // One term of the substitution below: t_i -= G_ij t_j, with G_ij broadcast from lane j of every 16
 #define LQ_SUBST(OP, JJ) "v_fmac_f32_dpp %0, -%1, %" #OP " row_newbcast:" #JJ " row_mask:0xf bank_mask:0xf\n"
 #define LQ_SUBST4 LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) LQ_SUBST(5, 3)

@@ -25,7 +25,8 @@ __global__ __launch_bounds__(256) void cumsum_scalar_kernel(const float* __restr
 }
 
 // The same scan for the chunk sizes the callers use (C = 64, 128, 192 or 256): 64 values of a thread are requested before the first
-// is added (the loop above waits for each load in turn: C round trips), summed in the same order.
+// is added (the loop above waits for each load in turn: C round trips), summed in the same order; 64 tokens as the kernels that make
+// the sum themselves do it (zoo_cumsum64).
 template <int C>
 __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* __restrict__ g, float* __restrict__ gc, int H,
                                                                   int64_t total) {
@@ -38,6 +39,13 @@ __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* _
     float v[64];
 #pragma unroll
     for (int t = 0; t < 64; ++t) v[t] = g[base + (int64_t)(t0 + t) * H];
+    if constexpr (C == 64) {
+      float o[64];
+      zoo_cumsum64(v, o);
+#pragma unroll
+      for (int t = 0; t < 64; ++t) gc[base + (int64_t)t * H] = o[t];
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < 64; ++t) {
       run += (double)v[t];

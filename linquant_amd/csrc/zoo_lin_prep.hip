@@ -104,18 +104,11 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
     kraw[u] = *(const lq_v4i*)(src + ((t0 + 4 * kq + u) * H + h) * K + 8 * kc);
     vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * vq + u) * H + h) * V + 8 * vc);
   }
-  // ---- per-token factors: lane t of wave 0 adds the log decays of tokens 0 .. t in fp64, in the order of lq_zoo_cumsum
+  // ---- per-token factors
   if (wave == 0) {
     float fk = 1.0f, fv = 1.0f;
     if constexpr (SCALAR) {
-      const float gr = p.g[(t0 + lane) * H + h];
-      double run = 0.0;
-#pragma unroll 8
-      for (int t = 0; t < 64; ++t) {
-        const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gr), t));
-        run += (double)(t <= lane ? x : 0.0f);
-      }
-      const float gc = (float)run;
+      const float gc = zoo_cumsum64(p.g[(t0 + lane) * H + h]);
       const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gc), 63)) - gc;
       fk = zoo_exp((1.0f - p.eta) * d), fv = zoo_exp(p.eta * d);
       gs_s[lane] = gc;

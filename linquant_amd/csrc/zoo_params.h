@@ -161,7 +161,8 @@ struct ZooScanParams {
 };
 int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, hipStream_t stream);
 
-// WY prep, no / scalar decay.  scan (with the write codes and `local`): wq and U in operand order, the codes of q and A, no Hw
+// WY prep, no / scalar decay.  scan (with the write codes and `local`): wq and U in operand order, the codes of q and A, no Hw; its g
+// is not cumulated
 struct ZooWyLocal {
   const void* q;
   int8_t* qc;   // zoo_op_codes
@@ -177,7 +178,7 @@ struct ZooWyParams {
   const _Float16* k;
   const _Float16* v;
   const float* beta;
-  const float* g;
+  const float* g;  // scalar decay: cumulated over the chunk; what zoo_scan.hip wants made: log decay per token
   _Float16* Hw;
   _Float16* W;
   _Float16* U;

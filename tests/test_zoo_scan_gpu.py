@@ -101,3 +101,38 @@ def test_a_chain_in_segments_equals_the_staged_kernels(cuda, cell, NT, B, H, K, 
     (131, 1, 3, 128, 128, torch.float16, ("dqk",)), (64, 1, 41, 64, 64, torch.float16, ("signs_qk",)), (65, 1, 41, 64, 64, torch.float16, ("signs_qk",))])
 def test_a_chain_in_segments_behind_the_prologue_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts):
     test_operand_prologue_in_the_one_call_forward_equals_the_staged_kernels(cuda, cell, NT, B, H, K, V, dtype, parts)
+
+
+# the running sum of a 64-token chunk by its thread-wide form (lq_zoo_cumsum) against fp64: the orders differ by fp64 roundings only, which
+# move an fp32 result by one unit in the last place at most; one token that forgets everything, in each 16 of the chunk
+@pytest.mark.parametrize("at", [None, 0, 15, 16, 40, 63])
+def test_cumulative_scalar_decay_of_64_tokens(cuda, at):
+    from linquant_amd.kernels.zoo import _common as C
+
+    B, NT, H = 3, 5, 7
+    g = -torch.rand(B, 64 * NT, H, generator=torch.Generator().manual_seed(3)) ** 4 * 8
+    if at is not None:
+        g[1, 128 + at, 2] = float("-inf")
+    out = C.cumsum(g.to(cuda), B, 64 * NT, H, 0)[0].cpu().view(B, NT, 64, H)
+    ref = g.double().view(B, NT, 64, H).cumsum(2)
+    assert torch.equal(torch.isinf(out), torch.isinf(ref))
+    fin = torch.isfinite(ref)
+    assert ((out[fin].double() - ref[fin]).abs() <= ref[fin].abs() * 2.0 ** -23).all()
+
+
+# the same sum across the lanes of a wave, in the launches that make it themselves: what a decay of minus infinity cuts off is cut off
+@pytest.mark.parametrize("cell", ["mamba2", "gated_deltanet"])
+@pytest.mark.parametrize("at", [0, 15, 16, 40, 63])
+def test_a_scalar_decay_that_forgets_everything_equals_the_staged_kernels(cuda, cell, at):
+    from linquant_amd.kernels import zoo
+
+    B, T, H, K, V = 1, 192, 3, 64, 64
+    q, k, v, g, beta = [t.to(cuda) if t is not None else None for t in zc.inputs(cell, B=B, T=T, H=H, K=K, V=V, seed=at, dtype=torch.float16)]
+    g[0, 64 + at, 1] = -200.0
+    sc = {n: torch.full((H,), x, device=cuda) for n, x in (("q", 0.002), ("k", 0.008), ("w", 0.03))}
+    sc.update(kw=torch.full((H, K), 0.01, device=cuda), **{n: torch.full((H, V), 0.03, device=cuda) for n in ("vw", "vl", "el", "ew", "state")})
+    fn, args = (zoo.chunk_simple_gla_int8, (q, k, v, g, sc)) if cell == "mamba2" else (zoo.chunk_delta_int8, (q, k, v, g, beta, sc))
+    o1, h1 = fn(*args, eta=0.25, output_final_state=True)
+    o0, h0 = fn(*args, eta=0.25, output_final_state=True, _staged=True)
+    assert float(o1.float().abs().max()) > 0 and torch.isfinite(o1).all()
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
