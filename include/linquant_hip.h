@@ -513,6 +513,11 @@ typedef struct {
   void* workspace;           /* device memory, 256-byte aligned, lq_zoo_chunk_forward_workspace_bytes() bytes; contents
                                 undefined on entry and on return */
   int64_t workspace_bytes;
+  /* 64-token chunks under per-channel decay: the tables as a caller holds them, 16-byte aligned; what would take a launch of its own
+   * in front of this call is done where they are read */
+  const float* rot_f32;      /* instead of rot: (K,K) fp32, rounded to fp16; or NULL */
+  void* rot_ws;              /* K * K * 2 bytes more of workspace: with it larger calls lay R_QK out as operands first; or NULL */
+  const float* dqk;          /* instead of dq and dq_rcp (KDA): (H,K) D_QK, its reciprocals rounded once; or NULL */
 } lq_zoo_chunk_forward_args;
 int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* args, hipStream_t stream);
 /* workspace size for the dims, family, decay and chunk size in `args` (pointers are not read), written to *bytes */

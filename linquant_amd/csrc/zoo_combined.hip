@@ -259,6 +259,12 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   return LQ_OK;
 }
 
+// R_QK laid out as operands by a launch of its own (4.5 us), or read by every chunk and head as the caller holds it (32 requests of 4 or,
+// fp32, 8 bytes a lane, rows apart, in the place of eight of 16)?  Whole calls: GLA B4 T4096 H16 (4096 of them) 196.8 us laid out, 217.6
+// as fp32, 199.6 as fp16 behind a conversion launch; KDA B1 T2048 H8 (256) 45.6 as fp32, 47.2 behind a launch.  Reading fp32 costs 5 ns for
+// each of them, so the line is at the launch's 4.5 us.
+bool rot_operand(const lq_zoo_chunk_forward_args* a) { return (int64_t)a->batch * a->nheads * (a->seqlen / 64) >= 1024; }
+
 }  // namespace
 
 extern "C" int lq_zoo_chunk_forward_workspace_bytes(const lq_zoo_chunk_forward_args* a, int64_t* bytes) {
@@ -281,8 +287,10 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   if (delta && (!a->beta || !a->sw)) return LQ_ERR_NULL;
   if (!a->sk) return LQ_ERR_NULL;
   if ((a->dq != nullptr) != (a->dq_rcp != nullptr)) return LQ_ERR_NULL;
-  if (a->dq && (!delta || !diag || big)) return LQ_ERR_SHAPE;  // D_QK at load: KDA, 64-token chunks
+  if ((a->dq || a->dqk) && (!delta || !diag || big)) return LQ_ERR_SHAPE;  // D_QK at load: KDA, 64-token chunks
   if (a->rot && !diag) return LQ_ERR_SHAPE;
+  if (a->rot_f32 && (!diag || big)) return LQ_ERR_SHAPE;  // rounded in the launch in front of the recurrence
+  if ((a->rot && a->rot_f32) || (a->dq && a->dqk)) return LQ_ERR_SHAPE;
   if (!big && (rc = check_scan(a->q, a->k, a->v, a->o, a->ss, a->svl, a->batch, a->seqlen, a->nheads, a->kdim, a->vdim, a->qmax, a->act_dtype)) != LQ_OK)
     return rc;
   if (a->workspace_bytes < l.total || ((uintptr_t)a->workspace % kAlign) != 0) return LQ_ERR_SHAPE;
@@ -309,11 +317,16 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
   float* cross = big ? (float*)(ws + l.cross) : nullptr;
 
   if (diag && !big) {  // everything in front of the recurrence in one launch
-    for (const void* x : {(const void*)a->rot, (const void*)a->dq, (const void*)a->dq_rcp, delta ? (const void*)a->skw : nullptr})
+    for (const void* x : {(const void*)a->rot, (const void*)a->rot_f32, (const void*)a->dq, (const void*)a->dq_rcp, (const void*)a->dqk,
+                          (const void*)a->rot_ws, delta ? (const void*)a->skw : nullptr})
       if (!zoo_al(x, 16)) return LQ_ERR_SHAPE;
     ZooDiagParams d = {};
     d.q = (const _Float16*)a->q, d.k = (const _Float16*)a->k, d.v = (const _Float16*)a->v, d.g = a->g, d.beta = a->beta;
-    d.rot = (const _Float16*)a->rot, d.dq = a->dq, d.dk_div = a->dq, d.dk_rcp = a->dq_rcp;
+    if ((a->rot || a->rot_f32) && a->rot_ws && rot_operand(a)) {
+      if ((rc = zoo_rot_operand_launch(a->rot_f32 ? a->rot_f32 : a->rot, a->rot_f32, (_Float16*)a->rot_ws, a->kdim, stream)) != LQ_OK) return rc;
+      d.rot_op = (const _Float16*)a->rot_ws;
+    }
+    d.rot = (const _Float16*)a->rot, d.rot_f = a->rot_f32, d.dq = d.dk_div = a->dqk ? a->dqk : a->dq, d.dk_rcp = a->dq_rcp;
     d.sq = a->sq, d.sk = a->sk, d.skw = a->skw, d.sw = a->sw, d.svw = a->svw, d.svl = a->svl;
     d.A = (_Float16*)A, d.qc = qg, d.kqT = kqT, d.wq = wq, d.vqT = vqT, d.vcT = vcT, d.U = (_Float16*)U, d.gam = gam, d.pack = pack;
     d.sigma = a->sigma, d.tau = a->tau, d.eta = a->eta, d.scale = a->scale, d.qmax = a->qmax, d.bf = a->act_dtype == LQ_DT_BF16;

@@ -41,6 +41,9 @@
 // during which its SIMD issues no vector instruction (the half-precision MFMA costs them only its issue), yet splitting their operands in
 // three would cost more.  Persistent workgroups with the next chunk's requests ahead spilled (KDA 714), three workgroups a compute unit for
 // GLA too (194).
+// R_QK comes in fp16, in fp32 or (larger calls) laid out as operands; D_QK's reciprocals are formed here.  As launches in front these were
+// 4.5 us for R_QK and 9.5 for the reciprocals: whole calls KDA B1 T2048 H8 47.2 -> 45.6, KDA B2 T8192 H32 with D_QK 532.8 -> 524.7, GLA B4
+// T4096 H16 199.6 -> 196.8 (there laid out as operands in the place of converted: kernel 144.6 -> 140.3 of its box).
 // Spilled registers: DIAG_KDA at K = 128 with the gate (sigma < 1, tau > 0) keeps Hw beside k over the key operands and spills 13 to 19
 // of its 128 in fp16 and up to 15 in bf16 (56 to 80 and up to 64 bytes a lane; about 300 of the 972 MB read and of the 730 MB written at
 // sigma = 0.5 above); without the gate at most one (bf16 with D_QK); the other forms and K = 64 none.
@@ -198,7 +201,10 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   if (tid < K) {
     if constexpr (L::KQ) iskw_s[tid] = codes ? 1.0f / p.skw[h * K + tid] : 0.0f;
     if constexpr (DK && DO_A) dq_s[tid] = p.dq[h * K + tid];
-    if constexpr (DK && DELTA) dkd_s[tid] = p.dk_div[h * K + tid], dkr_s[tid] = p.dk_rcp[h * K + tid];
+    if constexpr (DK && DELTA) {
+      const float d = p.dk_div[h * K + tid];
+      dkd_s[tid] = d, dkr_s[tid] = p.dk_rcp ? p.dk_rcp[h * K + tid] : 1.0f / d;
+    }
   }
 
   // ---- 1: cumulative log decay of the chunk into LDS
@@ -595,15 +601,37 @@ __global__ __launch_bounds__(512, 4) void zoo_diag_prep_kernel(ZooDiagParams p) 
   const int strip = wave % NS, part_of = wave / NS;
   lq_v4i rop[ROT ? 2 : 1][KS];
   if constexpr (ROT) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      uint32_t w[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(p.rot + (32 * ks + 8 * kg + e) * K + 32 * strip + 2 * rl);
+    auto operand = [&](const uint32_t (&w)[8], int ks) __attribute__((always_inline)) {
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         rop[0][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x05040100u);
         rop[1][ks][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1], w[2 * d], 0x07060302u);
+      }
+    };
+    const int at0 = 8 * kg * K + 32 * strip + 2 * rl;
+    if (FUSED && p.rot_op) {  // (uniform over the launch)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) rop[t][ks] = *(const lq_v4i*)(p.rot_op + (((strip * 2 + t) * KS + ks) * 64 + lane) * 8);
+    } else if (FUSED && p.rot_f) {  // fp32, rounded here
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const zoo_v2f x = *(const zoo_v2f*)(p.rot_f + at0 + (32 * ks + e) * K);
+          w[e] = zoo_pack_h2(x[0], x[1]);
+        }
+        operand(w, ks);
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(p.rot + at0 + (32 * ks + e) * K);
+        operand(w, ks);
       }
     }
   }
@@ -921,7 +949,7 @@ int launch_bf(const ZooDiagParams& p, hipStream_t stream) {
 template <int K, int MODE, bool DK>
 int launch_rot(const ZooDiagParams& p, hipStream_t stream) {
   if constexpr (MODE != DIAG_WY) {
-    if (p.rot) return launch_bf<K, true, MODE, DK>(p, stream);
+    if (p.rot || p.rot_f || p.rot_op) return launch_bf<K, true, MODE, DK>(p, stream);
   }
   return launch_bf<K, false, MODE, DK>(p, stream);
 }

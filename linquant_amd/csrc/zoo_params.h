@@ -222,7 +222,9 @@ struct ZooDiagParams {
   const float* beta;
   const float* logenv;    // DIAG_WY with write codes
   const _Float16* rot;    // (K,K) local R_QK, or nullptr
-  const float* dq;        // (H,K) D_QK for q, and for k with its reciprocal, or nullptr
+  const float* rot_f;     // fused forms: the same in fp32, to be rounded to fp16 (instead of rot), or nullptr
+  const _Float16* rot_op; // fused forms: the same as zoo_rot_operand_launch leaves it (before the others), or nullptr
+  const float* dq;        // (H,K) D_QK for q, and for k with its reciprocal (nullptr: formed here), or nullptr
   const float* dk_div;
   const float* dk_rcp;
   const float* sq;
@@ -254,6 +256,8 @@ int zoo_diag_a_launch(const ZooDiagParams& p, int K, hipStream_t stream);
 int zoo_diag_wy_launch(const ZooDiagParams& p, int K, hipStream_t stream);
 int zoo_diag_gla_launch(const ZooDiagParams& p, int K, hipStream_t stream);
 int zoo_diag_kda_launch(const ZooDiagParams& p, int K, hipStream_t stream);
+// R_QK (fp16, or fp32: rounded) in the operand order of the fused forms, K * K halves; defined in zoo_rot_operand.hip
+int zoo_rot_operand_launch(const void* rot, bool f32, _Float16* op, int K, hipStream_t stream);
 
 // Operand pre-pass of the linear family with no / scalar decay for zoo_scan.hip; defined in zoo_lin_prep.hip
 struct ZooLinPrepParams {

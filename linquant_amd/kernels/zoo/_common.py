@@ -141,6 +141,11 @@ def unrot_matrix(unrot, V):
     return unrot.to(torch.float16).contiguous()
 
 
+def rot_f16(rot):
+    """The local R_QK as the stage kernels read it."""
+    return None if rot is None else rot.to(torch.float16).contiguous()
+
+
 def cumsum(g, B, T, H, kdim, write=None, span=CHUNK):
     """Chunk-local cumulative log decay (fp32) over chunks of ``span`` tokens and, for per-channel decay, the log envelope.  ``write`` = dict(k, v, skw,
     svw, eta, qmax) (per-channel decay, linear family): the launch also makes the state kernel's write operands while
@@ -333,9 +338,10 @@ _FORWARD_WS = {}
 
 
 def one_call_forward(family, decay, q, k, v, g, beta, sc, dims, span, *, sigma=1.0, tau=1.0, eta, scale, qmax, final_state,
-                     out_dtype, rot=None, dq=None, dq_rcp=None):
+                     out_dtype, rot=None, dqk=None):
     """lq_zoo_chunk_forward: every stage of a chunk forward (GLA, DeltaNet, Gated DeltaNet, KDA; rotated storage) from one
-    foreign call over one workspace.  ``sc``: fp32 scales by role ('q','k','w','kw', value write 'vw' / 'ew', value local
+    foreign call over one workspace.  ``rot`` (K,K) R_QK in any float type, ``dqk`` (H,K) D_QK (64-token chunks): fp32 tables go in as they
+    are.  ``sc``: fp32 scales by role ('q','k','w','kw', value write 'vw' / 'ew', value local
     'vl' / 'el', 'state').  Returns (o, final fp32 state or None)."""
     import ctypes
 
@@ -344,6 +350,16 @@ def one_call_forward(family, decay, q, k, v, g, beta, sc, dims, span, *, sigma=1
     delta = family == FAMILY_DELTA
     svw, svl = (sc["ew"], sc["el"]) if delta else (sc["vw"], sc["vl"])
     svl, ss, skw = _lib.aligned(svl), _lib.aligned(sc["state"]), _lib.aligned(sc["kw"])
+    rot_f = None
+    if rot is not None:
+        assert tuple(rot.shape) == (K, K), "rot: (K, K) R_QK"
+        if span == CHUNK and rot.dtype == torch.float32 and rot.is_contiguous():
+            rot, rot_f = None, _lib.aligned(rot)
+        else:
+            rot = rot_f16(rot)
+    if dqk is not None:
+        dqk = _lib.aligned(f32(dqk))
+        assert tuple(dqk.shape) == (H, K), f"dqk: (H, K) = ({H}, {K}) positive factors"
     key = (family, decay, B, T, H, K, V, span)
     nbytes = _FORWARD_WS.get(key)
     if nbytes is None:
@@ -354,13 +370,14 @@ def one_call_forward(family, decay, q, k, v, g, beta, sc, dims, span, *, sigma=1
         if rc != 0:
             raise _lib.LinQuantHipError(f"lq_zoo_chunk_forward_workspace_bytes failed with code {rc}")
         nbytes = _FORWARD_WS[key] = n.value
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    extra = 2 * K * K if span == CHUNK and (rot is not None or rot_f is not None) else 0  # R_QK as operands
+    ws = torch.empty(nbytes + extra, dtype=torch.uint8, device=dev)
     o = out_buffer(v, out_dtype)
     ht = torch.empty(B, H, K, V, dtype=torch.float32, device=dev) if final_state else None
     _lib.call("lq_zoo_chunk_forward", dev, q=_lib.ptr(q), k=_lib.ptr(k), v=_lib.ptr(v), g=_lib.ptr(g), beta=_lib.ptr(beta),
               o=_lib.ptr(o), o_is_f32=int(o.dtype == torch.float32), ht=_lib.ptr(ht), sq=_lib.ptr(sc["q"]), sk=_lib.ptr(sc["k"]),
               sw=_lib.ptr(sc.get("w")), skw=_lib.ptr(skw), svw=_lib.ptr(svw), svl=_lib.ptr(svl), ss=_lib.ptr(ss), rot=_lib.ptr(rot),
-              dq=_lib.ptr(dq), dq_rcp=_lib.ptr(dq_rcp), sigma=float(sigma), tau=float(tau), eta=float(eta), scale=float(scale),
+              rot_f32=_lib.ptr(rot_f), rot_ws=ws.data_ptr() + nbytes if extra else None, dqk=_lib.ptr(dqk), sigma=float(sigma), tau=float(tau), eta=float(eta), scale=float(scale),
               qmax=int(qmax), family=family, decay=decay, batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=span,
               act_dtype=act_code(v), workspace=_lib.ptr(ws), workspace_bytes=nbytes)
     return o, ht

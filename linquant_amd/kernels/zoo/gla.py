@@ -28,21 +28,20 @@ def chunk_gla_int8(q, k, v, g, scales, *, eta=0.0, scale=None, chunk_size=64, ou
     B, T, H, K, V = dims
     assert chunk_size % BC == 0
     Ru = C.unrot_matrix(unrot, V)
-    R = None if rot is None else rot.to(torch.float16).contiguous()
     scale = K0 ** -0.5 if scale is None else scale
     qmax = 2 ** (bits - 1) - 1
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "kw", "vw", "vl", "state")}
     if unrot is None and _debug is None and not _staged:
         # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
         o, ht = C.one_call_forward(C.FAMILY_LINEAR, C.DECAY_DIAGONAL, q, k, v, C.f32(g), None, sc, dims, span, eta=eta, scale=scale,
-                                   qmax=qmax, final_state=output_final_state, out_dtype=out_dtype, rot=R)
+                                   qmax=qmax, final_state=output_final_state, out_dtype=out_dtype, rot=rot)
         return C.cut_values(restore(o), C.cut_keys(ht, K0), V0)
     # the cumsum launch also makes the state kernel's write operands (it holds the chunk's decay tile): no pre-pass
     if span == C.CHUNK:
         gc, logenv, codes = C.cumsum(g, B, T, H, K, write=dict(k=k, v=v, skw=sc["kw"], svw=sc["vw"], eta=eta, qmax=qmax))
     else:
         (gc, logenv), codes = C.cumsum(g, B, T, H, K, span=span), None
-    A, qg = C.run_gla_A(q, k, gc, sc["q"], sc["k"], scale, qmax, dims, rot=R, span=span)
+    A, qg = C.run_gla_A(q, k, gc, sc["q"], sc["k"], scale, qmax, dims, rot=C.rot_f16(rot), span=span)
     NT = T // span
     h_i8 = torch.empty(B, NT, H, V, K, dtype=torch.int8, device=q.device)
     ht = torch.empty(B, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None

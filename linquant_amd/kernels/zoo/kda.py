@@ -41,17 +41,16 @@ def chunk_kda_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=0.0, sca
     B, T, H, K, V = dims
     assert chunk_size % BC == 0 and beta.shape == (B, T, H)
     Ru = C.unrot_matrix(unrot, V)
-    R = None if rot is None else rot.to(torch.float16).contiguous()
     scale = K0 ** -0.5 if scale is None else scale
     qmax = 2 ** (bits - 1) - 1
     sc = {n: C.f32(scales[n]) for n in ("q", "k", "w", "kw", "el", "ew", "state")}
-    dq, dq_rcp = C.dqk_tables(dqk, H, K)
     if unrot is None and _debug is None and not _staged:
         # the whole forward as one C call over one workspace (the bits of the stage-by-stage route below)
         o, ht = C.one_call_forward(C.FAMILY_DELTA, C.DECAY_DIAGONAL, q, k, v, C.f32(g), C.f32(beta), sc, dims, span, sigma=sigma,
                                    tau=tau, eta=eta, scale=scale, qmax=qmax, final_state=output_final_state, out_dtype=out_dtype,
-                                   rot=R, dq=dq, dq_rcp=dq_rcp)
+                                   rot=rot, dqk=dqk)
         return C.cut_values(restore(o), C.cut_keys(ht, K0), V0)
+    dq, dq_rcp = C.dqk_tables(dqk, H, K)
     gc, logenv = C.cumsum(g, B, T, H, K, span=span)
     # one launch makes Hw, U, fw and the state kernel's write-operand codes; W leaves the chip only for a caller that asks
     if span == C.CHUNK:
@@ -60,7 +59,7 @@ def chunk_kda_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=0.0, sca
                                             keep_W=_debug is not None, dk=(dq, dq_rcp))
     else:  # (D_QK was applied up front; the write-operand codes come from the pre-pass launch)
         Hw, W, U, fw, codes = C.run_wy_prep(k, v, C.f32(beta), gc, sigma, tau, dims, C.DECAY_DIAGONAL, span=span)
-    A, qg = C.run_gla_A(q, Hw, gc, sc["q"], sc["k"], scale, qmax, dims, rot=R, dq=dq, span=span)
+    A, qg = C.run_gla_A(q, Hw, gc, sc["q"], sc["k"], scale, qmax, dims, rot=C.rot_f16(rot), dq=dq, span=span)
     NT = T // span
     h_i8 = torch.empty(B, NT, H, V, K, dtype=torch.int8, device=q.device)
     e_out = torch.empty_like(v)

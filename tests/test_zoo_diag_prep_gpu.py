@@ -72,3 +72,26 @@ def test_halves_of_a_sub_block_that_decide_apart_match_the_oracle(cuda, cell, K,
     scales = qz.kernel_scales(0, H, K, V, delta=cell == "kda")
     out = zc.run_kernel(cell, tensors, scales, eta=0.0, rot=R, debug={} if staged else None)[0]
     zc.check(out, run, qz, f"{cell} K={K} rot={rot} staged={staged}")
+
+
+# every way in which R_QK comes to the launch, below and from its line (1024 chunks and heads) on: fp32 as it is, fp32 that is not on a
+# 16-byte boundary, fp32 whose rows are not contiguous, fp16, fp64; a matrix without symmetry, so that a transposed operand shows
+@pytest.mark.parametrize("cell", ["gla", "kda"])
+@pytest.mark.parametrize("NT,H,K", [(31, 33, 64), (32, 32, 64), (33, 31, 128), (16, 64, 128)])
+@pytest.mark.parametrize("form", ["fp32", "unaligned", "transposed", "fp16", "fp64"])
+def test_every_form_of_the_local_rotation_equals_the_stages(cuda, cell, NT, H, K, form):
+    from linquant_amd.kernels import zoo
+
+    q, k, v, g, beta = [t if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=64 * NT, H=H, K=K, V=64, seed=NT, dtype=torch.float16)]
+    R = torch.linalg.qr(torch.randn(K, K, generator=torch.Generator().manual_seed(K), dtype=torch.float64))[0].to(cuda)
+    R = {"fp32": R.float(), "transposed": R.float().T, "fp16": R.half(), "fp64": R,
+         "unaligned": torch.cat([torch.zeros(1, device=cuda), R.float().flatten()])[1:].view(K, K)}[form]
+    assert R.is_contiguous() == (form != "transposed") and (form != "unaligned" or R.data_ptr() % 16 == 4)
+    full = lambda x, *shape: torch.full(shape, x, device=cuda)  # noqa: E731
+    sc = {"q": full(0.002, H), "k": full(0.008, H), "w": full(0.03, H), "kw": full(0.01, H, K)}
+    sc.update({n: full(0.03, H, 64) for n in ("vw", "vl", "el", "ew", "state")})
+    kw = dict(eta=0.25, output_final_state=True, rot=R)
+    call = lambda **x: zoo.chunk_kda_int8(q, k, v, g, beta, sc, dqk=full(0.75, H, K), **kw, **x) if cell == "kda" else zoo.chunk_gla_int8(q, k, v, g, sc, **kw, **x)  # noqa: E731
+    (o1, h1), (o0, h0) = call(), call(_staged=True)
+    assert float(o1.float().abs().max()) > 0
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
