@@ -83,7 +83,7 @@ def test_every_form_of_the_local_rotation_equals_the_stages(cuda, cell, NT, H, K
     from linquant_amd.kernels import zoo
 
     q, k, v, g, beta = [t if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=64 * NT, H=H, K=K, V=64, seed=NT, dtype=torch.float16)]
-    R = torch.linalg.qr(torch.randn(K, K, generator=torch.Generator().manual_seed(K), dtype=torch.float64))[0].to(cuda)
+    R = torch.linalg.qr(torch.randn(K, K, generator=torch.Generator().manual_seed(K), dtype=torch.float64))[0].contiguous().to(cuda)
     R = {"fp32": R.float(), "transposed": R.float().T, "fp16": R.half(), "fp64": R,
          "unaligned": torch.cat([torch.zeros(1, device=cuda), R.float().flatten()])[1:].view(K, K)}[form]
     assert R.is_contiguous() == (form != "transposed") and (form != "unaligned" or R.data_ptr() % 16 == 4)
