@@ -13,6 +13,9 @@ from pathlib import Path
 ROOT = Path(__file__).resolve().parent
 HEADER = ROOT.parent / "include" / "linquant_hip.h"
 LIB_PATH = ROOT / "csrc" / "liblinquant_hip.so"
+_NATIVE_ENTRIES = ("lq_zoo_simple_gla", "lq_zoo_simple_gla_workspace_bytes", "lq_zoo_chunk_forward",
+                   "lq_zoo_chunk_forward_workspace_bytes", "lq_zoo_rotate_qkv", "lq_split_rotate_quant_xBC", "lq_ssd_combined",
+                   "lq_ssd_combined_workspace_bytes")
 ABI_VERSION = 21
 
 LQ_DT_F16, LQ_DT_F32, LQ_DT_I8, LQ_DT_BF16 = 0, 1, 2, 3
@@ -93,6 +96,27 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The wrappers' short calls in native code (csrc/binding.cpp): functions that return None for what they do not serve."""
+    global _native
+    if _native is None:
+        lib = load()
+        try:
+            from linquant_amd import _binding
+        except ImportError as e:
+            raise LinQuantHipError("linquant_amd/_binding.so is missing: build it with `python -m linquant_amd.build`") from e
+        _binding.init(raise_failed, {fn: ctypes.cast(getattr(lib, fn), ctypes.c_void_p).value for fn in _NATIVE_ENTRIES})
+        _native = _binding
+    return _native
+
+
+def raise_failed(fn, rc):
+    raise LinQuantHipError(f"{fn} failed with code {rc}: {_ERRORS.get(rc, 'unknown error')}")
+
+
 def ptr(t):
     """Device pointer of a torch tensor (None -> NULL)."""
     return None if t is None else t.data_ptr()
@@ -147,7 +171,7 @@ def launch(fn: str, device, st):
         with torch.cuda.device(device):
             rc = getattr(lib, fn)(ctypes.byref(st), current_stream(device))
     if rc != 0:
-        raise LinQuantHipError(f"{fn} failed with code {rc}: {_ERRORS.get(rc, 'unknown error')}")
+        raise_failed(fn, rc)
 
 
 def call(fn: str, device, **fields):

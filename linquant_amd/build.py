@@ -1,4 +1,4 @@
-"""Build liblinquant_hip.so (all HIP kernels + the C ABI) for gfx950 with hipcc.
+"""Build liblinquant_hip.so (all HIP kernels + the C ABI) for gfx950 with hipcc, and the wrappers' native host code.
 
 ``python -m linquant_amd.build`` compiles in-tree; the library lands next to the sources so it travels with
 the repository snapshot.  hipcc cross-compiles without a GPU.
@@ -15,6 +15,7 @@ from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB_PATH = CSRC / "liblinquant_hip.so"
+BINDING_PATH = CSRC.parent / "_binding.so"
 ARCH = "gfx950"
 
 # -ffp-contract=off: every fp32 multiply/add that feeds an INT8 code is rounded on its own (the CPU checker
@@ -41,6 +42,23 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{res.stderr}")
 
 
+def _compile_binding() -> None:
+    """csrc/binding.cpp (host code only) against the installed torch."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__path__[0])
+    inc = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include", sysconfig.get_paths()["include"],
+           Path(_hipcc()).resolve().parents[1] / "include"]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{i}" for i in inc), str(CSRC / "binding.cpp"),
+           "-o", str(BINDING_PATH), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on binding.cpp:\n{res.stderr}")
+
+
 def build(force: bool = True, jobs: int | None = None, verbose: bool = False) -> Path:
     """Compile every .hip source and link the shared library. Returns the library path."""
     srcs = sources()
@@ -56,8 +74,13 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     jobs = jobs or min(8, max(1, (os.cpu_count() or 2)))
     if verbose:
         print(f"[linquant_amd.build] compiling {len(todo)}/{len(srcs)} sources with {jobs} jobs", flush=True)
+    bind = CSRC / "binding.cpp"
+    stale = force or not BINDING_PATH.exists() or BINDING_PATH.stat().st_mtime < max(bind.stat().st_mtime, newest_hdr)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        binding = ex.submit(_compile_binding) if stale else None
         list(ex.map(lambda so: _compile(*so), todo))
+        if binding is not None:
+            binding.result()
     objs = [str(objdir / (s.stem + ".o")) for s in srcs]
     cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", str(LIB_PATH)]
     res = subprocess.run(cmd, capture_output=True, text=True)

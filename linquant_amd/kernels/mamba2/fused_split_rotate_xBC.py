@@ -32,6 +32,11 @@ def fused_split_rotate_quant_xBC(xBC, r_signs, nheads, ngroups, d_state, headdim
     ``kronecker_hadamard_fwd`` of the [dqk-scaled] B lanes, so a key-side caller saves that second launch.  With
     ``return_b_rowmax`` as well a fifth: max_n |b_fp| per (batch, token, group), fp32, the table the key-side chunk state
     uses to leave out all-zero slabs (its ``b_rowmax``), which saves that stage's pre-pass over B."""
+    if dqk_b is None:
+        done = _lib.native().split_rotate(xBC, r_signs, nheads, ngroups, d_state, headdim, B_inv_scale, C_inv_scale, return_b_fp,
+                                          return_b_rowmax)
+        if done is not None:
+            return done
     batch, seq_len, xBC_dim = xBC.shape
     d_ssm = nheads * headdim
     g_n = ngroups * d_state

@@ -34,10 +34,17 @@ def _quant_mamba_chunk_scan_combined_fwd(x_fp, q_dt, dt_scale, q_A_log, A_log_sc
     fixed-point recurrence, INT8 CB on ``static_cb_scale``, INT8 chunk scan. Returns (out fp16 (B,L,H,P), None).
     ``b_rowmax`` (not in the reference; key side, optional): the per-token max |b_fp| that the prologue can return beside
     ``b_fp``; without it the chunk state stage computes the table itself.  Same result either way."""
+    rebound = _stages_rebound()
+    if not rebound:
+        out = _lib.native().ssd(x_fp, q_dt, dt_scale, q_A_log, A_log_scale, q_B, B_scale, q_C, C_scale, chunk_size, q_D, D_scale,
+                                dt_bias, dt_softplus, dt_limit, static_state_scale, static_cb_scale, alpha_hp, bscale_g, keyside,
+                                x_scale_hp, b_fp, b_gate_scale, b_rowmax, _GATE_SHIFT)
+        if out is not None:
+            return out, None
     batch, seqlen, nheads, headdim = x_fp.shape
     _, _, ngroups, dstate = q_B.shape
 
-    if not _stages_rebound():
+    if not rebound:
         return _one_call(x_fp, q_dt, dt_scale, q_A_log, A_log_scale, q_B, B_scale, q_C, C_scale, chunk_size, q_D, D_scale,
                          dt_bias, dt_softplus, dt_limit, static_state_scale, static_cb_scale, alpha_hp, bscale_g, keyside,
                          x_scale_hp, b_fp, b_gate_scale, b_rowmax=b_rowmax), None

@@ -6,6 +6,7 @@ import torch
 
 from linquant_amd import _lib
 
+native = _lib.native
 FAMILY_LINEAR, FAMILY_DELTA = 0, 1
 DECAY_NONE, DECAY_SCALAR, DECAY_DIAGONAL = 0, 1, 2
 CHUNK = 64

@@ -19,6 +19,10 @@ def chunk_delta_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=1.0, s
     scales: 'q','k','w' (H,), 'kw' (H,K), 'el','ew','state' (H,V). Returns (o, final fp32 state or None).
     ``chunk_size``: up to 64 (padded to 64 tokens), or up to 128 (padded to 128: the WY transform then
     runs over 128 x 128 Gram matrices in a kernel of its own, the state and output kernels walk a chunk as two halves)."""
+    if chunk_size == C.CHUNK and unrot is None and _debug is None and not _staged and (g is None or g.dim() == 3):
+        done = C.native().chunk_forward(q, k, v, g, beta, scales, sigma, tau, eta, scale, output_final_state, bits, out_dtype, None, None)
+        if done is not None:
+            return done
     span = C.chunk_span(chunk_size)
     q, k, v, g, beta, restore = C.pad_chunks(chunk_size, q, k, v, g, beta, span=span)
     q, k, g, scales, _, K0 = C.pad_keys(q, k, g, scales)

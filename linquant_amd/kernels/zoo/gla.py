@@ -18,6 +18,10 @@ def chunk_gla_int8(q, k, v, g, scales, *, eta=0.0, scale=None, chunk_size=64, ou
     """q,k [B,T,H,K], v [B,T,H,V] fp16, g [B,T,H,K] fp32 per-channel log decay. scales as chunk_simple_gla_int8.
     Returns (o, final fp32 state or None).  ``chunk_size``: a multiple of 16 up to 64, or up to 128 (the
     kernels walk a chunk of more than 64 tokens as two 64-token halves, padded to 128 tokens; the sub-block anchoring over its eight sub-blocks is the reference's)."""
+    if chunk_size == C.CHUNK and unrot is None and _debug is None and not _staged:
+        done = C.native().chunk_forward(q, k, v, g, None, scales, 1.0, 1.0, eta, scale, output_final_state, bits, out_dtype, rot, None)
+        if done is not None:
+            return done
     assert g.shape == q.shape
     span = C.chunk_span(chunk_size)
     q, k, v, g, _, restore = C.pad_chunks(chunk_size, q, k, v, g, span=span)

@@ -21,6 +21,10 @@ def chunk_kda_int8(q, k, v, g, beta, scales, *, sigma=1.0, tau=1.0, eta=0.0, sca
     (q' = q D, k' = k / D, rounded to the activation dtype) applied inside the kernels as they load q and k, with the
     result of calling ``rotate_qkv(q, k, None, dqk=dqk)`` first, bit for bit, and without that launch.
     ``chunk_size``: a multiple of 16 up to 64, or up to 128 (as ``chunk_delta_int8``)."""
+    if chunk_size == C.CHUNK and unrot is None and _debug is None and not _staged and beta is not None and g.dim() == 4:
+        done = C.native().chunk_forward(q, k, v, g, beta, scales, sigma, tau, eta, scale, output_final_state, bits, out_dtype, rot, dqk)
+        if done is not None:
+            return done
     assert g.shape == q.shape
     span = C.chunk_span(chunk_size)
     if dqk is not None and q.shape[-1] in (64, 128) and span != C.CHUNK:

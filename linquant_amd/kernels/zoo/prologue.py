@@ -32,6 +32,10 @@ def rotate_qkv(q=None, k=None, v=None, *, signs_qk=None, signs_v=None, dqk=None,
     of R_QK / R_V (``rotation_signs``), None = that rotation is left out.  ``dqk`` (H,K) fp32, finite and positive: q is
     multiplied by it and k divided (the quotient rounded once, as the division of linquant/harness.py:86 rounds it).  Returns the tuple (q', k', v') of new tensors (None where the
     input was None); ``out=(q_out, k_out, v_out)`` supplies the destinations (an input itself for in-place)."""
+    if dqk is None and out is None:
+        done = C.native().rotate_qkv(q, k, v, signs_qk, signs_v)
+        if done is not None:
+            return done
     ref = next(t for t in (q, k, v) if t is not None)
     B, T, H = ref.shape[:3]
     K = q.shape[-1] if q is not None else (k.shape[-1] if k is not None else 0)

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import torch
 
+from ... import _lib
 from . import _common as C
 
 
@@ -24,6 +25,10 @@ def chunk_simple_gla_int8(q, k, v, g, scales, *, eta=1.0, scale=None, chunk_size
     ``chunk_size``: up to 256 in rotated storage, up to 128 in canonical storage (padded to the next multiple of 64):
     above 64 the kernels walk every chunk as two to four 64-token pieces, with one stored state, one carry update (the INT8
     write product summed over the chunk's tokens) and one fp32 local accumulation per chunk."""
+    if chunk_size == C.CHUNK and unrot is None and _debug is None and not _staged:
+        done = C.native().simple_gla(q, k, v, g, scales, eta, scale, output_final_state, bits, out_dtype, prologue)
+        if done is not None:
+            return done
     span = C.chunk_span(chunk_size, pieces=2 if unrot is not None else 4)
     if prologue is not None and (q.shape[-1] not in (64, 128) or v.shape[-1] not in (64, 128) or unrot is not None or span != C.CHUNK):
         from .prologue import rotate_qkv  # shapes the fused launch is not built for: rotate up front
@@ -82,8 +87,6 @@ def _one_call(q, k, v, g, scales, eta, scale, qmax, dims, span, final_state, out
               dqk=None):
     """lq_zoo_simple_gla: the whole forward from one foreign call, 64-token chunks with the operand rotations in it."""
     import ctypes
-
-    from ... import _lib
 
     B, T, H, K, V = dims
     dev = q.device

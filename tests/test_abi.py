@@ -280,3 +280,17 @@ def test_route_of_the_linear_family_at_the_lines_of_its_rule(B, H, T, K, V, one)
     st, n = _lib.fill("lq_zoo_simple_gla_args", batch=B, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=64), ctypes.c_int64(0)
     assert _lib.load().lq_zoo_simple_gla_workspace_bytes(ctypes.byref(st), ctypes.byref(n)) == 0
     assert scan != staged and n.value == (scan if one else staged)
+
+
+def test_native_calls_leave_everything_but_gpu_tensors_to_the_general_path():
+    """csrc/binding.cpp returns None, without an exception and without entering the library, for arguments that are no tensors, for tensors
+    on the CPU and for subclasses."""
+    n = _lib.native()
+    t = torch.zeros(1, 64, 1, 64, dtype=torch.float16)
+    sub = torch.zeros(1).as_subclass(type("Sub", (torch.Tensor,), {}))
+    for first in (None, 3, "x", t, sub):
+        assert n.simple_gla(first, t, t, None, {}, 1.0, None, False, 8, None, None) is None
+        assert n.chunk_forward(first, t, t, None, t, {}, 1.0, 1.0, 1.0, None, False, 8, None, None, None) is None
+        assert n.rotate_qkv(first, t, None, None, None) is None
+        assert n.split_rotate(first, None, 1, 1, 64, 64, t, t, False, False) is None
+        assert n.ssd(first, *[None] * 24) is None
