@@ -5,11 +5,15 @@
 // caller asks for them, the operand rotations and the D_QK rescaling (bench/zoo_kernels.py:135-140, linquant/harness.py:68-88), with
 // the arithmetic of lq_zoo_cumsum, lq_zoo_rotate_quant and lq_zoo_output in their order: the same bits.
 //
-// One 8-wave workgroup per (chunk, batch*head), two to a compute unit (registers): load (a thread takes four adjacent tokens x 8
-// channels; every row is read once) while one wave forms the cumulative decay | rotate and quantize into LDS | operands
-// out as whole 1 KB tiles and 64-byte rows, blocks of A on the INT8 MFMA.  Linear attention with the rotations, B4 T4096 H16 K = V =
-// 128: 85 to 93 us for 201 MB read and 168 MB written (4.0 to 4.3 TB/s), vector instructions 70 us of it; with zoo_scan.hip 157 us for
-// the whole call, 176 as operand, state and output launches.  The Mamba-2 cell B1 T2048 H8 K = V = 64: 28.0 -> 23.4 us.
+// One 8-wave workgroup per (chunk, batch*head), three to a compute unit (80 registers, 49 KB of LDS): load (a thread takes four adjacent
+// tokens x 8 channels; every row is read once) while one wave forms the cumulative decay | rotate and quantize q and k into LDS, then v,
+// requested when their rows have left the registers | operands out as whole 1 KB tiles and 64-byte rows, blocks of A on the INT8 MFMA.
+// What holds the registers at 80: one token after the other, with the tables of its channels (scales, signs) read from LDS anew for each,
+// and one copy of the pass over value columns, with nothing that follows from the thread's number kept across it.  Linear attention with
+// the rotations, B4 T4096 H16 K = V = 128: 95.3 -> 84 to 87 us for 201 MB read and 168 MB written (4.3 TB/s; two workgroups to a compute
+// unit at 127 registers before), vector instructions 70 us of it; whole call 146.6 -> 136 to 138.
+// B4 T4096 H16 K 64, V 128: whole call 106.2 -> 93.2 (100.6 with two workgroups and v requested first), Mamba-2 cell K = V = 64 of the same
+// size even.
 #include <type_traits>
 
 #include "zoo_params.h"
@@ -43,11 +47,17 @@ LQ_DEV int lp_q8(float x, float inv, int qmax) {
   return r;
 }
 
-// rotation of a row of 8 * LPR channels, as lq_zoo_rotate_qkv forms it before it rounds
-template <int LPR>
-LQ_DEV void lp_rotate(float (&x)[8], int sub, const float* signs) {
-  constexpr float norm = LPR == 16 ? 0.08838834764831845f : 0.125f;  // 1 / sqrt(128), 1 / sqrt(64)
-  zoo_fwht<LPR>(x, sub);
+// tokens one after the other, the tables of the eight channels read anew for each
+LQ_DEV void token_end() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// rotation of a row of 128 (wide: uniform over the workgroup) or 64 channels, as lq_zoo_rotate_qkv forms it before it rounds
+LQ_DEV void lp_rotate(float (&x)[8], int sub, const float* signs, bool wide) {
+  const float norm = wide ? 0.08838834764831845f : 0.125f;  // 1 / sqrt(128), 1 / sqrt(64)
+  zoo_fwht<8>(x, sub);
+  if (wide) zoo_fwht_stage<8>(x, sub);
   const lq_v4f s0 = *(const lq_v4f*)(signs + 8 * sub), s1 = *(const lq_v4f*)(signs + 8 * sub + 4);
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = (x[e] * norm) * (e < 4 ? s0[e & 3] : s1[e & 3]);
@@ -71,11 +81,12 @@ LQ_DEV lq_v2i lp_pack8(const int (&c)[8]) {
 }
 
 template <bool SCALAR, int K, bool BF>
-__global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p) {
+__global__ __launch_bounds__(512, K == 128 ? 6 : 4) void zoo_lin_prep_kernel(ZooLinPrepParams p) {
   constexpr int QS = K == 128 ? 160 : 80;  // bytes per row of the code tiles
   __shared__ __align__(16) unsigned char qI[64 * QS], kI[64 * QS];
   __shared__ __align__(16) uint32_t cK[lp_ct_size(K)], cW[lp_ct_size(128)], cL[lp_ct_size(128)];
   __shared__ float fk_s[64], fv_s[64], gs_s[64], iskw_s[K], isvw_s[128], isvl_s[128];
+  __shared__ __align__(16) float sqk_s[K], sv_s[128];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -87,22 +98,24 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
   const int64_t t0 = (int64_t)b * p.T + (int64_t)ct * 64;
   const int64_t cb = ((int64_t)b * p.NT + ct) * H + h;
 
-  // ---- requests: a thread takes a token quad x 8 channels of q or k (the first or second half of the first K / 16 waves) and of v
-  // (from wave 0 on beside 128 keys, from wave 4 on beside 64)
+  // ---- requests: a thread takes a token quad x 8 channels of q or k (the first or second half of the first K / 16 waves)
   constexpr int KP = K / 8;
   const bool is_k = wave >= K / 32;
   const int kt = tid & (16 * KP - 1), kq = kt / KP, kc = kt % KP;
   const bool kact = wave < K / 16;
-  const int vt = K == 128 ? tid : max(tid - 256, 0);
-  int vp = min(V, 128) / 8;  // 16-byte pieces of a value row per pass
-  bool vact = (K == 128 || wave >= 4) && vt < 16 * vp;  // (wave-uniform)
-  int vq = (vt / vp) & 15, vc = vt % vp;
-  lq_v4i kraw[4], vraw[4];
+  lq_v4i kraw[4];
   const _Float16* src = is_k ? p.k : p.q;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    kraw[u] = *(const lq_v4i*)(src + ((t0 + 4 * kq + u) * H + h) * K + 8 * kc);
-    vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * vq + u) * H + h) * V + 8 * vc);
+  for (int u = 0; u < 4; ++u) kraw[u] = *(const lq_v4i*)(src + ((t0 + 4 * kq + u) * H + h) * K + 8 * kc);
+  constexpr bool EARLY = K == 64;
+  lq_v4i vraw[4];
+  auto request_v = [&](int vb, int quad, int piece) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * quad + u) * H + h) * V + vb + 8 * piece);
+  };
+  if constexpr (EARLY) {
+    const int vp = min(V, 128) / 8, vt = max(tid - 256, 0);
+    request_v(0, (vt / vp) & 15, vt % vp);
   }
   // ---- per-token factors
   if (wave == 0) {
@@ -117,10 +130,16 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
     fk_s[lane] = fk, fv_s[lane] = fv;
   } else if (wave == 1 || wave == 2) {
     const int n = tid - 64;
-    if (n < K) iskw_s[n] = 1.0f / p.skw[(int64_t)h * K + n];
+    if (n < K) {
+      iskw_s[n] = 1.0f / p.skw[(int64_t)h * K + n];
+      if (p.signs_qk) sqk_s[n] = p.signs_qk[n];
+    }
   } else if (wave == 3 || wave == 4) {
     const int n = tid - 192;
-    if (n < V) isvw_s[n] = 1.0f / p.svw[(int64_t)h * V + n];
+    if (n < V) {
+      isvw_s[n] = 1.0f / p.svw[(int64_t)h * V + n];
+      if (p.signs_v) sv_s[n] = p.signs_v[n];
+    }
   } else if (wave == 5 || wave == 6) {
     const int n = tid - 320;
     if (n < V) isvl_s[n] = 1.0f / p.svl[(int64_t)h * V + n];
@@ -143,7 +162,7 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = is_k ? zoo_div_rn(x[e], p.dq[n + e], p.dq_rcp[n + e]) : zoo_mul_rn(x[e], p.dq[n + e]);
       }
-      if (p.signs_qk) lp_rotate<KP>(x, kc, p.signs_qk);
+      if (p.signs_qk) lp_rotate(x, kc, sqk_s, K == 128);
       if (p.dq || p.signs_qk) lp_round<BF>(x);
       int c[8];
       if (is_k) {  // (wave-uniform)
@@ -158,47 +177,67 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
         for (int e = 0; e < 8; ++e) c[e] = lp_q8(x[e] * p.scale, inv, qmax);
       }
       *(lq_v2i*)(codes + t * QS + 8 * kc) = lp_pack8(c);
+      token_end();
     });
     if (is_k) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) cK[lp_ct(8 * kc + e, kq)] = wc[e];
     }
   }
-  // ---- values: write and local codes by channel
-  auto value_codes = [&]() __attribute__((always_inline)) {
-    if (!vact) return;
-    uint32_t ww[8], wl[8];
-    lp_quad([&](auto u_c) __attribute__((always_inline)) {
-      constexpr int u = decltype(u_c)::value;
-      float x[8];
-      lp_dec<BF>(vraw[u], x);
-      if (p.signs_v) {  // (V is 64 or 128: one pass)
-        if (vp == 16) lp_rotate<16>(x, vc, p.signs_v); else lp_rotate<8>(x, vc, p.signs_v);
-        lp_round<BF>(x);
+  // ---- values, up to 128 columns a pass: write and local codes by channel.  A thread takes a token quad x 8 channels, from wave 0 on
+  // beside 128 keys, from wave 4 on beside 64.
+#pragma unroll 1
+  for (int vb = 0; vb < V; vb += 128) {
+    int own = tid;
+    asm volatile("" : "+v"(own));  // (nothing that follows from it is to wait in registers from in front of the loop on)
+    const int tid = own, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, kg = lane >> 4;
+    const int vt = K == 128 ? tid : max(tid - 256, 0);
+    const int vp = min(V - vb, 128) / 8;  // 16-byte pieces of a value row
+    const bool vact = (K == 128 || wave >= 4) && vt < 16 * vp;  // (wave-uniform)
+    const int vq = (vt / vp) & 15, vc = vt % vp;
+    __builtin_amdgcn_sched_barrier(0);  // (requested behind the codes of q and k, whose rows leave their registers)
+    if (!EARLY || vb > 0) request_v(vb, vq, vc);
+    if (vb > 0) {
+      __syncthreads();  // the tiles have been read
+      if (tid < 8 * vp) {
+        isvw_s[tid] = 1.0f / p.svw[(int64_t)h * V + vb + tid];
+        isvl_s[tid] = 1.0f / p.svl[(int64_t)h * V + vb + tid];
       }
-      const float f = fv_s[4 * vq + u];
+      __syncthreads();
+    }
+    if (vact) {
+      uint32_t ww[8], wl[8];
+      lp_quad([&](auto u_c) __attribute__((always_inline)) {
+        constexpr int u = decltype(u_c)::value;
+        float x[8];
+        lp_dec<BF>(vraw[u], x);
+        if (p.signs_v) {  // (V is 64 or 128: one pass)
+          lp_rotate(x, vc, sv_s, vp == 16);
+          lp_round<BF>(x);
+        }
+        const float f = fv_s[4 * vq + u];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          wl[e] = lp_put<u>(wl[e], lp_q8(x[e], isvl_s[8 * vc + e], qmax));
+          ww[e] = lp_put<u>(ww[e], lp_q8(SCALAR ? x[e] * f : x[e], isvw_s[8 * vc + e], qmax));
+        }
+        token_end();
+      });
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        wl[e] = lp_put<u>(wl[e], lp_q8(x[e], isvl_s[8 * vc + e], qmax));
-        ww[e] = lp_put<u>(ww[e], lp_q8(SCALAR ? x[e] * f : x[e], isvw_s[8 * vc + e], qmax));
+        const int at = lp_ct(8 * vc + e, vq);
+        cW[at] = ww[e], cL[at] = wl[e];
       }
-    });
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int at = lp_ct(8 * vc + e, vq);
-      cW[at] = ww[e], cL[at] = wl[e];
     }
-  };
-  auto value_store = [&](int vb) __attribute__((always_inline)) {
-    if (tid >= 32 * vp) return;  // four 16-byte pieces per channel (wave-uniform)
-    *(lq_v4i*)(p.vqT + (cb * V + vb) * 64 + 16 * tid) = *(const lq_v4i*)(cW + lp_ct(tid >> 2, 4 * (tid & 3)));
-    // operand order: wave w has the even or odd channels of tile w >> 1, tokens 8 kg .. and 32 + 8 kg ..
-    const uint32_t* row = cL + lp_ct(32 * (wave >> 1) + 2 * rl + (wave & 1), 2 * kg);
-    const lq_v2i lo = *(const lq_v2i*)row, hi = *(const lq_v2i*)(row + 8);
-    *(lq_v4i*)(p.vcT + cb * 64 * V + 64 * vb + 16 * tid) = lq_v4i{lo[0], lo[1], hi[0], hi[1]};
-  };
-  value_codes();
-  __syncthreads();
+    __syncthreads();
+    if (tid < 32 * vp) {  // four 16-byte pieces per channel (wave-uniform)
+      *(lq_v4i*)(p.vqT + (cb * V + vb) * 64 + 16 * tid) = *(const lq_v4i*)(cW + lp_ct(tid >> 2, 4 * (tid & 3)));
+      // operand order: wave w has the even or odd channels of tile w >> 1, tokens 8 kg .. and 32 + 8 kg ..
+      const uint32_t* row = cL + lp_ct(32 * (wave >> 1) + 2 * rl + (wave & 1), 2 * kg);
+      const lq_v2i lo = *(const lq_v2i*)row, hi = *(const lq_v2i*)(row + 8);
+      *(lq_v4i*)(p.vcT + cb * 64 * V + 64 * vb + 16 * tid) = lq_v4i{lo[0], lo[1], hi[0], hi[1]};
+    }
+  }
 
   // ---- operands out
   if (tid < 4 * K) {
@@ -206,7 +245,6 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
     const int tb = wave / (K / 64), ks = wave % (K / 64);  // 16 tokens x 64 channels
     *(lq_v4i*)(p.qc + cb * 64 * K + 16 * tid) = *(const lq_v4i*)(qI + (16 * tb + rl) * QS + 64 * ks + 16 * kg);
   }
-  value_store(0);
   // ---- blocks of A: (0,0) (1,0) (1,1) (2,0) .. (3,3) of the lower triangle, then zeros above it
   const float sqk = p.sq[h] * p.sk[h];
   for (int n = wave; n < 16; n += 8) {
@@ -234,23 +272,6 @@ __global__ __launch_bounds__(512, 4) void zoo_lin_prep_kernel(ZooLinPrepParams p
       out = lq_v2i{(int)zoo_pack_h2(x[0], x[1]), (int)zoo_pack_h2(x[2], x[3])};
     }
     *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(i, j0)) = out;
-  }
-  // ---- further passes of up to 128 value columns
-  for (int vb = 128; vb < V; vb += 128) {
-    vp = min(V - vb, 128) / 8;
-    vact = (K == 128 || wave >= 4) && vt < 16 * vp;
-    vq = (vt / vp) & 15, vc = vt % vp;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * vq + u) * H + h) * V + vb + 8 * vc);
-    __syncthreads();
-    if (tid < 8 * vp) {
-      isvw_s[tid] = 1.0f / p.svw[(int64_t)h * V + vb + tid];
-      isvl_s[tid] = 1.0f / p.svl[(int64_t)h * V + vb + tid];
-    }
-    __syncthreads();
-    value_codes();
-    __syncthreads();
-    value_store(vb);
   }
 }
 
