@@ -27,6 +27,10 @@
 // every step wait for the operands it had just requested (seen in its assembly: vmcnt(2) .. vmcnt(4)
 // where vmcnt(27) is meant).
 //
+// An output wave's products take the local value codes of all 64 tokens as fp16.  Converted by each of the four waves they were 40 of its
+// vector instructions a step; an operand to a wave, handed on through LDS at the rendezvous that is there, they are 10: linear attention
+// and GLA B4 T4096 H16 K = V = 128, kernel 64.7 -> 62.1 us, whole calls 136.9 -> 133.8 and 196.8 -> 194.8.
+//
 // The linear family keeps two operand sets and at most 128 registers, so that two workgroups fit a compute unit.  With five sets
 // (199 .. 236 registers, one workgroup) 257 to 511 workgroups took two rounds of the chip, the second nearly empty, and lost to the
 // two launches that this one replaces; the second workgroup hides more than the three further sets did.  Linear attention K = V = 128,
@@ -83,7 +87,6 @@ template <bool DELTA, bool SCALAR, int K, int BV>
 struct OutOps {
   lq_v4i qop[K / 64];                     // codes of q: token 16*w + (lane & 15)
   lq_v4i aop[2];                          // A (fp16): the same token, columns 32 js + 8 kg ..
-  lq_v4i vop[DELTA ? 1 : BV / 16];        // linear: local value codes of column NJ rl + jj (NJ = BV / 16), tokens 8 kg .. and 32 + 8 kg ..
   lq_v4f g;                               // scalar decay: cumulative log decay of tokens 16*w + 4 kg ..
 };
 
@@ -128,6 +131,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
   __shared__ __align__(16) unsigned char eT[DELTA ? BV * ES : 16];
   __shared__ __align__(16) unsigned char eB[DELTA ? BV * LS : 16];  // E in the activation dtype, channel-major
   __shared__ __align__(16) unsigned char eL[DELTA ? BV * LS : 16];  // its local codes as fp16, channel-major
+  __shared__ __align__(16) unsigned char vL[DELTA ? 16 : 2 * BV * 128];  // linear: local value codes as fp16, operand by operand
   __shared__ __align__(16) unsigned char ue_lds[DELTA ? 4 * 16 * US : 16];
   __shared__ __align__(16) float misc_lds[256];                     // 64 floats per chain wave
 
@@ -363,10 +367,6 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = *(const lq_v4i*)(p.qc + cb * 64 * K + ((w * (K / 64) + ks) * 64 + lane) * 16);
 #pragma unroll
       for (int js = 0; js < 2; ++js) o.aop[js] = *(const lq_v4i*)(p.A + cb * 4096 + ((w * 2 + js) * 64 + lane) * 8);
-      if constexpr (!DELTA) {
-#pragma unroll
-        for (int jj = 0; jj < NJ; ++jj) o.vop[jj] = *(const lq_v4i*)(p.vcT + cb * 64 * V + zoo_op_values(v0 + NJ * rl + jj, 8 * kg));
-      }
       if constexpr (SCALAR) o.g = *(const lq_v4f*)(p.gpk + cb * 64 + 16 * w + 4 * kg);
     };
     float of[NJ][4];
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
           if constexpr (DELTA)
             x = *(const lq_v8h*)(eL + (NJ * rl + jj) * LS + 2 * (32 * js + 8 * kg));
           else
-            x = scan_i8x8_to_f16x8(lq_v2i{o.vop[jj][2 * js], o.vop[jj][2 * js + 1]});
+            x = *(const lq_v8h*)(vL + (ct & 1) * BV * 128 + ((jj * 2 + js) * 64 + lane) * 16);
           loc[jj] = lq_mfma_f16(aop, x, loc[jj]);
         }
       }
@@ -442,32 +442,50 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       }
       *(Raw*)(eL + at) = o;
     };
+    // linear family: the local value codes become fp16 once for all four waves, an operand to a wave (column NJ rl + jj, tokens 32 js + 8 kg
+    // .., of jj = w & 1, js = w >> 1; 16 columns: an operand to two of them), a step ahead of their use and requested two
+    const int ojj = NJ == 2 ? w & 1 : 0, ojs = w >> 1;
+    lq_v2i vraw[2];
+    auto load_v = [&](int ct, lq_v2i& o) __attribute__((always_inline)) {
+      if constexpr (!DELTA)
+        o = *(const lq_v2i*)(p.vcT + (((int64_t)b * NT + ct) * H + h) * 64 * V + zoo_op_values(v0 + NJ * rl + ojj, 8 * kg) + 8 * ojs);
+    };
+    auto convert_v = [&](int ct, const lq_v2i& raw) __attribute__((always_inline)) {
+      if constexpr (!DELTA) *(lq_v8h*)(vL + (ct & 1) * BV * 128 + ((ojj * 2 + ojs) * 64 + lane) * 16) = scan_i8x8_to_f16x8(raw);
+    };
     // One step: `cur` holds chunk ct, `prev` chunk ct - 1, into which chunk ct + D - 1 is requested once its last use is past.
-    auto do_step = [&](auto first_c, int ct, Ops& cur, Ops& prev) __attribute__((always_inline)) {
+    auto do_step = [&](auto first_c, int ct, Ops& cur, Ops& prev, lq_v2i& vnext, lq_v2i& vafter) __attribute__((always_inline)) {
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();  // the stored copy of chunk ct is in LDS
       if constexpr (DELTA && !decltype(first_c)::value) finish(ct - 1, prev);
       load(min(ct + D - 1, c1 - 1), prev);
+      load_v(min(ct + 2, c1 - 1), vafter);
       read_state(ct, cur);
       if constexpr (DELTA) {
         __syncthreads();  // E of chunk ct is in LDS
         convert();
       } else {
         finish(ct, cur);
+        convert_v(ct + 1, vnext);
       }
     };
     Ops st[D];
+    load_v(c0, vraw[0]);
+    load_v(min(c0 + 1, c1 - 1), vraw[1]);
     load(c0, st[0]);
     scan_for<D - 1>([&](auto i) __attribute__((always_inline)) { st[i + 1] = st[0]; });
     scan_for<D - 2>([&](auto i) __attribute__((always_inline)) { load(min(c0 + i + 1, c1 - 1), st[i + 1]); });
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
     asm volatile("" ::: "memory");
-    do_step(std::true_type{}, c0, st[0], st[D - 1]);
+    // (linear family, D = 2: the value codes of chunk c0 + n are requested into vraw[n % 2])
+    convert_v(c0, vraw[0]);
+    do_step(std::true_type{}, c0, st[0], st[D - 1], vraw[1], vraw[0]);
     int ct = c0 + 1;
-    for (; ct + D <= c1; ct += D) scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]); });
+    for (; ct + D <= c1; ct += D)
+      scan_for<D>([&](auto i) __attribute__((always_inline)) { do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i], vraw[i % 2], vraw[(i + 1) % 2]); });
     scan_for<D - 1>([&](auto i) __attribute__((always_inline)) {
-      if (ct + i < c1) do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i]);
+      if (ct + i < c1) do_step(std::false_type{}, ct + i, st[(i + 1) % D], st[i], vraw[i % 2], vraw[(i + 1) % 2]);
     });
     if constexpr (DELTA) {
       __syncthreads();  // the local codes of the last chunk, written by all four output waves
