@@ -31,6 +31,9 @@
 // vector instructions a step; an operand to a wave, handed on through LDS at the rendezvous that is there, they are 10: linear attention
 // and GLA B4 T4096 H16 K = V = 128, kernel 64.7 -> 62.1 us, whole calls 136.9 -> 133.8 and 196.8 -> 194.8.
 //
+// Addresses are a scalar base and a lane's 32-bit offset, and an output's place is formed once: kernel 62.1 -> 59.0 us for the linear family
+// (its output waves multiplied by H V in the vector unit for each store), 86.2 -> 83.7 for Gated DeltaNet B4 T4096 H16.
+//
 // The linear family keeps two operand sets and at most 128 registers, so that two workgroups fit a compute unit.  With five sets
 // (199 .. 236 registers, one workgroup) 257 to 511 workgroups took two rounds of the chip, the second nearly empty, and lost to the
 // two launches that this one replaces; the second workgroup hides more than the three further sets did.  Linear attention K = V = 128,
@@ -110,6 +113,13 @@ LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
   return __builtin_bit_cast(lq_v8h, lq_v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]});
 }
 
+// 16, 8 or 4 bytes at a lane's offset from a place that is the same for the whole wave: a scalar base and 32 bits of a vector register
+// (with a signed or a 64-bit offset every request forms its 64-bit address in the vector unit)
+template <typename T, typename P>
+LQ_DEV T scan_at(const P* base, uint32_t byte) {
+  return *(const T*)((const char*)base + byte);
+}
+
 // Operand sets in rotation: a set is requested D - 1 steps ahead of its use, and the loop is unrolled by D so that the sets
 // keep their registers.  Its body has no exit in it (what does not fill D steps follows behind): an exit inside merged, in the
 // compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
@@ -182,27 +192,29 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     }
     using Ops = ChainOps<DELTA, K, BV>;
     using URaw = decltype(Ops::uraw);
+    // float of a lane: per-token factors (delta) in lanes 0 .. 31, chunk decays of the wave's carry rows behind
+    const uint32_t misc_at = 4 * (DELTA ? (lane < 32 ? 64 * (lane >> 4) + 16 * wave + (lane & 15) : 128 + KR * wave + min(lane - 32, KR - 1))
+                                        : KR * wave + min(max(lane - 32, 0), KR - 1));
     // part: 0 = everything, 1 = key codes, decays and per-token factors, 2 = state-read codes and U
     auto load_part = [&](auto part_c, int ct, Ops& o) __attribute__((always_inline)) {
       constexpr int part = decltype(part_c)::value;
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
       if constexpr (part == 0 || part == 1) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) o.kop[kt] = *(const lq_v4i*)(p.kqT + (cb * K + KR * wave + 16 * kt + rl) * 64 + 16 * kg);
+        for (int kt = 0; kt < KT; ++kt) o.kop[kt] = scan_at<lq_v4i>(p.kqT + cb * K * 64, (KR * wave + 16 * kt + rl) * 64 + 16 * kg);
         if constexpr (DELTA) {  // fw[64] | ev[64] | gam[K]
-          const float* pk = p.pack + cb * (128 + K);
-          o.misc = *(lane < 32 ? pk + 64 * (lane >> 4) + 16 * wave + (lane & 15) : pk + 128 + KR * wave + min(lane - 32, KR - 1));
+          o.misc = scan_at<float>(p.pack + cb * (128 + K), misc_at);
         } else {
-          o.misc = p.gam[cb * K + KR * wave + min(max(lane - 32, 0), KR - 1)];
+          o.misc = scan_at<float>(p.gam + cb * K, misc_at);
 #pragma unroll
-          for (int vt = 0; vt < VT; ++vt) o.vop[vt] = *(const lq_v4i*)(p.vqT + (cb * V + v0 + 16 * vt + rl) * 64 + 16 * kg);
+          for (int vt = 0; vt < VT; ++vt) o.vop[vt] = scan_at<lq_v4i>(p.vqT + (cb * V + v0) * 64, (16 * vt + rl) * 64 + 16 * kg);
         }
       }
       if constexpr (DELTA && (part == 0 || part == 2)) {
 #pragma unroll
         for (int ks = 0; ks < K / 64; ++ks)
-          o.wop[ks] = *(const lq_v4i*)(p.wq + cb * 64 * K + ((wave * (K / 64) + ks) * 64 + lane) * 16);
-        o.uraw = *(const URaw*)(p.u + cb * 64 * V + zoo_op_U(16 * wave + (lane >> 2), v0 + BV / 4 * (lane & 3)));
+          o.wop[ks] = scan_at<lq_v4i>(p.wq + cb * 64 * K, ((wave * (K / 64) + ks) * 64 + lane) * 16);
+        o.uraw = scan_at<URaw>(p.u + cb * 64 * V + zoo_op_U(0, v0), 2 * zoo_op_U(16 * wave + (lane >> 2), BV / 4 * (lane & 3)));
       }
     };
     float hc[KT][VT][4];
@@ -364,12 +376,17 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     auto load = [&](int ct, Ops& o) __attribute__((always_inline)) {
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
 #pragma unroll
-      for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = *(const lq_v4i*)(p.qc + cb * 64 * K + ((w * (K / 64) + ks) * 64 + lane) * 16);
+      for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = scan_at<lq_v4i>(p.qc + cb * 64 * K, ((w * (K / 64) + ks) * 64 + lane) * 16);
 #pragma unroll
-      for (int js = 0; js < 2; ++js) o.aop[js] = *(const lq_v4i*)(p.A + cb * 4096 + ((w * 2 + js) * 64 + lane) * 8);
-      if constexpr (SCALAR) o.g = *(const lq_v4f*)(p.gpk + cb * 64 + 16 * w + 4 * kg);
+      for (int js = 0; js < 2; ++js) o.aop[js] = scan_at<lq_v4i>(p.A + cb * 4096, ((w * 2 + js) * 64 + lane) * 16);
+      if constexpr (SCALAR) o.g = scan_at<lq_v4f>(p.gpk + cb * 64, 4 * (16 * w + 4 * kg));
     };
     float of[NJ][4];
+    // outputs: elements between tokens, this lane's place in a chunk (once: formed anew for each store, the products by H V took 16 to 25
+    // instructions of a quarter of the rate a step)
+    const int64_t orow = (int64_t)H * V;
+    int64_t olane = (16 * w + 4 * kg) * orow + (int64_t)h * V + v0 + NJ * rl;
+    asm volatile("" : "+v"(olane));
     // state read of chunk ct
     auto read_state = [&](int ct, const Ops& o) __attribute__((always_inline)) {
       const unsigned char* hTb = hT + (DELTA ? 0 : (ct & 1) * BV * HS);
@@ -412,10 +429,10 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
           loc[jj] = lq_mfma_f16(aop, x, loc[jj]);
         }
       }
-      const int64_t t0 = (int64_t)b * T + (int64_t)ct * 64;
+      const int64_t chunk = ((int64_t)b * T + (int64_t)ct * 64) * orow;  // (uniform)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t off = ((t0 + 16 * w + 4 * kg + r) * H + h) * V + v0 + NJ * rl;
+        const int64_t off = chunk + r * orow + olane;
         float res[NJ];
 #pragma unroll
         for (int jj = 0; jj < NJ; ++jj) res[jj] = of[jj][r] + loc[jj][r] * svl_o[jj];
@@ -445,10 +462,12 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     // linear family: the local value codes become fp16 once for all four waves, an operand to a wave (column NJ rl + jj, tokens 32 js + 8 kg
     // .., of jj = w & 1, js = w >> 1; 16 columns: an operand to two of them), a step ahead of their use and requested two
     const int ojj = NJ == 2 ? w & 1 : 0, ojs = w >> 1;
+    const int vcol = zoo_op_values(v0 & ~31, 0);
+    const uint32_t vlane = zoo_op_values((v0 & 31) + NJ * rl + ojj, 8 * kg) + 8 * ojs;
     lq_v2i vraw[2];
     auto load_v = [&](int ct, lq_v2i& o) __attribute__((always_inline)) {
       if constexpr (!DELTA)
-        o = *(const lq_v2i*)(p.vcT + (((int64_t)b * NT + ct) * H + h) * 64 * V + zoo_op_values(v0 + NJ * rl + ojj, 8 * kg) + 8 * ojs);
+        o = scan_at<lq_v2i>(p.vcT + (((int64_t)b * NT + ct) * H + h) * 64 * V + vcol, vlane);
     };
     auto convert_v = [&](int ct, const lq_v2i& raw) __attribute__((always_inline)) {
       if constexpr (!DELTA) *(lq_v8h*)(vL + (ct & 1) * BV * 128 + ((ojj * 2 + ojs) * 64 + lane) * 16) = scan_i8x8_to_f16x8(raw);
