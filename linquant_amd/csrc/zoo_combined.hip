@@ -154,7 +154,7 @@ extern "C" int lq_zoo_simple_gla(const lq_zoo_simple_gla_args* a, hipStream_t st
     s.o = a->o, s.o_is_f32 = a->o_is_f32, s.ht = a->ht;
     s.skw = a->skw, s.svw = a->svw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
     s.qmax = a->qmax, s.bf = bf, s.B = w.B, s.T = w.T, s.H = w.H, s.V = w.V, s.NT = w.NT;
-    return zoo_scan_launch(s, false, a->g != nullptr, a->kdim, stream);
+    return zoo_scan_launch(s, false, decay, a->kdim, stream);
   }
   float* gc = a->g ? (float*)(ws + l.gc) : nullptr;
 
@@ -374,7 +374,7 @@ extern "C" int lq_zoo_chunk_forward(const lq_zoo_chunk_forward_args* a, hipStrea
     s.skw = a->skw, s.svw = a->svw, s.sw = a->sw, s.ss = a->ss, s.sq = a->sq, s.svl = a->svl;
     s.qmax = a->qmax, s.bf = a->act_dtype == LQ_DT_BF16;
     s.B = a->batch, s.T = a->seqlen, s.H = a->nheads, s.V = a->vdim, s.NT = a->seqlen / 64;
-    return zoo_scan_launch(s, delta, a->decay == LQ_DECAY_SCALAR, a->kdim, stream);
+    return zoo_scan_launch(s, delta, a->decay, a->kdim, stream);
   }
   {
     lq_zoo_state_args s = {};

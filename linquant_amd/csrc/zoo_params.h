@@ -159,7 +159,7 @@ struct ZooScanParams {
   int bf;
   int B, T, H, V, NT;
 };
-int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, hipStream_t stream);
+int zoo_scan_launch(const ZooScanParams& p, bool delta, int decay, int K, hipStream_t stream);  // decay: LQ_DECAY_*
 
 // WY prep, no / scalar decay.  scan (with the write codes and `local`): wq and U in operand order, the codes of q and A, no Hw; its g
 // is not cumulated

@@ -125,8 +125,9 @@ LQ_DEV T scan_at(const P* base, uint32_t byte) {
 // compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
 constexpr int scan_sets(bool delta) { return delta ? 3 : 2; }
 
-template <bool DELTA, bool SCALAR, int K, int BV, bool BF, bool OF32>
+template <bool DELTA, int DECAY, int K, int BV, bool BF, bool OF32>
 __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams p, ScanCuts cuts) {
+  constexpr bool SCALAR = DECAY == LQ_DECAY_SCALAR;
   constexpr int D = scan_sets(DELTA), DU = scan_update_sets(K, BV);
   constexpr int KR = K / 4;        // carry rows per chain wave
   constexpr int KT = K / 64;       // 16-row tiles per chain wave
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
         if constexpr (DELTA) {  // fw[64] | ev[64] | gam[K]
           o.misc = scan_at<float>(p.pack + cb * (128 + K), misc_at);
         } else {
-          o.misc = scan_at<float>(p.gam + cb * K, misc_at);
+          if constexpr (DECAY != LQ_DECAY_NONE) o.misc = scan_at<float>(p.gam + cb * K, misc_at);
 #pragma unroll
           for (int vt = 0; vt < VT; ++vt) o.vop[vt] = scan_at<lq_v4i>(p.vqT + (cb * V + v0) * 64, (16 * vt + rl) * 64 + 16 * kg);
         }
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
 
     // write product and carry update
     auto update = [&](const Ops& cur) __attribute__((always_inline)) {
-      if constexpr (!DELTA) misc_s[lane] = cur.misc;  // (no earlier: with one set in flight the step would start with this wait)
+      if constexpr (!DELTA && DECAY != LQ_DECAY_NONE) misc_s[lane] = cur.misc;  // (no earlier: with one set in flight the step would start with this wait)
 #pragma unroll
       for (int vt = 0; vt < VT; ++vt) {
         lq_v4i bop;
@@ -240,12 +241,14 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
           const lq_v4i a = lq_mfma_i8(cur.kop[kt], bop, lq_v4i{0, 0, 0, 0});
-          const lq_v4f gam4 = *(const lq_v4f*)(misc_s + 32 + 16 * kt + 4 * kg);
+          lq_v4f gam4;
+          if constexpr (DECAY != LQ_DECAY_NONE) gam4 = *(const lq_v4f*)(misc_s + 32 + 16 * kt + 4 * kg);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             float prod = (float)a[r] * skw_r[kt][r];
             prod = prod * svw_c[vt];
-            hc[kt][vt][r] = hc[kt][vt][r] * gam4[r] + prod;
+            if constexpr (DECAY != LQ_DECAY_NONE) hc[kt][vt][r] = hc[kt][vt][r] * gam4[r];  // (no decay: times one)
+            hc[kt][vt][r] = hc[kt][vt][r] + prod;
           }
         }
       }
@@ -531,38 +534,39 @@ ScanCuts scan_cuts(int64_t tiles, int NT, int step) {
   return c;
 }
 
-template <bool DELTA, bool SCALAR, int K, int BV>
+template <bool DELTA, int DECAY, int K, int BV>
 int launch(const ScanParams& p, hipStream_t stream) {
   const int64_t tiles = (int64_t)p.B * p.H * (p.V / BV);
   const ScanCuts cuts = DELTA || tiles > 128 ? ScanCuts{1, {0, p.NT}} : scan_cuts(tiles, p.NT, scan_update_sets(K, BV));
   const dim3 grid(8 * (p.V / BV), (p.B * p.H * cuts.n + 7) / 8), block(512);
   if (DELTA && p.o_is_f32 && p.bf)  // (the linear family reads codes only: the activation dtype is that of the output)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, DELTA, true>), grid, block, 0, stream, p, cuts);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, DECAY, K, BV, DELTA, true>), grid, block, 0, stream, p, cuts);
   else if (p.o_is_f32)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, true>), grid, block, 0, stream, p, cuts);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, DECAY, K, BV, false, true>), grid, block, 0, stream, p, cuts);
   else if (p.bf)
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, true, false>), grid, block, 0, stream, p, cuts);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, DECAY, K, BV, true, false>), grid, block, 0, stream, p, cuts);
   else
-    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, SCALAR, K, BV, false, false>), grid, block, 0, stream, p, cuts);
+    hipLaunchKernelGGL((zoo_scan_kernel<DELTA, DECAY, K, BV, false, false>), grid, block, 0, stream, p, cuts);
   return lq_check_launch();
 }
 
-template <bool DELTA, bool SCALAR, int K>
+template <bool DELTA, int DECAY, int K>
 int launch_bv(const ScanParams& p, hipStream_t stream) {
   const int64_t tiles = (int64_t)p.B * p.H * (p.V / 32);
   // linear family: a tile of 32 columns in more segments is the better use of the same compute units once the chain is long
   const bool few = tiles <= (DELTA || p.NT <= 12 ? 128 : (p.NT <= 32 ? 64 : (p.NT <= 256 ? 42 : 32)));
-  return few ? launch<DELTA, SCALAR, K, 16>(p, stream) : launch<DELTA, SCALAR, K, 32>(p, stream);
+  return few ? launch<DELTA, DECAY, K, 16>(p, stream) : launch<DELTA, DECAY, K, 32>(p, stream);
 }
 
-template <bool DELTA, bool SCALAR>
+template <bool DELTA, int DECAY>
 int launch_k(const ScanParams& p, int K, hipStream_t stream) {
-  return K == 128 ? launch_bv<DELTA, SCALAR, 128>(p, stream) : launch_bv<DELTA, SCALAR, 64>(p, stream);
+  return K == 128 ? launch_bv<DELTA, DECAY, 128>(p, stream) : launch_bv<DELTA, DECAY, 64>(p, stream);
 }
 
 }  // namespace
 
-int zoo_scan_launch(const ZooScanParams& p, bool delta, bool scalar, int K, hipStream_t stream) {
-  if (delta) return scalar ? launch_k<true, true>(p, K, stream) : launch_k<true, false>(p, K, stream);
-  return scalar ? launch_k<false, true>(p, K, stream) : launch_k<false, false>(p, K, stream);
+int zoo_scan_launch(const ZooScanParams& p, bool delta, int decay, int K, hipStream_t stream) {
+  if (decay == LQ_DECAY_NONE) return delta ? launch_k<true, LQ_DECAY_NONE>(p, K, stream) : launch_k<false, LQ_DECAY_NONE>(p, K, stream);
+  if (decay == LQ_DECAY_SCALAR) return delta ? launch_k<true, LQ_DECAY_SCALAR>(p, K, stream) : launch_k<false, LQ_DECAY_SCALAR>(p, K, stream);
+  return delta ? launch_k<true, LQ_DECAY_DIAGONAL>(p, K, stream) : launch_k<false, LQ_DECAY_DIAGONAL>(p, K, stream);
 }
