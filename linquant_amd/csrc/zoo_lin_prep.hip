@@ -81,7 +81,7 @@ LQ_DEV lq_v2i lp_pack8(const int (&c)[8]) {
 }
 
 template <bool SCALAR, int K, bool BF>
-__global__ __launch_bounds__(512, K == 128 ? 6 : 4) void zoo_lin_prep_kernel(ZooLinPrepParams p) {
+__global__ __launch_bounds__(512, 6) void zoo_lin_prep_kernel(ZooLinPrepParams p) {
   constexpr int QS = K == 128 ? 160 : 80;  // bytes per row of the code tiles
   __shared__ __align__(16) unsigned char qI[64 * QS], kI[64 * QS];
   __shared__ __align__(16) uint32_t cK[lp_ct_size(K)], cW[lp_ct_size(128)], cL[lp_ct_size(128)];
@@ -107,16 +107,6 @@ __global__ __launch_bounds__(512, K == 128 ? 6 : 4) void zoo_lin_prep_kernel(Zoo
   const _Float16* src = is_k ? p.k : p.q;
 #pragma unroll
   for (int u = 0; u < 4; ++u) kraw[u] = *(const lq_v4i*)(src + ((t0 + 4 * kq + u) * H + h) * K + 8 * kc);
-  constexpr bool EARLY = K == 64;
-  lq_v4i vraw[4];
-  auto request_v = [&](int vb, int quad, int piece) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * quad + u) * H + h) * V + vb + 8 * piece);
-  };
-  if constexpr (EARLY) {
-    const int vp = min(V, 128) / 8, vt = max(tid - 256, 0);
-    request_v(0, (vt / vp) & 15, vt % vp);
-  }
   // ---- per-token factors
   if (wave == 0) {
     float fk = 1.0f, fv = 1.0f;
@@ -196,7 +186,9 @@ __global__ __launch_bounds__(512, K == 128 ? 6 : 4) void zoo_lin_prep_kernel(Zoo
     const bool vact = (K == 128 || wave >= 4) && vt < 16 * vp;  // (wave-uniform)
     const int vq = (vt / vp) & 15, vc = vt % vp;
     __builtin_amdgcn_sched_barrier(0);  // (requested behind the codes of q and k, whose rows leave their registers)
-    if (!EARLY || vb > 0) request_v(vb, vq, vc);
+    lq_v4i vraw[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * vq + u) * H + h) * V + vb + 8 * vc);
     if (vb > 0) {
       __syncthreads();  // the tiles have been read
       if (tid < 8 * vp) {
