@@ -36,6 +36,20 @@ LQ_DEV uint32_t zoo_pack_h2(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// What lies at a lane's byte offset from a place that is the same for the whole wave: a scalar base and 32 bits of a vector register (with a
+// signed or a 64-bit offset every request forms its 64-bit address in the vector unit)
+template <typename T, typename P>
+LQ_DEV T zoo_at(const P* base, uint32_t byte) {
+  return *(const T*)((const char*)base + byte);
+}
+template <typename T, typename P>
+LQ_DEV void zoo_put(P* base, uint32_t byte, T x) {
+  *(T*)((char*)base + byte) = x;
+}
+// Elements from the first of a chunk's 64 rows of K channels to another: H K is below 2^24 (every entry point asks for B H <= 65535, K <=
+// 128), so the multiplication is one of full rate
+LQ_DEV uint32_t zoo_rows(int rows, int H, int K) { return __umul24((uint32_t)rows, (uint32_t)(H * K)); }
+
 static inline bool zoo_al(const void* q, int n) { return ((uintptr_t)q % n) == 0; }
 
 // exp on the hardware exp2 unit (x * log2(e), then v_exp_f32): the arithmetic tl.exp lowers to in the reference's

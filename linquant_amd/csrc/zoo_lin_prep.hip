@@ -106,12 +106,12 @@ __global__ __launch_bounds__(512, 6) void zoo_lin_prep_kernel(ZooLinPrepParams p
   lq_v4i kraw[4];
   const _Float16* src = is_k ? p.k : p.q;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) kraw[u] = *(const lq_v4i*)(src + ((t0 + 4 * kq + u) * H + h) * K + 8 * kc);
+  for (int u = 0; u < 4; ++u) kraw[u] = zoo_at<lq_v4i>(src + (t0 * H + h) * K, 2 * (zoo_rows(4 * kq + u, H, K) + 8 * kc));
   // ---- per-token factors
   if (wave == 0) {
     float fk = 1.0f, fv = 1.0f;
     if constexpr (SCALAR) {
-      const float gc = zoo_cumsum64(p.g[(t0 + lane) * H + h]);
+      const float gc = zoo_cumsum64(zoo_at<float>(p.g + t0 * H + h, 4 * zoo_rows(lane, H, 1)));
       const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gc), 63)) - gc;
       fk = zoo_exp((1.0f - p.eta) * d), fv = zoo_exp(p.eta * d);
       gs_s[lane] = gc;
@@ -182,13 +182,15 @@ __global__ __launch_bounds__(512, 6) void zoo_lin_prep_kernel(ZooLinPrepParams p
     asm volatile("" : "+v"(own));  // (nothing that follows from it is to wait in registers from in front of the loop on)
     const int tid = own, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, kg = lane >> 4;
     const int vt = K == 128 ? tid : max(tid - 256, 0);
-    const int vp = min(V - vb, 128) / 8;  // 16-byte pieces of a value row
+    const int vsh = V - vb >= 128 ? 4 : 3, vp = 1 << vsh;  // 16-byte pieces of a value row (V is a multiple of 64)
     const bool vact = (K == 128 || wave >= 4) && vt < 16 * vp;  // (wave-uniform)
-    const int vq = (vt / vp) & 15, vc = vt % vp;
+    const int vq = (vt >> vsh) & 15, vc = vt & (vp - 1);
     __builtin_amdgcn_sched_barrier(0);  // (requested behind the codes of q and k, whose rows leave their registers)
     lq_v4i vraw[4];
+    const int64_t vstep = (int64_t)H * V;  // (uniform)
+    const _Float16* const vrow = p.v + (t0 * vstep + (int64_t)h * V + vb) + 4 * vq * vstep + 8 * vc;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 4 * vq + u) * H + h) * V + vb + 8 * vc);
+    for (int u = 0; u < 4; ++u) vraw[u] = *(const lq_v4i*)(vrow + u * vstep);
     if (vb > 0) {
       __syncthreads();  // the tiles have been read
       if (tid < 8 * vp) {
@@ -223,19 +225,19 @@ __global__ __launch_bounds__(512, 6) void zoo_lin_prep_kernel(ZooLinPrepParams p
     }
     __syncthreads();
     if (tid < 32 * vp) {  // four 16-byte pieces per channel (wave-uniform)
-      *(lq_v4i*)(p.vqT + (cb * V + vb) * 64 + 16 * tid) = *(const lq_v4i*)(cW + lp_ct(tid >> 2, 4 * (tid & 3)));
+      zoo_put(p.vqT + (cb * V + vb) * 64, 16 * tid, *(const lq_v4i*)(cW + lp_ct(tid >> 2, 4 * (tid & 3))));
       // operand order: wave w has the even or odd channels of tile w >> 1, tokens 8 kg .. and 32 + 8 kg ..
       const uint32_t* row = cL + lp_ct(32 * (wave >> 1) + 2 * rl + (wave & 1), 2 * kg);
       const lq_v2i lo = *(const lq_v2i*)row, hi = *(const lq_v2i*)(row + 8);
-      *(lq_v4i*)(p.vcT + cb * 64 * V + 64 * vb + 16 * tid) = lq_v4i{lo[0], lo[1], hi[0], hi[1]};
+      zoo_put(p.vcT + cb * 64 * V + 64 * vb, 16 * tid, lq_v4i{lo[0], lo[1], hi[0], hi[1]});
     }
   }
 
   // ---- operands out
   if (tid < 4 * K) {
-    *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(cK + lp_ct(tid >> 2, 4 * (tid & 3)));
+    zoo_put(p.kqT + cb * K * 64, 16 * tid, *(const lq_v4i*)(cK + lp_ct(tid >> 2, 4 * (tid & 3))));
     const int tb = wave / (K / 64), ks = wave % (K / 64);  // 16 tokens x 64 channels
-    *(lq_v4i*)(p.qc + cb * 64 * K + 16 * tid) = *(const lq_v4i*)(qI + (16 * tb + rl) * QS + 64 * ks + 16 * kg);
+    zoo_put(p.qc + cb * 64 * K, 16 * tid, *(const lq_v4i*)(qI + (16 * tb + rl) * QS + 64 * ks + 16 * kg));
   }
   // ---- blocks of A: (0,0) (1,0) (1,1) (2,0) .. (3,3) of the lower triangle, then zeros above it
   const float sqk = p.sq[h] * p.sk[h];
@@ -263,7 +265,7 @@ __global__ __launch_bounds__(512, 6) void zoo_lin_prep_kernel(ZooLinPrepParams p
       }
       out = lq_v2i{(int)zoo_pack_h2(x[0], x[1]), (int)zoo_pack_h2(x[2], x[3])};
     }
-    *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(i, j0)) = out;
+    zoo_put(p.A + cb * 4096, 2 * zoo_op_A(i, j0), out);
   }
 }
 

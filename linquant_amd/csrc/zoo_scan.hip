@@ -113,13 +113,6 @@ LQ_DEV lq_v8h scan_i8x8_to_f16x8(lq_v2i c) {
   return __builtin_bit_cast(lq_v8h, lq_v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]});
 }
 
-// 16, 8 or 4 bytes at a lane's offset from a place that is the same for the whole wave: a scalar base and 32 bits of a vector register
-// (with a signed or a 64-bit offset every request forms its 64-bit address in the vector unit)
-template <typename T, typename P>
-LQ_DEV T scan_at(const P* base, uint32_t byte) {
-  return *(const T*)((const char*)base + byte);
-}
-
 // Operand sets in rotation: a set is requested D - 1 steps ahead of its use, and the loop is unrolled by D so that the sets
 // keep their registers.  Its body has no exit in it (what does not fill D steps follows behind): an exit inside merged, in the
 // compiler's count of outstanding requests, paths that had requested less, and the first step of every trip waited for all.
@@ -202,20 +195,20 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
       if constexpr (part == 0 || part == 1) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) o.kop[kt] = scan_at<lq_v4i>(p.kqT + cb * K * 64, (KR * wave + 16 * kt + rl) * 64 + 16 * kg);
+        for (int kt = 0; kt < KT; ++kt) o.kop[kt] = zoo_at<lq_v4i>(p.kqT + cb * K * 64, (KR * wave + 16 * kt + rl) * 64 + 16 * kg);
         if constexpr (DELTA) {  // fw[64] | ev[64] | gam[K]
-          o.misc = scan_at<float>(p.pack + cb * (128 + K), misc_at);
+          o.misc = zoo_at<float>(p.pack + cb * (128 + K), misc_at);
         } else {
-          if constexpr (DECAY != LQ_DECAY_NONE) o.misc = scan_at<float>(p.gam + cb * K, misc_at);
+          if constexpr (DECAY != LQ_DECAY_NONE) o.misc = zoo_at<float>(p.gam + cb * K, misc_at);
 #pragma unroll
-          for (int vt = 0; vt < VT; ++vt) o.vop[vt] = scan_at<lq_v4i>(p.vqT + (cb * V + v0) * 64, (16 * vt + rl) * 64 + 16 * kg);
+          for (int vt = 0; vt < VT; ++vt) o.vop[vt] = zoo_at<lq_v4i>(p.vqT + (cb * V + v0) * 64, (16 * vt + rl) * 64 + 16 * kg);
         }
       }
       if constexpr (DELTA && (part == 0 || part == 2)) {
 #pragma unroll
         for (int ks = 0; ks < K / 64; ++ks)
-          o.wop[ks] = scan_at<lq_v4i>(p.wq + cb * 64 * K, ((wave * (K / 64) + ks) * 64 + lane) * 16);
-        o.uraw = scan_at<URaw>(p.u + cb * 64 * V + zoo_op_U(0, v0), 2 * zoo_op_U(16 * wave + (lane >> 2), BV / 4 * (lane & 3)));
+          o.wop[ks] = zoo_at<lq_v4i>(p.wq + cb * 64 * K, ((wave * (K / 64) + ks) * 64 + lane) * 16);
+        o.uraw = zoo_at<URaw>(p.u + cb * 64 * V + zoo_op_U(0, v0), 2 * zoo_op_U(16 * wave + (lane >> 2), BV / 4 * (lane & 3)));
       }
     };
     float hc[KT][VT][4];
@@ -379,10 +372,10 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     auto load = [&](int ct, Ops& o) __attribute__((always_inline)) {
       const int64_t cb = ((int64_t)b * NT + ct) * H + h;
 #pragma unroll
-      for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = scan_at<lq_v4i>(p.qc + cb * 64 * K, ((w * (K / 64) + ks) * 64 + lane) * 16);
+      for (int ks = 0; ks < K / 64; ++ks) o.qop[ks] = zoo_at<lq_v4i>(p.qc + cb * 64 * K, ((w * (K / 64) + ks) * 64 + lane) * 16);
 #pragma unroll
-      for (int js = 0; js < 2; ++js) o.aop[js] = scan_at<lq_v4i>(p.A + cb * 4096, ((w * 2 + js) * 64 + lane) * 16);
-      if constexpr (SCALAR) o.g = scan_at<lq_v4f>(p.gpk + cb * 64, 4 * (16 * w + 4 * kg));
+      for (int js = 0; js < 2; ++js) o.aop[js] = zoo_at<lq_v4i>(p.A + cb * 4096, ((w * 2 + js) * 64 + lane) * 16);
+      if constexpr (SCALAR) o.g = zoo_at<lq_v4f>(p.gpk + cb * 64, 4 * (16 * w + 4 * kg));
     };
     float of[NJ][4];
     // outputs: elements between tokens, this lane's place in a chunk (once: formed anew for each store, the products by H V took 16 to 25
@@ -470,7 +463,7 @@ __global__ __launch_bounds__(512, DELTA ? 2 : 4) void zoo_scan_kernel(ScanParams
     lq_v2i vraw[2];
     auto load_v = [&](int ct, lq_v2i& o) __attribute__((always_inline)) {
       if constexpr (!DELTA)
-        o = scan_at<lq_v2i>(p.vcT + (((int64_t)b * NT + ct) * H + h) * 64 * V + vcol, vlane);
+        o = zoo_at<lq_v2i>(p.vcT + (((int64_t)b * NT + ct) * H + h) * 64 * V + vcol, vlane);
     };
     auto convert_v = [&](int ct, const lq_v2i& raw) __attribute__((always_inline)) {
       if constexpr (!DELTA) *(lq_v8h*)(vL + (ct & 1) * BV * 128 + ((ojj * 2 + ojs) * 64 + lane) * 16) = scan_i8x8_to_f16x8(raw);

@@ -133,25 +133,27 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
   constexpr int KP = K / 8;  // 16-byte pieces of a key row
   const int krp = tid / KP, kc = tid % KP;
   const bool kact = K == 128 || tid < 256;
-  const int vp = min(V, 128) / 8;  // pieces of a value row per pass
-  const int vrp = tid / vp, vc8 = tid % vp;
+  const int vsh = V >= 128 ? 4 : 3;  // (V is a multiple of 64: 16 or 8 pieces of a value row per pass)
+  const int vrp = tid >> vsh, vc8 = tid & ((1 << vsh) - 1);
   const bool vact = vrp < 32;
   lq_v4i kraw[2], qraw[2], vraw[2];
+  const int64_t head = (t0 * H + h) * K, vstep = (int64_t)H * V;  // (uniform)
+  const _Float16* const vrow = p.v + (t0 * vstep + (int64_t)h * V) + (vact ? 2 * vrp : 0) * vstep + 8 * vc8;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int64_t row = (t0 + 2 * (kact ? krp : 0) + u) * H + h;
-    kraw[u] = *(const lq_v4i*)(p.k + row * K + 8 * kc);
-    if constexpr (SCAN) qraw[u] = *(const lq_v4i*)(p.q + row * K + 8 * kc);
-    vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * (vact ? vrp : 0) + u) * H + h) * V + 8 * vc8);
+    const uint32_t at = 2 * (zoo_rows(2 * (kact ? krp : 0) + u, H, K) + 8 * kc);
+    kraw[u] = zoo_at<lq_v4i>(p.k + head, at);
+    if constexpr (SCAN) qraw[u] = zoo_at<lq_v4i>(p.q + head, at);
+    vraw[u] = *(const lq_v4i*)(vrow + u * vstep);
   }
   // ---- per-token factors
   if (tid < 64) {
-    const float bt = p.beta[(t0 + tid) * H + h];
+    const float bt = zoo_at<float>(p.beta + t0 * H + h, 4 * zoo_rows(tid, H, 1));
     const float bs = wn_powb(bt, p.sigma);
     const float fwv = wn_powb(bt, (1.0f - p.sigma) * (1.0f - p.tau));
     float gv = 0.0f, gl = 0.0f;
     if constexpr (SCALAR && SCAN) {
-      gv = zoo_cumsum64(p.g[(t0 + tid) * H + h]);
+      gv = zoo_cumsum64(zoo_at<float>(p.g + t0 * H + h, 4 * zoo_rows(tid, H, 1)));
       gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gv), 63));
     } else if constexpr (SCALAR) {
       gv = p.g[(t0 + tid) * H + h], gl = p.g[(t0 + 63) * H + h];
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
         // way than the stored Hw in some of the instantiations, and its code with it)
         hw[d] = (int)zoo_enc2(zoo_mul_rn(bw, x0), zoo_mul_rn(bw, x1), bf);
       }
-      if constexpr (!SCAN) *(lq_v4i*)(p.Hw + ((t0 + t) * H + h) * K + 8 * kc) = hw;
+      if constexpr (!SCAN) zoo_put(p.Hw + head, 2 * (zoo_rows(t, H, K) + 8 * kc), hw);
       if constexpr (CODES) {
         int ck[8], cq[8];
 #pragma unroll
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
 
   // ---- the write codes leave as whole rows
   if constexpr (CODES) {
-    if (tid < K * 4) *(lq_v4i*)(p.kqT + cb * K * 64 + 16 * tid) = *(const lq_v4i*)(cT + wn_ct(tid >> 2, 16 * (tid & 3)));
+    if (tid < K * 4) zoo_put(p.kqT + cb * K * 64, 16 * tid, *(const lq_v4i*)(cT + wn_ct(tid >> 2, 16 * (tid & 3))));
   }
   // ---- Gram blocks (tasks 0..9) and, MODE_SCAN, A blocks (tasks 10..19): task t belongs to wave t % 8
   // block n of the lower triangle: (0,0) (1,0) (1,1) (2,0) (2,1) (2,2) (3,0) ..
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
         if (SCALAR) x[r] = x[r] * zoo_exp(gs_s[i] - gs_s[j0 + r]);
         x[r] = j0 + r <= i ? x[r] : 0.0f;
       }
-      *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(i, j0)) = lq_v2i{(int)zoo_pack_h2(x[0], x[1]), (int)zoo_pack_h2(x[2], x[3])};
+      zoo_put(p.A + cb * 4096, 2 * zoo_op_A(i, j0), lq_v2i{(int)zoo_pack_h2(x[0], x[1]), (int)zoo_pack_h2(x[2], x[3])});
     }
     // zero blocks above the diagonal (waves 4 .. 7, which have a task less) and the codes of q, operand by operand (waves 0 .. 3)
     if (wave >= 4) {
@@ -294,12 +296,12 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
         const int n = wave - 4 + 4 * s;  // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
         if (n >= 6) continue;
         const int I = n < 3 ? 0 : (n < 5 ? 1 : 2), J = n < 3 ? n + 1 : (n < 5 ? n - 1 : 3);
-        *(lq_v2i*)(p.A + cb * 4096 + zoo_op_A(16 * I + rl, 16 * J + 4 * kg)) = lq_v2i{0, 0};
+        zoo_put(p.A + cb * 4096, 2 * zoo_op_A(16 * I + rl, 16 * J + 4 * kg), lq_v2i{0, 0});
       }
     } else {
 #pragma unroll
       for (int ks = 0; ks < K / 64; ++ks)
-        *(lq_v4i*)(p.qc + cb * 64 * K + ((wave * (K / 64) + ks) * 64 + lane) * 16) = *(const lq_v4i*)(qI + (16 * wave + rl) * QS + 64 * ks + 16 * kg);
+        zoo_put(p.qc + cb * 64 * K, ((wave * (K / 64) + ks) * 64 + lane) * 16, *(const lq_v4i*)(qI + (16 * wave + rl) * QS + 64 * ks + 16 * kg));
     }
   }
   __syncthreads();  // raw keys, codes and transposed codes are dead
@@ -450,21 +452,21 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
     lq_v2i o;
     o[0] = (int)zoo_enc2(a[0] * un, a[1] * un, bf);
     o[1] = (int)zoo_enc2(a[2] * un, a[3] * un, bf);
-    const int64_t woff = ((t0 + 16 * I + rl) * H + h) * K + 16 * nt + 4 * kg;
-    if (!SCAN && (!CODES || p.W)) *(lq_v2i*)(p.W + woff) = o;
+    const uint32_t wat = zoo_rows(16 * I + rl, H, K) + 16 * nt + 4 * kg;  // (token-major forms)
+    if (!SCAN && (!CODES || p.W)) zoo_put(p.W + head, 2 * wat, o);
     if constexpr (CODES) {  // state-read codes of the rounded W
       float w0, w1, w2, w3;
       zoo_dec2((uint32_t)o[0], bf, w0, w1);
       zoo_dec2((uint32_t)o[1], bf, w2, w3);
-      *(uint32_t*)(SCAN ? p.wq + cb * 64 * K + zoo_op_codes(16 * I + rl, 16 * nt + 4 * kg, K) : p.wq + woff) =
-          zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax), zoo_q8(w3, inv_sw, qmax));
+      zoo_put(p.wq + (SCAN ? cb * 64 * K : head), SCAN ? (uint32_t)zoo_op_codes(16 * I + rl, 16 * nt + 4 * kg, K) : wat,
+              zoo_pack_codes(zoo_q8(w0, inv_sw, qmax), zoo_q8(w1, inv_sw, qmax), zoo_q8(w2, inv_sw, qmax), zoo_q8(w3, inv_sw, qmax)));
     }
   }
   if constexpr (SCALAR) t_pieces(bs_s, t, un);  // (no decay: W and U share T . diag(bs))
   for (int vb = 0; vb < V; vb += 128) {  // passes of up to 128 value columns
     if (vb > 0 && vact && vc8 < min(V - vb, 128) / 8) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(p.v + ((t0 + 2 * vrp + u) * H + h) * V + vb + 8 * vc8);
+      for (int u = 0; u < 2; ++u) vraw[u] = *(const lq_v4i*)(vrow + u * vstep + vb);
     }
     __syncthreads();  // the tile has been read
     if (vact && vc8 < min(V - vb, 128) / 8) stage(vraw, vc8, vrp);
@@ -476,8 +478,10 @@ __global__ __launch_bounds__(512, 6) void zoo_wy_ns_kernel(ZooWyParams p) {
       lq_v2i o;
       o[0] = (int)zoo_enc2(a[0] * un, a[1] * un, bf);
       o[1] = (int)zoo_enc2(a[2] * un, a[3] * un, bf);
-      *(lq_v2i*)(SCAN ? p.U + cb * 64 * V + zoo_op_U(16 * I + rl, vb + 16 * nt + 4 * kg)
-                      : p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
+      if constexpr (SCAN)
+        zoo_put(p.U + cb * 64 * V + zoo_op_U(0, vb), 2 * zoo_op_U(16 * I + rl, 16 * nt + 4 * kg), o);
+      else
+        *(lq_v2i*)(p.U + ((t0 + 16 * I + rl) * H + h) * V + vb + 16 * nt + 4 * kg) = o;
     }
   }
 }
