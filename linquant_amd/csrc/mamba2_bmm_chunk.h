@@ -38,6 +38,7 @@ struct BmmParams {
   int seqlen, G, Q, nchunks;
   uint32_t tiles_magic, g_magic, tpc, tpc_magic, ncg, ncg_magic;
   int by_xcd;
+  int causal;      // only the tiles on and below the diagonal
   uint32_t tiles;  // in all
 };
 
@@ -54,8 +55,14 @@ LQ_DEV void bmm_chunk_tile(const BmmParams& p, uint32_t x, uint32_t j, int lane)
   // a unit's tiles run on one XCD, one after the other.
   const uint32_t uh = p.tpc_magic ? __umulhi(j, p.tpc_magic) : j;
   const uint32_t tile = j - uh * p.tpc, unit = p.by_xcd ? uh * 8u + x : uh;
-  const int mt64 = p.tiles_magic ? (int)__umulhi(tile, p.tiles_magic) : (int)tile;
-  const int kt64 = (int)tile - mt64 * (Q >> 6);
+  int mt64, kt64;
+  if (p.causal) {  // (wave-uniform, at most eight rows of tiles)
+    mt64 = 0, kt64 = (int)tile;
+    while (kt64 > mt64) kt64 -= ++mt64;
+  } else {
+    mt64 = p.tiles_magic ? (int)__umulhi(tile, p.tiles_magic) : (int)tile;
+    kt64 = (int)tile - mt64 * (Q >> 6);
+  }
   const int b = p.ncg_magic ? (int)__umulhi(unit, p.ncg_magic) : (int)unit;
   const uint32_t cg = unit - (uint32_t)b * p.ncg;
   const int c = p.g_magic ? (int)__umulhi(cg, p.g_magic) : (int)cg;
@@ -140,8 +147,8 @@ LQ_DEV void bmm_chunk_tile(const BmmParams& p, uint32_t x, uint32_t j, int lane)
 
 inline bool bmm_al(const void* q, int n) { return ((uintptr_t)q % n) == 0; }
 
-// Parameters of a call, or the reason to refuse it
-inline int bmm_plan(const lq_bmm_chunk_args* a, BmmParams* p) {
+// Parameters of a call (causal: for a caller that reads nothing above the diagonal tiles), or the reason to refuse it
+inline int bmm_plan(const lq_bmm_chunk_args* a, BmmParams* p, bool causal = false) {
   if (!a || !a->a || !a->b || !a->a_scale || !a->b_scale || !a->cb_scale || !a->out) return LQ_ERR_NULL;
   if (a->batch <= 0 || a->seqlen <= 0 || a->ngroups <= 0 || a->batch > 65535) return LQ_ERR_SHAPE;
   const int Q = a->chunk_size, N = a->dstate;
@@ -159,14 +166,14 @@ inline int bmm_plan(const lq_bmm_chunk_args* a, BmmParams* p) {
   if ((int64_t)nchunks * a->ngroups > 65535) return LQ_ERR_SHAPE;
   const uint32_t shift = Q == 64 ? 0u : (uint32_t)(0x100000000ull / (uint32_t)(Q / 64)) + 1u;  // tiles per row, as a multiplier
   const uint32_t g_magic = a->ngroups == 1 ? 0u : (uint32_t)(0x100000000ull / (uint32_t)a->ngroups) + 1u;
-  const uint32_t tpc = (uint32_t)((Q / 64) * (Q / 64)), ncg = (uint32_t)(nchunks * a->ngroups);
+  const uint32_t tpc = (uint32_t)(causal ? (Q / 64) * (Q / 64 + 1) / 2 : (Q / 64) * (Q / 64)), ncg = (uint32_t)(nchunks * a->ngroups);
   const uint64_t units = (uint64_t)a->batch * ncg, total = units * tpc;
   if (total >= (1ull << 31) || total * tpc >= (1ull << 32) || units * ncg >= (1ull << 32)) return LQ_ERR_SHAPE;
   auto magic = [](uint32_t d) { return d == 1 ? 0u : (uint32_t)(0x100000000ull / d) + 1u; };
   const int by_xcd = units % 8 == 0;
   *p = BmmParams{a->a, a->a_stride_b, a->a_stride_l, a->a_stride_g, a->b, a->b_stride_b, a->b_stride_l, a->b_stride_g, a->a_scale,
                  a->b_scale, a->cb_scale, a->out, a->seqlen, a->ngroups, Q, nchunks, shift, g_magic, tpc, magic(tpc), ncg, magic(ncg),
-                 by_xcd, (uint32_t)total};
+                 by_xcd, causal, (uint32_t)total};
   return LQ_OK;
 }
 

@@ -66,31 +66,31 @@ LQ_DEV void chunk_cumsum_fixed(const CumsumParams& p, uint32_t block, float* til
   constexpr int Q = 64 * E, NIT = Q * kHG / (kWaves * 64);
   const Where wh = where(block, p.hg, p.nchunks, p.by_xcd);
   const int h0 = wh.h0, c = wh.c, b = wh.b;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int limit = min(Q, p.seqlen - c * Q);
   // ---- requests: the (token, head) tile (consecutive lanes read consecutive heads of one token; positions past the
   // sequence end or the last head re-read a valid neighbour and are zeroed below), then the per-head constants
+  // The tile's first element is a scalar; a lane's offset from it fits 32 bits in bytes and its factors 24 (cumsum_fixed_e), a multiply of
+  // full rate: 64-bit products for each request were 47 vector instructions of a quarter of it.
   float raw[NIT];
-  int64_t offs[NIT];
+  uint32_t offs[NIT];
+  const int64_t first = (int64_t)b * p.sdt_b + (int64_t)c * Q * p.sdt_l + (int64_t)h0 * p.sdt_h;
+  const uint32_t hoff = __umul24((uint32_t)min(tid % kHG, p.nheads - 1 - h0), (uint32_t)p.sdt_h);
 #pragma unroll
-  for (int i = 0; i < NIT; ++i) {
-    const int it = tid + i * kWaves * 64;
-    const int pos = min(it / kHG, limit - 1), hh = min(it % kHG, p.nheads - 1 - h0);
-    offs[i] = (int64_t)b * p.sdt_b + (int64_t)(c * Q + pos) * p.sdt_l + (int64_t)(h0 + hh) * p.sdt_h;
-  }
+  for (int i = 0; i < NIT; ++i) offs[i] = __umul24((uint32_t)min((tid + i * kWaves * 64) / kHG, limit - 1), (uint32_t)p.sdt_l) + hoff;
   if (p.dt_dtype == LQ_DT_F16) {  // one uniform branch around all requests of a dtype, not one per request
     _Float16 r[NIT];
 #pragma unroll
-    for (int i = 0; i < NIT; ++i) r[i] = ((const _Float16*)p.dt_in)[offs[i]];
+    for (int i = 0; i < NIT; ++i) r[i] = *(const _Float16*)((const char*)((const _Float16*)p.dt_in + first) + 2u * offs[i]);
 #pragma unroll
     for (int i = 0; i < NIT; ++i) raw[i] = (float)r[i];
   } else if (p.dt_dtype == LQ_DT_F32) {
 #pragma unroll
-    for (int i = 0; i < NIT; ++i) raw[i] = ((const float*)p.dt_in)[offs[i]];
+    for (int i = 0; i < NIT; ++i) raw[i] = *(const float*)((const char*)((const float*)p.dt_in + first) + 4u * offs[i]);
   } else {
     int8_t r[NIT];
 #pragma unroll
-    for (int i = 0; i < NIT; ++i) r[i] = ((const int8_t*)p.dt_in)[offs[i]];
+    for (int i = 0; i < NIT; ++i) r[i] = *((const int8_t*)p.dt_in + first + offs[i]);
 #pragma unroll
     for (int i = 0; i < NIT; ++i) raw[i] = (float)r[i];
   }
@@ -140,15 +140,18 @@ LQ_DEV void chunk_cumsum_fixed(const CumsumParams& p, uint32_t block, float* til
     }
     float ex = __shfl_up(t, 1, 64);
     if (lane == 0) ex = 0.0f;
-    const int64_t base = (((int64_t)b * p.nheads + h) * p.nchunks + c) * Q + lane * E;
+    const int64_t base = (((int64_t)b * p.nheads + h) * p.nchunks + c) * Q;
+    char* const dto = (char*)(p.dt_out + base);
+    char* const dAo = (char*)(p.dA_cs + base);
+    const uint32_t at = 4u * E * lane;
     if constexpr (E == 4) {
-      *(lq_v4f*)(p.dt_out + base) = lq_v4f{dtv[0], dtv[1], dtv[2], dtv[3]};
-      *(lq_v4f*)(p.dA_cs + base) = lq_v4f{ex + pre[0], ex + pre[1], ex + pre[2], ex + pre[3]};
+      *(lq_v4f*)(dto + at) = lq_v4f{dtv[0], dtv[1], dtv[2], dtv[3]};
+      *(lq_v4f*)(dAo + at) = lq_v4f{ex + pre[0], ex + pre[1], ex + pre[2], ex + pre[3]};
     } else {
 #pragma unroll
       for (int i = 0; i < E; ++i) {
-        p.dt_out[base + i] = dtv[i];
-        p.dA_cs[base + i] = ex + pre[i];
+        *(float*)(dto + (at + 4u * i)) = dtv[i];
+        *(float*)(dAo + (at + 4u * i)) = ex + pre[i];
       }
     }
   }
@@ -178,6 +181,9 @@ inline int cumsum_plan(const lq_chunk_cumsum_args* a, CumsumParams* p, uint32_t*
 inline int cumsum_fixed_e(const lq_chunk_cumsum_args* a) {
   const int Q = a->chunk_size;
   const bool vec_ok = ((uintptr_t)a->dt_out % 16 == 0) && ((uintptr_t)a->dA_cumsum % 16 == 0);
+  // lane offsets of the tile: 24-bit factors, 32 bits of bytes
+  const int64_t sl = a->dt_stride_l, sh = a->dt_stride_h;
+  if (sl < 0 || sh < 0 || sl >= (1 << 24) || sh >= (1 << 24) || (Q - 1) * sl + (kHG - 1) * sh >= (1ll << 30)) return 0;
   return Q == 64 || Q == 128 || Q == 512 || (Q == 256 && vec_ok) ? Q / 64 : 0;
 }
 

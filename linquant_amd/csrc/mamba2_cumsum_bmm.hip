@@ -1,7 +1,10 @@
 // Cumulative sum and C.B^T of the Mamba-2 SSD in one launch: neither reads what the other writes, and both are a few microseconds of
 // work behind a launch and a memory round trip.  The first workgroups take the dt tiles (mamba2_cumsum.h, the longer chain), the others
 // one to eight C.B^T tiles each (mamba2_bmm_chunk.h), the bits of the two stand-alone launches.
-// Bound by latency.  Kernel us, two launches -> one: B1 L512 H80 6.4 + 5.9 -> 6.4, B3 L5000 H80 11.0 + 7.5 -> 13.2, B4 L2048 H80
+// The scan reads nothing above the diagonal 64 x 64 tiles of C.B^T: those (6 of 16 at 256-token chunks) are not formed here.  With them, and
+// with 64-bit lane offsets for dt (mamba2_cumsum.h): B4 L8192 H80 whole call 253.2 -> 252 us, B3 L5000 H80 193.6 -> 192.2, B8 L2048 H64
+// value side 138.8 -> 137.7.
+// Bound by latency.  Kernel us before that, two launches -> one: B1 L512 H80 6.4 + 5.9 -> 6.4, B3 L5000 H80 11.0 + 7.5 -> 13.2, B4 L2048 H80
 // 7.0 + 6.0 -> 8.3, B8 L2048 H64 value side 7.1 + 6.0 -> 9.8, B4 L8192 H80 12.6 + 10.2 -> 19.6 .. 22.7.
 #include "mamba2_bmm_chunk.h"
 #include "mamba2_cumsum.h"
@@ -50,7 +53,7 @@ int lq_cumsum_bmm(const lq_chunk_cumsum_args* cs, const lq_bmm_chunk_args* bm, h
   BmmParams b;
   uint32_t cblocks;
   int rc;
-  if ((rc = cumsum_plan(cs, &c, &cblocks)) != LQ_OK || (rc = bmm_plan(bm, &b)) != LQ_OK) return rc;
+  if ((rc = cumsum_plan(cs, &c, &cblocks)) != LQ_OK || (rc = bmm_plan(bm, &b, true)) != LQ_OK) return rc;
   const int E = cumsum_fixed_e(cs), N64 = bm->dstate / 64;
   const uint32_t cpad = (cblocks + 7u) / 8u * 8u;
   // as few tiles to a workgroup as keep everything in the 512 places of one round (two workgroups per compute unit): 32 tiles eight to
