@@ -145,9 +145,10 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(Params p) {
   float rmv[4];
   {
     const float* rmp = elide ? p.rowmax + ((int64_t)b * p.seqlen + (int64_t)c * Q) * p.G + g : p.dt + cs;
-    const int rstride = elide ? p.G : 0;
+    const uint32_t rstride = elide ? p.G : 0;  // (24 bits, as the token)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rmv[i] = rmp[(int64_t)min(max(64 * (nslab_all - 2 - i), 0) + lane, limit - 1) * rstride];
+    for (int i = 0; i < 4; ++i)
+      rmv[i] = *(const float*)((const char*)rmp + 4u * __umul24((uint32_t)min(max(64 * (nslab_all - 2 - i), 0) + lane, limit - 1), rstride));
   }
   const float bs_t = KEYSIDE ? 0.0f : p.bscale_g[(int64_t)g * p.sbs_g];
 
@@ -184,15 +185,26 @@ __global__ __launch_bounds__(256, 2) void chunk_state_kernel(Params p) {
   }
   auto load_slab = [&](int k0, lq_v2i (&xr)[4], lq_v4i (&br)[4]) {
     const uint32_t xk = (uint32_t)(k0 * sxl) * 2u, bk = (uint32_t)(k0 * bst);  // scalar
+    uint32_t ox[4], ob[4];
+    if (ragged) {  // (one branch around all of them: a select per request became a branch in front of each)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        ox[t] = (uint32_t)__mul24(min(k0 + 4 * kqx + t, last), sxl) * 2u + xlane;
+        ob[t] = (uint32_t)__mul24(min(k0 + 4 * kqb + t, last), bst) + blane;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ox[t] = xo[t] + xk, ob[t] = bo4[t] + bk;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(ox[t]), "+v"(ob[t]));
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const uint32_t ox = ragged ? (uint32_t)__mul24(min(k0 + 4 * kqx + t, last), sxl) * 2u + xlane : xo[t] + xk;
-      const uint32_t ob = ragged ? (uint32_t)__mul24(min(k0 + 4 * kqb + t, last), bst) + blane : bo4[t] + bk;
-      xr[t] = *(const lq_v2i*)((const char*)xg + ox);
+      xr[t] = *(const lq_v2i*)((const char*)xg + ox[t]);
       if (KEYSIDE) {
-        br[t] = *(const lq_v4i*)(bg0 + ob);
+        br[t] = *(const lq_v4i*)(bg0 + ob[t]);
       } else {
-        const lq_v2i v = *(const lq_v2i*)(bg0 + ob);
+        const lq_v2i v = *(const lq_v2i*)(bg0 + ob[t]);
         br[t][0] = v[0], br[t][1] = v[1];
       }
     }
