@@ -68,7 +68,8 @@ LQ_DEV void arrived(lq_v4i& v) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"m
 // IT = 16-byte pieces per lane (g <= 4 IT); NT = 16-column tiles of had, KS = 32-chunk contraction steps that follow
 // NORM: gate + RMSNorm in front; QHAD: Hadamard + INT8 behind (false: the kernel ends after storing the normalized row)
 // GATE: z is given; EXACT: g = 4 IT, every lane owns IT whole pieces and no access needs a guard
-template <int IT, bool NORM, bool QHAD, bool GATE, bool EXACT>
+// W32: the weight is fp32 (else fp16; a select per element of both forms cost two of its 30 instructions)
+template <int IT, bool NORM, bool QHAD, bool GATE, bool EXACT, bool W32>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(IT <= 10 ? 3 : 2, IT <= 10 ? 3 : 2))) void epilogue_kernel(
     EpiParams p) {
   constexpr int kIt = IT, NT = (IT + 3) / 4, KS = (IT + 7) / 8;
@@ -182,21 +183,17 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(IT 
       }
       __syncthreads();
     }
-    // Weights without a branch on their dtype (a load inside a branch is waited for inside it: one memory round trip per
-    // piece): two 16-byte requests per piece, the whole fp16 piece twice or the two halves of the fp32 piece, and a
-    // select per element.  (float)h * f rounds once either way, so both dtypes share y = (a * rstd) * w.
-    const bool wf32 = p.weight_f32;
+    // (float)h * f rounds once either way, so both weight dtypes share y = (a * rstd) * w
     const char* wbase = (const char*)p.weight;
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
-      const char* wp = wbase + (int64_t)pcc[it] * (wf32 ? 32 : 16);
+      const char* wp = wbase + (uint32_t)pcc[it] * (W32 ? 32u : 16u);
       const lq_v4i wa = *(const lq_v4i*)wp;
-      const lq_v4i wb = *(const lq_v4i*)(wp + (wf32 ? 16 : 0));
+      const lq_v4i wb = W32 ? *(const lq_v4i*)(wp + 16) : wa;
       const lq_v8h wh = __builtin_bit_cast(lq_v8h, wa);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float w32 = __int_as_float(e < 4 ? wa[e & 3] : wb[e & 3]);
-        const float w = wf32 ? w32 : (float)wh[e];
+        const float w = W32 ? __int_as_float(e < 4 ? wa[e & 3] : wb[e & 3]) : (float)wh[e];
         float y = (gated(it, e) * rstd[it]) * w;
         asm("" : "+v"(y));  // keeps the fp32 rounding of the product: no multiply fused into the fp16 conversion
         xv[it][e] = (_Float16)y;
@@ -349,14 +346,14 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(IT 
 
 bool al(const void* q, int n) { return ((uintptr_t)q % n) == 0; }
 
-template <bool NORM, bool QHAD, bool GATE>
-int launch(const EpiParams& p, hipStream_t stream) {
+template <bool NORM, bool QHAD, bool GATE, bool W32>
+int launch_as(const EpiParams& p, hipStream_t stream) {
   const int g = p.g, g8 = (g + 7) & ~7;
   const size_t lds = QHAD || (NORM && p.dim / p.group_size > 1) ? (size_t)kWaves * g8 * kLS * 2 : 0;
   const dim3 grid((unsigned)((p.rows + kWaves - 1) / kWaves)), block(64 * kWaves);
 #define LQ_EPI_LAUNCH_(IT_, EX_)                                                                                  \
   do {                                                                                                            \
-    auto kern = &epilogue_kernel<IT_, NORM, QHAD, GATE, EX_>;                                                     \
+    auto kern = &epilogue_kernel<IT_, NORM, QHAD, GATE, EX_, W32>;                                                \
     if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                                   \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)   \
       return LQ_ERR_LAUNCH;                                                                                       \
@@ -376,6 +373,14 @@ int launch(const EpiParams& p, hipStream_t stream) {
 #undef LQ_EPI_EXACT
 #undef LQ_EPI_LAUNCH_
   return lq_check_launch();
+}
+
+template <bool NORM, bool QHAD, bool GATE>
+int launch(const EpiParams& p, hipStream_t stream) {
+  if constexpr (NORM) {
+    if (p.weight_f32) return launch_as<NORM, QHAD, GATE, true>(p, stream);
+  }
+  return launch_as<NORM, QHAD, GATE, false>(p, stream);
 }
 
 int check_row_tensor(const void* x, int64_t stride, int dim) {

@@ -54,11 +54,11 @@ __global__ __launch_bounds__(256) void fp16_to_int8_kernel(const _Float16* __res
 
 constexpr int kTL = 16;  // tokens per thread: the W-1 halo rows are re-read once per 16 outputs
 
-template <int W>
+template <int W, bool SILU>
 __global__ __launch_bounds__(256) void causal_conv1d_kernel(const _Float16* __restrict__ x, int64_t sx_b, int64_t sx_l,
                                                             const _Float16* __restrict__ weight,
                                                             const _Float16* __restrict__ bias, _Float16* __restrict__ out,
-                                                            int L, int D, int silu) {
+                                                            int L, int D) {
   const int c8n = D >> 3;
   const int idx = blockIdx.x * 256 + threadIdx.x;  // (token block, channel group), channel groups fastest
   const int cg = idx % c8n, tb = idx / c8n;
@@ -74,18 +74,19 @@ __global__ __launch_bounds__(256) void causal_conv1d_kernel(const _Float16* __re
 #pragma unroll
   for (int j = 0; j < W; ++j) wraw[j] = *(const lq_v8h*)(weight + (int64_t)c * W + 8 * j);
   const lq_v8h braw = *(const lq_v8h*)(bias ? bias + c : weight + (int64_t)c * W);
-  const _Float16* xp = x + (int64_t)b * sx_b + c;
+  // rows from one 64-bit product by sums: a product for each of the rows and stores was 35 of them, at a quarter of the rate
+  const _Float16* xp = x + (int64_t)b * sx_b + (int64_t)t0 * sx_l + c;
   lq_v8h halo[W - 1];
 #pragma unroll
-  for (int j = 0; j < W - 1; ++j) halo[j] = *(const lq_v8h*)(xp + (int64_t)max(t0 - (W - 1) + j, 0) * sx_l);
-  _Float16* op = out + ((int64_t)b * L) * D + c;
+  for (int j = 0; j < W - 1; ++j) halo[j] = *(const lq_v8h*)(xp - (t0 > 0 ? (W - 1 - j) * sx_l : 0));  // (a block is longer than the halo)
+  _Float16* op = out + ((int64_t)b * L + t0) * D + c;
   // all rows of the block are requested before the first one is used (the clamped row index keeps a ragged last block
   // inside the sequence; its surplus rows are computed and not stored)
   lq_v8h rows[kTL];
 #pragma unroll
   for (int i = 0; i < kTL; ++i) {
-    const int t = t0 + i < L ? t0 + i : L - 1;
-    rows[i] = *(const lq_v8h*)(xp + (int64_t)t * sx_l);
+    if (i > 0) xp += t0 + i < L ? sx_l : 0;
+    rows[i] = *(const lq_v8h*)xp;
   }
   float w[W][8], bv[8];
 #pragma unroll
@@ -115,10 +116,11 @@ __global__ __launch_bounds__(256) void causal_conv1d_kernel(const _Float16* __re
       float a = bv[e];
 #pragma unroll
       for (int j = 0; j < W; ++j) a = a + w[j][e] * win[j][e];
-      if (silu) a = a * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896340736f));
+      if constexpr (SILU) a = a * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896340736f));
       o[e] = (_Float16)a;
     }
-    if (t < L) __builtin_nontemporal_store(o, (lq_v8h*)(op + (int64_t)t * D));
+    if (t < L) __builtin_nontemporal_store(o, (lq_v8h*)op);
+    op += D;
   }
 }
 
@@ -154,10 +156,9 @@ extern "C" int lq_causal_conv1d(const lq_causal_conv1d_args* a, hipStream_t stre
   const _Float16* wt = (const _Float16*)a->weight;
   const _Float16* bs = (const _Float16*)a->bias;
   _Float16* out = (_Float16*)a->out;
-  switch (a->width) {
-    case 2: hipLaunchKernelGGL(causal_conv1d_kernel<2>, grid, dim3(256), 0, stream, x, a->x_stride_b, a->x_stride_l, wt, bs, out, a->seqlen, a->dim, a->silu); break;
-    case 3: hipLaunchKernelGGL(causal_conv1d_kernel<3>, grid, dim3(256), 0, stream, x, a->x_stride_b, a->x_stride_l, wt, bs, out, a->seqlen, a->dim, a->silu); break;
-    default: hipLaunchKernelGGL(causal_conv1d_kernel<4>, grid, dim3(256), 0, stream, x, a->x_stride_b, a->x_stride_l, wt, bs, out, a->seqlen, a->dim, a->silu); break;
-  }
+  auto kernel = a->width == 2 ? (a->silu ? causal_conv1d_kernel<2, true> : causal_conv1d_kernel<2, false>)
+                              : (a->width == 3 ? (a->silu ? causal_conv1d_kernel<3, true> : causal_conv1d_kernel<3, false>)
+                                               : (a->silu ? causal_conv1d_kernel<4, true> : causal_conv1d_kernel<4, false>));
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, a->x_stride_b, a->x_stride_l, wt, bs, out, a->seqlen, a->dim);
   return lq_check_launch();
 }
