@@ -12,7 +12,7 @@
 // HBM-bound byte work, no matrix core needed.  A row is spread over N/8 lanes, 8 contiguous channels
 // (16 bytes) per lane; butterfly stages 1,2,4 run in registers, the rest through wave shuffles, in the
 // fixed order 1,2,4,...,BS/2 and then the H2 step across the halves.
-#include "lq_common.h"
+#include "zoo_common.h"
 #include "../../include/linquant_hip.h"
 
 namespace {
@@ -30,6 +30,34 @@ LQ_DEV float load_sign(const void* s, int64_t i, int dtype) {
   return (float)((const int8_t*)s)[i];
 }
 
+// value of lane ^ M: up to 8 by lane permutations of the vector unit, further through the LDS crossbar.  (All of them through the crossbar,
+// 40 a lane, SSD calls of N = 128 took 1 to 2 us longer: B4 L8192 259.3 -> 257.5, B8 L2048 139.3 -> 138.0.)
+template <int M>
+LQ_DEV float lane_xor(float v) {
+  if constexpr (M <= 8) return zoo_lane_xor<M>(v);
+  return __shfl_xor(v, M, 64);
+}
+// butterflies across lanes M, 2 M, .. below LIMIT: lanes whose bit is set hold the difference o - v, the others the sum
+template <int M, int LIMIT>
+LQ_DEV void lane_stages(float* v, int sub) {
+  if constexpr (M < LIMIT) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float o = lane_xor<M>(v[i]);
+      v[i] = (sub & M) ? (o - v[i]) : (v[i] + o);
+    }
+    lane_stages<2 * M, LIMIT>(v, sub);
+  }
+}
+template <int M, int LIMIT>
+LQ_DEV float lane_max(float m) {  // a NaN wins
+  if constexpr (M < LIMIT) {
+    const float t = lane_xor<M>(m);
+    return lane_max<2 * M, LIMIT>((t > m || t != t) ? t : m);
+  }
+  return m;
+}
+
 // v[8]: this lane's 8 channels of one row; sub = lane index inside the row (0 .. N/8-1); LPH = lanes per half.
 // Returns the rotated row in place: w * kron for both halves combined by the H2 step.
 template <int LPH>
@@ -43,21 +71,12 @@ LQ_DEV void fwht_row(float* v, int sub, float hb, float kron) {
         v[i] = a + b;
         v[i + h] = a - b;
       }
-#pragma unroll
-  for (int m = 1; m < LPH; m <<= 1)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float o = __shfl_xor(v[i], m, 64);
-      v[i] = (sub & m) ? (o - v[i]) : (v[i] + o);
-    }
+  lane_stages<1, LPH>(v, sub);
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = v[i] * hb;
+  lane_stages<LPH, 2 * LPH>(v, sub);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float o = __shfl_xor(v[i], LPH, 64);
-    const float s = (sub & LPH) ? (o - v[i]) : (v[i] + o);
-    v[i] = s * kron;
-  }
+  for (int i = 0; i < 8; ++i) v[i] = v[i] * kron;
 }
 
 // VEC: signs and dqk are 16-byte aligned, so a lane's eight entries are fetched as whole pieces, requested together with
@@ -143,11 +162,7 @@ __global__ __launch_bounds__(256) void rotate_kernel(const _Float16* __restrict_
       const float a = __builtin_fabsf((float)(_Float16)v[i]);
       rmax = (a > rmax || a != a) ? a : rmax;
     }
-#pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) {
-      const float t2 = __shfl_xor(rmax, o, 64);
-      rmax = (t2 > rmax || t2 != t2) ? t2 : rmax;
-    }
+    rmax = lane_max<1, LPR>(rmax);
   }
   if (!live) return;
   if (QUANT) {
