@@ -4,7 +4,7 @@
 // and for what is to be refused: the caller then takes the wrapper's general path, which converts, pads, copies or raises.  Nothing is
 // kept from one call for the next.
 //
-// Host time of a call on one box, general path -> here (the C entry with its launches in brackets): Mamba-2 cell B1 T2048 H8 26.5 ->
+// Host time of a call on one machine, general path -> here (the C entry with its launches in brackets): Mamba-2 cell B1 T2048 H8 26.5 ->
 // 10.1 us (7.3 for two launches), KDA B1 T2048 H8 26.6 -> 10.3 (6.6), SSD layer B1 L512 H80, prologue and forward, 56 -> 25.3 (20.6 for
 // five).  That was longer than the kernels of the first and the last (17 and 30 us): a ctypes struct of 30 to 60 fields, their conversions
 // and attribute reads of tensors.  Whole calls 24.1 -> 16.7 and 52.3 -> 28.0.

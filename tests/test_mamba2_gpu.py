@@ -350,6 +350,13 @@ def test_state_passing_in_place(cuda, nc):
     assert_same_codes(fin, rfin, "final")
 
 
+@pytest.mark.parametrize("nc", [7, 8, 9, 15, 16, 17, 20])
+def test_state_passing_in_place_group_edges(cuda, nc):
+    """Chunk counts around multiples of the ring of eight requests: the last requests of a ragged count read the last
+    chunk's slot again."""
+    test_state_passing_in_place(cuda, nc)
+
+
 def test_state_passing_noncontiguous(cuda):
     from linquant_amd.kernels.mamba2.state_passing import _fixedpoint_state_passing_fwd
 
