@@ -29,8 +29,8 @@ INT8_PEAK_TOPS = 5000.0  # published dense INT8 MFMA rate of MI355X; the measure
 STAGE_SOURCES = {
     "c5": {"prologue": "prologue_rotate_quant.hip", "chunk_cumsum": "mamba2_cumsum.h", "chunk_state": "mamba2_chunk_state.hip",
            "state_passing": "mamba2_state_passing.hip", "bmm_chunk": "mamba2_bmm_chunk.h", "chunk_scan": "mamba2_chunk_scan.hip"},
-    "zoo": {"rotate": "zoo_rotate.hip", "cumsum": "zoo_cumsum.hip", "wy_ns": "zoo_wy_ns.hip", "diag_prep": "zoo_diag_prep.h",
-            "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
+    "zoo": {"rotate": "zoo_rotate.hip", "rot_operand": "zoo_rot_operand.hip", "cumsum": "zoo_cumsum.hip", "wy_ns": "zoo_wy_ns.hip",
+            "diag_prep": "zoo_diag_prep.h", "lin_prep": "zoo_lin_prep.hip", "scan": "zoo_scan.hip", "write_codes": "zoo_write_codes.hip",
             "state": "zoo_state.hip", "output": "zoo_output.hip", "rotate_quant": "zoo_rotate_quant.hip"},
 }
 COUNTER_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "hbm_traffic_and_mfma_counters.md")
@@ -145,10 +145,9 @@ def zoo_launch_bytes(workload):
     gam, pack = tok * K // 64, tok * (128 + K) // 64
     sc = tok if dec == "scalar" else 0
     out = {"rotate": 2 * qk * 2}
-    if dec == "scalar":
-        out["cumsum"] = 2 * tok
     if dec == "diagonal":
         g = tok * K
+        out["rot_operand"] = K * K * (4 + 2)
         out["diag_prep"] = 2 * qk + vv + g + A + 2 * kc + (tok + kc + vv + pack if fam == "delta" else 2 * vc + gam)
     out["wy_ns"] = 2 * qk + vv + tok + sc + 3 * kc + vv + A + pack + sc
     out["lin_prep"] = 2 * qk + vv + sc + 2 * kc + 2 * vc + A + gam + sc
@@ -173,9 +172,9 @@ def launch_times(fn, reps):
         torch.cuda.synchronize()
     out = {}
     for e in sorted((e for e in prof.events() if e.device_type == DeviceType.CUDA), key=lambda e: e.time_range.start):
-        m = re.search(r"(\w+)_kernel\b", e.name)
-        if m and (m.group(1).startswith("zoo_") or m.group(1).startswith("cumsum_")):
-            label = "cumsum" if m.group(1).startswith("cumsum_") else m.group(1)[4:]
+        m = re.search(r"(zoo_\w+?|cumsum_\w+?|rot_operand)_kernel", e.name)
+        if m:
+            label = "cumsum" if m.group(1).startswith("cumsum_") else m.group(1).removeprefix("zoo_")
             out.setdefault(label, []).append(e.time_range.elapsed_us() * 1e-3)
     return out
 
