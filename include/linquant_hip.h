@@ -40,7 +40,8 @@ typedef struct ihipStream_t* hipStream_t;
 #define LQ_DT_I8 2
 #define LQ_DT_BF16 3
 
-/* ABI version; bumped whenever a struct layout, or what a call asks of its caller, changes. */
+/* ABI version; bumped whenever a struct layout, or what a call asks of its caller, changes.  The function gives the library's. */
+#define LQ_ABI_VERSION 21
 int lq_abi_version(void);
 /* sizeof() of the named args struct as compiled into the library (negative if unknown); lets a binding
  * check its own struct layout before the first call. */

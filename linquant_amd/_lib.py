@@ -15,7 +15,7 @@ HEADER = ROOT.parent / "include" / "linquant_hip.h"
 LIB_PATH = ROOT / "csrc" / "liblinquant_hip.so"
 _NATIVE_ENTRIES = ("lq_zoo_simple_gla", "lq_zoo_simple_gla_workspace_bytes", "lq_zoo_chunk_forward",
                    "lq_zoo_chunk_forward_workspace_bytes", "lq_zoo_rotate_qkv", "lq_split_rotate_quant_xBC", "lq_ssd_combined",
-                   "lq_ssd_combined_workspace_bytes")
+                   "lq_ssd_combined_workspace_bytes", "lq_abi_version", "lq_args_size")
 ABI_VERSION = 21
 
 LQ_DT_F16, LQ_DT_F32, LQ_DT_I8, LQ_DT_BF16 = 0, 1, 2, 3
@@ -108,7 +108,10 @@ def native():
             from linquant_amd import _binding
         except ImportError as e:
             raise LinQuantHipError("linquant_amd/_binding.so is missing: build it with `python -m linquant_amd.build`") from e
-        _binding.init(raise_failed, {fn: ctypes.cast(getattr(lib, fn), ctypes.c_void_p).value for fn in _NATIVE_ENTRIES})
+        try:
+            _binding.init(raise_failed, {fn: ctypes.cast(getattr(lib, fn), ctypes.c_void_p).value for fn in _NATIVE_ENTRIES})
+        except RuntimeError as e:
+            raise LinQuantHipError(f"linquant_amd/_binding.so was built for another liblinquant_hip.so ({e}): rebuild") from e
         _native = _binding
     return _native
 

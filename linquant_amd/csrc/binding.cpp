@@ -430,6 +430,22 @@ PyObject* ssd(PyObject*, PyObject* const* arg, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// whether the library was built from the header that this file was: its ABI version and the structs that are filled here
+bool same_abi(decltype(&lq_abi_version) version, decltype(&lq_args_size) size) {
+  const int v = version();
+  if (v != LQ_ABI_VERSION) return PyErr_Format(PyExc_RuntimeError, "ABI version %d, the library has %d", LQ_ABI_VERSION, v), false;
+#define LQ_SAME_SIZE(T)                                                                                                          \
+  if (const int n = size(#T); n != (int)sizeof(T))                                                                               \
+    return PyErr_Format(PyExc_RuntimeError, #T ": sizeof %d, the library has %d", (int)sizeof(T), n), false
+  LQ_SAME_SIZE(lq_zoo_simple_gla_args);
+  LQ_SAME_SIZE(lq_zoo_chunk_forward_args);
+  LQ_SAME_SIZE(lq_zoo_rotate_qkv_args);
+  LQ_SAME_SIZE(lq_split_rotate_quant_xBC_args);
+  LQ_SAME_SIZE(lq_ssd_combined_args);
+#undef LQ_SAME_SIZE
+  return true;
+}
+
 // init(raise_failed, {entry point: address})
 PyObject* init(PyObject*, PyObject* const* arg, Py_ssize_t n) {
   if (n != 2 || !PyCallable_Check(arg[0]) || !PyDict_Check(arg[1])) {
@@ -437,6 +453,13 @@ PyObject* init(PyObject*, PyObject* const* arg, Py_ssize_t n) {
     return nullptr;
   }
   auto entry = [&](const char* name) { PyObject* o = PyDict_GetItemString(arg[1], name); return o ? PyLong_AsVoidPtr(o) : nullptr; };
+  const auto version = (decltype(&lq_abi_version))entry("lq_abi_version");
+  const auto size = (decltype(&lq_args_size))entry("lq_args_size");
+  if (!version || !size) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_KeyError, "lq_abi_version or lq_args_size is missing");
+    return nullptr;
+  }
+  if (!same_abi(version, size)) return nullptr;
   simple_gla_entry = (decltype(simple_gla_entry))entry("lq_zoo_simple_gla");
   simple_gla_bytes = (decltype(simple_gla_bytes))entry("lq_zoo_simple_gla_workspace_bytes");
   split_rotate_entry = (decltype(split_rotate_entry))entry("lq_split_rotate_quant_xBC");

@@ -294,3 +294,26 @@ def test_native_calls_leave_everything_but_gpu_tensors_to_the_general_path():
         assert n.rotate_qkv(first, t, None, None, None) is None
         assert n.split_rotate(first, None, 1, 1, 64, 64, t, t, False, False) is None
         assert n.ssd(first, *[None] * 24) is None
+
+
+@pytest.mark.parametrize("odd", ["lq_abi_version", "lq_zoo_simple_gla_args", "lq_zoo_chunk_forward_args", "lq_zoo_rotate_qkv_args",
+                                 "lq_split_rotate_quant_xBC_args", "lq_ssd_combined_args"])
+def test_native_calls_refuse_a_library_of_another_abi(monkeypatch, odd):
+    """csrc/binding.cpp fills its structs by the header it was compiled with; a library with another version, or another size of one of
+    them, would read its fields in the wrong places."""
+    lib = _lib.load()
+    version = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: lib.lq_abi_version() + (odd == "lq_abi_version"))
+    size = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p)(lambda name: lib.lq_args_size(name) + 8 * (name == odd.encode()))
+
+    class Library:
+        lq_abi_version, lq_args_size = version, size
+
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "_lib", Library())
+    with pytest.raises(_lib.LinQuantHipError, match=odd if odd.endswith("args") else "ABI version"):
+        _lib.native()
+    monkeypatch.setattr(_lib, "_lib", lib)
+    assert _lib.native() is not None
