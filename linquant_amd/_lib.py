@@ -108,6 +108,11 @@ def native():
             from linquant_amd import _binding
         except ImportError as e:
             raise LinQuantHipError("linquant_amd/_binding.so is missing: build it with `python -m linquant_amd.build`") from e
+        from linquant_amd.build import built_for
+
+        theirs = getattr(_binding, "built_for", "something unknown")
+        if theirs != built_for():
+            raise LinQuantHipError(f"linquant_amd/_binding.so was built for {theirs}, this is {built_for()}: rebuild")
         try:
             _binding.init(raise_failed, {fn: ctypes.cast(getattr(lib, fn), ctypes.c_void_p).value for fn in _NATIVE_ENTRIES})
         except RuntimeError as e:

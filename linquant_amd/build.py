@@ -42,6 +42,21 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{res.stderr}")
 
 
+def built_for() -> str:
+    """What binding.cpp is compiled against besides its own sources: torch's and Python's binary interfaces.  The compiled file holds
+    this text."""
+    import sysconfig
+
+    import torch
+
+    return f"torch {torch.__version__}, {sysconfig.get_config_var('SOABI')}"
+
+
+def _binding_stale(newest_src: float) -> bool:
+    return (not BINDING_PATH.exists() or BINDING_PATH.stat().st_mtime < newest_src
+            or built_for().encode() not in BINDING_PATH.read_bytes())
+
+
 def _compile_binding() -> None:
     """csrc/binding.cpp (host code only) against the installed torch."""
     import sysconfig
@@ -52,7 +67,7 @@ def _compile_binding() -> None:
     inc = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include", sysconfig.get_paths()["include"],
            Path(_hipcc()).resolve().parents[1] / "include"]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{i}" for i in inc), str(CSRC / "binding.cpp"),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DLQ_BUILT_FOR="{built_for()}"', *(f"-I{i}" for i in inc), str(CSRC / "binding.cpp"),
            "-o", str(BINDING_PATH), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -75,7 +90,7 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     if verbose:
         print(f"[linquant_amd.build] compiling {len(todo)}/{len(srcs)} sources with {jobs} jobs", flush=True)
     bind = CSRC / "binding.cpp"
-    stale = force or not BINDING_PATH.exists() or BINDING_PATH.stat().st_mtime < max(bind.stat().st_mtime, newest_hdr)
+    stale = force or _binding_stale(max(bind.stat().st_mtime, newest_hdr))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         binding = ex.submit(_compile_binding) if stale else None
         list(ex.map(lambda so: _compile(*so), todo))

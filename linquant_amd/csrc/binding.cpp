@@ -488,4 +488,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__binding() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", LQ_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
+}

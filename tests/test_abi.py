@@ -317,3 +317,18 @@ def test_native_calls_refuse_a_library_of_another_abi(monkeypatch, odd):
         _lib.native()
     monkeypatch.setattr(_lib, "_lib", lib)
     assert _lib.native() is not None
+
+
+def test_native_calls_refuse_another_torch(monkeypatch, tmp_path):
+    """The file unpacks torch's tensors by the headers that it was compiled with: it is not used with, and rebuilt for, another torch."""
+    from linquant_amd import build
+
+    here = tmp_path / "_binding.so"
+    here.write_bytes(build.BINDING_PATH.read_bytes())
+    monkeypatch.setattr(build, "BINDING_PATH", here)
+    assert not build._binding_stale(0.0)
+    monkeypatch.setattr(torch, "__version__", "1.0")
+    monkeypatch.setattr(_lib, "_native", None)
+    assert build._binding_stale(0.0)
+    with pytest.raises(_lib.LinQuantHipError, match="built for torch"):
+        _lib.native()
