@@ -13,6 +13,7 @@ from pathlib import Path
 ROOT = Path(__file__).resolve().parent
 HEADER = ROOT.parent / "include" / "linquant_hip.h"
 LIB_PATH = ROOT / "csrc" / "liblinquant_hip.so"
+BINDING_PATH = ROOT / "_binding.so"
 _NATIVE_ENTRIES = ("lq_zoo_simple_gla", "lq_zoo_simple_gla_workspace_bytes", "lq_zoo_chunk_forward",
                    "lq_zoo_chunk_forward_workspace_bytes", "lq_zoo_rotate_qkv", "lq_split_rotate_quant_xBC", "lq_ssd_combined",
                    "lq_ssd_combined_workspace_bytes", "lq_abi_version", "lq_args_size")
@@ -104,10 +105,14 @@ def native():
     global _native
     if _native is None:
         lib = load()
+        import torch  # noqa: F401  (loads the libraries that the binding needs)
+
+        if not BINDING_PATH.exists():
+            raise LinQuantHipError(f"{BINDING_PATH} is missing: build it with `python -m linquant_amd.build`")
         try:
             from linquant_amd import _binding
         except ImportError as e:
-            raise LinQuantHipError("linquant_amd/_binding.so is missing: build it with `python -m linquant_amd.build`") from e
+            raise LinQuantHipError(f"{BINDING_PATH} does not load: {e}") from e
         from linquant_amd.build import built_for
 
         theirs = getattr(_binding, "built_for", "something unknown")

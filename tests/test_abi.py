@@ -332,3 +332,26 @@ def test_native_calls_refuse_another_torch(monkeypatch, tmp_path):
     assert build._binding_stale(0.0)
     with pytest.raises(_lib.LinQuantHipError, match="built for torch"):
         _lib.native()
+
+
+def test_native_calls_load_without_torch_imported_first():
+    import subprocess
+    import sys
+
+    res = subprocess.run([sys.executable, "-c", "from linquant_amd import _lib; _lib.native()"], cwd=ROOT, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+
+
+def test_native_calls_report_why_they_do_not_load(monkeypatch, tmp_path):
+    import sys
+
+    import linquant_amd
+
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(linquant_amd, "_binding", raising=False)
+    monkeypatch.setitem(sys.modules, "linquant_amd._binding", None)  # (its import raises)
+    with pytest.raises(_lib.LinQuantHipError, match="does not load: .*_binding"):
+        _lib.native()
+    monkeypatch.setattr(_lib, "BINDING_PATH", tmp_path / "_binding.so")
+    with pytest.raises(_lib.LinQuantHipError, match="is missing"):
+        _lib.native()
