@@ -74,8 +74,14 @@ def _compile_binding() -> None:
         raise RuntimeError(f"g++ failed on binding.cpp:\n{res.stderr}")
 
 
+def _bind(force: bool, newest_src: float) -> None:
+    if force or _binding_stale(newest_src):
+        _compile_binding()
+
+
 def build(force: bool = True, jobs: int | None = None, verbose: bool = False) -> Path:
-    """Compile every .hip source and link the shared library. Returns the library path."""
+    """Compile every .hip source and link the shared library, then report the native host code if that failed: the C library needs
+    hipcc alone. Returns the library path."""
     srcs = sources()
     objdir = CSRC / "build"
     objdir.mkdir(exist_ok=True)
@@ -90,17 +96,17 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     if verbose:
         print(f"[linquant_amd.build] compiling {len(todo)}/{len(srcs)} sources with {jobs} jobs", flush=True)
     bind = CSRC / "binding.cpp"
-    stale = force or _binding_stale(max(bind.stat().st_mtime, newest_hdr))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        binding = ex.submit(_compile_binding) if stale else None
+        binding = ex.submit(_bind, force, max(bind.stat().st_mtime, newest_hdr))
         list(ex.map(lambda so: _compile(*so), todo))
-        if binding is not None:
-            binding.result()
     objs = [str(objdir / (s.stem + ".o")) for s in srcs]
     cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", str(LIB_PATH)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
+    failure = binding.exception()
+    if failure is not None:
+        raise RuntimeError(f"{LIB_PATH.name} is built, the Python wrappers' {BINDING_PATH.name} is not: {failure}") from failure
     return LIB_PATH
 
 

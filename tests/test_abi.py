@@ -355,3 +355,33 @@ def test_native_calls_report_why_they_do_not_load(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "BINDING_PATH", tmp_path / "_binding.so")
     with pytest.raises(_lib.LinQuantHipError, match="is missing"):
         _lib.native()
+
+
+@pytest.mark.parametrize("why", ["no g++", "no torch", "does not compile"])
+def test_the_c_library_builds_without_the_native_calls(monkeypatch, tmp_path, why):
+    """hipcc is all that liblinquant_hip.so needs: it is linked, and then the binding's failure raised."""
+    import subprocess
+    import types
+
+    from linquant_amd import build
+
+    def run(cmd, **_):
+        if cmd[0] == "g++":
+            if why == "no g++":
+                raise FileNotFoundError("g++")
+            return subprocess.CompletedProcess(cmd, 1, "", "error")
+        Path(cmd[cmd.index("-o") + 1]).write_bytes(b"linked")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(build, "subprocess", types.SimpleNamespace(run=run))
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build, "_compile", lambda src, obj: None)
+    monkeypatch.setattr(build, "LIB_PATH", tmp_path / "liblinquant_hip.so")
+    monkeypatch.setattr(build, "BINDING_PATH", tmp_path / "_binding.so")
+    if why == "no torch":
+        import sys
+
+        monkeypatch.setitem(sys.modules, "torch", None)
+    with pytest.raises(RuntimeError, match="_binding.so is not"):
+        build.build(force=why != "no torch")
+    assert build.LIB_PATH.read_bytes() == b"linked"
