@@ -341,7 +341,7 @@ _FORWARD_WS = {}
 def one_call_forward(family, decay, q, k, v, g, beta, sc, dims, span, *, sigma=1.0, tau=1.0, eta, scale, qmax, final_state,
                      out_dtype, rot=None, dqk=None):
     """lq_zoo_chunk_forward: every stage of a chunk forward (GLA, DeltaNet, Gated DeltaNet, KDA; rotated storage) from one
-    foreign call over one workspace.  ``rot`` (K,K) R_QK in any float type, ``dqk`` (H,K) D_QK (64-token chunks): fp32 tables go in as they
+    foreign call over one workspace.  ``rot`` (K,K) R_QK in any float type (its entries in that order, whatever the shape), ``dqk`` (H,K) D_QK (64-token chunks): fp32 tables go in as they
     are.  ``sc``: fp32 scales by role ('q','k','w','kw', value write 'vw' / 'ew', value local
     'vl' / 'el', 'state').  Returns (o, final fp32 state or None)."""
     import ctypes
@@ -353,7 +353,7 @@ def one_call_forward(family, decay, q, k, v, g, beta, sc, dims, span, *, sigma=1
     svl, ss, skw = _lib.aligned(svl), _lib.aligned(sc["state"]), _lib.aligned(sc["kw"])
     rot_f = None
     if rot is not None:
-        assert tuple(rot.shape) == (K, K), "rot: (K, K) R_QK"
+        assert rot.numel() == K * K, "rot: (K, K) R_QK"
         if span == CHUNK and rot.dtype == torch.float32 and rot.is_contiguous():
             rot, rot_f = None, _lib.aligned(rot)
         else:

@@ -385,3 +385,26 @@ def test_the_c_library_builds_without_the_native_calls(monkeypatch, tmp_path, wh
     with pytest.raises(RuntimeError, match="_binding.so is not"):
         build.build(force=why != "no torch")
     assert build.LIB_PATH.read_bytes() == b"linked"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64])
+@pytest.mark.parametrize("family", ["gla", "kda"])
+@pytest.mark.parametrize("span", [64, 128])
+def test_a_rotation_of_another_shape_is_taken_as_its_entries(dtype, family, span):
+    """K * K entries of R_QK in any shape reach the call (which refuses the CPU tensors of this test); another number does not."""
+    from linquant_amd.kernels import zoo
+
+    q, g, beta = torch.zeros(1, 128, 1, 64, dtype=torch.float16), torch.zeros(1, 128, 1, 64), torch.zeros(1, 128, 1)
+    sc = {n: torch.ones(1) if n in ("q", "k", "w") else torch.ones(1, 64) for n in ("q", "k", "w", "kw", "vw", "vl", "el", "ew", "state")}
+
+    def call(rot):
+        if family == "gla":
+            return zoo.chunk_gla_int8(q, q, q, g, sc, rot=rot, chunk_size=span)
+        return zoo.chunk_kda_int8(q, q, q, g, beta, sc, rot=rot, chunk_size=span)
+
+    eye = torch.eye(64, dtype=dtype)
+    for rot in (eye, eye[None], eye.flatten()):
+        with pytest.raises(ValueError, match="expected tensors on a GPU"):
+            call(rot)
+    with pytest.raises(AssertionError, match="R_QK"):
+        call(eye[:32])
