@@ -95,3 +95,48 @@ def test_every_form_of_the_local_rotation_equals_the_stages(cuda, cell, NT, H, K
     (o1, h1), (o0, h0) = call(), call(_staged=True)
     assert float(o1.float().abs().max()) > 0
     assert torch.equal(o0, o1) and torch.equal(h0, h1)
+
+
+# what only callers of the C entry choose, below and from the line of R_QK's operand launch (1024 chunks and heads) on: fp16 or fp32 R_QK,
+# without room for its operands too, and KDA's D_QK with reciprocals of the caller's or without
+@pytest.mark.parametrize("cell,tables", [("gla", None), ("kda", "dqk"), ("kda", "dq")])
+@pytest.mark.parametrize("NT,H,K", [(31, 33, 64), (32, 32, 128)])
+@pytest.mark.parametrize("rot", ["rot", "rot_f32"])
+@pytest.mark.parametrize("room", [False, True])
+def test_tables_of_the_c_entry_equal_the_wrapper(cuda, cell, tables, NT, H, K, rot, room):
+    import ctypes
+
+    from linquant_amd import _lib
+    from linquant_amd.kernels import zoo
+
+    T, V = 64 * NT, 64
+    q, k, v, g, beta = [t if t is None else t.to(cuda) for t in zc.inputs(cell, B=1, T=T, H=H, K=K, V=V, seed=NT, dtype=torch.float16)]
+    gen = torch.Generator().manual_seed(K)
+    r = lambda *shape, lo, hi: (torch.rand(*shape, generator=gen) * (hi - lo) + lo).to(cuda)  # noqa: E731
+    R = torch.linalg.qr(torch.randn(K, K, generator=gen))[0].contiguous().to(cuda)
+    D = r(H, K, lo=0.25, hi=1.75)
+    sc = {"q": r(H, lo=0.001, hi=0.003), "k": r(H, lo=0.005, hi=0.01), "w": r(H, lo=0.02, hi=0.04), "kw": r(H, K, lo=0.005, hi=0.015)}
+    sc.update({n: r(H, V, lo=0.02, hi=0.05) for n in ("vw", "vl", "el", "ew", "state")})
+    kda = cell == "kda"
+    fn = (lambda **x: zoo.chunk_kda_int8(q, k, v, g, beta, sc, dqk=D, **x)) if kda else (lambda **x: zoo.chunk_gla_int8(q, k, v, g, sc, **x))
+    o1, h1 = fn(eta=0.25, output_final_state=True, rot=R)
+
+    dims = dict(family=int(kda), decay=2, batch=1, seqlen=T, nheads=H, kdim=K, vdim=V, chunk_size=64)
+    n = ctypes.c_int64(0)
+    st = _lib.fill("lq_zoo_chunk_forward_args", **dims)
+    assert _lib.load().lq_zoo_chunk_forward_workspace_bytes(ctypes.byref(st), ctypes.byref(n)) == 0
+    ws, ops = torch.empty(n.value, dtype=torch.uint8, device=cuda), torch.empty(2 * K * K, dtype=torch.uint8, device=cuda)
+    o0, h0 = torch.zeros_like(v), torch.zeros(1, H, K, V, device=cuda)
+    Rt, rcp = R if rot == "rot_f32" else R.half(), 1.0 / D
+    extra = {rot: Rt.data_ptr()}
+    if room:
+        extra["rot_ws"] = ops.data_ptr()
+    if kda:
+        extra.update(beta=beta.data_ptr(), sw=sc["w"].data_ptr())
+        extra.update({"dqk": D.data_ptr()} if tables == "dqk" else {"dq": D.data_ptr(), "dq_rcp": rcp.data_ptr()})
+    p = lambda name: sc[name].data_ptr()  # noqa: E731
+    _lib.call("lq_zoo_chunk_forward", q.device, q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), g=g.data_ptr(), o=o0.data_ptr(), ht=h0.data_ptr(),
+              sq=p("q"), sk=p("k"), skw=p("kw"), svw=p("ew" if kda else "vw"), svl=p("el" if kda else "vl"), ss=p("state"), sigma=1.0, tau=1.0,
+              eta=0.25, scale=K ** -0.5, qmax=127, act_dtype=_lib.LQ_DT_F16, workspace=ws.data_ptr(), workspace_bytes=n.value, **dims, **extra)
+    assert float(o1.float().abs().max()) > 0
+    assert torch.equal(o0, o1) and torch.equal(h0, h1)
