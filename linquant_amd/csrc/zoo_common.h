@@ -196,29 +196,6 @@ LQ_DEV float zoo_cumsum64(float g) {
   x = zoo_dpp_add<0x143, 0xc>(x);  // row_bcast:31: the last lane of row 1 into rows 2 and 3
   return (float)x;
 }
-// the same sums of one thread that holds all 64 tokens
-LQ_DEV void zoo_cumsum64(const float (&g)[64], float (&o)[64]) {
-  double last[2] = {0.0, 0.0};  // the sum that rows 0, 1 end with, and the total of row 2
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    double x[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) x[t] = (double)g[16 * r + t];
-#pragma unroll
-    for (int s = 1; s < 16; s <<= 1)
-#pragma unroll
-      for (int t = 15; t >= s; --t) x[t] += x[t - s];
-    const double total = x[15];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      if (r == 3) x[t] += last[1];
-      if (r > 0) x[t] += last[0];
-      o[16 * r + t] = (float)x[t];
-    }
-    if (r < 2) last[0] = x[15]; else last[1] = total;
-  }
-}
-
 // One term of the substitution below: t_i -= G_ij t_j, with G_ij broadcast from lane j of every 16
 #define LQ_SUBST(OP, JJ) "v_fmac_f32_dpp %0, -%1, %" #OP " row_newbcast:" #JJ " row_mask:0xf bank_mask:0xf\n"
 #define LQ_SUBST4 LQ_SUBST(2, 0) LQ_SUBST(3, 1) LQ_SUBST(4, 2) LQ_SUBST(5, 3)

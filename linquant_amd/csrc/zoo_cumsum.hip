@@ -24,9 +24,8 @@ __global__ __launch_bounds__(256) void cumsum_scalar_kernel(const float* __restr
   }
 }
 
-// The same scan for the chunk sizes the callers use (C = 64, 128, 192 or 256): 64 values of a thread are requested before the first
-// is added (the loop above waits for each load in turn: C round trips), summed in the same order; 64 tokens as the kernels that make
-// the sum themselves do it (zoo_cumsum64).
+// The same scan for the longer chunks the callers use (C = 128, 192 or 256): 64 values of a thread are requested before the first
+// is added (the loop above waits for each load in turn: C round trips), summed in the same order.
 template <int C>
 __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* __restrict__ g, float* __restrict__ gc, int H,
                                                                   int64_t total) {
@@ -39,18 +38,41 @@ __global__ __launch_bounds__(256) void cumsum_scalar_fixed_kernel(const float* _
     float v[64];
 #pragma unroll
     for (int t = 0; t < 64; ++t) v[t] = g[base + (int64_t)(t0 + t) * H];
-    if constexpr (C == 64) {
-      float o[64];
-      zoo_cumsum64(v, o);
-#pragma unroll
-      for (int t = 0; t < 64; ++t) gc[base + (int64_t)t * H] = o[t];
-      return;
-    }
 #pragma unroll
     for (int t = 0; t < 64; ++t) {
       run += (double)v[t];
       gc[base + (int64_t)(t0 + t) * H] = (float)run;
     }
+  }
+}
+
+// Chunks of 64 tokens, by the sums of the kernels that cumulate a chunk themselves (zoo_cumsum64): a wave to 16 tokens of 64 columns,
+// the totals of the 16s through LDS.  Bound by latency.  (A thread to a column, with these sums and their 250 additions, took 3.4 us where
+// 64 additions one after the other take 3.1; this one 2.7: T4096 B4 H16.  With heads that do not fill a line, T1088 B3 H5, 9.4 -> 4.1.)
+__global__ __launch_bounds__(256) void cumsum_scalar64_kernel(const float* g, float* gc, int H, int64_t total) {
+  __shared__ double total_s[3][64];
+  const int lane = threadIdx.x & 63, row = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t idx = (int64_t)blockIdx.x * 64 + lane, col = min(idx, total - 1);  // (b, chunk, h)
+  const int64_t base = (col / H * 64 + 16 * row) * H + col % H;
+  float v[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) v[t] = g[base + (int64_t)t * H];
+  double x[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) x[t] = (double)v[t];
+#pragma unroll
+  for (int s = 1; s < 16; s <<= 1)
+#pragma unroll
+    for (int t = 15; t >= s; --t) x[t] += x[t - s];
+  if (row < 3) total_s[row][lane] = x[15];
+  __syncthreads();
+  if (idx >= total) return;
+  const double t0 = total_s[0][lane], t1 = total_s[1][lane], t2 = total_s[2][lane];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    if (row == 3) x[t] += t2;
+    if (row > 0) x[t] += row == 1 ? t0 : t1 + t0;
+    gc[base + (int64_t)t * H] = (float)x[t];
   }
 }
 
@@ -229,8 +251,8 @@ extern "C" int lq_zoo_cumsum(const lq_zoo_cumsum_args* a, hipStream_t stream) {
   if (a->kdim == 0) {
     const int64_t total = (int64_t)a->batch * NT * a->nheads;
     if (a->chunk_size == 64)
-      hipLaunchKernelGGL(cumsum_scalar_fixed_kernel<64>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, a->g,
-                         a->gc, a->nheads, total);
+      hipLaunchKernelGGL(cumsum_scalar64_kernel, dim3((unsigned)((total + 63) / 64)), dim3(256), 0, stream, a->g, a->gc, a->nheads,
+                         total);
     else if (a->chunk_size == 128)
       hipLaunchKernelGGL(cumsum_scalar_fixed_kernel<128>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, a->g,
                          a->gc, a->nheads, total);

@@ -5,6 +5,7 @@ in the same order, so outputs and final states are equal bit for bit."""
 import pytest
 import torch
 
+from linquant_amd import _lib
 from tests import zoo_cases as zc
 
 pytestmark = pytest.mark.gpu
@@ -118,6 +119,25 @@ def test_cumulative_scalar_decay_of_64_tokens(cuda, at):
     assert torch.equal(torch.isinf(out), torch.isinf(ref))
     fin = torch.isfinite(ref)
     assert ((out[fin].double() - ref[fin]).abs() <= ref[fin].abs() * 2.0 ** -23).all()
+
+
+# its order, to the bit: inside each 16 tokens by sums over the last 1, 2, 4, 8 values, then the totals of the 16s before; columns that fill
+# a workgroup's 64 and that do not, also where the result takes the place of the input
+@pytest.mark.parametrize("B,NT,H", [(1, 1, 1), (1, 3, 21), (2, 2, 16), (5, 13, 1), (3, 17, 5), (1, 5, 130)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_cumulative_scalar_decay_takes_the_order_of_the_waves(cuda, B, NT, H, in_place):
+    g = -torch.rand(B, 64 * NT, H, generator=torch.Generator().manual_seed(H)) ** 4 * 8
+    x = g.double().view(B, NT, 4, 16, H)
+    for s in (1, 2, 4, 8):
+        x = torch.cat([x[..., :s, :], x[..., s:, :] + x[..., :-s, :]], 3)
+    t0, t1, t2 = x[:, :, :3, -1:].clone().unbind(2)
+    x[:, :, 1] += t0
+    x[:, :, 3] += t2
+    x[:, :, 2:] += (t1 + t0)[:, :, None]
+    gin = g.to(cuda)
+    out = gin if in_place else torch.empty_like(gin)
+    _lib.call("lq_zoo_cumsum", gin.device, g=gin.data_ptr(), gc=out.data_ptr(), batch=B, seqlen=64 * NT, nheads=H, kdim=0, chunk_size=64)
+    assert torch.equal(out.cpu(), x.float().view(g.shape))
 
 
 # the same sum across the lanes of a wave, in the launches that make it themselves: what a decay of minus infinity cuts off is cut off
