@@ -30,6 +30,13 @@ LQ_DEV float load_sign(const void* s, int64_t i, int dtype) {
   return (float)((const int8_t*)s)[i];
 }
 
+// x * d rounded once to fp16 (left to the compiler it is that or fp32 in between, from one instantiation and element to the next)
+LQ_DEV float mul_f16(float x, float d) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(x), "v"(d));
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)r);
+}
+
 // value of lane ^ M: up to 8 by lane permutations of the vector unit, further through the LDS crossbar.  (All of them through the crossbar,
 // 40 a lane, SSD calls of N = 128 took 1 to 2 us longer: B4 L8192 259.3 -> 257.5, B8 L2048 139.3 -> 138.0.)
 template <int M>
@@ -76,12 +83,18 @@ LQ_DEV void fwht_row(float* v, int sub, float hb, float kron) {
   for (int i = 0; i < 8; ++i) v[i] = v[i] * hb;
   lane_stages<LPH, 2 * LPH>(v, sub);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = v[i] * kron;
+  for (int i = 0; i < 8; ++i) {
+    v[i] = v[i] * kron;
+    asm("" : "+v"(v[i]));  // keeps the fp32 rounding of the product: no multiply fused into the fp16 conversion
+  }
 }
 
 // VEC: signs and dqk are 16-byte aligned, so a lane's eight entries are fetched as whole pieces, requested together with
 // its row piece before anything is used (element by element, behind a run-time dtype switch, they formed a chain of
-// memory round trips several times longer than the transform itself).
+// memory round trips several times longer than the transform itself).  An empty statement that takes all of them holds the
+// order: without it the row was waited for and converted in front of the other requests.  Operands that are not there are
+// not requested (uniform branches; from a dummy address they cost rows without signs 2 to 8 %: B4 L4096 N128 G8
+// 21.2 -> 19.1 us without b_fp, 24.3 -> 22.9 with the row maxima; with signs and D_QK 38.9 -> 34.9).
 // BF: the rows are bf16 in and out (stand-alone rotation only; the fused prologue rounds through fp16 by definition).
 template <int N, bool QUANT, bool VEC, bool BF = false>
 __global__ __launch_bounds__(256) void rotate_kernel(const _Float16* __restrict__ src, int64_t s_b, int64_t s_t,
@@ -104,28 +117,30 @@ __global__ __launch_bounds__(256) void rotate_kernel(const _Float16* __restrict_
   const int tt = live ? t : T - 1;  // inactive rows still take part in the shuffles
 
   const _Float16* sp = src + (int64_t)b * s_b + (int64_t)tt * s_t + side * side_off + (int64_t)seg * s_seg + sub * 8;
-  const lq_v4i hraw = *(const lq_v4i*)sp;
-  const lq_v8h hv = __builtin_bit_cast(lq_v8h, hraw);
-  float xin[8];  // the row piece as fp32
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    xin[i] = BF ? __uint_as_float(((uint32_t)hraw[i >> 1] >> (16 * (i & 1))) << 16) : (float)hv[i];
+  lq_v4i hraw = *(const lq_v4i*)sp;
   float v[8];
+  auto convert = [&]() __attribute__((always_inline)) {  // the row piece as fp32
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[i] = BF ? __uint_as_float(((uint32_t)hraw[i >> 1] >> (16 * (i & 1))) << 16) : (float)__builtin_bit_cast(lq_v8h, hraw)[i];
+  };
   const float* dqk = side ? dqk1 : dqk0;
   if constexpr (VEC) {
-    // absent operands are read from a valid dummy address (the start of the row) and ignored
     const int64_t e0 = (int64_t)seg * N + sub * 8;
-    const float* dq = (QUANT && dqk) ? dqk + e0 : (const float*)(sp - sub * 8);
-    const lq_v4f d0 = *(const lq_v4f*)dq, d1 = *(const lq_v4f*)(dq + 4);
     const int es = signs_dtype == LQ_DT_F16 ? 2 : (signs_dtype == LQ_DT_F32 ? 4 : 1);
-    const char* sgp = signs ? (const char*)signs + e0 * es : (const char*)(sp - sub * 8);
-    const lq_v4i s0 = *(const lq_v4i*)(es == 1 ? sgp - ((uintptr_t)sgp & 8) : sgp);          // int8: the aligned 16 bytes around the 8
-    const lq_v4i s1 = *(const lq_v4i*)(es == 4 ? sgp + 16 : sgp - ((uintptr_t)sgp & 15));    // fp32: second half
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = xin[i];
+    const char* sgp = (const char*)signs + e0 * es;
+    lq_v4f d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0;
+    lq_v4i s0 = {0, 0, 0, 0}, s1 = s0;
+    if (QUANT && dqk) d0 = *(const lq_v4f*)(dqk + e0), d1 = *(const lq_v4f*)(dqk + e0 + 4);
+    if (signs) {
+      s0 = *(const lq_v4i*)(es == 1 ? sgp - ((uintptr_t)sgp & 8) : sgp);        // int8: the aligned 16 bytes around the 8
+      s1 = *(const lq_v4i*)(es == 4 ? sgp + 16 : sgp - ((uintptr_t)sgp & 15));  // fp32: second half
+    }
+    asm volatile("" : "+v"(hraw), "+v"(d0), "+v"(d1), "+v"(s0), "+v"(s1));  // one wait for all of them
+    convert();
     if (QUANT && dqk) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (float)(_Float16)(v[i] * (i < 4 ? d0[i & 3] : d1[i & 3]));
+      for (int i = 0; i < 8; ++i) v[i] = mul_f16(v[i], i < 4 ? d0[i & 3] : d1[i & 3]);
     }
     if (signs) {
       const lq_v8h sh = __builtin_bit_cast(lq_v8h, s0);
@@ -141,11 +156,10 @@ __global__ __launch_bounds__(256) void rotate_kernel(const _Float16* __restrict_
       fwht_row<LPH>(v, sub, hb, kron);
     }
   } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = xin[i];
+    convert();
     if (QUANT && dqk) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (float)(_Float16)(v[i] * dqk[seg * N + sub * 8 + i]);
+      for (int i = 0; i < 8; ++i) v[i] = mul_f16(v[i], dqk[seg * N + sub * 8 + i]);
     }
     if (signs) {
 #pragma unroll
