@@ -259,11 +259,21 @@ int fplan(const lq_zoo_chunk_forward_args* a, FLayout* l) {
   return LQ_OK;
 }
 
-// R_QK laid out as operands by a launch of its own (4.5 us), or read by every chunk and head as the caller holds it (32 requests of 4 or,
-// fp32, 8 bytes a lane, rows apart, in the place of eight of 16)?  Whole calls: GLA B4 T4096 H16 (4096 of them) 196.8 us laid out, 217.6
-// as fp32, 199.6 as fp16 behind a conversion launch; KDA B1 T2048 H8 (256) 45.6 as fp32, 47.2 behind a launch.  Reading fp32 costs 5 ns for
-// each of them, so the line is at the launch's 4.5 us.
-bool rot_operand(const lq_zoo_chunk_forward_args* a) { return (int64_t)a->batch * a->nheads * (a->seqlen / 64) >= 1024; }
+// R_QK laid out as operands by a launch of its own (2 us in a stream of launches), or read by every chunk and head as the caller holds it (32
+// requests of 4 or, fp32, 8 bytes a lane at K = 128, rows apart, in the place of eight of 16)?  GPU us of the whole call, as it is / laid out
+// (H 16 or 32, 64 value columns):
+//   chunks and heads     1024            2048            4096            8192
+//   GLA fp32, K = 64     41.0 / 41.8     64.7 / 62.5     118 / 111       233 / 216
+//             K = 128    58.4 / 57.1     98.3 / 91.7     185 / 169       349 / 312
+//   KDA fp32, K = 64     75.2 / 76.3     104.6 / 103.9   179 / 172       342 / 323
+//             K = 128    100.9 / 100.1   146.1 / 143.0   269 / 253       489 / 455
+//   GLA fp16, K = 64     40.0 / 41.7     61.0 / 62.5     110.2 / 111.3   218.0 / 215.6
+//             K = 128    55.1 / 57.1     90.6 / 92.1     169.5 / 168.5   315.2 / 311.9
+//   KDA fp16, K = 64     74.5 / 76.3     103.0 / 104.0   172.0 / 171.6   326.2 / 322.2
+//             K = 128    99.2 / 100.4    142.8 / 143.0   254.9 / 252.2   460.5 / 455.2
+bool rot_operand(const lq_zoo_chunk_forward_args* a) {
+  return (int64_t)a->batch * a->nheads * (a->seqlen / 64) >= (a->rot_f32 ? 1024 : 4096);
+}
 
 }  // namespace
 

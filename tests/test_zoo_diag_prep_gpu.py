@@ -97,10 +97,10 @@ def test_every_form_of_the_local_rotation_equals_the_stages(cuda, cell, NT, H, K
     assert torch.equal(o0, o1) and torch.equal(h0, h1)
 
 
-# what only callers of the C entry choose, below and from the line of R_QK's operand launch (1024 chunks and heads) on: fp16 or fp32 R_QK,
-# without room for its operands too, and KDA's D_QK with reciprocals of the caller's or without
+# what only callers of the C entry choose, below and from the lines of R_QK's operand launch (1024 chunks and heads fp32, 4096 fp16) on: fp16
+# or fp32 R_QK, without room for its operands too, and KDA's D_QK with reciprocals of the caller's or without
 @pytest.mark.parametrize("cell,tables", [("gla", None), ("kda", "dqk"), ("kda", "dq")])
-@pytest.mark.parametrize("NT,H,K", [(31, 33, 64), (32, 32, 128)])
+@pytest.mark.parametrize("NT,H,K", [(31, 33, 64), (32, 32, 128), (63, 65, 64), (64, 64, 64)])
 @pytest.mark.parametrize("rot", ["rot", "rot_f32"])
 @pytest.mark.parametrize("room", [False, True])
 def test_tables_of_the_c_entry_equal_the_wrapper(cuda, cell, tables, NT, H, K, rot, room):
