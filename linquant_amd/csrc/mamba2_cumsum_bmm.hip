@@ -2,8 +2,8 @@
 // work behind a launch and a memory round trip.  The first workgroups take the dt tiles (mamba2_cumsum.h, the longer chain), the others
 // one to eight C.B^T tiles each (mamba2_bmm_chunk.h), the bits of the two stand-alone launches.
 // The scan reads nothing above the diagonal 64 x 64 tiles of C.B^T: those (6 of 16 at 256-token chunks) are not formed here.  With them, and
-// with 64-bit lane offsets for dt (mamba2_cumsum.h): B4 L8192 H80 whole call 253.2 -> 252 us, B3 L5000 H80 193.6 -> 192.2, B8 L2048 H64
-// value side 138.8 -> 137.7.
+// with 64-bit lane offsets for dt (mamba2_cumsum.h), kernel us on one card in turn: B4 L8192 H80 20.5 -> 19.6, B3 L5000 H80 13.3 -> 11.9, B8
+// L2048 H64 value side 9.7 -> 9.3, B4 L2048 H80 8.7 -> 8.5, B1 L512 H80 even (6.4).
 // Bound by latency.  Kernel us before that, two launches -> one: B1 L512 H80 6.4 + 5.9 -> 6.4, B3 L5000 H80 11.0 + 7.5 -> 13.2, B4 L2048 H80
 // 7.0 + 6.0 -> 8.3, B8 L2048 H64 value side 7.1 + 6.0 -> 9.8, B4 L8192 H80 12.6 + 10.2 -> 19.6 .. 22.7.
 #include "mamba2_bmm_chunk.h"

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void state_passing_kernel(
 
   // whole groups with chunks behind them: every request and every store of the steady state is unconditional, which keeps the
   // compiler's count of outstanding operations exact (with guards around them, as counts that DEPTH does not divide once had
-  // them, it drained the whole ring once per group: B3 H80 dim 8192, 20 chunks, 24 us, now 18).  The last of them, where less
+  // them, it drained the whole ring once per group: B3 H80 dim 8192, 20 chunks, 24 us, now 19).  The last of them, where less
   // than a group is left to request, asks for the last chunk once more instead (in place that slot is never stored to); with
   // that minimum in every group 112 chunks of H24 took 29 us, without 27.
   int c0 = 0;

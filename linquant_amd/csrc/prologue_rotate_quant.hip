@@ -38,7 +38,7 @@ LQ_DEV float mul_f16(float x, float d) {
 }
 
 // value of lane ^ M: up to 8 by lane permutations of the vector unit, further through the LDS crossbar.  (All of them through the crossbar,
-// 40 a lane, SSD calls of N = 128 took 1 to 2 us longer: B4 L8192 259.3 -> 257.5, B8 L2048 139.3 -> 138.0.)
+// 40 a lane: N = 128, kernel us on one card in turn, B4 L8192 13.7 -> 13.1, B1 L512 4.0 -> 3.5, B4 L2048 5.8 -> 5.4.)
 template <int M>
 LQ_DEV float lane_xor(float v) {
   if constexpr (M <= 8) return zoo_lane_xor<M>(v);

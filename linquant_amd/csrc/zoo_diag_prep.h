@@ -42,8 +42,9 @@
 // three would cost more.  Persistent workgroups with the next chunk's requests ahead spilled (KDA 714), three workgroups a compute unit for
 // GLA too (194).
 // R_QK comes in fp16, in fp32 or (larger calls) laid out as operands; D_QK's reciprocals are formed here.  As launches in front these were
-// 4.5 us for R_QK and 9.5 for the reciprocals: whole calls KDA B1 T2048 H8 47.2 -> 45.6, KDA B2 T8192 H32 with D_QK 532.8 -> 524.7, GLA B4
-// T4096 H16 199.6 -> 196.8 (there laid out as operands in the place of converted: kernel 144.6 -> 140.3).
+// 4.6 us for R_QK and 9.3 for the reciprocals.  On one card in turn, with the steps of zoo_scan.hip since: whole calls KDA B1 T2048 H8 47.3
+// -> 45.1 (this kernel 23.0 -> 23.6, R_QK read as fp32), KDA B2 T8192 H32 with D_QK 566 -> 558, GLA B4 T4096 H16 207 -> 204 (there R_QK is
+// laid out as operands in the place of converted, a launch of 4.6 as before).
 // Spilled registers: DIAG_KDA at K = 128 with the gate (sigma < 1, tau > 0) keeps Hw beside k over the key operands and spills 13 to 19
 // of its 128 in fp16 and up to 15 in bf16 (56 to 80 and up to 64 bytes a lane; about 300 of the 972 MB read and of the 730 MB written at
 // sigma = 0.5 above); without the gate at most one (bf16 with D_QK); the other forms and K = 64 none.

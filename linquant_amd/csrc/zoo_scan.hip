@@ -60,6 +60,11 @@ using ScanParams = ZooScanParams;
 // with R_QK, K = V = 128, H4 T4096 / T16384 49.3 -> 30.3 / 132 -> 75.5 us, H16 60.3 -> 49.9 / 231 -> 187; K = V = 64 H8 T2048 / T16384
 // 24.2 -> 16.6 / 110 -> 67.4; GLA K = V = 128 H4 T16384 162 -> 90, H5 T8192 96.3 -> 59.4.  Decay of the segments' lengths by 0.2 or 0.4
 // in the place of 0.3: at most 4 % slower.
+// All of this takes the compute units that one call leaves idle for free.  Where other work fills them, the repeated updates cost it: GPU us
+// a call, one segment or two launches -> segments, with 1 / 2 / 4 / 8 streams of the same call: Mamba-2 cell H8 T16384 116 -> 65 / 63 -> 63 /
+// 45 -> 60 / 45 -> 60, H8 T2048 24 -> 18 / 17 -> 12 / 9.5 -> 7.6 / 9.3 -> 7.4; linear attention H4 T16384 132 -> 71 / 76 -> 66 / 55 -> 63 /
+// 67 -> 64, H4 T4096 46 -> 29 / 30 -> 19 / 18 -> 15 / 17 -> 15; GLA H4 T16384 155 -> 91 / 107 -> 79 / 84 -> 76 / 95 -> 80, H8 T4096 56 -> 41 /
+// 55 -> 40 / 24 -> 29.  A call cannot see what else runs; the lines are those of one call at a time.
 constexpr int scan_update_sets(int K, int BV) { return K == 128 && BV == 32 ? 3 : 4; }  // (four spill there)
 constexpr int kMaxCuts = 16;
 struct ScanCuts {

@@ -26,9 +26,9 @@
 // blocks by forward substitution | block columns of T, one wave each, in registers | W | values transposed | U.  Keys and then values
 // pass through one transposed tile, the rows waiting in registers (every row is read once), and G and T lie in 16 blocks in the place of
 // the raw keys and codes.  With a tile each for keys and values and square G and T (77 KB) two workgroups fitted, which did not cover each
-// other's waits between eight barriers: 128.8 -> 117.4 us at B4 T4096 H16 with scalar decay (fp16), 59.3 -> 57.7 at B8 T2048 H8 without
-// (bf16; 2.7 rounds of the chip for four), whole calls 260.9 -> 248.7 and 94.7 -> 89.8, although there are two barriers more.  Bound by no
-// unit alone: 410 MB are 81 us at the rate of a large copy and the vector instructions 82 us.
+// other's waits between eight barriers: on one card in turn 130.4 -> 116 to 120 us at B4 T4096 H16 with scalar decay (fp16), 61.3 -> 56.5 at B8
+// T2048 H8 without (bf16; 2.7 rounds of the chip for four), although there are two barriers more.  Bound by no unit alone: 410 MB are 81 us
+// at the rate of a large copy and the vector instructions 82 us.
 #include "zoo_params.h"
 
 namespace {

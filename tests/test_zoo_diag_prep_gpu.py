@@ -74,7 +74,7 @@ def test_halves_of_a_sub_block_that_decide_apart_match_the_oracle(cuda, cell, K,
     zc.check(out, run, qz, f"{cell} K={K} rot={rot} staged={staged}")
 
 
-# every way in which R_QK comes to the launch, below and from its line (1024 chunks and heads) on: fp32 as it is, fp32 that is not on a
+# every way in which R_QK comes to the launch, below and from fp32's line (1024 chunks and heads) on: fp32 as it is, fp32 that is not on a
 # 16-byte boundary, fp32 whose rows are not contiguous, fp16, fp64; a matrix without symmetry, so that a transposed operand shows
 @pytest.mark.parametrize("cell", ["gla", "kda"])
 @pytest.mark.parametrize("NT,H,K", [(31, 33, 64), (32, 32, 64), (33, 31, 128), (16, 64, 128)])
